@@ -18,91 +18,215 @@
 
 namespace fo {
 
-constexpr int kSFChunk = 4;   // (b,c) entries per thread per chunk
-constexpr int kSFTile = 32;   // atoms per LDS tile
-
-FO_DEV double2 phase64(double kfrac_times2) {
-  // e^{-i pi * kfrac_times2}
-  double s, c;
-  sincospi(kfrac_times2, &s, &c);
-  return make_double2(c, -s);
+typedef double v4d __attribute__((ext_vector_type(4)));
+FO_DEV v4d mfma64(double a, double b, v4d c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// One workgroup per (x-index a of the k-cube, pair).
-__global__ void __launch_bounds__(256) k_per_sf(
+// One k-vector's weighted overlap product: sum over the groups of C1 conj(C2)
+// in this fused order, then the weight.  Every path to Cprod uses these two
+// (the same coefficients give the same product to the last bit).
+FO_DEV void overlap_add(double2& s, double2 c1, double2 c2) {
+  s.x = __builtin_fma(c1.x, c2.x, __builtin_fma(c1.y, c2.y, s.x));
+  s.y = __builtin_fma(c1.y, c2.x, __builtin_fma(-c1.x, c2.y, s.y));
+}
+FO_DEV double overlap_weight(const PerPair& d, int a, int b, int c) {
+  const double kx = 2.0 * kPi * a / d.box[0];
+  const double ky = 2.0 * kPi * b / d.box[1];
+  const double kz = 2.0 * kPi * c / d.box[2];
+  return exp(-(__builtin_fma(kx, kx, __builtin_fma(ky, ky, kz * kz))) * d.scale * d.scale);
+}
+
+// ---------------------------------------------------------------------------
+// Structure factors on the matrix cores.  With cos / sin of a x, b y, c z
+// (a, b, c >= 0, angles in units of the box) the sums over a group's atoms
+//   S[X][Y][Z](a, b, c) = sum_j X_j(a) Y_j(b) Z_j(c),   X, Y, Z in {cos, sin},
+// are NB^3 real numbers (NB = 2 nk + 1; sin(0) drops out) that give C(k) for
+// every sign of a, b, c, and C(-k) = conj C(k) exactly: an eighth of the
+// multiply-adds of the complex sum over the full cube.  Per a they are a
+// real product over the atoms, rows (X, Y(b)) by columns Z(c).
+//
+// One workgroup per (a >= 0, pair), waves 0-3 on the first and 4-7 on the
+// second structure.  Per tile of kSFTile atoms the phases of both structures
+// go to LDS ([atom]: cos/sin a x, the NB values of y, the NB values of z),
+// then v_mfma_f64_16x16x4f64 over four atoms a step: wave w owns row tile(s)
+// w & 3 (+ 4) and all CT column tiles, the A operand X_j Y_j(b) is formed
+// from two LDS reads.  The group's S of both structures then meet in LDS,
+// where one thread forms C1, C2 of each (b, c) and adds their product.
+//
+// CT = ceil(NB / 16) column tiles; 2 NB rows are at most 4 tiles for CT <= 2
+// and 8 above (two per wave).  Bound: the latency of the phase stage, which
+// every a repeats (one sincospi per atom and axis, multiples by products) and
+// its barriers; the products take 23 us of the 114 below at the matrix rate
+// (34 of 48 rows and 17 of 32 columns used at nk = 8).  Against the complex
+// VALU sum over the full cube: 256 atoms, nk = 8: 145 -> 23 us for one pair,
+// 565 -> 114 us for 128; 24 pairs of 601..1024 atoms, nk = 14: 1428 -> 145 us;
+// relative error against 64-bit-exact phases 1.6e-15 -> 0.8e-15 (256 atoms).
+// ---------------------------------------------------------------------------
+constexpr int kSFTile = 64;   // atoms per LDS tile
+constexpr int kSFThreads = 512;
+
+FO_HD int sf_stride(int NB) { return 2 * NB + 3; }  // doubles per atom (odd)
+
+template <int CT>
+__global__ void __launch_bounds__(kSFThreads) k_per_sf(
     const PerPair* __restrict__ pd, const PerGroup* __restrict__ grp,
     const int* __restrict__ atoms, const double* __restrict__ pos1,
     const double* __restrict__ pos2, int nk, double2* __restrict__ Cprod,
     double2* __restrict__ C1out, double2* __restrict__ C2out) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int NB = 2 * nk + 1;
+  constexpr int RTW = CT <= 2 ? 1 : 2;                         // row tiles per wave
+  constexpr int kMaxNB = 16 * CT - 1;                          // NB is odd
+  constexpr int ITEMS = (kMaxNB * kMaxNB + kSFThreads - 1) / kSFThreads;
+  extern __shared__ __align__(16) double sf_lds[];
+  const int NB = 2 * nk + 1, SR = sf_stride(NB);
   const int a = blockIdx.x, p = blockIdx.y, t = threadIdx.x;
   const PerPair d = pd[p];
-  double2* ex = (double2*)smem;          // [kSFTile]
-  double2* ey = ex + kSFTile;            // [kSFTile][NB]
-  double2* ez = ey + kSFTile * NB;       // [kSFTile][NB]
-  const long long plane = (long long)NB * NB;
-  const long long cube = plane * NB;
-  for (int e0 = 0; e0 < NB * NB; e0 += kSFChunk * blockDim.x) {
-    double2 prod[kSFChunk];
-    for (int q = 0; q < kSFChunk; ++q) prod[q] = make_double2(0.0, 0.0);
-    for (int g = 0; g < d.ngroups; ++g) {
-      const PerGroup G = grp[d.group_off + g];
-      double2 acc[2][kSFChunk];
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6), st = wv >> 2, wr = wv & 3;
+  const int ln = t & 63, col = ln & 15, kq = ln >> 4;
+  const int rows = a > 0 ? 2 * NB : NB;  // rows (X, beta): X * NB + beta; sin(0) = 0
+  const int nrt = (rows + 15) >> 4;
+  // this lane's A operand: LDS offsets of X and Y of row 16 rt + col (rows
+  // beyond the last read the last row and are not stored)
+  int ox[RTW], oy[RTW], oz[CT];
+#pragma unroll
+  for (int q = 0; q < RTW; ++q) {
+    const int r = min(16 * (wr + 4 * q) + col, rows - 1);
+    ox[q] = r >= NB ? 1 : 0;
+    oy[q] = 2 + (r >= NB ? r - NB : r);
+  }
+#pragma unroll
+  for (int c = 0; c < CT; ++c) oz[c] = 2 + NB + min(16 * c + col, NB - 1);
+  double* const tile = sf_lds + st * kSFTile * SR;
+  // phase stage: wave pj = (structure, axis), lane = atom of the tile
+  static_assert(kSFTile == 64 && kSFThreads >= 6 * 64, "a wave per structure and axis");
+  const int pj = wv, ps = pj >= 3 ? 1 : 0, pax = pj - 3 * ps, pa = ln;
+  const double pbox = d.box[pj < 6 ? pax : 0];
+  double2 prod[ITEMS];
+#pragma unroll
+  for (int q = 0; q < ITEMS; ++q) prod[q] = make_double2(0.0, 0.0);
+  const long long plane = (long long)NB * NB, cube = plane * NB;
+  for (int g = 0; g < d.ngroups; ++g) {
+    const PerGroup G = grp[d.group_off + g];
+    v4d acc[RTW][CT];
+#pragma unroll
+    for (int q = 0; q < RTW; ++q)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) acc[q][c] = v4d{0.0, 0.0, 0.0, 0.0};
+    // thread (s, axis, atom) of the phase stage; the next tile's coordinate is
+    // loaded before the products of this one
+    auto coord = [&](int j) {
+      return pj < 2 * 3 && j < G.size
+                 ? (ps ? pos2 : pos1)[3LL * (d.atom_off + atoms[G.atom_list_off + j]) + pax]
+                 : 0.0;
+    };
+    double xnext = coord(pa);
+    for (int j0 = 0; j0 < G.size; j0 += kSFTile) {
+      const int jt = min(kSFTile, G.size - j0), jp = (jt + 3) & ~3;  // padded to MFMA steps
+      __syncthreads();  // readers of the previous tile (or of S) are done
+      if (pj < 2 * 3) {
+        double* o = sf_lds + (ps * kSFTile + pa) * SR;
+        const bool ok = pa < jt;  // padding atoms add nothing
+        // x / box as its fraction of the nearest integer plus the quotient's
+        // remainder: the base angle is as accurate as its last bit
+        const double q = xnext / pbox, f = (q - rint(q)) + __builtin_fma(-q, pbox, xnext) / pbox;
+        double sn, cs;
+        sincospi(2.0 * (pax == 0 ? a : 1) * f, &sn, &cs);
+        if (!ok) sn = cs = 0.0;
+        if (pax == 0) {
+          o[0] = cs;
+          o[1] = sn;
+        } else {
+          o += pax == 1 ? 2 : 2 + NB;
+          o[0] = ok ? 1.0 : 0.0;
+          if (nk > 0) {
+            o[1] = cs;
+            o[2] = sn;
+          }
+          // e^{i m f} = e^{i h f} e^{i (m - h) f}, h = m / 2
+          for (int m = 2; m <= nk; ++m) {
+            const int h = m >> 1, k = m - h;
+            const double hc = o[2 * h - 1], hs = o[2 * h], kc = o[2 * k - 1], ks = o[2 * k];
+            o[2 * m - 1] = hc * kc - hs * ks;
+            o[2 * m] = hc * ks + hs * kc;
+          }
+        }
+        xnext = coord(j0 + kSFTile + pa);
+      }
+      __syncthreads();
+      if (wr < nrt) {  // wave-uniform
+#pragma unroll 2
+        for (int s4 = 0; s4 < jp; s4 += 4) {
+          const double* o = tile + (s4 + kq) * SR;
+          double zv[CT], av[RTW];
+#pragma unroll
+          for (int c = 0; c < CT; ++c) zv[c] = o[oz[c]];
+#pragma unroll
+          for (int q = 0; q < RTW; ++q) av[q] = o[ox[q]] * o[oy[q]];
+#pragma unroll
+          for (int q = 0; q < RTW; ++q) {
+            if (q > 0 && wr + 4 * q >= nrt) continue;  // wave-uniform
+#pragma unroll
+            for (int c = 0; c < CT; ++c) acc[q][c] = mfma64(av[q], zv[c], acc[q][c]);
+          }
+        }
+      }
+    }
+    // S of both structures -> LDS [structure][row][gamma] (over the tiles)
+    __syncthreads();
+    double* const S = sf_lds + (long long)st * 2 * plane;
+#pragma unroll
+    for (int q = 0; q < RTW; ++q)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 16 * (wr + 4 * q) + 4 * i + kq, gm = 16 * c + col;
+          if (r < rows && gm < NB) S[r * NB + gm] = acc[q][c][i];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < ITEMS; ++q) {
+      const int e = t + q * kSFThreads;
+      if (e >= plane) continue;
+      const int b = e / NB - nk, c = e % NB - nk;
+      const int ab = abs(b), ac = abs(c);
+      const double sb = b < 0 ? -1.0 : 1.0, sc = c < 0 ? -1.0 : 1.0;
+      const int bc = ab ? 2 * ab - 1 : 0, cc = ac ? 2 * ac - 1 : 0;
+      double2 C[2];
+#pragma unroll
       for (int s = 0; s < 2; ++s) {
-        const double* pos = (s ? pos2 : pos1) + 3LL * d.atom_off;
-        for (int q = 0; q < kSFChunk; ++q) acc[s][q] = make_double2(0.0, 0.0);
-        for (int j0 = 0; j0 < G.size; j0 += kSFTile) {
-          const int jt = min(kSFTile, G.size - j0);
-          __syncthreads();
-          for (int w = t; w < jt * (1 + 2 * NB); w += blockDim.x) {
-            const int j = w / (1 + 2 * NB), r = w % (1 + 2 * NB);
-            const int at = atoms[G.atom_list_off + j0 + j];
-            const double* x = pos + 3LL * at;
-            if (r == 0) {
-              ex[j] = phase64(2.0 * (a - nk) * x[0] / d.box[0]);
-            } else if (r <= NB) {
-              ey[j * NB + r - 1] = phase64(2.0 * (r - 1 - nk) * x[1] / d.box[1]);
-            } else {
-              ez[j * NB + r - 1 - NB] = phase64(2.0 * (r - 1 - NB - nk) * x[2] / d.box[2]);
-            }
-          }
-          __syncthreads();
-          // e^{-i kx x} (fixed kx per workgroup) folded into the y phases once
-          // per tile: the product the sum below used to form per entry
-          for (int w = t; w < jt * NB; w += blockDim.x) ey[w] = cmul(ex[w / NB], ey[w]);
-          __syncthreads();
-          for (int q = 0; q < kSFChunk; ++q) {
-            const int e = e0 + q * blockDim.x + t;
-            if (e >= NB * NB) break;
-            const int b = e / NB, c = e % NB;
-            double2 sacc = acc[s][q];
-            for (int j = 0; j < jt; ++j) sacc = cadd(sacc, cmul(ey[j * NB + b], ez[j * NB + c]));
-            acc[s][q] = sacc;
-          }
-        }
+        // row / column of the cosine; the sine follows it (none at 0)
+        const double* Z = sf_lds + s * 2 * plane + bc * NB + cc;
+        const int nb1 = ab ? NB : 0, nx = a > 0 ? (int)plane : 0;
+        const double hb = ab ? sb : 0.0, hc = ac ? sc : 0.0, hx = a > 0 ? 1.0 : 0.0;
+        const int z1 = ac ? 1 : 0;
+        const double ccc = Z[0], ccs = Z[z1], csc = Z[nb1], css = Z[nb1 + z1];
+        const double scc = Z[nx], scs = Z[nx + z1], ssc = Z[nx + nb1], sss = Z[nx + nb1 + z1];
+        // (cx - i sx)(cy - i hb sy)(cz - i hc sz), the sine sums signed by b, c
+        C[s].x = ccc - hx * hb * ssc - hb * hc * css - hx * hc * scs;
+        C[s].y = -(hb * csc + hx * scc + hc * ccs - hx * hb * hc * sss);
       }
-      for (int q = 0; q < kSFChunk; ++q) {
-        const int e = e0 + q * blockDim.x + t;
-        if (e >= NB * NB) break;
-        prod[q] = cadd(prod[q], cmul(acc[0][q], cconj(acc[1][q])));
-        if (C1out) {
-          const long long o = (long long)(d.group_off + g) * cube + a * plane + e;
-          C1out[o] = acc[0][q];
-          C2out[o] = acc[1][q];
+      overlap_add(prod[q], C[0], C[1]);
+      if (C1out) {
+        const long long o = (long long)(d.group_off + g) * cube;
+        const long long kp = (nk + a) * plane + e, km = (nk - a) * plane + (plane - 1 - e);
+        C1out[o + kp] = C[0];
+        C2out[o + kp] = C[1];
+        if (a > 0) {
+          C1out[o + km] = cconj(C[0]);
+          C2out[o + km] = cconj(C[1]);
         }
       }
     }
-    for (int q = 0; q < kSFChunk; ++q) {
-      const int e = e0 + q * blockDim.x + t;
-      if (e >= NB * NB) break;
-      const int b = e / NB, c = e % NB;
-      const double kx = 2.0 * kPi * (a - nk) / d.box[0];
-      const double ky = 2.0 * kPi * (b - nk) / d.box[1];
-      const double kz = 2.0 * kPi * (c - nk) / d.box[2];
-      const double w = exp(-(kx * kx + ky * ky + kz * kz) * d.scale * d.scale);
-      Cprod[d.c_off + a * plane + e] = cscale(prod[q], w);
-    }
+  }
+#pragma unroll
+  for (int q = 0; q < ITEMS; ++q) {
+    const int e = t + q * kSFThreads;
+    if (e >= plane) continue;
+    const double2 v = cscale(prod[q], overlap_weight(d, a, e / NB - nk, e % NB - nk));
+    double2* o = Cprod + d.c_off;
+    o[(nk + a) * plane + e] = v;
+    if (a > 0) o[(nk - a) * plane + (plane - 1 - e)] = cconj(v);
   }
 }
 
@@ -120,12 +244,9 @@ __global__ void k_per_product(const PerPair* __restrict__ pd, int nk,
     double2 s = make_double2(0.0, 0.0);
     for (int g = 0; g < d.ngroups; ++g) {
       const long long o = (long long)(d.group_off + g) * cube + e;
-      s = cadd(s, cmul(C1[o], cconj(C2[o])));
+      overlap_add(s, C1[o], C2[o]);
     }
-    const double kx = 2.0 * kPi * (a - nk) / d.box[0];
-    const double ky = 2.0 * kPi * (b - nk) / d.box[1];
-    const double kz = 2.0 * kPi * (c - nk) / d.box[2];
-    Cprod[d.c_off + e] = cscale(s, exp(-(kx * kx + ky * ky + kz * kz) * d.scale * d.scale));
+    Cprod[d.c_off + e] = cscale(s, overlap_weight(d, a - nk, b - nk, c - nk));
   }
 }
 
@@ -146,11 +267,8 @@ __global__ void k_per_product_indexed(const PerPair* __restrict__ pd, int nk,
     const int a = (int)(e / (NB * NB)), b = (int)((e / NB) % NB), c = (int)(e % NB);
     double2 s = make_double2(0.0, 0.0);
     for (int g = 0; g < d.ngroups; ++g)
-      s = cadd(s, cmul(A[(long long)g * cube + e], cconj(B[(long long)g * cube + e])));
-    const double kx = 2.0 * kPi * (a - nk) / d.box[0];
-    const double ky = 2.0 * kPi * (b - nk) / d.box[1];
-    const double kz = 2.0 * kPi * (c - nk) / d.box[2];
-    Cprod[d.c_off + e] = cscale(s, exp(-(kx * kx + ky * ky + kz * kz) * d.scale * d.scale));
+      overlap_add(s, A[(long long)g * cube + e], B[(long long)g * cube + e]);
+    Cprod[d.c_off + e] = cscale(s, overlap_weight(d, a - nk, b - nk, c - nk));
   }
 }
 
@@ -562,13 +680,30 @@ namespace fo {
 
 static inline int pcdiv(long long a, long long b) { return (int)((a + b - 1) / b); }
 
-size_t per_sf_smem(int nk) { return sizeof(double2) * (size_t)kSFTile * (1 + 2 * (2 * nk + 1)); }
+// the larger of the phase tiles and the group sums S of both structures
+size_t per_sf_smem(int nk) {
+  const size_t NB = 2 * (size_t)nk + 1;
+  return sizeof(double) * std::max(2 * (size_t)kSFTile * sf_stride((int)NB), 4 * NB * NB);
+}
 
 void launch_per_sf(hipStream_t s, int P, int nk, const PerPair* pd, const PerGroup* grp,
                    const int* atoms, const double* pos1, const double* pos2, double2* Cprod,
                    double2* C1out, double2* C2out) {
-  hipLaunchKernelGGL(k_per_sf, dim3(2 * nk + 1, P), dim3(256), per_sf_smem(nk), s, pd, grp, atoms,
-                     pos1, pos2, nk, Cprod, C1out, C2out);
+  const dim3 g(nk + 1, P), b(kSFThreads);
+  const size_t sm = per_sf_smem(nk);
+  const int ct = (2 * nk + 1 + 15) / 16;
+#define FO_SF(CT)                                                                             \
+  hipLaunchKernelGGL(k_per_sf<CT>, g, b, sm, s, pd, grp, atoms, pos1, pos2, nk, Cprod, C1out, \
+                     C2out)
+  if (ct == 1)
+    FO_SF(1);
+  else if (ct == 2)
+    FO_SF(2);
+  else if (ct == 3)
+    FO_SF(3);
+  else
+    FO_SF(4);
+#undef FO_SF
 }
 
 void launch_per_product(hipStream_t s, int P, int nk, const PerPair* pd, const double2* C1,

@@ -147,3 +147,40 @@ def test_dropin_repeated_calls_reuse_the_batch(gpu):
         np.testing.assert_array_equal(perm, permf)
         np.testing.assert_array_equal(disp, dispf)
         np.testing.assert_array_equal(X2, X2f)
+
+
+@pytest.mark.parametrize("sizes,nk", [((1,), 0), ((3, 2), 1), ((64, 1), 7), ((65, 0, 4), 8),
+                                      ((63,), 15), ((130, 5), 16), ((66,), 24), ((7, 68), 31)])
+def test_structure_factors_tiles_and_product(gpu, sizes, nk):
+    """Structure factors at the edges of the 64-atom tiles and of the 16-wide
+    column tiles (2 nk + 1 = 15, 17, 31, 33, 49, 63), with empty groups,
+    unwrapped positions and a box that is not a cube; Hermitian to the last
+    bit, and the product is the one from the same coefficients supplied."""
+    say(f"case: groups {sizes} nk={nk}")
+    rng = np.random.default_rng(100 + nk)
+    N = sum(sizes)
+    box = np.array([5.0, 6.1, 4.3])
+    pos = [(2.0 * rng.random((N, 3)) - 0.5) * box for _ in range(2)]
+    at = np.concatenate([[0], np.cumsum(sizes)])
+    perm = rng.permutation(N)
+    groups = [perm[at[i]:at[i + 1]] for i in range(len(sizes))]
+    F = max(2 * nk + 1, 4)
+    with PeriodicBatch([N], box, 0.3, nk, F, [groups], 10, _lib.PER_KEEP_COEFFS) as b:
+        b.set_positions(*pos)
+        b.run(_lib.PSTAGE_SF)
+        C, Cp = b.coeffs(), b.product()[0]
+    with PeriodicBatch([N], box, 0.3, nk, F, [groups], 10, _lib.PER_INPUT_COEFFS) as b:
+        b.set_positions(*pos)
+        b.set_coeffs(*C)
+        b.run(_lib.PSTAGE_SF)
+        np.testing.assert_array_equal(b.product()[0], Cp)
+    k = np.arange(-nk, nk + 1)
+    for Cs, x in zip(C, pos):
+        e = [np.exp(-2j * np.pi * np.outer(x[:, q] / box[q], k)) for q in range(3)]
+        for Cg, g in zip(Cs, groups):
+            ref = np.einsum("ja,jb,jc->abc", e[0][g], e[1][g], e[2][g])
+            # per atom and axis the reference's angle, below 2 pi nk 1.5, is
+            # off by at most three roundings of it; a dozen roundings besides
+            tol = len(g) * 3 * (2 * np.pi * nk * 1.5 * 3 + 12) * 2.0 ** -53
+            assert np.abs(Cg - ref).max() <= tol
+            np.testing.assert_array_equal(Cg[::-1, ::-1, ::-1], Cg.conj())

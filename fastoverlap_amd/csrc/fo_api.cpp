@@ -84,8 +84,8 @@ int find_peaks_max_window();
 void launch_per_select(hipStream_t, int, int, int, const PerPair*, const double2*, const double2*,
                        const PlaneCand*, double2*, long long, PerPeak*);
 void launch_per_refine(hipStream_t, int, int, const PerPair*, const PerGroup*, const int*,
-                       const double*, const double*, const PerPeak*, int, int*, int*, int*,
-                       double*, double*, PerResult*);
+                       const double*, const double*, const PerPeak*, int, int, NearRec*, int*,
+                       int*, int*, double*, double*, PerResult*);
 void launch_lap_align(hipStream_t, int, const double*, const double*, int, const int*, const int*,
                       const int*, int, const double*, int, int*, int*, double*);
 }  // namespace fo
@@ -1558,7 +1558,7 @@ struct fo_per_batch {
   fo_context* ctx = nullptr;
   hipStream_t stream = nullptr;
   const PerTw* tw = nullptr;
-  int P = 0, nk = 0, F = 0, niter = 10, flags = 0, maxgroup = 1, gsum = 0;
+  int P = 0, nk = 0, F = 0, niter = 10, flags = 0, maxgroup = 1, maxgath = 0, gsum = 0;
   long long Ntot = 0, cube = 0;
   std::vector<PerPair> hp;
   std::vector<PerGroup> hg;
@@ -1624,7 +1624,8 @@ static int per_enqueue(fo_per_batch* b, int stages) {
   mark(3);
   if (stages & FO_PSTAGE_REFINE)
     launch_per_refine(s, b->P, b->maxgroup, b->pd, b->grp, b->atoms, b->pos1, b->pos2, b->peaks,
-                      b->niter, b->perm, b->saveperm, b->rowsol, b->X1out, b->X2out, b->res);
+                      b->niter, b->maxgath, (NearRec*)b->scr, b->perm, b->saveperm, b->rowsol,
+                      b->X1out, b->X2out, b->res);
   mark(4);
   FO_CHECK_LAUNCH();
   return FO_OK;
@@ -1688,6 +1689,9 @@ int per_batch_plan(fo_context* c, const fo_per_batch_desc* d, fo_per_batch** out
       ga += sz;
       b->maxgroup = std::max(b->maxgroup, sz);
     }
+    int gath = 0;
+    for (int q = 0; q < pp.ngroups; ++q) gath += b->hg[gq + q].size;
+    b->maxgath = std::max(b->maxgath, gath);
     gq += pp.ngroups;
     Ntot += N;
   }
@@ -1718,7 +1722,10 @@ int per_batch_plan(fo_context* c, const fo_per_batch_desc* d, fo_per_batch** out
   o.perm = lay.add<int>(Ntot);
   o.sp = lay.add<int>(Ntot);
   o.rs = lay.add<int>(Ntot + 1);
-  o.scr = lay.add<double2>((size_t)b->P * b->scr_stride);
+  // the selection's scratch, then the refinement's nearest rows (one per
+  // entry of the group lists)
+  o.scr = lay.add<double2>(std::max<size_t>((size_t)b->P * b->scr_stride,
+                                            (b->hatoms.size() * sizeof(NearRec) + 15) / 16));
   o.grid = (b->flags & FO_PER_KEEP_GRID) ? lay.add<float>((size_t)b->P * b->F * b->F * b->F) : 0;
   o.cgrid = (b->flags & FO_PER_KEEP_FFT) ? lay.add<float2>((size_t)b->P * b->F * b->F * b->F) : 0;
   b->bytes = lay.off;

@@ -185,30 +185,12 @@ FO_DEV void block_argmax(T& v, int& i, T* sv, int* si) {
   for (int w = 1; w < nw; ++w) argmax_merge(v, i, sv[w], si[w]);
 }
 
-// Block argmin with ties -> smaller index.
+// Argmin with ties -> smaller index.
 FO_DEV void argmin_merge(double& v, int& i, double ov, int oi) {
   if (ov < v || (ov == v && oi < i)) {
     v = ov;
     i = oi;
   }
-}
-FO_DEV void block_argmin(double& v, int& i, double* sv, int* si) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int nw = (blockDim.x + 63) >> 6;
-  for (int off = 32; off > 0; off >>= 1) {
-    double ov = __shfl_xor(v, off, 64);
-    int oi = __shfl_xor(i, off, 64);
-    argmin_merge(v, i, ov, oi);
-  }
-  __syncthreads();
-  if (lane == 0) {
-    sv[wid] = v;
-    si[wid] = i;
-  }
-  __syncthreads();
-  v = sv[0];
-  i = si[0];
-  for (int w = 1; w < nw; ++w) argmin_merge(v, i, sv[w], si[w]);
 }
 
 }  // namespace fo

@@ -565,11 +565,114 @@ __global__ void __launch_bounds__(256) k_per_select(
 // semantics: Euclidean minimum-image cost with rows = X1, X2[perm] ~ X1.
 // ---------------------------------------------------------------------------
 FO_DEV double pwrap(double v, double box) { return v - rint(v / box) * box; }
+// squared minimum-image length (ib = 1 / box)
+FO_DEV double pdist2(double dx, double dy, double dz, const double box[3], const double ib[3]) {
+  dx -= rint(dx * ib[0]) * box[0];
+  dy -= rint(dy * ib[1]) * box[1];
+  dz -= rint(dz * ib[2]) * box[2];
+  return dx * dx + dy * dy + dz * dz;
+}
+
+// The nearest row of every column (structure 2's atoms, displaced by the
+// peak) over its group, for the refinement's first assignment.  64 entries of
+// the pair's group lists per workgroup, four lanes a column; the rows of the
+// workgroup's groups pass through LDS in tiles.  In the refinement's single
+// workgroup this scan of all size^2 distances took most of its time (one
+// wavefront a SIMD, every distance waiting on gathered loads).  Both kernels
+// together against that: one pair of 256 atoms 226 -> 29 us, 24 pairs of
+// 601..1024 atoms 1826 -> 82 us (a search over cells of the box inside the
+// refinement took 661: its short, divergent loops wait on LDS).  Bound: the
+// FP64 vector rate, 20 operations a distance.
+constexpr int kNearCols = 64;
+constexpr int kNearTile = 256;
+__global__ void __launch_bounds__(256) k_per_nearest(
+    const PerPair* __restrict__ pd, const PerGroup* __restrict__ grp,
+    const int* __restrict__ atoms, const double* __restrict__ pos1,
+    const double* __restrict__ pos2, const PerPeak* __restrict__ peaks,
+    NearRec* __restrict__ near) {
+  __shared__ double rows[kNearTile][3];
+  __shared__ int s_range[2];
+  const int p = blockIdx.y, t = threadIdx.x;
+  const PerPair d = pd[p];
+  if (d.ngroups < 1) return;
+  const PerGroup* G = grp + d.group_off;
+  const int base = G[0].atom_list_off;  // the pair's list entries are contiguous
+  const int total = G[d.ngroups - 1].atom_list_off + G[d.ngroups - 1].size - base;
+  const int e0 = blockIdx.x * kNearCols;
+  if (e0 >= total) return;  // whole workgroup
+  const int e = e0 + (t >> 2), part = t & 3;
+  // the last group that starts at or before entry e (empty groups before it
+  // start there too)
+  int q = 0, hi = d.ngroups;
+  const int ec = min(e, total - 1);
+  while (hi - q > 1) {
+    const int mid = (q + hi) >> 1;
+    if (G[mid].atom_list_off - base <= ec)
+      q = mid;
+    else
+      hi = mid;
+  }
+  const int r0 = G[q].atom_list_off - base, r1 = r0 + G[q].size;
+  if (t == 0) s_range[0] = r0;
+  if (t == 255) s_range[1] = r1;
+  const double* x = pos1 + 3LL * d.atom_off;
+  const int* ga = atoms + base;
+  const double box[3] = {d.box[0], d.box[1], d.box[2]};
+  const double ib[3] = {1.0 / box[0], 1.0 / box[1], 1.0 / box[2]};
+  const double* Y = pos2 + 3LL * (d.atom_off + ga[ec]);
+  const double b0 = Y[0] - peaks[p].disp[0], b1 = Y[1] - peaks[p].disp[1],
+               b2 = Y[2] - peaks[p].disp[2];
+  auto root = [](double k) { return sqrt(k); };
+  ColMin m;
+  __syncthreads();
+  const int lo = s_range[0], end = s_range[1];
+  for (int k0 = lo; k0 < end; k0 += kNearTile) {
+    __syncthreads();  // readers of the previous tile are done
+    for (int w = t; w < 3 * min(kNearTile, end - k0); w += 256)
+      rows[w / 3][w % 3] = x[3 * ga[k0 + w / 3] + w % 3];
+    __syncthreads();
+    const int i1 = min(r1, k0 + kNearTile) - k0;
+    int i = max(r0, k0) - k0;
+    // rows of this lane: the group's row index modulo 4 is its part
+    i += (part - (i + k0 - r0)) & 3;
+    auto key = [&](int r) {
+      return pdist2(rows[r][0] - b0, rows[r][1] - b1, rows[r][2] - b2, box, ib);
+    };
+    for (; i + 12 < i1; i += 16) {
+      const double c0 = key(i), c1 = key(i + 4), c2 = key(i + 8), c3 = key(i + 12);
+      if (fmin(fmin(c0, c1), fmin(c2, c3)) < m.key2) {
+        m.add(c0, i + k0 - r0 + 1, root);
+        m.add(c1, i + k0 - r0 + 5, root);
+        m.add(c2, i + k0 - r0 + 9, root);
+        m.add(c3, i + k0 - r0 + 13, root);
+      }
+    }
+    for (; i < i1; i += 4) m.add(key(i), i + k0 - r0 + 1, root);
+  }
+  m.join(4);
+  if (part == 0 && e < total) {
+    NearRec r;
+    r.mn = m.mn;
+    r.gap = sqrt(m.key2) - sqrt(m.key);  // +inf for one row; NaN: never used
+    r.mi = m.mi;
+    r.pad = 0;
+    near[base + e] = r;
+  }
+}
+
+// LDS of the refinement beside the assignment arrays: the positions of the
+// largest group's rows and displaced columns, when they fit
+static inline size_t refine_lds_bytes(int nmax, bool staged) {
+  const size_t lap = (lap_lds_bytes(nmax) + 15) & ~(size_t)15;
+  return staged ? lap + 6 * sizeof(double) * (size_t)nmax : lap;
+}
+constexpr size_t kRefineLds = 160 * 1024;
 
 __global__ void __launch_bounds__(256) k_per_refine(
     const PerPair* __restrict__ pd, const PerGroup* __restrict__ grp,
     const int* __restrict__ atoms, const double* __restrict__ pos1,
-    const double* __restrict__ pos2, const PerPeak* __restrict__ peaks, int niter, int lap_nmax,
+    const double* __restrict__ pos2, const PerPeak* __restrict__ peaks,
+    const NearRec* __restrict__ near, int niter, int lap_nmax, int staged,
     int* __restrict__ perm, int* __restrict__ saveperm, int* __restrict__ rowsol,
     double* __restrict__ X1out, double* __restrict__ X2out, PerResult* __restrict__ res) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -588,27 +691,67 @@ __global__ void __launch_bounds__(256) k_per_refine(
   double disp[3] = {peaks[p].disp[0], peaks[p].disp[1], peaks[p].disp[2]};
   LapShared ls = lap_carve(smem, lap_nmax);
 
+  const double box[3] = {bx, by, bz}, ib[3] = {1.0 / bx, 1.0 / by, 1.0 / bz};
+  // group positions in LDS: rows x, columns y - disp
+  double* g1 = (double*)(smem + ((lap_lds_bytes(lap_nmax) + 15) & ~(size_t)15));
+  double* g2 = g1 + 3 * lap_nmax;
+  // Column minima: the first assignment takes k_per_nearest's.  A later one
+  // differs by a displacement e, which moves no minimum-image distance by
+  // more than |e|: a column whose second nearest row was more than 2 |e|
+  // farther keeps its nearest row, and only that distance is formed again;
+  // the others scan their rows.
+  const double start[3] = {disp[0], disp[1], disp[2]};
+  bool first = true;
+
   auto hungarian = [&](int* out) {
     for (int a = t; a < N; a += blockDim.x) out[a] = a;
     __threadfence_block();
     __syncthreads();
+    auto root = [](double k) { return sqrt(k); };
+    const double e0 = disp[0] - start[0], e1 = disp[1] - start[1], e2 = disp[2] - start[2];
+    const double safe = 2.0 * (1.0 + 1e-9) * sqrt(e0 * e0 + e1 * e1 + e2 * e2) +
+                        1e-12 * (bx + by + bz);
     for (int g = 0; g < d.ngroups; ++g) {
       const PerGroup G = grp[d.group_off + g];
+      const int n = G.size;
       const int* ga = atoms + G.atom_list_off;
-      const double d0 = disp[0], d1 = disp[1], d2 = disp[2];
-      auto cost = [&](int i, int j) {
-        const double* A = x + 3 * ga[i];
-        const double* B = y + 3 * ga[j];
-        const double dx = pwrap(A[0] - (B[0] - d0), bx);
-        const double dy = pwrap(A[1] - (B[1] - d1), by);
-        const double dz = pwrap(A[2] - (B[2] - d2), bz);
-        return sqrt(dx * dx + dy * dy + dz * dz);
+      const NearRec* nr = near + G.atom_list_off;
+      auto solve = [&](auto key) {
+        lap_solve(n, key, root,
+                  [&](int j, ColMin& m) {
+                    const NearRec r = nr[j];
+                    m.mi = r.mi;
+                    m.mn = r.mn;
+                    if (first) return true;
+                    if (!(r.mi > 0 && r.gap > safe)) return false;
+                    m.mn = root(key(r.mi - 1, j));
+                    return true;
+                  },
+                  ls, rs, red, redi);
       };
-      lap_solve(G.size, cost, ls, rs, red, redi);
-      for (int i = t; i < G.size; i += blockDim.x) out[ga[i]] = ga[rs[i]];
+      if (staged) {
+        for (int e = t; e < 3 * n; e += blockDim.x) {
+          const int i = e / 3, k = e - 3 * i;
+          g1[e] = x[3 * ga[i] + k];
+          g2[e] = y[3 * ga[i] + k] - (k == 0 ? disp[0] : (k == 1 ? disp[1] : disp[2]));
+        }
+        __syncthreads();
+        solve([&](int i, int j) {
+          const double *A = g1 + 3 * i, *B = g2 + 3 * j;
+          return pdist2(A[0] - B[0], A[1] - B[1], A[2] - B[2], box, ib);
+        });
+      } else {
+        const double d0 = disp[0], d1 = disp[1], d2 = disp[2];
+        solve([&](int i, int j) {
+          const double *A = x + 3 * ga[i], *B = y + 3 * ga[j];
+          return pdist2(A[0] - (B[0] - d0), A[1] - (B[1] - d1), A[2] - (B[2] - d2), box, ib);
+        });
+      }
+      for (int i = t; i < n; i += blockDim.x) out[ga[i]] = ga[rs[i]];
       __threadfence_block();
       __syncthreads();
     }
+    first = false;
   };
   auto mean_shift = [&](const int* pr) {
     double s[3] = {0, 0, 0};
@@ -618,7 +761,8 @@ __global__ void __launch_bounds__(256) k_per_refine(
       s[1] += pwrap(x[3 * a + 1] - (B[1] - disp[1]), by);
       s[2] += pwrap(x[3 * a + 2] - (B[2] - disp[2]), bz);
     }
-    for (int k = 0; k < 3; ++k) disp[k] -= block_sum(s[k], red) / (double)N;
+    block_sum_n<3>(s, red);
+    for (int k = 0; k < 3; ++k) disp[k] -= s[k] / (double)N;
   };
 
   hungarian(sp);
@@ -743,11 +887,16 @@ void launch_per_select(hipStream_t s, int P, int nk, int F, const PerPair* pd,
 
 void launch_per_refine(hipStream_t s, int P, int lap_nmax, const PerPair* pd, const PerGroup* grp,
                        const int* atoms, const double* pos1, const double* pos2,
-                       const PerPeak* peaks, int niter, int* perm, int* saveperm, int* rowsol,
-                       double* X1out, double* X2out, PerResult* res) {
-  hipLaunchKernelGGL(k_per_refine, dim3(P), dim3(256), lap_lds_bytes(lap_nmax), s, pd, grp, atoms,
-                     pos1, pos2, peaks, niter, lap_nmax, perm, saveperm, rowsol, X1out, X2out,
-                     res);
+                       const PerPeak* peaks, int niter, int maxgath, NearRec* near, int* perm,
+                       int* saveperm, int* rowsol, double* X1out, double* X2out, PerResult* res) {
+  if (maxgath > 0)
+    hipLaunchKernelGGL(k_per_nearest, dim3(pcdiv(maxgath, kNearCols), P), dim3(256), 0, s, pd, grp,
+                       atoms, pos1, pos2, peaks, near);
+  // (the reduction scratch is static, beside the dynamic part)
+  const bool staged = refine_lds_bytes(lap_nmax, true) + 1024 <= kRefineLds;
+  hipLaunchKernelGGL(k_per_refine, dim3(P), dim3(256), refine_lds_bytes(lap_nmax, staged), s, pd,
+                     grp, atoms, pos1, pos2, peaks, near, niter, lap_nmax, staged ? 1 : 0, perm,
+                     saveperm, rowsol, X1out, X2out, res);
 }
 
 }  // namespace fo
@@ -778,19 +927,15 @@ __global__ void __launch_bounds__(256) k_lap_align(int N, const double* __restri
   __syncthreads();
   for (int g = 0; g < ngroups; ++g) {
     const int* ga = gatoms + goff[g];
-    auto cost = [&](int i, int j) {
+    const double box[3] = {bx, by, bz}, ib[3] = {1.0 / bx, 1.0 / by, 1.0 / bz};
+    auto key = [&](int i, int j) {
       const double* A = X1 + 3 * ga[i];
       const double* B = X2 + 3 * ga[j];
-      double dx = A[0] - B[0], dy = A[1] - B[1], dz = A[2] - B[2];
-      if (metric == 1) {
-        dx = pwrap(dx, bx);
-        dy = pwrap(dy, by);
-        dz = pwrap(dz, bz);
-        return sqrt(dx * dx + dy * dy + dz * dz);
-      }
-      return dx * dx + dy * dy + dz * dz;
+      const double dx = A[0] - B[0], dy = A[1] - B[1], dz = A[2] - B[2];
+      return metric == 1 ? pdist2(dx, dy, dz, box, ib) : dx * dx + dy * dy + dz * dz;
     };
-    lap_solve(gsize[g], cost, ls, rowsol, red, redi);
+    lap_solve(gsize[g], key, [&](double k) { return metric == 1 ? sqrt(k) : k; },
+              [](int, ColMin&) { return false; }, ls, rowsol, red, redi);
     for (int i = t; i < gsize[g]; i += blockDim.x) perm[ga[i]] = ga[rowsol[i]];
     __threadfence_block();
     __syncthreads();

@@ -20,7 +20,7 @@ struct LapShared {
   int* p;
   int* way;
   int* used;
-  int* ra;  // column assigned to row i by the initial column reduction (0: free)
+  int* ra;  // column assigned to row i by the initial column reduction (n + 1: free)
 };
 FO_HD size_t lap_lds_bytes(int nmax) {
   return (size_t)(nmax + 1) * (3 * sizeof(double) + 4 * sizeof(int));
@@ -69,112 +69,192 @@ FO_DEV void wave_argmin_dpp(double& v, int& i) {
   i = ri;
 }
 
-// Minimum-cost assignment of an n x n cost matrix given by cost(i, j)
-// (0-based).  rowsol[i] = column assigned to row i.  Ties in the column
-// search are broken toward the smaller column index, so the result does not
-// depend on the launch width.  Every thread of the block must call this;
-// a one-wavefront block reduces without LDS or barrier.
+// Cost of an assignment problem: cost(i, j) = fin(key(i, j)) with fin
+// non-decreasing (squared distance and its square root, or the identity), so
+// a column's minimum is searched on the keys and fin is taken of the few
+// that improve it.  The result is the minimum of the costs at its smallest
+// row, as if every cost had been formed.
+struct ColMin {
+  double key = INFINITY, key2 = INFINITY;  // smallest two keys
+  double mn = kLapInf;
+  int mi = 0;  // 1-based row, 0: none finite
+  template <class Fin>
+  FO_DEV void add(double k, int row, Fin fin) {
+    key2 = fmin(key2, fmax(key, k));
+    if (k < key) {
+      key = k;
+      const double c = fin(k);
+      if (c < mn) {
+        mn = c;
+        mi = row;
+      }
+    }
+  }
+  // across the S lanes (a power of two) that scanned one column's rows
+  FO_DEV void join(int S) {
+    for (int o = 1; o < S; o <<= 1) {
+      const double om = __shfl_xor(mn, o, 64), ok = __shfl_xor(key, o, 64),
+                   o2 = __shfl_xor(key2, o, 64);
+      const int oi = __shfl_xor(mi, o, 64);
+      key2 = fmin(fmin(key2, o2), fmax(key, ok));
+      key = fmin(key, ok);
+      if (om < mn || (om == mn && oi && (!mi || oi < mi))) {
+        mn = om;
+        mi = oi;
+      }
+    }
+  }
+};
+
+// Column j's nearest row as a wide kernel found it: cost and (1-based) row,
+// and how much farther the second nearest row is.
+struct NearRec {
+  double mn, gap;
+  int mi, pad;
+};
+
+// Minimum-cost assignment of an n x n cost matrix given by key(i, j) and fin
+// (0-based, see ColMin).  rowsol[i] = column assigned to row i.  Ties in the
+// column search are broken toward the smaller column index, so the result
+// does not depend on the launch width.  near(j, m) may leave column j's
+// minimum in m and return true, or return false to have all rows scanned.
+// Costs are formed where they are used; the serial parts (the row of each
+// column, the list of free rows) go over all threads or 64 rows a step: at
+// 716 rows the walk over the rows alone took 36 us.
+// Every thread of the block (at most eight wavefronts; red_v, red_i: 16
+// entries of LDS) must call this; a one-wavefront block reduces without LDS or
+// barrier.
 // Returns false (rowsol = identity) if a non-finite cost stops the search.
-template <class CostF>
-FO_DEV bool lap_solve(int n, CostF cost, LapShared s, int* rowsol, double* red_v,
-                      int* red_i) {
+template <class KeyF, class Fin, class Near>
+FO_DEV bool lap_solve(int n, KeyF key, Fin fin, Near near, LapShared s, int* rowsol,
+                      double* red_v, int* red_i) {
   const int t = threadIdx.x, bd = blockDim.x;
+  auto cost = [&](int i, int j) { return fin(key(i, j)); };
   // column reduction (Jonker & Volgenant 1987): v[j] = min_i c(i, j), and
   // column j goes to its minimising row (ties: smallest row) unless an
   // earlier column took that row.  The duals (u = 0, v) are feasible and
   // tight on these pairs, so the search below only runs for the free rows.
-  for (int j = t; j <= n; j += bd) {
-    double mn = 0.0;
-    int mi = 0;
-    if (j > 0) {
-      mn = kLapInf;
-      for (int i = 1; i <= n; ++i) {
-        const double c = cost(i - 1, j - 1);
-        if (c < mn) {
-          mn = c;
-          mi = i;
+  // S lanes share a column when the block has lanes to spare.
+  int S = 1;
+  while (2 * S <= 16 && 2 * S * n <= bd) S *= 2;
+  const int part = t & (S - 1);
+  for (int j = t / S; j < n; j += bd / S) {
+    ColMin m;
+    if (!near(j, m)) {
+      m = ColMin{};
+      int i = part;
+      for (; i + 3 * S < n; i += 4 * S) {
+        const double k0 = key(i, j), k1 = key(i + S, j), k2 = key(i + 2 * S, j),
+                     k3 = key(i + 3 * S, j);
+        if (fmin(fmin(k0, k1), fmin(k2, k3)) < m.key) {
+          m.add(k0, i + 1, fin);
+          m.add(k1, i + S + 1, fin);
+          m.add(k2, i + 2 * S + 1, fin);
+          m.add(k3, i + 3 * S + 1, fin);
         }
       }
-      if (!(mn < kLapInf)) mn = 0.0;  // non-finite column: left to the search
+      for (; i < n; i += S) m.add(key(i, j), i + 1, fin);
+      m.join(S);
     }
-    s.u[j] = 0.0;
-    s.v[j] = mn;
-    s.p[j] = 0;
-    s.way[j] = mi;  // candidate row, read once below
-    s.ra[j] = 0;
+    if (part == 0) {
+      s.u[j + 1] = 0.0;
+      s.v[j + 1] = m.mn < kLapInf ? m.mn : 0.0;  // non-finite column: left to the search
+      s.p[j + 1] = 0;
+      s.way[j + 1] = m.mi;  // candidate row, read once below
+      s.ra[j + 1] = n + 1;  // row j + 1: free
+    }
+  }
+  if (t == 0) {
+    s.u[0] = s.v[0] = 0.0;
+    s.p[0] = s.way[0] = 0;
   }
   __syncthreads();
-  if (t == 0)
-    for (int j = 1; j <= n; ++j) {
-      const int i = s.way[j];
-      if (i > 0 && !s.ra[i]) {
-        s.ra[i] = j;
-        s.p[j] = i;
-      }
-    }
+  for (int j = 1 + t; j <= n; j += bd)
+    if (s.way[j] > 0) atomicMin(&s.ra[s.way[j]], j);
   __syncthreads();
-  for (int i = 1; i <= n; ++i) {
-    if (s.ra[i]) continue;  // uniform: every thread reads the same LDS word
-    for (int j = t; j <= n; j += bd) {
-      s.minv[j] = kLapInf;
-      s.used[j] = 0;
-    }
-    if (t == 0) s.p[0] = i;
-    __syncthreads();
-    int j0 = 0;
-    for (;;) {
-      if (t == 0) s.used[j0] = 1;
-      __syncthreads();
-      const int i0 = s.p[j0];
-      const double ui0 = s.u[i0];
-      double best = kLapInf;
-      int bj = 0x7fffffff;
-      for (int j = 1 + t; j <= n; j += bd) {
-        if (!s.used[j]) {
-          double cur = cost(i0 - 1, j - 1) - ui0 - s.v[j];
-          double mv = s.minv[j];
-          if (cur < mv) {
-            mv = cur;
-            s.minv[j] = cur;
-            s.way[j] = j0;
-          }
-          if (mv < best || (mv == best && j < bj)) {
-            best = mv;
-            bj = j;
-          }
-        }
-      }
-      if (bd == 64)
-        wave_argmin_dpp(best, bj);
-      else
-        block_argmin(best, bj, red_v, red_i);
-      if (bj == 0x7fffffff || !(best < kLapInf)) {
-        // no finite reduced cost left: the costs are not finite numbers
-        for (int k = t; k < n; k += bd) rowsol[k] = k;
-        __syncthreads();
-        return false;
-      }
-      const double delta = best;
+  for (int j = 1 + t; j <= n; j += bd)
+    if (s.way[j] > 0 && s.ra[s.way[j]] == j) s.p[j] = s.way[j];
+  __syncthreads();
+  int half = 0;
+  // the free rows in order, 64 at a time (every wavefront reads the same LDS
+  // words, so the masks agree)
+  for (int i64 = 0; i64 < n; i64 += 64) {
+    const int ir = i64 + (t & 63) + 1;
+    unsigned long long freem = __ballot(ir <= n && s.ra[ir] > n);
+    while (freem) {
+      const int i = i64 + __ffsll(freem);
+      freem &= freem - 1;
       for (int j = t; j <= n; j += bd) {
-        if (s.used[j]) {
-          s.u[s.p[j]] += delta;
-          s.v[j] -= delta;
-        } else {
-          s.minv[j] -= delta;
+        s.minv[j] = kLapInf;
+        s.used[j] = 0;
+      }
+      if (t == 0) s.p[0] = i;
+      __syncthreads();
+      int j0 = 0;
+      for (;;) {
+        if (t == 0) s.used[j0] = 1;
+        __syncthreads();
+        const int i0 = s.p[j0];
+        const double ui0 = s.u[i0];
+        double best = kLapInf;
+        int bj = 0x7fffffff;
+        for (int j = 1 + t; j <= n; j += bd) {
+          if (!s.used[j]) {
+            double cur = cost(i0 - 1, j - 1) - ui0 - s.v[j];
+            double mv = s.minv[j];
+            if (cur < mv) {
+              mv = cur;
+              s.minv[j] = cur;
+              s.way[j] = j0;
+            }
+            if (mv < best || (mv == best && j < bj)) {
+              best = mv;
+              bj = j;
+            }
+          }
         }
+        wave_argmin_dpp(best, bj);
+        if (bd > 64) {
+          // the wavefronts' minima, in the half of the scratch that the
+          // previous step did not use (its readers may still be at it)
+          half ^= 8;
+          if ((t & 63) == 0) {
+            red_v[half + (t >> 6)] = best;
+            red_i[half + (t >> 6)] = bj;
+          }
+          __syncthreads();
+          best = red_v[half];
+          bj = red_i[half];
+          for (int w = 1; w < bd >> 6; ++w) argmin_merge(best, bj, red_v[half + w], red_i[half + w]);
+        }
+        if (bj == 0x7fffffff || !(best < kLapInf)) {
+          // no finite reduced cost left: the costs are not finite numbers
+          for (int k = t; k < n; k += bd) rowsol[k] = k;
+          __syncthreads();
+          return false;
+        }
+        const double delta = best;
+        for (int j = t; j <= n; j += bd) {
+          if (s.used[j]) {
+            s.u[s.p[j]] += delta;
+            s.v[j] -= delta;
+          } else {
+            s.minv[j] -= delta;
+          }
+        }
+        __syncthreads();
+        j0 = bj;
+        if (s.p[j0] == 0) break;
+      }
+      if (t == 0) {
+        do {
+          int j1 = s.way[j0];
+          s.p[j0] = s.p[j1];
+          j0 = j1;
+        } while (j0);
       }
       __syncthreads();
-      j0 = bj;
-      if (s.p[j0] == 0) break;
     }
-    if (t == 0) {
-      do {
-        int j1 = s.way[j0];
-        s.p[j0] = s.p[j1];
-        j0 = j1;
-      } while (j0);
-    }
-    __syncthreads();
   }
   for (int j = 1 + t; j <= n; j += bd) rowsol[s.p[j] - 1] = j - 1;
   __syncthreads();

@@ -2678,13 +2678,14 @@ __global__ void __launch_bounds__(256) k_sph_finish(
       }
       __syncthreads();
     }
-    auto cost = [&](int i, int j) {
+    auto key = [&](int i, int j) {
       const double* A = pos_lds ? g1 + 3 * i : x1 + 3 * ga[i];
       const double* B = pos_lds ? g2 + 3 * j : xr + 3 * ga[j];
       const double dx = A[0] - B[0], dy = A[1] - B[1], dz = A[2] - B[2];
       return dx * dx + dy * dy + dz * dz;
     };
-    lap_solve(G.size, cost, ls, rs, red, redi);
+    lap_solve(G.size, key, [](double k) { return k; }, [](int, ColMin&) { return false; }, ls, rs,
+              red, redi);
     for (int i = t; i < G.size; i += blockDim.x) pm[ga[i]] = ga[rs[i]];
     __threadfence_block();
     __syncthreads();

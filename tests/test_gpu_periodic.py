@@ -184,3 +184,66 @@ def test_structure_factors_tiles_and_product(gpu, sizes, nk):
             tol = len(g) * 3 * (2 * np.pi * nk * 1.5 * 3 + 12) * 2.0 ** -53
             assert np.abs(Cg - ref).max() <= tol
             np.testing.assert_array_equal(Cg[::-1, ::-1, ::-1], Cg.conj())
+
+
+def _refine_reference(x, y, box, groups, disp, niter):
+    """The LAP + mean-shift iteration with scipy's assignment solver."""
+    from scipy.optimize import linear_sum_assignment
+
+    def wrap(v):
+        return v - np.round(v / box) * box
+
+    def assign(d):
+        perm = np.arange(len(x))
+        for g in groups:
+            c = np.linalg.norm(wrap(x[g][:, None] - (y[g] - d)[None]), axis=2)
+            perm[g] = g[linear_sum_assignment(c)[1]]
+        return perm
+
+    def shift(d, perm):
+        return d - wrap(x - (y[perm] - d)).mean(0)
+
+    perm = assign(disp)
+    for _ in range(niter):
+        disp = shift(disp, perm)
+        new = assign(disp)
+        same = np.array_equal(new, perm)
+        perm = new
+        if same:
+            break
+    disp = shift(disp, perm)
+    return perm, disp, np.linalg.norm(wrap(x - (y[perm] - disp)))
+
+
+@pytest.mark.parametrize("sizes,noise,niter", [
+    ((1,), 0.02, 10), ((63, 0, 2), 0.02, 10), ((64,), 0.3, 10), ((65, 1, 64), 0.3, 10),
+    ((256,), 0.02, 0), ((257, 130), 0.25, 10), ((2000,), 0.02, 1)])
+def test_refine_nearest_rows_and_assignment(gpu, sizes, noise, niter):
+    """The refinement from a given displacement at the edges of the nearest-row
+    kernel's 64 columns and 256-row tiles, with empty and one-atom groups,
+    with many free rows (noise 0.25 and above: later assignments rescan
+    columns) and with positions too many for LDS (2000)."""
+    say(f"case: groups {sizes} noise {noise} niter {niter}")
+    rng = np.random.default_rng(sum(sizes) + niter)
+    N = sum(sizes)
+    box = np.array([1.0, 1.15, 0.9]) * (N / 1.1) ** (1 / 3) + 0.5
+    at = np.concatenate([[0], np.cumsum(sizes)])
+    order = rng.permutation(N)
+    groups = [order[at[i]:at[i + 1]] for i in range(len(sizes))]
+    x = rng.random((N, 3)) * box
+    perm = np.arange(N)
+    for g in groups:
+        perm[g] = rng.permutation(g)
+    y = x[perm] + 0.4 + rng.normal(scale=noise, size=x.shape)
+    d0 = np.full(3, 0.4 + 0.01)
+    with PeriodicBatch([N], box, 0.3, 2, 12, [groups], niter) as b:
+        b.set_positions(x, y)
+        b.set_disp(d0)
+        b.run(_lib.PSTAGE_REFINE)
+        r = b.results()
+    rp, rd, dist = _refine_reference(x, y, box, groups, d0, niter)
+    np.testing.assert_array_equal(r["perm"][0], rp)
+    # sums of N terms below the box length
+    tol = 8 * N * box.max() * 2.0 ** -53
+    np.testing.assert_allclose(r["disp"][0], rd, rtol=0, atol=tol)
+    assert abs(r["dist"][0] - dist) <= tol

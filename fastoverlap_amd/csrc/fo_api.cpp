@@ -75,14 +75,14 @@ void launch_per_product(hipStream_t, int, int, const PerPair*, const double2*, c
                         double2*);
 size_t per_plane_smem(int, int);
 void launch_per_plane(hipStream_t, int, int, int, const PerPair*, const double2*, const float2*,
-                      PlaneCand*, float*, float2*);
+                      PlaneCand*, double*, float*, float2*);
 void launch_per_product_indexed(hipStream_t, int, int, const PerPair*, const double2*, const int*,
                                 const int*, double2*);
 void launch_find_peaks(hipStream_t, int, const float*, long long, float*, int, int, int, int, int,
                        double*, int*);
 int find_peaks_max_window();
 void launch_per_select(hipStream_t, int, int, int, const PerPair*, const double2*, const double2*,
-                       const PlaneCand*, double2*, long long, PerPeak*);
+                       const PlaneCand*, const double*, double2*, long long, PerPeak*);
 void launch_per_refine(hipStream_t, int, int, const PerPair*, const PerGroup*, const int*,
                        const double*, const double*, const PerPeak*, int, int, NearRec*, int*,
                        int*, int*, double*, double*, PerResult*);
@@ -1571,6 +1571,7 @@ struct fo_per_batch {
   double *pos1 = nullptr, *pos2 = nullptr, *X1out = nullptr, *X2out = nullptr;
   double2 *Cprod = nullptr, *C1 = nullptr, *C2 = nullptr, *scr = nullptr;
   PlaneCand* cand = nullptr;
+  double* abound = nullptr;  // per pair: sum |C|
   PerPeak* peaks = nullptr;
   PerResult* res = nullptr;
   int *perm = nullptr, *saveperm = nullptr, *rowsol = nullptr;
@@ -1581,7 +1582,8 @@ struct fo_per_batch {
   hipEvent_t ev[5] = {};
   bool ev_made = false;
   struct {
-    size_t pd, grp, at, p1, p2, x1, x2, cp, c1, c2, cand, pk, res, perm, sp, rs, scr, grid, cgrid;
+    size_t pd, grp, at, p1, p2, x1, x2, cp, c1, c2, cand, ab, pk, res, perm, sp, rs, scr, grid,
+        cgrid;
   } off{};
   bool keepc = false;
   bool own_mem = false, own_stream = false;
@@ -1613,11 +1615,11 @@ static int per_enqueue(fo_per_batch* b, int stages) {
   }
   mark(1);
   if (stages & FO_PSTAGE_GRID) {
-    launch_per_plane(s, b->P, b->nk, b->F, b->pd, b->Cprod, b->tw->tw32, b->cand, b->grid,
-                     b->cgrid);
+    launch_per_plane(s, b->P, b->nk, b->F, b->pd, b->Cprod, b->tw->tw32, b->cand, b->abound,
+                     b->grid, b->cgrid);
     mark(2);
-    launch_per_select(s, b->P, b->nk, b->F, b->pd, b->Cprod, b->tw->tw64, b->cand, b->scr,
-                      b->scr_stride, b->peaks);
+    launch_per_select(s, b->P, b->nk, b->F, b->pd, b->Cprod, b->tw->tw64, b->cand, b->abound,
+                      b->scr, b->scr_stride, b->peaks);
   } else {
     mark(2);
   }
@@ -1717,6 +1719,7 @@ int per_batch_plan(fo_context* c, const fo_per_batch_desc* d, fo_per_batch** out
   o.c1 = b->keepc ? lay.add<double2>((size_t)std::max(gsum, 1) * b->cube) : 0;
   o.c2 = b->keepc ? lay.add<double2>((size_t)std::max(gsum, 1) * b->cube) : 0;
   o.cand = lay.add<PlaneCand>((size_t)b->P * b->F);
+  o.ab = lay.add<double>(b->P);
   o.pk = lay.add<PerPeak>(b->P);
   o.res = lay.add<PerResult>(b->P);
   o.perm = lay.add<int>(Ntot);
@@ -1758,6 +1761,7 @@ int per_batch_bind(fo_per_batch* b, void* mem, hipStream_t stream) {
   b->C1 = b->keepc ? (double2*)(B + o.c1) : nullptr;
   b->C2 = b->keepc ? (double2*)(B + o.c2) : nullptr;
   b->cand = (PlaneCand*)(B + o.cand);
+  b->abound = (double*)(B + o.ab);
   b->peaks = (PerPeak*)(B + o.pk);
   b->res = (PerResult*)(B + o.res);
   b->perm = (int*)(B + o.perm);

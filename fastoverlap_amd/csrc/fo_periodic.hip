@@ -272,13 +272,24 @@ __global__ void k_per_product_indexed(const PerPair* __restrict__ pd, int nk,
   }
 }
 
+// sum |C| of one pair, for the selection's error bound, by the workgroup of
+// 256 threads that takes the pair's first plane
+FO_DEV void product_abound(const double2* C, int cube, double* out) {
+  __shared__ double sa[4];
+  double v = 0.0;
+#pragma unroll 8
+  for (int e = threadIdx.x; e < cube; e += 256) v += sqrt(C[e].x * C[e].x + C[e].y * C[e].y);
+  v = block_sum(v, sa);
+  if (threadIdx.x == 0) *out = v;
+}
+
 // |f(x,y,z)|, f = sum_{a,b,c} C[a,b,c] e^{-2 pi i (a x + b y + c z)/F}, for
 // one x-plane per workgroup (numpy fftn with C at the array corner,
 // fastoverlap/periodicAlignment.py:439-440).
 __global__ void __launch_bounds__(256) k_per_plane(
     const PerPair* __restrict__ pd, int nk, int F, const double2* __restrict__ Cprod,
-    const float2* __restrict__ twg, PlaneCand* __restrict__ cand, float* __restrict__ grid,
-    float2* __restrict__ cgrid) {
+    const float2* __restrict__ twg, PlaneCand* __restrict__ cand, double* __restrict__ abound,
+    float* __restrict__ grid, float2* __restrict__ cgrid) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int NB = 2 * nk + 1;
   const int x = blockIdx.x, p = blockIdx.y, t = threadIdx.x, bd = blockDim.x;
@@ -368,6 +379,7 @@ __global__ void __launch_bounds__(256) k_per_plane(
   out.rest[0] = fmaxf(fifth, dm);
   for (int r = 1; r < kCandPerPlane; ++r) out.rest[r] = -INFINITY;
   if (t == 0) cand[(long long)p * F + x] = out;
+  if (x == 0) product_abound(C, NB * NB * NB, abound + p);
 }
 
 struct PerGridCtx {
@@ -376,20 +388,80 @@ struct PerGridCtx {
   const double2* tw64;
 };
 
-// FP64 |f| at one grid point (workgroup cooperative)
-FO_DEV double per_eval64(const PerGridCtx& c, int x, int y, int z, double* red) {
-  const int NB = c.NB, F = c.F;
-  double sx = 0.0, sy = 0.0;
-  for (int e = threadIdx.x; e < NB * NB * NB; e += blockDim.x) {
-    const int a = e / (NB * NB), b = (e / NB) % NB, cc = e % NB;
-    const int ph = (int)(((long long)a * x + (long long)b * y + (long long)cc * z) % F);
-    const double2 v = cmul(c.C[e], c.tw64[ph]);
-    sx += v.x;
-    sy += v.y;
+// FP64 |f| at up to kSelPoints grid points with at most three x and five
+// (x, y) values among them, in one pass over the product: H[x][b, c] =
+// sum_a C w^{a x} (XB of the x values a pass, coalesced over (b, c)), then
+// G[x, y][c] = sum_b H w^{b y} and the points' sums over c, a wavefront each.
+// tw: the F twiddles in LDS; H: [XB][NB^2], G: [kSelPairs][NB].  Every thread
+// must call it (kSelThreads).
+constexpr int kSelThreads = 512;
+constexpr int kSelPoints = 7, kSelPairs = 5, kSelXs = 3;
+struct SelPoints {
+  int np, nxy, nx;
+  int x[kSelXs];                       // distinct x
+  int xy_x[kSelPairs], xy_y[kSelPairs];  // (index into x, y)
+  int pt_xy[kSelPoints], pt_z[kSelPoints];
+  double val[kSelPoints];
+};
+template <int XB>
+FO_DEV void per_eval64(const PerGridCtx& c, SelPoints& s, const double2* tw, double2* H,
+                       double2* G) {
+  const int NB = c.NB, F = c.F, plane = NB * NB, t = threadIdx.x;
+  for (int x0 = 0; x0 < s.nx; x0 += XB) {
+    int xs[XB];
+#pragma unroll
+    for (int q = 0; q < XB; ++q) xs[q] = s.x[min(x0 + q, s.nx - 1)];
+    for (int e = t; e < plane; e += kSelThreads) {
+      double2 acc[XB];
+      int ph[XB];
+#pragma unroll
+      for (int q = 0; q < XB; ++q) {
+        acc[q] = make_double2(0.0, 0.0);
+        ph[q] = 0;
+      }
+#pragma unroll 8
+      for (int a = 0; a < NB; ++a) {
+        const double2 v = c.C[(long long)a * plane + e];
+#pragma unroll
+        for (int q = 0; q < XB; ++q) {
+          acc[q] = cadd(acc[q], cmul(v, tw[ph[q]]));
+          ph[q] += xs[q];
+          if (ph[q] >= F) ph[q] -= F;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < XB; ++q) H[q * plane + e] = acc[q];
+    }
+    __syncthreads();
+    for (int e = t; e < s.nxy * NB; e += kSelThreads) {
+      const int k = e / NB, cc = e - k * NB, q = s.xy_x[k] - x0, y = s.xy_y[k];
+      if (q < 0 || q >= XB) continue;
+      double2 acc = make_double2(0.0, 0.0);
+      int ph = 0;
+#pragma unroll 4
+      for (int b = 0; b < NB; ++b) {
+        acc = cadd(acc, cmul(H[q * plane + b * NB + cc], tw[ph]));
+        ph += y;
+        if (ph >= F) ph -= F;
+      }
+      G[e] = acc;
+    }
+    __syncthreads();
   }
-  sx = block_sum(sx, red);
-  sy = block_sum(sy, red);
-  return sqrt(sx * sx + sy * sy);
+  const int w = t >> 6, ln = t & 63;
+  if (w < s.np) {
+    // NB <= 63: one term a lane
+    double2 v = make_double2(0.0, 0.0);
+    if (ln < NB) v = cmul(G[s.pt_xy[w] * NB + ln], tw[(ln * s.pt_z[w]) % F]);
+    const double vx = wave_sum(v.x), vy = wave_sum(v.y);
+    if (ln == 0) s.val[w] = sqrt(vx * vx + vy * vy);
+  }
+  __syncthreads();
+}
+// doubles of LDS: twiddles, H, G
+static inline size_t per_select_smem(int nk, int F) {
+  const size_t NB = 2 * (size_t)nk + 1, xb = nk <= 15 ? 3 : 1;
+  return sizeof(double2) * (F + xb * NB * NB + kSelPairs * NB);
 }
 
 FO_DEV void per_plane64(const PerGridCtx& c, int x, double2* Hg, double2* Gg, double* red,
@@ -431,10 +503,19 @@ FO_DEV void per_plane64(const PerGridCtx& c, int x, double2* Hg, double2* Gg, do
 // twiddles and of three DFT passes of NB terms each stays below
 // (4 NB + 32) 2^-24 A.  Candidates within 2 delta of the FP32 maximum are
 // re-evaluated in FP64.
-__global__ void __launch_bounds__(256) k_per_select(
+// The product is read once for the argmax and its six neighbours when a single
+// candidate is listed (the common case); as seven separate sums over the cube
+// and one for A, each a chain of loads, this took 61 us for one pair of nk = 8
+// and 255 us for 24 of nk = 14, now 11 and 30.  Bound: load latency of one
+// workgroup per pair.
+template <int XB>
+__global__ void __launch_bounds__(kSelThreads) k_per_select(
     const PerPair* __restrict__ pd, int nk, int F, const double2* __restrict__ Cprod,
     const double2* __restrict__ tw64, const PlaneCand* __restrict__ cand,
-    double2* __restrict__ scratch, long long scratch_stride, PerPeak* __restrict__ peaks) {
+    const double* __restrict__ abound, double2* __restrict__ scratch, long long scratch_stride,
+    PerPeak* __restrict__ peaks) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ SelPoints sp;
   __shared__ double red[16];
   __shared__ int redi[16];
   __shared__ float rv[16];
@@ -450,15 +531,17 @@ __global__ void __launch_bounds__(256) k_per_select(
   c.F = F;
   c.C = Cprod + d.c_off;
   c.tw64 = tw64;
+  double2* tw = (double2*)smem;
+  double2* H = tw + F;
+  double2* G = H + XB * NB * NB;
+  for (int q = t; q < F; q += kSelThreads) tw[q] = tw64[q];
   const PlaneCand* pc = cand + (long long)p * F;
   float mv = -INFINITY;
   int mi = 0x7fffffff;
   for (int b = t; b < F; b += blockDim.x)
     for (int r = 0; r < kCandPerPlane; ++r) argmax_merge(mv, mi, pc[b].val[r], pc[b].idx[r]);
   block_argmax(mv, mi, rv, ri);
-  double A = 0.0;
-  for (int e = t; e < NB * NB * NB; e += blockDim.x) A += hypot(c.C[e].x, c.C[e].y);
-  A = block_sum(A, red);
+  const double A = abound[p];
   const double delta = (4.0 * NB + 32.0) * 5.9604644775390625e-08 * A;
   const double thr = (double)mv - 2.0 * delta;
   if (t == 0) {
@@ -515,7 +598,10 @@ __global__ void __launch_bounds__(256) k_per_select(
       second = v;
     }
   };
-  if (cand_overflow) {
+  const bool merged = !cand_overflow && novf == 0 && ncand == 1;
+  if (merged) {
+    besti = s_cand[0];
+  } else if (cand_overflow) {
     for (int x = 0; x < F; ++x) {
       double v;
       int i;
@@ -525,7 +611,18 @@ __global__ void __launch_bounds__(256) k_per_select(
   } else {
     for (int q = 0; q < ncand; ++q) {
       const int f = s_cand[q];
-      take(per_eval64(c, f / (F * F), (f / F) % F, f % F, red), f);
+      if (t == 0) {
+        sp.np = sp.nxy = sp.nx = 1;
+        sp.x[0] = f / (F * F);
+        sp.xy_x[0] = 0;
+        sp.xy_y[0] = (f / F) % F;
+        sp.pt_xy[0] = 0;
+        sp.pt_z[0] = f % F;
+      }
+      __syncthreads();
+      per_eval64<XB>(c, sp, tw, H, G);
+      take(sp.val[0], f);
+      __syncthreads();
     }
     for (int q = 0; q < novf; ++q) {
       double v;
@@ -535,13 +632,38 @@ __global__ void __launch_bounds__(256) k_per_select(
     }
   }
   const int ind[3] = {besti / (F * F), (besti / F) % F, besti % F};
+  // the argmax and its neighbours: points 0, then (+1, -1) per axis
+  if (t == 0) {
+    // (no listed point, as for a product that is not a number: ind is out of
+    // range and is folded back)
+    const int x0 = ind[0] % F, y0 = ind[1] % F, z0 = ind[2] % F;
+    const int xp = (ind[0] + 1) % F, xm = (ind[0] + F - 1) % F;
+    const int yp = (ind[1] + 1) % F, ym = (ind[1] + F - 1) % F;
+    const int zp = (ind[2] + 1) % F, zm = (ind[2] + F - 1) % F;
+    sp.np = kSelPoints;
+    sp.nxy = kSelPairs;
+    sp.nx = kSelXs;
+    sp.x[0] = x0;
+    sp.x[1] = xp;
+    sp.x[2] = xm;
+    const int ys[kSelPairs] = {y0, y0, y0, yp, ym};
+    const int xy[kSelPoints] = {0, 1, 2, 3, 4, 0, 0};
+    const int zs[kSelPoints] = {z0, z0, z0, z0, z0, zp, zm};
+    for (int q = 0; q < kSelPairs; ++q) {
+      sp.xy_x[q] = q < 3 ? q : 0;
+      sp.xy_y[q] = ys[q];
+    }
+    for (int q = 0; q < kSelPoints; ++q) {
+      sp.pt_xy[q] = xy[q];
+      sp.pt_z[q] = zs[q];
+    }
+  }
+  __syncthreads();
+  per_eval64<XB>(c, sp, tw, H, G);
+  if (merged) best = sp.val[0];
   double off[3];
   for (int ax = 0; ax < 3; ++ax) {
-    int ip[3] = {ind[0], ind[1], ind[2]}, im[3] = {ind[0], ind[1], ind[2]};
-    ip[ax] = (ind[ax] + 1) % F;
-    im[ax] = (ind[ax] + F - 1) % F;
-    const double y1 = per_eval64(c, ip[0], ip[1], ip[2], red);
-    const double y3 = per_eval64(c, im[0], im[1], im[2], red);
+    const double y1 = sp.val[1 + 2 * ax], y3 = sp.val[2 + 2 * ax];
     off[ax] = (y3 - y1) / (2.0 * (2.0 * best - y1 - y3));
   }
   if (t == 0) {
@@ -864,10 +986,10 @@ size_t per_plane_smem(int nk, int F) {
 }
 
 void launch_per_plane(hipStream_t s, int P, int nk, int F, const PerPair* pd,
-                      const double2* Cprod, const float2* tw32, PlaneCand* cand, float* grid,
-                      float2* cgrid) {
+                      const double2* Cprod, const float2* tw32, PlaneCand* cand, double* abound,
+                      float* grid, float2* cgrid) {
   hipLaunchKernelGGL(k_per_plane, dim3(F, P), dim3(256), per_plane_smem(nk, F), s, pd, nk, F,
-                     Cprod, tw32, cand, grid, cgrid);
+                     Cprod, tw32, cand, abound, grid, cgrid);
 }
 
 void launch_per_product_indexed(hipStream_t s, int P, int nk, const PerPair* pd,
@@ -880,9 +1002,16 @@ void launch_per_product_indexed(hipStream_t s, int P, int nk, const PerPair* pd,
 
 void launch_per_select(hipStream_t s, int P, int nk, int F, const PerPair* pd,
                        const double2* Cprod, const double2* tw64, const PlaneCand* cand,
-                       double2* scratch, long long scratch_stride, PerPeak* peaks) {
-  hipLaunchKernelGGL(k_per_select, dim3(P), dim3(256), 0, s, pd, nk, F, Cprod, tw64, cand,
-                     scratch, scratch_stride, peaks);
+                       const double* abound, double2* scratch, long long scratch_stride,
+                       PerPeak* peaks) {
+  // three x values a pass while their sums over a fit LDS (NB <= 31: 46 KB)
+  const size_t sm = per_select_smem(nk, F);
+  if (nk <= 15)
+    hipLaunchKernelGGL(k_per_select<3>, dim3(P), dim3(kSelThreads), sm, s, pd, nk, F, Cprod, tw64,
+                       cand, abound, scratch, scratch_stride, peaks);
+  else
+    hipLaunchKernelGGL(k_per_select<1>, dim3(P), dim3(kSelThreads), sm, s, pd, nk, F, Cprod, tw64,
+                       cand, abound, scratch, scratch_stride, peaks);
 }
 
 void launch_per_refine(hipStream_t s, int P, int lap_nmax, const PerPair* pd, const PerGroup* grp,

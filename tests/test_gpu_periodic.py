@@ -247,3 +247,40 @@ def test_refine_nearest_rows_and_assignment(gpu, sizes, noise, niter):
     tol = 8 * N * box.max() * 2.0 ** -53
     np.testing.assert_allclose(r["disp"][0], rd, rtol=0, atol=tol)
     assert abs(r["dist"][0] - dist) <= tol
+
+
+@pytest.mark.parametrize("nk,F,mirror", [(1, 4, False), (4, 9, True), (15, 31, False),
+                                         (15, 64, True), (16, 33, False), (16, 36, True),
+                                         (31, 63, True)])
+def test_selected_peak_and_neighbours(gpu, nk, F, mirror):
+    """The selected grid maximum, its value and the interpolated displacement
+    against a 64-bit FFT, on both sides of the k-cube where the selection
+    evaluates one x a pass (nk 15 / 16); inversion-symmetric structures
+    (mirror) give pairs of equal maxima, evaluated one by one."""
+    say(f"case: nk={nk} F={F} mirror={mirror}")
+    rng = np.random.default_rng(nk * F)
+    box = np.array([4.0, 4.4, 3.7])
+    x, y = (rng.random((20, 3)) - 0.5 for _ in range(2))
+    if mirror:
+        x, y = np.concatenate([x, -x]), np.concatenate([y, -y])
+    x, y = x * box, y * box
+    N = len(x)
+    with PeriodicBatch([N], box, 0.25, nk, F) as b:
+        b.set_positions(x, y)
+        b.run(_lib.PSTAGE_SF | _lib.PSTAGE_GRID)
+        C, pk = b.product()[0], b.peaks()
+    f = np.abs(np.fft.fftn(C, (F, F, F)))
+    i = pk["ind"][0]
+    # an FFT of F points a side: below 16 log2(F) roundings of sum |C|
+    tol = 16 * np.log2(F) * 2.0 ** -53 * np.abs(C).sum()
+    assert f[tuple(i)] >= f.max() - tol
+    assert abs(pk["value"][0] - f.max()) <= tol
+    disp = np.zeros(3)
+    for ax in range(3):
+        up, dn = i.copy(), i.copy()
+        up[ax], dn[ax] = (i[ax] + 1) % F, (i[ax] - 1) % F
+        y1, y2, y3 = f[tuple(up)], f[tuple(i)], f[tuple(dn)]
+        curv = 2 * (2 * y2 - y1 - y3)
+        disp[ax] = (i[ax] - (y3 - y1) / curv) * box[ax] / F
+        # numerator and denominator are each off by a few tol
+        assert abs(pk["disp"][0, ax] - disp[ax]) <= 16 * tol / abs(curv) * box[ax] / F + 1e-14

@@ -74,15 +74,16 @@ void launch_per_sf(hipStream_t, int, int, const PerPair*, const PerGroup*, const
 void launch_per_product(hipStream_t, int, int, const PerPair*, const double2*, const double2*,
                         double2*);
 size_t per_plane_smem(int, int);
-void launch_per_plane(hipStream_t, int, int, int, const PerPair*, const double2*, const float2*,
-                      PlaneCand*, double*, float*, float2*);
+void launch_per_plane(hipStream_t, int, int, int, int, const PerPair*, const double2*,
+                      const float2*, PlaneCand*, double*, float*, float2*);
+double per_plane_delta(int nk, int real);
 void launch_per_product_indexed(hipStream_t, int, int, const PerPair*, const double2*, const int*,
                                 const int*, double2*);
 void launch_find_peaks(hipStream_t, int, const float*, long long, float*, int, int, int, int, int,
                        double*, int*);
 int find_peaks_max_window();
 void launch_per_select(hipStream_t, int, int, int, const PerPair*, const double2*, const double2*,
-                       const PlaneCand*, const double*, double2*, long long, PerPeak*);
+                       const PlaneCand*, const double*, double, double2*, long long, PerPeak*);
 void launch_per_refine(hipStream_t, int, int, const PerPair*, const PerGroup*, const int*,
                        const double*, const double*, const PerPeak*, int, int, NearRec*, int*,
                        int*, int*, double*, double*, PerResult*);
@@ -1571,7 +1572,7 @@ struct fo_per_batch {
   double *pos1 = nullptr, *pos2 = nullptr, *X1out = nullptr, *X2out = nullptr;
   double2 *Cprod = nullptr, *C1 = nullptr, *C2 = nullptr, *scr = nullptr;
   PlaneCand* cand = nullptr;
-  double* abound = nullptr;  // per pair: sum |C|
+  double* abound = nullptr;  // per pair and slice a: sum |C|
   PerPeak* peaks = nullptr;
   PerResult* res = nullptr;
   int *perm = nullptr, *saveperm = nullptr, *rowsol = nullptr;
@@ -1615,11 +1616,13 @@ static int per_enqueue(fo_per_batch* b, int stages) {
   }
   mark(1);
   if (stages & FO_PSTAGE_GRID) {
-    launch_per_plane(s, b->P, b->nk, b->F, b->pd, b->Cprod, b->tw->tw32, b->cand, b->abound,
+    // the structure factors' product is Hermitian; supplied coefficients need not be
+    const int real = (b->flags & (FO_PER_INPUT_COEFFS | FO_PER_KEEP_FFT)) ? 0 : 1;
+    launch_per_plane(s, b->P, b->nk, b->F, real, b->pd, b->Cprod, b->tw->tw32, b->cand, b->abound,
                      b->grid, b->cgrid);
     mark(2);
     launch_per_select(s, b->P, b->nk, b->F, b->pd, b->Cprod, b->tw->tw64, b->cand, b->abound,
-                      b->scr, b->scr_stride, b->peaks);
+                      per_plane_delta(b->nk, real), b->scr, b->scr_stride, b->peaks);
   } else {
     mark(2);
   }
@@ -1719,7 +1722,7 @@ int per_batch_plan(fo_context* c, const fo_per_batch_desc* d, fo_per_batch** out
   o.c1 = b->keepc ? lay.add<double2>((size_t)std::max(gsum, 1) * b->cube) : 0;
   o.c2 = b->keepc ? lay.add<double2>((size_t)std::max(gsum, 1) * b->cube) : 0;
   o.cand = lay.add<PlaneCand>((size_t)b->P * b->F);
-  o.ab = lay.add<double>(b->P);
+  o.ab = lay.add<double>((size_t)b->P * NB);
   o.pk = lay.add<PerPeak>(b->P);
   o.res = lay.add<PerResult>(b->P);
   o.perm = lay.add<int>(Ntot);

@@ -193,4 +193,59 @@ FO_DEV void argmin_merge(double& v, int& i, double ov, int oi) {
   }
 }
 
+// DPP row shifts (within rows of 16 lanes): row_shl:S gives lane i the value
+// of lane i + S, row_shr:S that of lane i - S.
+template <int CTRL>
+FO_DEV float dpp_mov(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+
+// Records (largest value v, its flat index i, largest of the other values
+// s): larger value first, ties to the smaller index; the loser's largest
+// value joins the others (so s counts a repeated maximum).
+FO_DEV void top2_merge(float& v, int& i, float& s, float ov, int oi, float os) {
+  const bool take = ov > v || (ov == v && oi < i);
+  s = fmaxf(fmaxf(s, os), take ? v : ov);
+  v = take ? ov : v;
+  i = take ? oi : i;
+}
+// One butterfly of NO (v, i, s) records over a wavefront: inside each row of
+// 16 lanes by DPP (quad_perm [1,0,3,2], quad_perm [2,3,0,1], row_half_mirror,
+// row_mirror), the records interleaved, then the four row results through
+// readlane.  Every lane must be active and gets the wavefront's records.
+template <int CTRL, int NO>
+FO_DEV void top2_dpp_step(float (&v)[NO], int (&i)[NO], float (&s)[NO]) {
+  float ov[NO], os[NO];
+  int oi[NO];
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    ov[o] = dpp_mov<CTRL>(v[o]);
+    oi[o] = __builtin_amdgcn_update_dpp(0, i[o], CTRL, 0xf, 0xf, true);
+    os[o] = dpp_mov<CTRL>(s[o]);
+  }
+#pragma unroll
+  for (int o = 0; o < NO; ++o) top2_merge(v[o], i[o], s[o], ov[o], oi[o], os[o]);
+}
+template <int NO>
+FO_DEV void wave_top2(float (&v)[NO], int (&i)[NO], float (&s)[NO]) {
+  top2_dpp_step<0xB1>(v, i, s);
+  top2_dpp_step<0x4E>(v, i, s);
+  top2_dpp_step<0x141>(v, i, s);
+  top2_dpp_step<0x140>(v, i, s);
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    float rv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[o]), 0));
+    float rs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[o]), 0));
+    int ri = __builtin_amdgcn_readlane(i[o], 0);
+#pragma unroll
+    for (int r = 16; r < 64; r += 16)
+      top2_merge(rv, ri, rs, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[o]), r)),
+                 __builtin_amdgcn_readlane(i[o], r),
+                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[o]), r)));
+    v[o] = rv;
+    i[o] = ri;
+    s[o] = rs;
+  }
+}
+
 }  // namespace fo

@@ -272,20 +272,23 @@ __global__ void k_per_product_indexed(const PerPair* __restrict__ pd, int nk,
   }
 }
 
-// sum |C| of one pair, for the selection's error bound, by the workgroup of
-// 256 threads that takes the pair's first plane
-FO_DEV void product_abound(const double2* C, int cube, double* out) {
+// sum of |C| over the slice a = x of the product (workgroups x < NB), for the
+// selection's error bound
+FO_DEV void slice_abound(const double2* C, int x, int NB, double* out) {
   __shared__ double sa[4];
+  if (x >= NB) return;
+  const double2* S = C + (long long)x * NB * NB;
   double v = 0.0;
-#pragma unroll 8
-  for (int e = threadIdx.x; e < cube; e += 256) v += sqrt(C[e].x * C[e].x + C[e].y * C[e].y);
+  for (int e = threadIdx.x; e < NB * NB; e += 256) v += sqrt(S[e].x * S[e].x + S[e].y * S[e].y);
   v = block_sum(v, sa);
-  if (threadIdx.x == 0) *out = v;
+  if (threadIdx.x == 0) out[x] = v;
 }
 
 // |f(x,y,z)|, f = sum_{a,b,c} C[a,b,c] e^{-2 pi i (a x + b y + c z)/F}, for
 // one x-plane per workgroup (numpy fftn with C at the array corner,
-// fastoverlap/periodicAlignment.py:439-440).
+// fastoverlap/periodicAlignment.py:439-440).  For products that need not be
+// Hermitian (supplied coefficients) and where f itself is kept; k_per_plane_real
+// serves the others.
 __global__ void __launch_bounds__(256) k_per_plane(
     const PerPair* __restrict__ pd, int nk, int F, const double2* __restrict__ Cprod,
     const float2* __restrict__ twg, PlaneCand* __restrict__ cand, double* __restrict__ abound,
@@ -379,7 +382,165 @@ __global__ void __launch_bounds__(256) k_per_plane(
   out.rest[0] = fmaxf(fifth, dm);
   for (int r = 1; r < kCandPerPlane; ++r) out.rest[r] = -INFINITY;
   if (t == 0) cand[(long long)p * F + x] = out;
-  if (x == 0) product_abound(C, NB * NB * NB, abound + p);
+  slice_abound(C, x, NB, abound + (long long)p * NB);
+}
+
+// The same planes for a Hermitian product (structure factors of real
+// densities): up to a phase f is the real sum
+//   g(x,y,z) = sum_{|a|,|b|,|c| <= nk} C[a,b,c] e^{-2 pi i (a x + b y + c z)/F}.
+// Per plane x, with the real basis phi_0 = 1, phi_{2m-1} = cos m, phi_{2m} =
+// sin m over b and over c (NB functions each):
+//   1. H[b,c] = sum_a C w^{a x} for c >= 0 on the vector units, folded over
+//      +-b into the real coefficients R[r over c][k over b] (LDS);
+//   2. G[r][y] = sum_k R[r][k] phi_k(y)  and
+//   3. g[y][z] = sum_r G[r][y] phi_r(z)  on v_mfma_f32_16x16x4f32: a
+//      wavefront owns 16 columns y, and register i of lane group q, row
+//      r = 4 q + i of a result tile of 2, is the A operand of 3 at the step
+//      that takes the rows 4 q + i, q = 0..3 (any order of r will do).
+// phi: (NB + 1) rows of F in LDS, the last one zero (padding of r and k).
+// XP planes share the table; their products read C through the caches.
+// Rounding: the folds and the three sums of at most NB terms stay below
+// real_plane_delta(NB) sum |C|: stage 1 (2 NB + 4) u sum|C|, times sqrt 2 for each
+// of |cos| + |sin| in 2 and 3, whose own NB roundings add 3 NB u: 7.5 NB + 19
+// units u = 2^-24 in all.
+// Against the complex transform on the vector units, which formed every F^2 NB
+// term of a plane: 259 -> 75 us for 128 pairs of nk = 8, F = 64, 111 -> 36 us for
+// 24 of nk = 14, F = 60, 20 -> 12 us for one pair.  Bound: stage 1 (two FP64
+// products read, four conversions and eight FP32 operations a term) and the
+// candidate test of every value.
+constexpr int kPlaneXP = 4;
+typedef float v4f __attribute__((ext_vector_type(4)));
+FO_HD double real_plane_delta(int NB) { return (9.0 * NB + 64.0) * 5.9604644775390625e-08; }
+FO_HD int real_plane_fs(int F) { return ((F + 15) & ~15) + 4; }  // row stride of phi
+FO_HD int real_plane_ks(int NB) { return ((NB + 3) & ~3) + 1; }  // row stride of R
+
+template <int NT>
+__global__ void __launch_bounds__(256) k_per_plane_real(
+    const PerPair* __restrict__ pd, int nk, int F, int XP, const double2* __restrict__ Cprod,
+    const float2* __restrict__ twg, PlaneCand* __restrict__ cand, double* __restrict__ abound,
+    float* __restrict__ grid) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int NB = 2 * nk + 1, FS = real_plane_fs(F), KS = real_plane_ks(NB);
+  const int p = blockIdx.y, t = threadIdx.x, x0 = blockIdx.x * XP;
+  const PerPair d = pd[p];
+  float2* tw = (float2*)smem;         // [F], e^{-2 pi i j / F}
+  float* phi = (float*)(tw + F);      // [NB + 1][FS]
+  float* R = phi + (NB + 1) * FS;     // [XP][NB][KS]
+  for (int k = t; k < F; k += 256) tw[k] = twg[k];
+  __syncthreads();
+  const double2* C = Cprod + d.c_off;
+  const int nb = nk + 1, plane = NB * NB;
+  for (int e = t; e < XP * nb * nb; e += 256) {
+    const int xi = e / (nb * nb), r = e - xi * nb * nb, b = r / nb, c = r - b * nb;
+    const int x = min(x0 + xi, F - 1);
+    const double2* Cp = C + (nk + b) * NB + nk + c;
+    const double2* Cm = C + (nk - b) * NB + nk + c;
+    float2 hp = make_float2(0.f, 0.f), hm = hp;
+    int ph = (F - nk * x % F) % F;  // (-nk x) mod F
+#pragma unroll 4
+    for (int a = 0; a < NB; ++a) {
+      const double2 u = Cp[(long long)a * plane], v = Cm[(long long)a * plane];
+      const float2 w = tw[ph];
+      const float ux = (float)u.x, uy = (float)u.y, vx = (float)v.x, vy = (float)v.y;
+      hp.x += ux * w.x - uy * w.y;
+      hp.y += ux * w.y + uy * w.x;
+      hm.x += vx * w.x - vy * w.y;
+      hm.y += vx * w.y + vy * w.x;
+      ph += x;
+      if (ph >= F) ph -= F;
+    }
+    const float sc = c ? 2.f : 1.f;  // the terms of -c
+    float* re = R + ((long long)xi * NB + (c ? 2 * c - 1 : 0)) * KS;
+    float* im = re + KS;  // c > 0 only
+    if (b == 0) {
+      re[0] = sc * hp.x;
+      if (c) im[0] = sc * hp.y;
+    } else {
+      re[2 * b - 1] = sc * (hp.x + hm.x);
+      re[2 * b] = sc * (hp.y - hm.y);
+      if (c) {
+        im[2 * b - 1] = sc * (hp.y + hm.y);
+        im[2 * b] = -sc * (hp.x - hm.x);
+      }
+    }
+  }
+  for (int e = t; e < XP * NB * (KS - 1 - NB); e += 256) {
+    const int row = e / (KS - 1 - NB);
+    R[row * KS + NB + e - row * (KS - 1 - NB)] = 0.f;
+  }
+  for (int e = t; e < (NB + 1) * FS; e += 256) {
+    const int k = e / FS, j = e - k * FS;
+    float v = 0.f;
+    if (k < NB && j < F) {
+      const float2 w = tw[((k + 1) >> 1) * j % F];
+      v = (k & 1) || k == 0 ? w.x : -w.y;
+    }
+    phi[e] = v;
+  }
+  __syncthreads();
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6), ln = t & 63, col = ln & 15, q = ln >> 4;
+  const int nyt = (F + 15) >> 4, ksteps = (NB + 3) >> 2;
+  // this lane's rows of phi in stage 3, register i of tile tt: 16 tt + 4 q + i
+  for (int xi = 0; xi < XP; ++xi) {
+    const int x = x0 + xi;
+    if (x >= F) break;  // uniform
+    const float* Rx = R + (long long)xi * NB * KS;
+    float bv = -INFINITY, dm = -INFINITY;
+    int bi = 0x7fffffff;
+    for (int yt = wv; yt < nyt; yt += 4) {
+      v4f G[NT];
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) G[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < ksteps; ++s) {
+        const int k = 4 * s + q;
+        const float b = phi[min(k, NB) * FS + 16 * yt + col];
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) {
+          const float a = Rx[min(16 * tt + col, NB - 1) * KS + k];
+          G[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, G[tt], 0, 0, 0);
+        }
+      }
+      for (int zt = 0; zt < nyt; ++zt) {
+        const float* pz = phi + 16 * zt + col;
+        v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (16 * tt + i >= NB) continue;  // uniform
+            const float b = pz[min(16 * tt + 4 * q + i, NB) * FS];
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(G[tt][i], b, acc, 0, 0, 0);
+          }
+        const int z = 16 * zt + col;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int y = 16 * yt + 4 * q + i;
+          const float val = fabsf(acc[i]);
+          if (y < F && z < F) {
+            const int flat = (x * F + y) * F + z;
+            if (grid) grid[(long long)p * F * F * F + flat] = val;
+            if (val > bv) {
+              dm = fmaxf(dm, bv);
+              bv = val;
+              bi = flat;
+            } else {
+              dm = fmaxf(dm, val);
+            }
+          }
+        }
+      }
+    }
+    float v[1] = {bv}, r[1] = {dm};
+    int id[1] = {bi};
+    wave_top2(v, id, r);
+    if (ln == 0) {
+      PlaneCand* o = cand + (long long)p * F + x;
+      o->val[wv] = v[0];
+      o->idx[wv] = id[0];
+      o->rest[wv] = r[0];
+    }
+  }
+  for (int xi = 0; xi < XP; ++xi) slice_abound(C, x0 + xi, NB, abound + (long long)p * NB);
 }
 
 struct PerGridCtx {
@@ -458,39 +619,67 @@ FO_DEV void per_eval64(const PerGridCtx& c, SelPoints& s, const double2* tw, dou
   }
   __syncthreads();
 }
-// doubles of LDS: twiddles, H, G
+// LDS: twiddles, then H and G of the points or of a whole plane
+FO_HD size_t sel_points_lds(int nk) {
+  const size_t NB = 2 * (size_t)nk + 1, xb = nk <= 15 ? kSelXs : 1;
+  return sizeof(double2) * (xb * NB * NB + kSelPairs * NB);
+}
+FO_HD size_t sel_plane_lds(int nk, int F) {
+  const size_t NB = 2 * (size_t)nk + 1;
+  return sizeof(double2) * (NB * NB + NB * F);
+}
+constexpr size_t kSelLds = 64 * 1024;  // two workgroups a CU
 static inline size_t per_select_smem(int nk, int F) {
-  const size_t NB = 2 * (size_t)nk + 1, xb = nk <= 15 ? 3 : 1;
-  return sizeof(double2) * (F + xb * NB * NB + kSelPairs * NB);
+  const size_t pt = sel_points_lds(nk), pl = sel_plane_lds(nk, F);
+  return sizeof(double2) * F + std::max(pt, pl <= kSelLds ? pl : 0);
 }
 
-FO_DEV void per_plane64(const PerGridCtx& c, int x, double2* Hg, double2* Gg, double* red,
-                        int* redi, double& bestv, int& besti) {
-  const int NB = c.NB, F = c.F;
-  for (int e = threadIdx.x; e < NB * NB; e += blockDim.x) {
+// FP64 |f| over a whole plane x; returns its argmax (ties -> lower flat index).
+// H: [NB^2], G: [NB][F], in LDS when they fit (sel_plane_lds), else global; tw:
+// the twiddles in LDS, phases advance by integer steps.  Every thread must
+// call it.
+FO_DEV void per_plane64(const PerGridCtx& c, int x, double2* H, double2* G, const double2* tw,
+                        double* red, int* redi, double& bestv, int& besti) {
+  const int NB = c.NB, F = c.F, plane = NB * NB;
+  for (int e = threadIdx.x; e < plane; e += kSelThreads) {
     double2 acc = make_double2(0.0, 0.0);
-    for (int a = 0; a < NB; ++a)
-      acc = cadd(acc, cmul(c.C[(long long)a * NB * NB + e], c.tw64[(int)(((long long)a * x) % F)]));
-    Hg[e] = acc;
+    int ph = 0;
+#pragma unroll 8
+    for (int a = 0; a < NB; ++a) {
+      acc = cadd(acc, cmul(c.C[(long long)a * plane + e], tw[ph]));
+      ph += x;
+      if (ph >= F) ph -= F;
+    }
+    H[e] = acc;
   }
   __threadfence_block();
   __syncthreads();
-  for (int e = threadIdx.x; e < NB * F; e += blockDim.x) {
-    const int b = e / F, z = e % F;
+  for (int e = threadIdx.x; e < NB * F; e += kSelThreads) {
+    const int b = e / F, z = e - b * F;
     double2 acc = make_double2(0.0, 0.0);
-    for (int cc = 0; cc < NB; ++cc)
-      acc = cadd(acc, cmul(Hg[b * NB + cc], c.tw64[(int)(((long long)cc * z) % F)]));
-    Gg[e] = acc;
+    int ph = 0;
+#pragma unroll 4
+    for (int cc = 0; cc < NB; ++cc) {
+      acc = cadd(acc, cmul(H[b * NB + cc], tw[ph]));
+      ph += z;
+      if (ph >= F) ph -= F;
+    }
+    G[e] = acc;
   }
   __threadfence_block();
   __syncthreads();
   double bv = -INFINITY;
   int bi = 0x7fffffff;
-  for (int e = threadIdx.x; e < F * F; e += blockDim.x) {
-    const int y = e / F, z = e % F;
+  for (int e = threadIdx.x; e < F * F; e += kSelThreads) {
+    const int y = e / F, z = e - y * F;
     double2 acc = make_double2(0.0, 0.0);
-    for (int b = 0; b < NB; ++b)
-      acc = cadd(acc, cmul(Gg[b * F + z], c.tw64[(int)(((long long)b * y) % F)]));
+    int ph = 0;
+#pragma unroll 4
+    for (int b = 0; b < NB; ++b) {
+      acc = cadd(acc, cmul(G[b * F + z], tw[ph]));
+      ph += y;
+      if (ph >= F) ph -= F;
+    }
     argmax_merge(bv, bi, sqrt(acc.x * acc.x + acc.y * acc.y), (x * F + y) * F + z);
   }
   block_argmax(bv, bi, red, redi);
@@ -500,9 +689,9 @@ FO_DEV void per_plane64(const PerGridCtx& c, int x, double2* Hg, double2* Gg, do
 }
 
 // Error bound of the FP32 planes: |f| <= A = sum |C|; rounding of C, of the
-// twiddles and of three DFT passes of NB terms each stays below
-// (4 NB + 32) 2^-24 A.  Candidates within 2 delta of the FP32 maximum are
-// re-evaluated in FP64.
+// twiddles and of three DFT passes of NB terms each stays below delta =
+// rel_delta A (per_plane_delta).  Candidates within 2 delta of the FP32
+// maximum are re-evaluated in FP64.
 // The product is read once for the argmax and its six neighbours when a single
 // candidate is listed (the common case); as seven separate sums over the cube
 // and one for A, each a chain of loads, this took 61 us for one pair of nk = 8
@@ -512,8 +701,8 @@ template <int XB>
 __global__ void __launch_bounds__(kSelThreads) k_per_select(
     const PerPair* __restrict__ pd, int nk, int F, const double2* __restrict__ Cprod,
     const double2* __restrict__ tw64, const PlaneCand* __restrict__ cand,
-    const double* __restrict__ abound, double2* __restrict__ scratch, long long scratch_stride,
-    PerPeak* __restrict__ peaks) {
+    const double* __restrict__ abound, double rel_delta, double2* __restrict__ scratch,
+    long long scratch_stride, PerPeak* __restrict__ peaks) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ SelPoints sp;
   __shared__ double red[16];
@@ -541,8 +730,8 @@ __global__ void __launch_bounds__(kSelThreads) k_per_select(
   for (int b = t; b < F; b += blockDim.x)
     for (int r = 0; r < kCandPerPlane; ++r) argmax_merge(mv, mi, pc[b].val[r], pc[b].idx[r]);
   block_argmax(mv, mi, rv, ri);
-  const double A = abound[p];
-  const double delta = (4.0 * NB + 32.0) * 5.9604644775390625e-08 * A;
+  const double A = block_sum(t < NB ? abound[(long long)p * NB + t] : 0.0, red);
+  const double delta = rel_delta * A;
   const double thr = (double)mv - 2.0 * delta;
   if (t == 0) {
     s_cnt = 0;
@@ -587,7 +776,7 @@ __global__ void __launch_bounds__(kSelThreads) k_per_select(
   __syncthreads();
   double best = -INFINITY, second = -INFINITY;
   int besti = 0x7fffffff;
-  double2* Hg = scratch + (long long)p * scratch_stride;
+  double2* Hg = sel_plane_lds(nk, F) <= kSelLds ? H : scratch + (long long)p * scratch_stride;
   double2* Gg = Hg + NB * NB;
   auto take = [&](double v, int i) {
     if (v > best || (v == best && i < besti)) {
@@ -605,7 +794,7 @@ __global__ void __launch_bounds__(kSelThreads) k_per_select(
     for (int x = 0; x < F; ++x) {
       double v;
       int i;
-      per_plane64(c, x, Hg, Gg, red, redi, v, i);
+      per_plane64(c, x, Hg, Gg, tw, red, redi, v, i);
       take(v, i);
     }
   } else {
@@ -627,7 +816,7 @@ __global__ void __launch_bounds__(kSelThreads) k_per_select(
     for (int q = 0; q < novf; ++q) {
       double v;
       int i;
-      per_plane64(c, s_ovfl[q], Hg, Gg, red, redi, v, i);
+      per_plane64(c, s_ovfl[q], Hg, Gg, tw, red, redi, v, i);
       take(v, i);
     }
   }
@@ -985,11 +1174,47 @@ size_t per_plane_smem(int nk, int F) {
          16 * sizeof(int);
 }
 
-void launch_per_plane(hipStream_t s, int P, int nk, int F, const PerPair* pd,
+// real: the product is Hermitian and f itself is not kept
+double per_plane_delta(int nk, int real) {
+  const int NB = 2 * nk + 1;
+  return real ? real_plane_delta(NB) : (4.0 * NB + 32.0) * 5.9604644775390625e-08;
+}
+
+static size_t real_plane_smem(int nk, int F, int XP) {
+  const size_t NB = 2 * (size_t)nk + 1;
+  return sizeof(float2) * F +
+         sizeof(float) * ((NB + 1) * real_plane_fs(F) + XP * NB * real_plane_ks((int)NB));
+}
+
+void launch_per_plane(hipStream_t s, int P, int nk, int F, int real, const PerPair* pd,
                       const double2* Cprod, const float2* tw32, PlaneCand* cand, double* abound,
                       float* grid, float2* cgrid) {
-  hipLaunchKernelGGL(k_per_plane, dim3(F, P), dim3(256), per_plane_smem(nk, F), s, pd, nk, F,
-                     Cprod, tw32, cand, abound, grid, cgrid);
+  if (!real) {
+    hipLaunchKernelGGL(k_per_plane, dim3(F, P), dim3(256), per_plane_smem(nk, F), s, pd, nk, F,
+                       Cprod, tw32, cand, abound, grid, cgrid);
+    return;
+  }
+  // four planes a workgroup when there are planes enough to fill the chip
+  // that way (the basis table is made once for them), else one
+  const int XP = (long long)P * F >= 1024 * kPlaneXP &&
+                         real_plane_smem(nk, F, kPlaneXP) <= 64 * 1024
+                     ? kPlaneXP
+                     : 1;
+  const dim3 g((F + XP - 1) / XP, P), b(256);
+  const size_t sm = real_plane_smem(nk, F, XP);
+  const int nt = (2 * nk + 1 + 15) / 16;
+#define FO_PLANE(NT)                                                                          \
+  hipLaunchKernelGGL(k_per_plane_real<NT>, g, b, sm, s, pd, nk, F, XP, Cprod, tw32, cand, abound, \
+                     grid)
+  if (nt == 1)
+    FO_PLANE(1);
+  else if (nt == 2)
+    FO_PLANE(2);
+  else if (nt == 3)
+    FO_PLANE(3);
+  else
+    FO_PLANE(4);
+#undef FO_PLANE
 }
 
 void launch_per_product_indexed(hipStream_t s, int P, int nk, const PerPair* pd,
@@ -1002,16 +1227,16 @@ void launch_per_product_indexed(hipStream_t s, int P, int nk, const PerPair* pd,
 
 void launch_per_select(hipStream_t s, int P, int nk, int F, const PerPair* pd,
                        const double2* Cprod, const double2* tw64, const PlaneCand* cand,
-                       const double* abound, double2* scratch, long long scratch_stride,
-                       PerPeak* peaks) {
+                       const double* abound, double rel_delta, double2* scratch,
+                       long long scratch_stride, PerPeak* peaks) {
   // three x values a pass while their sums over a fit LDS (NB <= 31: 46 KB)
   const size_t sm = per_select_smem(nk, F);
   if (nk <= 15)
     hipLaunchKernelGGL(k_per_select<3>, dim3(P), dim3(kSelThreads), sm, s, pd, nk, F, Cprod, tw64,
-                       cand, abound, scratch, scratch_stride, peaks);
+                       cand, abound, rel_delta, scratch, scratch_stride, peaks);
   else
     hipLaunchKernelGGL(k_per_select<1>, dim3(P), dim3(kSelThreads), sm, s, pd, nk, F, Cprod, tw64,
-                       cand, abound, scratch, scratch_stride, peaks);
+                       cand, abound, rel_delta, scratch, scratch_stride, peaks);
 }
 
 void launch_per_refine(hipStream_t s, int P, int lap_nmax, const PerPair* pd, const PerGroup* grp,

@@ -1143,65 +1143,21 @@ FO_DEV void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// DPP row shifts (within rows of 16 lanes): row_shl:S gives lane i the value
-// of lane i + S, row_shr:S that of lane i - S.
-template <int CTRL>
-FO_DEV float dpp_mov(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
-}
-
-// Records (largest value v, its flat index i, largest of the other values
-// s): larger value first, ties to the smaller index; the loser's largest
-// value joins the others (so s counts a repeated maximum).
-FO_DEV void top2_merge(float& v, int& i, float& s, float ov, int oi, float os) {
-  const bool take = ov > v || (ov == v && oi < i);
-  s = fmaxf(fmaxf(s, os), take ? v : ov);
-  v = take ? ov : v;
-  i = take ? oi : i;
-}
 // Plane candidates of a 256-thread workgroup: wavefront w fills entry w of
 // the plane's record with its largest value and the largest of its other
-// values (no LDS, no barrier).  One butterfly of (v, i, s) records per
-// orientation inside each row of 16 lanes by DPP (quad_perm [1,0,3,2],
-// quad_perm [2,3,0,1], row_half_mirror, row_mirror), the orientations
-// interleaved, then the four row results through readlane.  Every thread
-// must call it.
-template <int CTRL>
-FO_DEV void top2_dpp_step(float (&v)[2], int (&i)[2], float (&s)[2]) {
-  float ov[2], os[2];
-  int oi[2];
-#pragma unroll
-  for (int o = 0; o < 2; ++o) {
-    ov[o] = dpp_mov<CTRL>(v[o]);
-    oi[o] = __builtin_amdgcn_update_dpp(0, i[o], CTRL, 0xf, 0xf, true);
-    os[o] = dpp_mov<CTRL>(s[o]);
-  }
-#pragma unroll
-  for (int o = 0; o < 2; ++o) top2_merge(v[o], i[o], s[o], ov[o], oi[o], os[o]);
-}
+// values (no LDS, no barrier).  Every thread must call it.
 FO_DEV void plane_candidates(const CandTrack& ct, int norient, PlaneCand* out, int ostride) {
   const int wl = threadIdx.x & 63, w = threadIdx.x >> 6;
   float v[2] = {ct.c0.bv, ct.c1.bv}, s[2] = {ct.c0.dm, ct.c1.dm};
   int i[2] = {ct.c0.bi, ct.c1.bi};
-  top2_dpp_step<0xB1>(v, i, s);
-  top2_dpp_step<0x4E>(v, i, s);
-  top2_dpp_step<0x141>(v, i, s);
-  top2_dpp_step<0x140>(v, i, s);
+  wave_top2(v, i, s);
 #pragma unroll
   for (int o = 0; o < 2; ++o) {
-    float rv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[o]), 0));
-    float rs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[o]), 0));
-    int ri = __builtin_amdgcn_readlane(i[o], 0);
-#pragma unroll
-    for (int r = 16; r < 64; r += 16)
-      top2_merge(rv, ri, rs, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[o]), r)),
-                 __builtin_amdgcn_readlane(i[o], r),
-                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[o]), r)));
     if (o < norient && wl == 0) {
       PlaneCand* dst = out + (long long)o * ostride;
-      dst->val[w] = rv;
-      dst->idx[w] = ri;
-      dst->rest[w] = rs;
+      dst->val[w] = v[o];
+      dst->idx[w] = i[o];
+      dst->rest[w] = s[o];
     }
   }
 }

@@ -284,3 +284,38 @@ def test_selected_peak_and_neighbours(gpu, nk, F, mirror):
         disp[ax] = (i[ax] - (y3 - y1) / curv) * box[ax] / F
         # numerator and denominator are each off by a few tol
         assert abs(pk["disp"][0, ax] - disp[ax]) <= 16 * tol / abs(curv) * box[ax] / F + 1e-14
+
+
+@pytest.mark.parametrize("nk,F,P", [(1, 3, 1), (7, 16, 2), (8, 17, 256), (8, 64, 64), (15, 45, 1),
+                                    (16, 36, 1), (23, 47, 1), (24, 81, 1), (31, 63, 66)])
+def test_real_planes_within_the_selection_bound(gpu, nk, F, P):
+    """|f| of the real-basis planes (structure factors) and of the complex ones
+    (the same coefficients supplied) against a 64-bit FFT at the edges of the
+    basis tiles (2 nk + 1 = 15, 17, 31, 33, 47, 49, 63), odd F, and with one
+    or four planes a workgroup: within the bound the selection relies on."""
+    say(f"case: nk={nk} F={F} P={P}")
+    rng = np.random.default_rng(nk + F)
+    box = np.array([4.0, 4.4, 3.7])
+    N = 12
+    x, y = rng.random((P, N, 3)) * box, rng.random((P, N, 3)) * box
+    NB = 2 * nk + 1
+    with PeriodicBatch([N] * P, box, 0.25, nk, F, None, 10,
+                       _lib.PER_KEEP_GRID | _lib.PER_KEEP_COEFFS) as b:
+        b.set_positions(list(x), list(y))
+        b.run(_lib.PSTAGE_SF | _lib.PSTAGE_GRID)
+        C, coef, pk = b.product(), b.coeffs(), b.peaks()
+        grids = {p: b.grid(p) for p in {0, P - 1}}
+    for p, g in grids.items():
+        f = np.abs(np.fft.fftn(C[p], (F, F, F)))
+        A = np.abs(C[p]).sum()
+        assert np.abs(g - f).max() <= (9 * NB + 64) * 2.0 ** -24 * A
+        assert abs(pk["delta"][p] - (9 * NB + 64) * 2.0 ** -24 * A) <= 1e-12 * A
+        assert f[tuple(pk["ind"][p])] >= f.max() * (1 - 1e-12)
+    with PeriodicBatch([N], box, 0.25, nk, F, None, 10,
+                       _lib.PER_KEEP_GRID | _lib.PER_INPUT_COEFFS) as b:
+        b.set_positions(x[0], y[0])
+        b.set_coeffs(coef[0][:1], coef[1][:1])
+        b.run(_lib.PSTAGE_SF | _lib.PSTAGE_GRID)
+        f = np.abs(np.fft.fftn(C[0], (F, F, F)))
+        A = np.abs(C[0]).sum()
+        assert np.abs(b.grid(0) - f).max() <= (4 * NB + 32) * 2.0 ** -24 * A

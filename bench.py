@@ -530,7 +530,7 @@ def main():
     # roofline of the dominant kernel (algorithmic flops / measured time)
     work = {
         "plane": ("k_isoft_fft", sum(isoft_flops(c["L"], c["grid_n"]) for c in pairs), FP32_PEAK),
-        "contract": ("k_sph_contract_low+k_sph_contract_mfma",
+        "contract": ("k_sph_contract",
                      sum(coeff_flops(c["groups"], c["L"]) for c in pairs), FP64_PEAK),
         "rotopt": ("k_sph_rotopt", sum(float((e * rotopt_eval_flops(L)[:, None]).sum())
                                        for e, L in zip(evs, Ls)), FP64_PEAK),

@@ -40,7 +40,7 @@ void launch_harm_coeffs(hipStream_t, int, int, int, int, const SphPair*, const S
                         float2*);
 void launch_coef_norm2(hipStream_t, int, const SphPair*, const double2*, double*);
 int harm_block_lx(int L, int nmax, int basis);
-void launch_sph_contract(hipStream_t, int, int, int, const SphPair*, const SphGroup*,
+void launch_sph_contract(hipStream_t, int, int, int, int, int, const SphPair*, const SphGroup*,
                          const double*, const double*, const double2*, const double2*,
                          const double*, const double*, double2*, float2*);
 size_t isoft_plane_smem(int, int, int);
@@ -555,8 +555,8 @@ static int sph_enqueue(fo_sph_batch* b, int stages) {
       launch_sph_radial(s, Pc, C.Lmax, C.maxjk, pdc, b->grp, b->rad, b->rad + b->hgath.size(), scc,
                         b->R, b->tune[2]);
       cmark(3 * c + 2);
-      launch_sph_contract(s, Pc, L.n, C.Lmax, pdc, b->grp, b->rad, b->rad + b->hgath.size(),
-                          b->Y1, b->Y2, b->R, scc, b->I64A, b->I32A);
+      launch_sph_contract(s, Pc, L.n, C.Lmax, L.mingath, L.maxgath, pdc, b->grp, b->rad,
+                          b->rad + b->hgath.size(), b->Y1, b->Y2, b->R, scc, b->I64A, b->I32A);
     }
     cmark(3 * b->chunks.size());
   }
@@ -652,7 +652,7 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
   b->harm_nmax = harm_nmax;
   b->harm_r0 = harm_r0;
   b->harm_basis = harm_basis ? 1 : 0;
-  int Lmax = 0, maxatoms = 0, maxgath = 0;
+  int Lmax = 0, maxatoms = 0, mingath = 1 << 30, maxgath = 0;
   long long maxjk = 0, Ntot = 0, Ktot = 0, C32tot = 0, radtot = 0, ylmtot = 0;
   long long radmax = 0, ylmmax = 0;  // largest chunk
   const size_t chunk_budget = coef_chunk_bytes();
@@ -738,6 +738,7 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
     ylmmax = std::max(ylmmax, ylmtot);
     Lmax = std::max(Lmax, Lp);
     maxatoms = std::max(maxatoms, N);
+    mingath = std::min(mingath, ng);
     maxgath = std::max(maxgath, ng);
     maxjk = std::max(maxjk, jk);
     Ntot += N;
@@ -765,6 +766,7 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
   lc.n = n;
   lc.Lmax = Lmax;
   lc.Lt = b->tab->Lt;
+  lc.mingath = mingath;
   lc.maxgath = maxgath;
   lc.maxatoms = maxatoms;
   lc.maxjk = maxjk;

@@ -41,7 +41,9 @@ FO_HD int qlm(int l, int m) { return l * (l + 1) / 2 + m; }
 //   L <= 7 :  L, L+1                    (block 0 = 0..L)
 //   L <= 15:  7, 8, L, L+1              (block 1 = 8..L)
 //   L >= 16:  7, 8, 15, 16, 17, ..., L  (degree l >= 16 in slot l - 13)
-// Block b reads slots 2b (its top degree) and 2b + 1 (one above).
+// Block b reads slots 2b (its top degree) and 2b + 1 (one above).  x =
+// r1 r2 / 2 s^2 below kMinRadX counts as kMinRadX.
+constexpr double kMinRadX = 0x1p-58;
 FO_HD int rad_slots(int L) { return L <= 7 ? 2 : (L <= 15 ? 4 : L - 12); }
 FO_HD int rad_slot_deg(int s, int L) {
   if (L <= 7) return L + s;
@@ -246,6 +248,51 @@ FO_DEV void wave_top2(float (&v)[NO], int (&i)[NO], float (&s)[NO]) {
     i[o] = ri;
     s[o] = rs;
   }
+}
+
+// XCD-aware decode of a 1-D launch of 8 ceil(P/8) per workgroups over
+// (pair, item): workgroup w serves pair (w % 8) + 8 (w / (8 per)) and item
+// (w / 8) % per.  Workgroups are dealt to the 8 XCDs round-robin, so all
+// items of a pair run on one XCD and share its L2.  False for the padding
+// workgroups (pair >= P).
+FO_DEV bool xcd_decode(int P, int per, int& p, int& item) {
+  const int w = blockIdx.x;
+  p = (w & 7) + 8 * (w / (8 * per));
+  item = (w >> 3) % per;
+  return p < P;
+}
+static inline unsigned xcd_grid(int P, int per) { return (unsigned)(8 * ((P + 7) / 8) * per); }
+
+// Raw buffer access (gfx9 descriptor): a per-lane byte offset plus a
+// wavefront-uniform one (scalar register); offsets at or beyond `bytes`
+// read zero.
+FO_DEV __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, bytes, 0x00020000);
+}
+FO_DEV float4 load_f4(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+  const u4 w = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+  return make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z),
+                     __uint_as_float(w.w));
+}
+
+FO_DEV double load_d(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+  const u2 w = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+  return __hiloint2double((int)w.y, (int)w.x);
+}
+FO_DEV double2 load_d2(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+  const u4 w = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+  return make_double2(__hiloint2double((int)w.y, (int)w.x), __hiloint2double((int)w.w, (int)w.z));
+}
+
+// FP64 matrix product step.  Lane layout: A operand lane -> (row lane%16, k
+// lane/16), B operand lane -> (k lane/16, col lane%16), result register i of
+// a lane -> (row 4 i + lane/16, col lane%16).
+typedef double v4d __attribute__((ext_vector_type(4)));
+FO_DEV v4d mfma64(double a, double b, v4d c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
 }  // namespace fo

@@ -116,6 +116,7 @@ struct SphLaunch {
   int n;               // grid side 2B
   int Lmax;            // max L over the pairs
   int Lt;              // degree of the resident Wigner table
+  int mingath;         // min gathered atoms over pairs
   int maxgath;         // max gathered atoms over pairs
   int maxatoms;        // max atoms over pairs
   long long maxjk;     // max sum of group size^2 over pairs

@@ -18,11 +18,6 @@
 
 namespace fo {
 
-typedef double v4d __attribute__((ext_vector_type(4)));
-FO_DEV v4d mfma64(double a, double b, v4d c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
 // One k-vector's weighted overlap product: sum over the groups of C1 conj(C2)
 // in this fused order, then the weight.  Every path to Cprod uses these two
 // (the same coefficients give the same product to the last bit).

@@ -5,7 +5,7 @@
 //   k_sph_prep       centroids, automatic kernel width
 //   k_sph_ylm        Y_lm of every grouped atom (FP64)
 //   k_sph_radial     scaled i_l(x) * Gaussian radial kernel (FP64)
-//   k_sph_contract   C^l = Y1 . K_l . Y2^H per degree (FP64)
+//   k_sph_contract   C^l = Y1 . K_l . Y2^H per degree (FP64, fo_contract.hip)
 //   k_isoft_fft      inverse SOFT of both orientations per beta plane (FP32),
 //                    two-pass register transforms (power-of-two n); k_isoft_plane
 //                    is the direct-DFT form for other n;
@@ -173,19 +173,6 @@ __global__ void k_sph_prep(const SphPair* __restrict__ pd, const double* __restr
 // recurrence in l with tabulated coefficients (k_leg_table).  An atom at the
 // centre takes theta = phi = 0 (only l = 0 survives there).
 // ---------------------------------------------------------------------------
-// XCD-aware decode of a 1-D launch of 8 ceil(P/8) per workgroups over
-// (pair, item): workgroup w serves pair (w % 8) + 8 (w / (8 per)) and item
-// (w / 8) % per.  Workgroups are dealt to the 8 XCDs round-robin, so all
-// items of a pair run on one XCD and share its L2.  False for the padding
-// workgroups (pair >= P).
-FO_DEV bool xcd_decode(int P, int per, int& p, int& item) {
-  const int w = blockIdx.x;
-  p = (w & 7) + 8 * (w / (8 * per));
-  item = (w >> 3) % per;
-  return p < P;
-}
-static inline unsigned xcd_grid(int P, int per) { return (unsigned)(8 * ((P + 7) / 8) * per); }
-
 __global__ void k_sph_ylm(const SphPair* __restrict__ pd, const int* __restrict__ gath,
                           const double* __restrict__ X1c, const double* __restrict__ X2c,
                           const double2* __restrict__ leg, const double* __restrict__ cm,
@@ -280,11 +267,6 @@ FO_DEV double radial_series(int l, double x, double exg) {
 // (0.93 -> 0.84 ms; the contraction's time unchanged).
 FO_DEV void radial_store(int L, double x, double gauss, double* out, long long stride) {
   const int ns = rad_slots(L);
-  if (x == 0.0) {
-    for (int s = 0; s < ns; ++s)
-      __builtin_nontemporal_store(rad_slot_deg(s, L) == 0 ? gauss : 0.0, &out[s * stride]);
-    return;
-  }
   if (x < 1.0) {
     const double exg = exp(-x) * gauss;
     for (int s = 0; s < ns; ++s)
@@ -354,677 +336,10 @@ __global__ void __launch_bounds__(256, 5) k_sph_radial(const SphPair* __restrict
     // |x| of the two atoms, as the harmonics kernel recorded them
     const double r1 = rad1[d.gath_off + g[q].gath_off + j];
     const double r2 = rad2[d.gath_off + g[q].gath_off + k];
-    const double x = r1 * r2 * i2s2;
+    const double x = fmax(r1 * r2 * i2s2, kMinRadX);
     const double gauss = exp(-(r1 - r2) * (r1 - r2) * i4s2);
     radial_store(d.L, x, gauss, R + d.rad_off + g[q].rad_off + (long long)j * Ns + k,
                  (long long)Ns * Ns);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Contraction I^l_{m1m2} = 4 pi^{5/2} s^3 sum_s sum_{j,k in s}
-//   Y1[l,m1,j] K_l[j,k] conj(Y2[l,m2,k])      (sphericalAlignment.py:273,:175)
-// Only rows m1 >= 0 are contracted: Y_l^{-m} = (-1)^m conj(Y_l^m) and K_l
-// is real, so I^l_{-m1,-m2} = (-1)^{m1+m2} conj(I^l_{m1m2}) and the m1 < 0
-// rows are stored from the computed ones.
-// ---------------------------------------------------------------------------
-// m1 rows per workgroup: 16 for the column-tile class of degrees <= 15
-// (at most 16 rows), 32 above
-template <int NCT>
-constexpr int contract_rows() {
-  return NCT <= 2 ? 16 : 32;
-}
-
-// ---------------------------------------------------------------------------
-// MFMA form of the contraction (v_mfma_f64_16x16x4f64).  One workgroup per
-// (pair, l, block of MB rows m1 >= 0).  Per species group and tile of kCT
-// atoms k of structure 2:
-//   stage Y2[m][k-tile] (built from P2, E2) in LDS
-//   A[rr][k] = sum_j Y1'[rr][j] K_l[j][k]: real rows rr = 2r + {Re, Im} of
-//              row m1a + r; j in chunks of kJC staged in LDS one chunk ahead
-//              (cooperative coalesced loads, double buffer); wave w computes
-//              rows 16w..16w+15 of both 16-wide column tiles
-//   A -> LDS (complex [row][k], aliasing the chunk buffers)
-//   C[r][m] += sum_k A[r][k] conj(Y2[m][k]) as four real products
-//              (Cr += Ar Y2r + Ai Y2i, Ci += Ai Y2r - Ar Y2i); complex 16x16
-//              tiles dealt to the waves round-robin.
-// MFMA lane layout: A operand lane -> (row lane%16, k lane/16), B operand
-// lane -> (k lane/16, col lane%16), result register i of a lane -> (row
-// 4 i + lane/16, col lane%16).  The reduction order of every output is
-// fixed, so results do not depend on the batch a pair is in.
-// ---------------------------------------------------------------------------
-typedef double v4d __attribute__((ext_vector_type(4)));
-
-FO_DEV v4d mfma64(double a, double b, v4d c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-constexpr int kCT = 32;  // atoms of structure 2 per tile
-constexpr int kJC = 16;  // atoms of structure 1 per staged chunk
-
-// LDS of one contraction workgroup; NCT = 16-wide column tiles of Y2.  The
-// chunk buffers of the first product and the A / Y2 tiles of the second are
-// never live together.
-template <int NCT, int MB = contract_rows<NCT>()>
-struct ContractLds {
-  union {
-    struct {
-      double y1[2][2 * MB][kJC + 1];   // [buffer][real row][j]
-      double kc[2][kJC][kCT + 1];      // [buffer][j][k]
-    } a;
-    struct {
-      double2 ac[MB][kCT + 1];         // A tile [row][k]
-      double2 ys[kCT][16 * NCT + 1];   // Y2 tile [k][m]
-    } b;
-  } u;
-};
-
-template <int NCT>
-FO_DEV void contract_mfma_body(const SphPair& d, int l, int b, const SphGroup* __restrict__ grp,
-                               const double2* __restrict__ Y1, const double2* __restrict__ Y2,
-                               const double* __restrict__ R, double sc,
-                               double2* __restrict__ I64, float2* __restrict__ I32, int n,
-                               ContractLds<NCT>& S) {
-  constexpr int MB = contract_rows<NCT>();  // m1 rows per workgroup
-  constexpr int MP = 16 * NCT;            // padded columns of Y2
-  constexpr int NY = kCT * MP / 256;      // staged Y2 entries per thread
-  const int M = 2 * l + 1;
-  const int m1a = b * MB;
-  const int rows = min(MB, l + 1 - m1a);
-  const int nrt = (rows + 15) >> 4;       // complex row tiles of C
-  const int nrtA = (2 * rows + 15) >> 4;  // real row tiles of A
-  const int nct = (M + 15) >> 4;          // column tiles of C
-  // the wave index is read into a scalar register so that the tile
-  // conditions below are uniform branches (MFMA needs all lanes active)
-  const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int ln = t & 63, col = ln & 15, kq = ln >> 4;
-  // first product: wave w owns A tiles (row tile (w >> 1) + 2 qa, column
-  // tile w & 1), qa < 2.  Second product: wave w computes the real (w even)
-  // or imaginary (w odd) part of complex C tiles (w >> 1) + 2 qb, qb < NCT.
-  const int actA = w & 1, part = w & 1;
-  v4d cacc[NCT];
-#pragma unroll
-  for (int q = 0; q < NCT; ++q) cacc[q] = v4d{0.0, 0.0, 0.0, 0.0};
-  const int Ng = d.ngath;
-  const double2* Y1l = Y1 + d.ylm_off;
-  const double2* Y2l = Y2 + d.ylm_off;
-  for (int g = 0; g < d.ngroups; ++g) {
-    const SphGroup G = grp[d.group_off + g];
-    const int Ns = G.size, go = G.gath_off;
-    // degree l >= 16 is stored in radial slot l - 13
-    const double* Rl = R + d.rad_off + G.rad_off + (long long)(l - 13) * Ns * Ns;
-    // staging roles of this thread:
-    //   Y1 chunk:  j = j0 + t % kJC, complex rows t / kJC + kYR i, i < kNY1
-    //              (each gives the real rows 2r and 2r + 1)
-    //   K chunk:   k = k0 + (t & 31), j = j0 + (t >> 5) + 8 i, i < kNK
-    //   Y2 tile:   k = k0 + (t & 31), m = (t >> 5) + 8 i, i < NY
-    constexpr int kYR = 256 / kJC;          // complex rows per Y1 staging round
-    constexpr int kNY1 = MB * kJC / 256;    // Y1 entries staged per thread
-    constexpr int kNK = kJC / 8;            // K entries staged per thread
-    const int yj = t % kJC, yr0 = t / kJC;
-    const int kk_t = t & 31, kj0 = t >> 5;
-    const double2* Y1g = Y1l + go;
-    const double2* Y2g = Y2l + go;
-    for (int k0 = 0; k0 < Ns; k0 += kCT) {
-      const int kt = k0 + kk_t;
-      const bool kok = kt < Ns;
-      double2 sy[kNY1];
-      double sk[kNK];
-      double2 yv[NY];
-#define FO_LOAD_CHUNK(J0)                                                           \
-  {                                                                                 \
-    const int j_ = (J0) + yj;                                                       \
-    _Pragma("unroll") for (int i = 0; i < kNY1; ++i) {                              \
-      const int r = yr0 + kYR * i;                                                  \
-      sy[i] = (r < rows && j_ < Ns) ? Y1g[qlm(l, m1a + r) * Ng + j_]                \
-                                    : make_double2(0.0, 0.0);                       \
-    }                                                                               \
-    _Pragma("unroll") for (int i = 0; i < kNK; ++i) {                               \
-      const int j = (J0) + kj0 + 8 * i;                                             \
-      sk[i] = (j < Ns && kok) ? Rl[j * Ns + kt] : 0.0;                              \
-    }                                                                               \
-  }
-#define FO_STORE_CHUNK(BUF)                                                         \
-  {                                                                                 \
-    _Pragma("unroll") for (int i = 0; i < kNY1; ++i) {                              \
-      S.u.a.y1[BUF][2 * (yr0 + kYR * i)][yj] = sy[i].x;                             \
-      S.u.a.y1[BUF][2 * (yr0 + kYR * i) + 1][yj] = sy[i].y;                         \
-    }                                                                               \
-    _Pragma("unroll") for (int i = 0; i < kNK; ++i) S.u.a.kc[BUF][kj0 + 8 * i][kk_t] = sk[i]; \
-  }
-// Y2 row m2 = m - l: Y_l^{m2} = P2 E2 for m2 >= 0, (-1)^|m2| conj(P2 E2) for m2 < 0.
-// Every lane loads (entries outside the tile read element 0 of the group's
-// block and are zeroed afterwards), so the loads issue back to back.
-#define FO_LOAD_Y2                                                                  \
-  {                                                                                 \
-    _Pragma("unroll") for (int i = 0; i < NY; ++i) {                                \
-      const int m = kj0 + 8 * i;                                                    \
-      const bool ok = m < M && kok;                                                 \
-      const int am = abs(m - l);                                                    \
-      yv[i] = Y2g[ok ? qlm(l, am) * Ng + kt : 0];                                   \
-    }                                                                               \
-    _Pragma("unroll") for (int i = 0; i < NY; ++i) {                                \
-      const int m = kj0 + 8 * i, m2 = m - l;                                        \
-      const bool ok = m < M && kok;                                                 \
-      const double sgn = (m2 < 0 && (m2 & 1)) ? -1.0 : 1.0;                         \
-      yv[i] = ok ? make_double2(sgn * yv[i].x, (m2 < 0 ? -sgn : 1.0) * yv[i].y)     \
-                 : make_double2(0.0, 0.0);                                          \
-    }                                                                               \
-  }
-      FO_LOAD_CHUNK(0);
-      __syncthreads();  // previous tile's readers of the union are done
-      FO_STORE_CHUNK(0);
-      __syncthreads();
-      v4d a0 = v4d{0.0, 0.0, 0.0, 0.0}, a1 = a0;
-      const int nch = (Ns + kJC - 1) / kJC;
-      for (int c = 0; c < nch; ++c) {
-        const int buf = c & 1;
-        if (c + 1 < nch) FO_LOAD_CHUNK((c + 1) * kJC);
-        // A tiles of this wave: rows 16 rt, columns 16 actA.  The row-tile
-        // conditions are wave-uniform and outside the k loop, so every LDS
-        // operand of the chunk is read before the first MFMA waits on one.
-        {
-          const int rt0 = w >> 1, rt1 = rt0 + 2;
-          double bv[kJC / 4], ya[kJC / 4], yb[kJC / 4];
-          if (rt0 < nrtA) {
-#pragma unroll
-            for (int s4 = 0; s4 < kJC / 4; ++s4) {
-              const int jj = 4 * s4 + kq;
-              bv[s4] = S.u.a.kc[buf][jj][16 * actA + col];
-              ya[s4] = S.u.a.y1[buf][16 * rt0 + col][jj];
-            }
-            if (rt1 < nrtA) {
-#pragma unroll
-              for (int s4 = 0; s4 < kJC / 4; ++s4)
-                yb[s4] = S.u.a.y1[buf][16 * rt1 + col][4 * s4 + kq];
-#pragma unroll
-              for (int s4 = 0; s4 < kJC / 4; ++s4) {
-                a0 = mfma64(ya[s4], bv[s4], a0);
-                a1 = mfma64(yb[s4], bv[s4], a1);
-              }
-            } else {
-#pragma unroll
-              for (int s4 = 0; s4 < kJC / 4; ++s4) a0 = mfma64(ya[s4], bv[s4], a0);
-            }
-          }
-        }
-        if (c + 1 < nch) FO_STORE_CHUNK(buf ^ 1);
-        __syncthreads();
-      }
-      FO_LOAD_Y2;
-#undef FO_LOAD_CHUNK
-#undef FO_STORE_CHUNK
-#undef FO_LOAD_Y2
-      // A and Y2 tiles -> LDS (the chunk buffers are free after the barrier)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int rt = (w >> 1) + 2 * h;
-        if (rt < nrtA) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int r2 = 16 * rt + 4 * i + kq;
-            double* e0 = (double*)&S.u.b.ac[r2 >> 1][16 * actA + col];
-            e0[r2 & 1] = h == 0 ? a0[i] : a1[i];
-          }
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < NY; ++i) S.u.b.ys[kk_t][kj0 + 8 * i] = yv[i];
-      __syncthreads();
-      // second product, k-steps outer so consecutive MFMAs update
-      // different accumulators.  Every k-step reads the operands of all NCT
-      // tile slots first (row clamped into the block, so the reads stay in
-      // the A tile), then issues the MFMAs of this wave's tiles, ctile =
-      // (w >> 1) + 2 qb below nrt * nct (wave-uniform).
-      {
-        const int ntl = nrt * nct;
-#pragma unroll 2
-        for (int s8 = 0; s8 < kCT / 4; ++s8) {
-          const int kk = 4 * s8 + kq;
-          double2 av[NCT], yw[NCT];
-#pragma unroll
-          for (int qb = 0; qb < NCT; ++qb) {
-            const int ctile = (w >> 1) + 2 * qb;
-            const int rt = min(ctile / nct, nrt - 1), ct = ctile % nct;
-            const int r = 16 * rt + col;
-            av[qb] = r < rows ? S.u.b.ac[r][kk] : make_double2(0.0, 0.0);
-            yw[qb] = S.u.b.ys[kk][16 * ct + col];
-          }
-#pragma unroll
-          for (int qb = 0; qb < NCT; ++qb) {
-            if ((w >> 1) + 2 * qb >= ntl) continue;  // wave-uniform
-            // real part: Ar Y2r + Ai Y2i; imaginary part: Ai Y2r - Ar Y2i
-            const double a0 = part ? av[qb].y : av[qb].x, a1 = part ? -av[qb].x : av[qb].y;
-            cacc[qb] = mfma64(a0, yw[qb].x, cacc[qb]);
-            cacc[qb] = mfma64(a1, yw[qb].y, cacc[qb]);
-          }
-        }
-      }
-    }
-  }
-  // C tiles: real parts in waves 0, 2, imaginary parts in waves 1, 3;
-  // exchange through LDS so one lane writes both parts of an entry
-  __syncthreads();
-  double2 (*cb)[kCT + 1] = S.u.b.ac;  // reuse as [MB][kCT + 1] staging per column tile pass
-  const double norm = 4.0 * pow(kPi, 2.5) * sc * sc * sc;
-  for (int ct = 0; ct < nct; ++ct) {
-    // tiles (rt, ct) for rt < nrt: ctile = rt * nct + ct
-#pragma unroll
-    for (int qb = 0; qb < NCT; ++qb) {
-      const int ctile = (w >> 1) + 2 * qb;
-      const int rt = ctile / nct, cc = ctile % nct;
-      if (rt >= nrt || cc != ct) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 16 * rt + 4 * i + kq;
-        double* e = (double*)&cb[r][col];
-        e[part] = cacc[qb][i];
-      }
-    }
-    __syncthreads();
-    for (int e = t; e < MB * 16; e += 256) {
-      const int r = e >> 4, mc = e & 15, m = 16 * ct + mc;
-      if (r < rows && m < M) {
-        const int m1 = m1a + r, m2 = m - l;
-        const long long id = d.coef_off + kidx(l, m1, m2);
-        const double2 cv = cb[r][mc];
-        const double2 v = make_double2(norm * cv.x, norm * cv.y);
-        I64[id] = v;
-        I32[d.c32_off + (long long)qlm(l, m1) * n + plane_pos(plane_k(m2, n), n)] =
-            make_float2((float)v.x, (float)v.y);
-      }
-    }
-    __syncthreads();
-  }
-  // Only rows m1 >= 0 are written: the selection and the refinement read
-  // nothing else, the m1 < 0 rows of I64 are filled by k_sph_mirror when the
-  // coefficients are read out, and the plane-layout entries |m2| > l stay
-  // at the zeros the batch was bound with.
-}
-
-// NCTMAX: column tiles of the largest degree in the launch (2l+1 <= 16 NCTMAX);
-// the launch covers the degrees l_lo..l_hi of every pair.
-template <int NCTMAX>
-__global__ void __launch_bounds__(256, NCTMAX <= 2 ? 5 : 3) k_sph_contract_mfma(
-    const SphPair* __restrict__ pd, const SphGroup* __restrict__ grp,
-    const double2* __restrict__ Y1, const double2* __restrict__ Y2,
-    const double* __restrict__ R, const double* __restrict__ scale_eff,
-    double2* __restrict__ I64, float2* __restrict__ I32, int n, int P, int nbl, int l_lo,
-    int l_hi) {
-  __shared__ ContractLds<NCTMAX> S;
-  int pp, b;
-  if (!xcd_decode(P, nbl, pp, b)) return;
-  const SphPair d = pd[pp];
-  const int L = min(d.L, l_hi);
-  int l = l_lo;
-  for (; l <= L; ++l) {
-    constexpr int MB = contract_rows<NCTMAX>();
-    const int nb = (l + 1 + MB - 1) / MB;
-    if (b < nb) break;
-    b -= nb;
-  }
-  if (l > L) return;
-  const double sc = scale_eff[pp];
-  contract_mfma_body<NCTMAX>(d, l, b, grp, Y1, Y2, R, sc, I64, I32, n, S);
-}
-
-// Raw buffer access (gfx9 descriptor): a per-lane byte offset plus a
-// wavefront-uniform one (scalar register); offsets at or beyond `bytes`
-// read zero.
-FO_DEV __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, bytes, 0x00020000);
-}
-FO_DEV float4 load_f4(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-  const u4 w = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-  return make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z),
-                     __uint_as_float(w.w));
-}
-
-FO_DEV double load_d(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  typedef unsigned int u2 __attribute__((ext_vector_type(2)));
-  const u2 w = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-  return __hiloint2double((int)w.y, (int)w.x);
-}
-FO_DEV double2 load_d2(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-  const u4 w = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-  return make_double2(__hiloint2double((int)w.y, (int)w.x), __hiloint2double((int)w.w, (int)w.z));
-}
-
-// ---------------------------------------------------------------------------
-// Degrees 0..15: radial factors and contraction in one pass.  The radial
-// kernel stored K at the top degree h of each block of eight (block 0:
-// 0..min(7, L), block 1: 8..min(15, L)) and at h + 1 (slots 2b, 2b + 1).
-// One workgroup per (pair, four degrees): quarter s of block b covers
-// degrees h - 4s down to max(8b, h - 4s - 3).  It starts from the stored
-// pair and descends with the radial kernel's recurrence
-// K_{l-1} = K_{l+1} + (2l+1)/x K_l (i_l is the minimal solution, stable
-// downwards), so the K_l of degrees <= 15 never pass through HBM.  Entries
-// with x < 2^-40, where the stored values of degree 16 can be subnormal
-// (x = 0: an atom at the centre), take the power series instead.
-// Per species group and tile of KT = 64 atoms k of structure 2:
-//   j in chunks of kJL: the Y1 rows of the four degrees are staged in LDS
-//   (the next chunk is loaded into registers meanwhile); wave w owns the
-//   column tile of atoms k0 + 16 w .. + 15 and every row tile of A (one for
-//   block 0, whose 2(l+1) <= 16 real rows fit one, two for block 1), so
-//   each lane steps the recurrence of the four (j, k) entries it supplies
-//   as the MFMA B operand once for all row tiles, and A_l += Y1'_l K_l
-//   accumulates per degree in registers.
-//   Then two degrees at a time: their A_l tiles and Y2_l rows -> LDS,
-//   C^l += A_l conj(Y2_l)^T as in k_sph_contract_mfma, one real or
-//   imaginary part of one column tile per wave (block 0: even degrees on
-//   waves 0-1, odd degrees on waves 2-3).
-// Each output's reduction order is fixed: j in order inside A, k in order
-// inside C, groups in order.
-// ---------------------------------------------------------------------------
-constexpr double kTinyX = 0x1p-40;
-constexpr int kJL = 16;  // atoms j per staged chunk
-static_assert(kJL == 16, "the chunk staging maps thread t to atom t & 15 of a chunk");
-constexpr int kNS4 = kJL / 4;  // MFMA k-steps per chunk
-// 1/(2l+1)!!, l = 0..15
-__constant__ double kInvDfact[16] = {
-    1.0, 1.0 / 3, 1.0 / 15, 1.0 / 105, 1.0 / 945, 1.0 / 10395, 1.0 / 135135, 1.0 / 2027025,
-    1.0 / 34459425, 1.0 / 654729075, 1.0 / 13749310575.0, 1.0 / 316234143225.0,
-    1.0 / 7905853580625.0, 1.0 / 213458046676875.0, 1.0 / 6190283353629375.0,
-    1.0 / 191898783962510625.0};
-
-template <int BLK>
-struct LowCfg {
-  static constexpr int RTW = BLK ? 2 : 1;     // real-row tiles of A per degree (per wave)
-  static constexpr int KT = 64;               // atoms k per tile: one column tile per wave
-  static constexpr int NQ = BLK ? 58 : 26;    // complex Y rows of four degrees (12..15, 4..7)
-  static constexpr int AR = BLK ? 16 : 8;     // complex rows m1 <= l
-  static constexpr int NMC = BLK ? 32 : 16;   // columns m = m2 + l (2l + 1 < NMC)
-  static constexpr int NC = BLK ? 4 : 2;      // C tile parts held per wave
-  static constexpr int NYI = (NQ * kJL + 255) / 256;  // staged Y1 entries per thread
-  static constexpr int NM = BLK ? 16 : 8;     // rows m2 = 0..l of Y2 (l < NM)
-  static constexpr int NYV = KT * NM / 256;           // staged Y2 entries per thread
-};
-
-template <int BLK>
-struct LowLds {
-  using Cf = LowCfg<BLK>;
-  union {
-    double y1[2 * Cf::NQ][kJL + 1];     // Y1 rows of a j chunk, [real row][j]
-    double2 ac[2][Cf::AR][Cf::KT + 1];  // A_l tiles of two degrees [degree][m1][k]
-  } u;
-  double2 ys[2][Cf::KT][Cf::NM + 1];    // Y2_l rows m2 >= 0 of two degrees [degree][k][m2]
-  double rj[kJL];                       // |x1_j| of the chunk's atoms (-1: none)
-  double irj[kJL];                      // 1/|x1_j| (0: none)
-};
-
-// A copy of v that the compiler cannot see through: lane-dependent index
-// arithmetic derived from it stays where it is used instead of being hoisted
-// out of the loops (where it would hold registers for the whole loop nest).
-FO_DEV int opaque_lane(int v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-
-template <int BLK>
-__global__ void __launch_bounds__(256, 2) k_sph_contract_low(
-    const SphPair* __restrict__ pd, const SphGroup* __restrict__ grp,
-    const double* __restrict__ rad1, const double* __restrict__ rad2,
-    const double2* __restrict__ Y1, const double2* __restrict__ Y2,
-    const double* __restrict__ R, const double* __restrict__ scale_eff,
-    double2* __restrict__ I64, float2* __restrict__ I32, int n, int P) {
-  using Cf = LowCfg<BLK>;
-  constexpr int KT = Cf::KT;
-  constexpr double kBig = 0x1p600;  // stands for 1/r of an atom at the centre
-  __shared__ LowLds<BLK> S;
-  int pp, qs;
-  if (!xcd_decode(P, 2, pp, qs)) return;
-  const SphPair d = pd[pp];
-  const int lo = 8 * BLK;
-  if (lo > d.L) return;
-  const int h = min(lo + 7, d.L), top = h - 4 * qs;
-  if (top < lo) return;
-  const int bot = max(lo, top - 3), nd = top - bot + 1;
-  const double sc = scale_eff[pp];
-  const double i2s2 = 1.0 / (2.0 * sc * sc), i4s2 = 1.0 / (4.0 * sc * sc), s2x2 = 2.0 * sc * sc;
-  const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int ln = t & 63, col = ln & 15, kq = ln >> 4;
-  const int ct = w;                             // A column tile of this wave (all row tiles)
-  const int part = w & 1;                       // C part: 0 real, 1 imaginary
-  const int ct2 = BLK ? (w >> 1) : 0;           // C column tile
-  const int q0 = qlm(bot, 0);
-  // Every workgroup steps four degrees top - dd; those below bot (dd >= nd,
-  // only when L < 15) are computed into accumulators that are never
-  // stored, so the degree loops carry no branches.  LDS offset of this
-  // lane's A operand rows per degree: real row 16 rt + col = 2 m1 + (Re, Im)
-  // of row tile rt (rows m1 > l read row l, degrees below bot read bot:
-  // never stored)
-  int arow[4][Cf::RTW];
-#pragma unroll
-  for (int dd = 0; dd < 4; ++dd) {
-    const int l = max(top - dd, bot);
-#pragma unroll
-    for (int rt = 0; rt < Cf::RTW; ++rt)
-      arow[dd][rt] = (2 * (qlm(l, min((16 * rt + col) >> 1, l)) - q0) + (col & 1)) * (kJL + 1);
-  }
-  v4d cacc[Cf::NC];
-#pragma unroll
-  for (int q = 0; q < Cf::NC; ++q) cacc[q] = v4d{0.0, 0.0, 0.0, 0.0};
-  const int Ng = d.ngath;
-  // Y1 of the pair (reads past its end return zero); this thread stages
-  // row (t >> 4) + 16 i of the quarter and atom t & 15 of each chunk
-  const __amdgpu_buffer_rsrc_t ry1 = buf_rsrc(Y1 + d.ylm_off, (int)(plane_rows(d.L) * Ng * 16));
-  const int vy1 = ((t >> 4) * Ng + (t & 15)) * 16;
-  for (int g = 0; g < d.ngroups; ++g) {
-    const SphGroup G = grp[d.group_off + g];
-    const int Ns = G.size, go = G.gath_off;
-    const long long ss = (long long)Ns * Ns;
-    // stored K_h and K_{h+1} of the group ([j][k]; reads past the end: zero)
-    const __amdgpu_buffer_rsrc_t rq0 = buf_rsrc(R + d.rad_off + G.rad_off + 2 * BLK * ss, (int)(ss * 8));
-    const __amdgpu_buffer_rsrc_t rq1 =
-        buf_rsrc(R + d.rad_off + G.rad_off + (2 * BLK + 1) * ss, (int)(ss * 8));
-    const double2* Y2g = Y2 + d.ylm_off + go;
-    const double* ra1 = rad1 + d.gath_off + go;  // |x| of the group's atoms
-    const double* ra2 = rad2 + d.gath_off + go;
-    for (int k0 = 0; k0 < Ns; k0 += KT) {
-      const int kk = k0 + 16 * ct + col;  // this lane's B operand column
-      const bool kok = kk < Ns;
-      const double r2 = kok ? ra2[kk] : 0.0;
-      // 1/x = (1/r1) (1/(r2 i2s2)): the second factor per lane, 0 for
-      // columns beyond the group (their entries stay zero)
-      const double ir2 = !kok ? 0.0 : (r2 > 0.0 ? s2x2 / r2 : kBig);
-      // byte offset of entry (4 s4 + kq, kk) of a chunk, past the end for
-      // columns beyond the group
-      const int vq = kok ? (kq * Ns + kk) * 8 : 0x7ff00000;
-      v4d acc[4][Cf::RTW];
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int rt = 0; rt < Cf::RTW; ++rt) acc[q][rt] = v4d{0.0, 0.0, 0.0, 0.0};
-      // registers of the next chunk: Y1 entries, the stored K_h, K_{h+1}
-      // of this lane's entries, one radius (-1: no atom)
-      double2 yb[Cf::NYI];
-      double kh[kNS4], kh1[kNS4], rjv = -1.0;
-#define FO_LOW_LOAD_CHUNK(J0)                                                               \
-  {                                                                                         \
-    const int j0_ = (J0);                                                                   \
-    _Pragma("unroll") for (int i = 0; i < Cf::NYI; ++i)                                     \
-      yb[i] = load_d2(ry1, vy1 + ((q0 + 16 * i) * Ng + go + j0_) * 16, 0);                  \
-    _Pragma("unroll") for (int s4 = 0; s4 < kNS4; ++s4) {                                   \
-      const int o_ = vq + (j0_ + 4 * s4) * Ns * 8;                                          \
-      kh[s4] = load_d(rq0, o_, 0);                                                          \
-      kh1[s4] = load_d(rq1, o_, 0);                                                         \
-    }                                                                                       \
-    if (t < kJL) rjv = j0_ + t < Ns ? ra1[j0_ + t] : -1.0;                                  \
-  }
-      const int nch = (Ns + kJL - 1) / kJL;
-      FO_LOW_LOAD_CHUNK(0);
-      for (int c = 0; c < nch; ++c) {
-        const int j0 = c * kJL;
-        __syncthreads();  // readers of the previous chunk (or tile) are done
-#pragma unroll
-        for (int i = 0; i < Cf::NYI; ++i) {
-          const int qq = (t >> 4) + 16 * i;
-          if (qq < Cf::NQ) {
-            S.u.y1[2 * qq][t & 15] = yb[i].x;
-            S.u.y1[2 * qq + 1][t & 15] = yb[i].y;
-          }
-        }
-        if (t < kJL) {
-          S.rj[t] = rjv;
-          S.irj[t] = rjv > 0.0 ? 1.0 / rjv : (rjv == 0.0 ? kBig : 0.0);
-        }
-        double cur[kNS4], up[kNS4];
-#pragma unroll
-        for (int s4 = 0; s4 < kNS4; ++s4) {
-          cur[s4] = kh[s4];
-          up[s4] = kh1[s4];
-        }
-        __syncthreads();
-        if (c + 1 < nch) FO_LOW_LOAD_CHUNK(j0 + kJL)
-        // entries (j0 + 4 s4 + kq, kk): cx = 1/x (0 for empty entries);
-        // for x < 2^-40 the series, which is x^l/(2l+1)!! e^{-x} g to FP64
-        // precision there (its next term is below 2^-81 relative, and
-        // e^{-x} = 1 - x): cx = e^{-x} g, and the recurrence values are
-        // replaced at every degree
-        double cx[kNS4];
-        int tiny = 0;
-#pragma unroll
-        for (int s4 = 0; s4 < kNS4; ++s4) {
-          cx[s4] = S.irj[4 * s4 + kq] * ir2;
-          if (cx[s4] > 0x1p40) {
-            tiny |= 1 << s4;
-            const double r1 = S.rj[4 * s4 + kq], x = r1 * r2 * i2s2;
-            cx[s4] = (1.0 - x) * exp(-(r1 - r2) * (r1 - r2) * i4s2);
-          }
-        }
-        // degrees above this quarter: recurrence only
-        for (int l = h; l > top; --l) {
-          const double cl = 2.0 * l + 1.0;
-#pragma unroll
-          for (int s4 = 0; s4 < kNS4; ++s4) {
-            const double nx = up[s4] + cl * cx[s4] * cur[s4];
-            up[s4] = cur[s4];
-            cur[s4] = nx;
-          }
-        }
-#pragma unroll
-        for (int dd = 0; dd < 4; ++dd) {
-          const int l = top - dd;
-          if (tiny) {
-            const int la = max(l, 0);
-#pragma unroll
-            for (int s4 = 0; s4 < kNS4; ++s4)
-              if (tiny & (1 << s4))
-                cur[s4] = ipow(S.rj[4 * s4 + kq] * r2 * i2s2, la) * cx[s4] * kInvDfact[la];
-          }
-          double ya[Cf::RTW][kNS4];
-#pragma unroll
-          for (int rt = 0; rt < Cf::RTW; ++rt)
-#pragma unroll
-            for (int s4 = 0; s4 < kNS4; ++s4) ya[rt][s4] = (&S.u.y1[0][0])[arow[dd][rt] + 4 * s4 + kq];
-#pragma unroll
-          for (int s4 = 0; s4 < kNS4; ++s4)
-#pragma unroll
-            for (int rt = 0; rt < Cf::RTW; ++rt) acc[dd][rt] = mfma64(ya[rt][s4], cur[s4], acc[dd][rt]);
-          const double cl = 2.0 * l + 1.0;
-#pragma unroll
-          for (int s4 = 0; s4 < kNS4; ++s4) {
-            const double nx = up[s4] + cl * cx[s4] * cur[s4];
-            up[s4] = cur[s4];
-            cur[s4] = nx;
-          }
-        }
-      }
-      // second product, two degrees at a time: their Y2_l rows m2 = 0..l
-      // (entry k = k0 + e % KT, m2 = e / KT, coalesced in k; the columns
-      // m2 < 0 are formed when read, Y_l^{-m} = (-1)^m conj(Y_l^m)) and
-      // their A_l tiles -> LDS (the A tiles aliasing the chunk buffer), then
-      // C^l += A_l conj(Y2_l)^T
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int tl = opaque_lane(t), cl_ = tl & 15, kq_ = (tl >> 4) & 3;
-        double2 yv[2][Cf::NYV];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int dd = 2 * hh + q, l_ = top - dd;
-#pragma unroll
-          for (int i = 0; i < Cf::NYV; ++i) {
-            const int e = tl + 256 * i, k = k0 + e % KT, m2 = e / KT;
-            yv[q][i] = (dd < nd && m2 <= l_ && k < Ns) ? Y2g[(long long)qlm(l_, m2) * Ng + k]
-                                                        : make_double2(0.0, 0.0);
-          }
-        }
-        __syncthreads();  // readers of the last chunk / the previous pair of degrees are done
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int dd = 2 * hh + q, l = top - dd;
-#pragma unroll
-          for (int rt = 0; rt < Cf::RTW; ++rt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int r = 16 * rt + 4 * i + kq_, m1 = r >> 1;
-              if (m1 <= l) ((double*)&S.u.ac[q][m1][16 * ct + cl_])[r & 1] = acc[dd][rt][i];
-            }
-#pragma unroll
-          for (int i = 0; i < Cf::NYV; ++i) {
-            const int e = tl + 256 * i;
-            S.ys[q][e % KT][e / KT] = yv[q][i];  // rows m2 > l hold zeros
-          }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int dd = 2 * hh + q, l = top - dd;
-          if (BLK || (w >> 1) == (dd & 1)) {  // uniform
-            v4d& cq = cacc[BLK ? dd : (dd >> 1)];
-            // column m = 16 ct2 + col of C: m2 = m - l, read as row |m2|
-            // (times -1 for odd negative m2, conjugated for negative m2)
-            const int m2 = 16 * ct2 + cl_ - l, am2 = min(abs(m2), Cf::NM - 1);
-            const double sr = (m2 < 0 && (m2 & 1)) ? -1.0 : 1.0;
-            const double si = m2 < 0 ? -sr : sr;
-            const bool rok = cl_ <= l;
-            const int ar = min(cl_, Cf::AR - 1);
-#pragma unroll 4
-            for (int s = 0; s < KT / 4; ++s) {
-              const int kk2 = 4 * s + kq_;
-              const double2 av = rok ? S.u.ac[q][ar][kk2] : make_double2(0.0, 0.0);
-              const double2 yr = S.ys[q][kk2][am2];
-              const double a0 = part ? av.y : av.x, a1 = part ? -av.x : av.y;
-              cq = mfma64(a0, sr * yr.x, cq);
-              cq = mfma64(a1, si * yr.y, cq);
-            }
-          }
-        }
-      }
-#undef FO_LOW_LOAD_CHUNK
-    }
-  }
-  // C^l of the four degrees: both parts of an entry through LDS, then one
-  // lane writes it (FP64 compact and FP32 plane layouts)
-  const double norm = 4.0 * pow(kPi, 2.5) * sc * sc * sc;
-#pragma unroll
-  for (int dd = 0; dd < 4; ++dd) {
-    if (dd < nd) {
-      const int l = top - dd, M = 2 * l + 1, tl = opaque_lane(t);
-      __syncthreads();
-      if (BLK || (w >> 1) == (dd & 1)) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 4 * i + ((tl >> 4) & 3);
-          if (r < Cf::AR)
-            ((double*)&S.u.ac[0][r][16 * ct2 + (tl & 15)])[part] = cacc[BLK ? dd : (dd >> 1)][i];
-        }
-      }
-      __syncthreads();
-      for (int e = tl; e < Cf::AR * Cf::NMC; e += 256) {
-        const int r = e / Cf::NMC, mc = e % Cf::NMC;
-        if (r <= l && mc < M) {
-          const int m2 = mc - l;
-          const double2 cv = S.u.ac[0][r][mc];
-          const double2 v = make_double2(norm * cv.x, norm * cv.y);
-          I64[d.coef_off + kidx(l, r, m2)] = v;
-          I32[d.c32_off + (long long)qlm(l, r) * n + plane_pos(plane_k(m2, n), n)] =
-              make_float2((float)v.x, (float)v.y);
-        }
-      }
-    }
   }
 }
 
@@ -2894,43 +2209,6 @@ void launch_sph_radial(hipStream_t s, int P, int Lmax, long long maxjk, const Sp
   (void)Lmax;  // one kernel for every degree
   hipLaunchKernelGGL(k_sph_radial, dim3(bx, P), dim3(256), 0, s, pd, grp, rad1, rad2, scale_eff,
                      R);
-}
-
-void launch_sph_contract(hipStream_t s, int P, int n, int Lmax, const SphPair* pd,
-                         const SphGroup* grp, const double* rad1, const double* rad2,
-                         const double2* Y1, const double2* Y2, const double* R,
-                         const double* scale_eff, double2* I64, float2* I32) {
-  // degrees 0..15: radial recurrence and contraction fused, one workgroup
-  // per (pair, block of eight degrees); degrees >= 16: one launch per
-  // column-tile class, workgroups per (pair, degree, block of 32 rows)
-  const dim3 b(256), gl(xcd_grid(P, 2));
-  hipLaunchKernelGGL(k_sph_contract_low<0>, gl, b, 0, s, pd, grp, rad1, rad2, Y1, Y2, R,
-                     scale_eff, I64, I32, n, P);
-  if (Lmax >= 8)
-    hipLaunchKernelGGL(k_sph_contract_low<1>, gl, b, 0, s, pd, grp, rad1, rad2, Y1, Y2, R,
-                       scale_eff, I64, I32, n, P);
-  auto launch = [&](int K, int lo, int hi) {
-    hi = std::min(hi, Lmax);
-    if (lo > hi) return;
-    int nb = 0;
-    const int MB = K <= 2 ? contract_rows<2>() : contract_rows<4>();
-    for (int l = lo; l <= hi; ++l) nb += (l + 1 + MB - 1) / MB;
-    const dim3 g(xcd_grid(P, nb));
-    if (K == 4)
-      hipLaunchKernelGGL(k_sph_contract_mfma<4>, g, b, 0, s, pd, grp, Y1, Y2, R, scale_eff, I64,
-                         I32, n, P, nb, lo, hi);
-    else if (K == 6)
-      hipLaunchKernelGGL(k_sph_contract_mfma<6>, g, b, 0, s, pd, grp, Y1, Y2, R, scale_eff, I64,
-                         I32, n, P, nb, lo, hi);
-    else
-      hipLaunchKernelGGL(k_sph_contract_mfma<8>, g, b, 0, s, pd, grp, Y1, Y2, R, scale_eff, I64,
-                         I32, n, P, nb, lo, hi);
-  };
-  // column-tile classes: 2l+1 <= 64 / 96 / 128 (the six-tile class holds two
-  // waves per SIMD and two workgroups per CU, the eight-tile class one)
-  launch(4, 16, 31);
-  launch(6, 32, 47);
-  launch(8, 48, 63);
 }
 
 // two-pass factorisation n = N1 N2 of the power-of-two grids (0: direct DFT)

@@ -602,3 +602,28 @@ def test_autotuner_shapes_give_identical_results(gpu):
             np.testing.assert_array_equal(a, e)
         for a, e in zip(got[2], ref[2]):
             np.testing.assert_array_equal(a, e)
+
+
+@pytest.mark.parametrize("L,sizes", [
+    (7, [1, 15]), (8, [16, 49]), (15, [17, 160]), (16, [33, 64, 0, 3]), (17, [31]), (23, [48, 16]),
+    (24, [65]), (31, [130, 31]), (32, [47]), (39, [16, 15]), (40, [161]), (47, [18]), (48, [5, 40]),
+    (49, [33])])
+def test_coefficients_across_row_classes(gpu, L, sizes):
+    """C^l at the edges of the contraction's row classes (eight degrees each, up
+    to the largest degree whose planes fit), of its 16-atom tiles and of the blocks of several
+    tiles, with an empty group, and on both sides of the size at which a
+    pair's items take four wavefronts (160 grouped atoms)."""
+    say(f"case: Jmax {L}, groups {sizes}")
+    rng = np.random.default_rng(L)
+    N = sum(sizes)
+    X1, X2 = (rng.normal(size=(N, 3)) * 1.3 for _ in range(2))
+    off = np.cumsum([0] + sizes)
+    order = rng.permutation(N)
+    groups = [order[off[i]:off[i + 1]] for i in range(len(sizes))]
+    with SphericalBatch([N], [L], 0.35, 64 if L <= 31 else 2 * (L + 1), [groups],
+                        _lib.SPH_NO_INVERT | _lib.SPH_NO_CENTER) as b:
+        b.set_positions(X1, X2)
+        b.run(_lib.STAGE_PREP | _lib.STAGE_COEFF)
+        got = compact_to_dense(b.coeffs()[0], L)
+    ref = O.so3_coeffs_species(X1, X2, [g for g in groups if len(g)], L, 0.35, fast=True)
+    np.testing.assert_allclose(got, ref, atol=1e-12 * np.abs(ref).max())

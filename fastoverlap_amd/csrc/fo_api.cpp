@@ -30,7 +30,7 @@ void launch_wigner_table(hipStream_t, int, int, double*, float*);
 void launch_twiddles(hipStream_t, int, double, double2*, float2*);
 void launch_sph_prep(hipStream_t, int, const SphPair*, const double*, const double*, double*,
                      double*, double*, int);
-void launch_sph_ylm(hipStream_t, int, const SphPair*, const int*, const double*, const double*,
+void launch_sph_ylm(hipStream_t, int, int, const SphPair*, const int*, const double*, const double*,
                     const double2*, const double*, double2*, double2*, double*, double*);
 void launch_sph_radial(hipStream_t, int, int, long long, const SphPair*, const SphGroup*,
                        const double*, const double*, const double*, double*, int);
@@ -542,7 +542,7 @@ static int sph_enqueue(fo_sph_batch* b, int stages) {
       const SphPair* pdc = b->pd + C.p0;
       const double* scc = b->scale + C.p0;
       cmark(3 * c);
-      launch_sph_ylm(s, Pc, pdc, b->gath, b->X1c, b->X2c, b->rect->leg, b->rect->cm, b->Y1, b->Y2,
+      launch_sph_ylm(s, Pc, L.maxgath, pdc, b->gath, b->X1c, b->X2c, b->rect->leg, b->rect->cm, b->Y1, b->Y2,
                      b->rad, b->rad + b->hgath.size());
       cmark(3 * c + 1);
       if (b->harm_nmax >= 0) {

@@ -168,42 +168,77 @@ __global__ void k_sph_prep(const SphPair* __restrict__ pd, const double* __restr
 // fastoverlap/sphericalAlignment.py:57-65), FP64, for m >= 0 only:
 //   Y[q(l,m)][g] = P_l^m(cos theta) e^{i m phi},  q(l,m) = l(l+1)/2 + m,
 // with P the normalised associated Legendre function (Condon-Shortley
-// phase); Y_l^{-m} = (-1)^m conj(Y_l^m) is formed where it is read.  One
-// thread per (atom, m): P_m^m = c_m sin^m(theta), then the three-term
-// recurrence in l with tabulated coefficients (k_leg_table).  An atom at the
-// centre takes theta = phi = 0 (only l = 0 survives there).
+// phase); Y_l^{-m} = (-1)^m conj(Y_l^m) is formed where it is read.  A
+// workgroup takes `atoms` atoms of one structure: first one lane per
+// atom forms the distance, the cosine and sine of theta and the unit phase
+// e^{i phi} = (x, y) / |(x, y)|, then one lane per (atom, m) raises the phase
+// and the sine to the power m by squaring and runs the three-term recurrence
+// in l with tabulated coefficients (k_leg_table).  An atom at the centre
+// takes theta = phi = 0 (only l = 0 survives there).  Bound by the writes
+// where a batch fills the chip: 64 pairs of 1000 atoms at L = 40 (1.8 GB) take
+// 322 us (790 with one workgroup per structure and a sine, cosine and
+// arctangent per (atom, m)), 4096 pairs of 13..147 atoms (2.6 GB) 660 us; one
+// pair of 38 atoms 6 us (10).
 // ---------------------------------------------------------------------------
-__global__ void k_sph_ylm(const SphPair* __restrict__ pd, const int* __restrict__ gath,
-                          const double* __restrict__ X1c, const double* __restrict__ X2c,
-                          const double2* __restrict__ leg, const double* __restrict__ cm,
-                          double2* __restrict__ Y1, double2* __restrict__ Y2,
-                          double* __restrict__ rad1, double* __restrict__ rad2) {
+constexpr int kYlmAtoms = 256;  // most atoms of a workgroup
+
+__global__ void __launch_bounds__(256) k_sph_ylm(
+    int atoms, const SphPair* __restrict__ pd, const int* __restrict__ gath,
+    const double* __restrict__ X1c, const double* __restrict__ X2c,
+    const double2* __restrict__ leg, const double* __restrict__ cm, double2* __restrict__ Y1,
+    double2* __restrict__ Y2, double* __restrict__ rad1, double* __restrict__ rad2) {
+  __shared__ double2 theta[kYlmAtoms];  // cos, sin
+  __shared__ double2 phase[kYlmAtoms];  // e^{i phi}
   const SphPair d = pd[blockIdx.x];
-  const double* X = blockIdx.y ? X2c : X1c;
-  double2* Yp = (blockIdx.y ? Y2 : Y1) + d.ylm_off;
-  double* rad = (blockIdx.y ? rad2 : rad1) + d.gath_off;
   const int L = d.L, Ng = d.ngath;
-  for (int w = threadIdx.x; w < Ng * (L + 1); w += blockDim.x) {
-    const int m = w / Ng, g = w % Ng;
+  const int g0 = blockIdx.z * atoms, na = min(Ng - g0, atoms);
+  if (na <= 0) return;
+  const double* X = blockIdx.y ? X2c : X1c;
+  double2* Yp = (blockIdx.y ? Y2 : Y1) + d.ylm_off + g0;
+  if ((int)threadIdx.x < na) {
+    const int g = g0 + threadIdx.x;
     const int a = gath[d.gath_off + g];
     const double x = X[3LL * (d.atom_off + a)], y = X[3LL * (d.atom_off + a) + 1],
                  z = X[3LL * (d.atom_off + a) + 2];
     const double rxy = sqrt(x * x + y * y), r = sqrt(x * x + y * y + z * z);
-    if (m == 0) rad[g] = r;  // |x| per grouped atom, for the fused contraction
-    double ct = 1.0, st = 0.0, phi = 0.0;
+    (blockIdx.y ? rad2 : rad1)[d.gath_off + g] = r;  // |x| per grouped atom
+    double ct = 1.0, st = 0.0, cp = 1.0, sp = 0.0;
     if (r > 0.0) {
       ct = z / r;
       st = rxy / r;
-      phi = atan2(y, x);
+      // scaled by a power of two, so that squares of the smallest
+      // coordinates keep their digits; one Newton step takes the modulus to
+      // 1 within rounding, as its error would grow with m
+      const double big = fmax(fabs(x), fabs(y));
+      if (big > 0.0) {
+        const int e = ilogb(big);
+        const double xs = ldexp(x, -e), ys = ldexp(y, -e);
+        const double h = sqrt(fma(xs, xs, ys * ys));
+        cp = xs / h;
+        sp = ys / h;
+        const double dev = 0.5 * fma(-sp, sp, fma(-cp, cp, 1.0));
+        cp = fma(cp, dev, cp);
+        sp = fma(sp, dev, sp);
+      }
     }
-    double sp, cp;
-    sincos((double)m * phi, &sp, &cp);
+    theta[threadIdx.x] = make_double2(ct, st);
+    phase[threadIdx.x] = make_double2(cp, sp);
+  }
+  __syncthreads();
+  for (int w = threadIdx.x; w < na * (L + 1); w += blockDim.x) {
+    const int m = w / na, g = w % na;
+    const double ct = theta[g].x, st = theta[g].y;
+    double2 b = phase[g], u = make_double2(1.0, 0.0);
+    for (int k = m; k; k >>= 1) {
+      if (k & 1) u = make_double2(fma(u.x, b.x, -u.y * b.y), fma(u.x, b.y, u.y * b.x));
+      b = make_double2(fma(b.x, b.x, -b.y * b.y), 2.0 * b.x * b.y);
+    }
     double p2 = 0.0, p1 = cm[m] * ipow(st, m);
-    Yp[(long long)qlm(m, m) * Ng + g] = make_double2(p1 * cp, p1 * sp);
+    Yp[(long long)qlm(m, m) * Ng + g] = make_double2(p1 * u.x, p1 * u.y);
     for (int l = m + 1; l <= L; ++l) {
       const double2 ab = leg[qlm(l, m)];
       const double pl = ab.x * (ct * p1 - ab.y * p2);
-      Yp[(long long)qlm(l, m) * Ng + g] = make_double2(pl * cp, pl * sp);
+      Yp[(long long)qlm(l, m) * Ng + g] = make_double2(pl * u.x, pl * u.y);
       p2 = p1;
       p1 = pl;
     }
@@ -2193,11 +2228,19 @@ void launch_sph_prep(hipStream_t s, int P, const SphPair* pd, const double* pos1
                      center);
 }
 
-void launch_sph_ylm(hipStream_t s, int P, const SphPair* pd, const int* gath, const double* X1c,
+void launch_sph_ylm(hipStream_t s, int P, int maxgath, const SphPair* pd, const int* gath, const double* X1c,
                     const double* X2c, const double2* leg, const double* cm, double2* Y1,
                     double2* Y2, double* rad1, double* rad2) {
-  hipLaunchKernelGGL(k_sph_ylm, dim3(P, 2), dim3(256), 0, s, pd, gath, X1c, X2c, leg, cm, Y1, Y2,
-                     rad1, rad2);
+  // The rows of Y are written in runs of a workgroup's atoms: as long as the
+  // batch fills the chip (2048 workgroups), as the lines that two workgroups
+  // share are written twice (the 4096-pair batch: 660 us at 256, 870 at 64,
+  // 1250 at 16), else short ones for more workgroups (96 pairs of 20..120
+  // atoms: 14 us at 16, 20 at 64; one pair: 6 and 9).  An element's value does
+  // not depend on the split.
+  int atoms = kYlmAtoms;
+  while (atoms > 16 && P * 2LL * cdiv(maxgath, atoms) < 2048) atoms /= 4;
+  hipLaunchKernelGGL(k_sph_ylm, dim3(P, 2, std::max(1, cdiv(maxgath, atoms))), dim3(256), 0, s,
+                     atoms, pd, gath, X1c, X2c, leg, cm, Y1, Y2, rad1, rad2);
 }
 
 void launch_sph_radial(hipStream_t s, int P, int Lmax, long long maxjk, const SphPair* pd,

@@ -627,3 +627,31 @@ def test_coefficients_across_row_classes(gpu, L, sizes):
         got = compact_to_dense(b.coeffs()[0], L)
     ref = O.so3_coeffs_species(X1, X2, [g for g in groups if len(g)], L, 0.35, fast=True)
     np.testing.assert_allclose(got, ref, atol=1e-12 * np.abs(ref).max())
+
+
+def test_harmonics_split_over_workgroups(gpu):
+    """Y_lm of a structure is the same, bit for bit, in a small batch (16 atoms
+    a workgroup) and in a large one (256), at the edges of both, with atoms at
+    the centre, on the z axis and so near it that the squares underflow."""
+    L, sizes = 6, [1, 15, 16, 17, 65, 257]
+    rng = np.random.default_rng(3)
+    Xs = [[rng.normal(size=(N, 3)) for _ in range(2)] for N in sizes]
+    for A, B in Xs[1:]:
+        A[0], A[1], A[2], B[3] = 0.0, (0, 0, -1.1), (3e-170, -1e-170, 0.7), (0, 0.8, 0)
+
+    def coeffs(reps):
+        P = reps * len(sizes)
+        with SphericalBatch(sizes * reps, [L] * P, 0.4, 16, [[np.arange(N)] for N in sizes] * reps,
+                            _lib.SPH_NO_INVERT | _lib.SPH_NO_CENTER) as b:
+            b.set_positions(np.concatenate([x[0] for x in Xs] * reps),
+                            np.concatenate([x[1] for x in Xs] * reps))
+            b.run(_lib.STAGE_PREP | _lib.STAGE_COEFF)
+            return b.coeffs()
+
+    say(f"case: {len(sizes)} pairs, then 180 times as many")
+    few, many = coeffs(1), coeffs(180)
+    for p in range(len(many)):
+        np.testing.assert_array_equal(many[p], few[p % len(sizes)])
+    for got, (A, B) in zip(few, Xs):
+        ref = O.so3_coeffs_species(A, B, [np.arange(len(A))], L, 0.4, fast=True)
+        np.testing.assert_allclose(compact_to_dense(got, L), ref, atol=1e-12 * np.abs(ref).max())

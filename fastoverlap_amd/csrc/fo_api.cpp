@@ -39,7 +39,6 @@ void launch_harm_coeffs(hipStream_t, int, int, int, int, const SphPair*, const S
                         const double*, const double2*, const double2*, double*, int, double2*,
                         float2*);
 void launch_coef_norm2(hipStream_t, int, const SphPair*, const double2*, double*);
-int harm_block_lx(int L, int nmax, int basis);
 void launch_sph_contract(hipStream_t, int, int, int, int, int, const SphPair*, const SphGroup*,
                          const double*, const double*, const double2*, const double2*,
                          const double*, const double*, double2*, float2*);
@@ -713,11 +712,11 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
     C32tot += plane_rows(Lp) * n;
     // coefficient chunks: K and Y offsets are relative to the pair's chunk
     // radial block: K_l[j][k] of every group, or for the harmonic basis
-    // D[j][l][n] of both structures then c[group][q(l,m)][n] of both
+    // the projections kept in memory, then c[group][q(l,m)][n] of both structures
     const long long nn = harm_nmax + 1;
-    const long long lx = harm_nmax >= 0 ? harm_block_lx(Lp, harm_nmax, b->harm_basis) : 0;
     const long long rs = harm_nmax >= 0
-                             ? 2 * ng * (lx + 1) * nn + 4 * (long long)sp.ngroups * plane_rows(Lp) * nn
+                             ? harm_proj_doubles(ng, Lp, harm_nmax, b->harm_basis) +
+                                   4 * (long long)sp.ngroups * plane_rows(Lp) * nn
                              : (long long)rad_slots(Lp) * jk;
     const long long ys = (long long)(Lp + 1) * (Lp + 2) / 2 * ng;
     b->maxgroups = std::max(b->maxgroups, sp.ngroups);
@@ -946,8 +945,8 @@ int fo_sph_batch_harmonic_coeffs(fo_sph_batch* b, int pair, double* c1, double* 
   const SphPair& d = b->hp[pair];
   const size_t nn = b->harm_nmax + 1;
   const size_t one = (size_t)d.ngroups * plane_rows(d.L) * nn;
-  const size_t lx = harm_block_lx(d.L, b->harm_nmax, b->harm_basis);
-  const double* base = b->R + d.rad_off + 2 * (size_t)d.ngath * (lx + 1) * nn;
+  const double* base =
+      b->R + d.rad_off + harm_proj_doubles(d.ngath, d.L, b->harm_nmax, b->harm_basis);
   FO_HIP(hipSetDevice(b->ctx->device));
   if (c1) FO_HIP(hipMemcpyAsync(c1, base, sizeof(double2) * one, hipMemcpyDeviceToHost, b->stream));
   if (c2)

@@ -32,6 +32,13 @@ struct SphGroup {
   long long rad_off;   // (L+1) * jk_off : offset inside the pair's radial block
 };
 
+// Doubles of a pair's block that hold the harmonic basis' projections of both
+// structures, D[atom][degree <= L + 2 nmax][n] (basis 1; basis 0 keeps its
+// projections in LDS).
+__host__ __device__ inline long long harm_proj_doubles(int ngath, int L, int nmax, int basis) {
+  return basis ? 2LL * ngath * (L + 2 * nmax + 1) * (nmax + 1) : 0;
+}
+
 // Per (pair, orientation, plane) candidate record written by the plane
 // kernels: the plane's values are split into kCandPerPlane parts (the
 // spherical kernels: one per wavefront) and entry r lists the largest value

@@ -36,6 +36,20 @@ def test_harmonic_coefficients_match_oracle(gpu):
     np.testing.assert_allclose(I, Io, rtol=0, atol=1e-10 * np.abs(Io).max())
 
 
+@pytest.mark.parametrize("N,Jmax,nmax", [(1, 0, 0), (63, 3, 1), (64, 12, 6), (65, 15, 15),
+                                         (129, 7, 0)])
+def test_harmonic_coefficients_over_atom_tiles(gpu, N, Jmax, nmax):
+    """Coefficients at the edges of the 64-atom tiles, of the radial degrees
+    and of the basis degrees (the bound is that of the test above)."""
+    print(f"case: {N} atoms, Jmax {Jmax}, nmax {nmax}", flush=True)
+    _, X = _cloud(N, N)
+    if N == 1:
+        X = X + 0.7
+    A = fo.SphericalHarmonicAlign(scale=0.35, harmscale=1.1, nmax=nmax, Jmax=Jmax)
+    o = O.harmonic_coeff(X, Jmax, nmax, 0.35, 1.1)
+    np.testing.assert_allclose(A.calcHarmCoeff(X), o, rtol=0, atol=1e-10 * np.abs(o).max())
+
+
 def _check(A, p1, p2, groups, Jmax, nmax, scale, r0):
     d, X1, X2 = A.align(p1, p2)
     o = O.harmonic_align(p1, p2, Jmax, nmax, scale=scale, r0=r0,

@@ -60,8 +60,7 @@ void launch_sph_finish(hipStream_t, int, int, const SphPair*, const SphGroup*, c
                        double*, SphResult*);
 void launch_coef_to_plane(hipStream_t, int, int, int, const SphPair*, const double2*, float2*);
 void launch_soft_forward(hipStream_t, int, long long, const double*, const double2*, const double2*,
-                         double*, double2*, double2*);
-size_t soft_forward_smem(int);
+                         double2*, double2*);
 void launch_sph_mirror(hipStream_t, int, int, const SphPair*, double2*);
 void launch_sph_energy(hipStream_t, int, const double2*, double, double, double, const double*,
                        const double*, int, double*);
@@ -122,6 +121,7 @@ static bool all_finite(const double* p, size_t n) {
   return true;
 }
 static constexpr int kMaxL = 63;
+static constexpr int kSoftMaxBw = 50;  // bandwidth of the forward transform of a grid
 static constexpr int kMaxGroup = 4096;
 static constexpr int kHarmMaxN = 40;  // harmonic basis radial degree
 
@@ -1474,7 +1474,7 @@ int fo_soft_forward(fo_context* c, int bw, const double* data, double* flmm) {
   if (!c || !data || !flmm || bw < 1 || bw - 1 > kMaxL)
     return set_err(FO_ERR_INVALID, "bad argument");
   const int n = 2 * bw, L = bw - 1, W = 2 * L + 1;
-  if (soft_forward_smem(n) > c->max_lds)
+  if (bw > kSoftMaxBw)
     return set_err(FO_ERR_UNSUPPORTED, "bandwidth too large for the forward transform");
   const SphTable* t = nullptr;
   int rc = get_sph_table(c, n, &t);
@@ -1484,24 +1484,23 @@ int fo_soft_forward(fo_context* c, int bw, const double* data, double* flmm) {
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
   const size_t n3 = (size_t)n * n * n, K = (size_t)kcount(L);
   const size_t bg = up(sizeof(double2) * n3), bs = up(sizeof(double2) * (size_t)W * n * W);
-  const size_t bk = up(sizeof(double2) * K), bw8 = up(sizeof(double) * n);
+  const size_t bk = up(sizeof(double2) * K);
   void* base = nullptr;
-  rc = ctx_alloc(c, bg + bs + bk + bw8, &base);
+  rc = ctx_alloc(c, bg + bs + bk, &base);
   if (rc) return rc;
   char* p = (char*)base;
   double2* dg = (double2*)p;
   double2* S2 = (double2*)(p + bg);
   double2* df = (double2*)(p + bg + bs);
-  double* w = (double*)(p + bg + bs + bk);
   hipError_t e = hipMemcpyAsync(dg, data, sizeof(double2) * n3, hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess) {
-    launch_soft_forward(c->stream, n, t->Kt, t->tab64, t->tw64, dg, w, S2, df);
+    launch_soft_forward(c->stream, n, t->Kt, t->tab64, t->tw64, dg, S2, df);
     e = hipGetLastError();
   }
   if (e == hipSuccess)
     e = hipMemcpyAsync(flmm, df, sizeof(double2) * K, hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  ctx_free(c, base, bg + bs + bk + bw8);
+  ctx_free(c, base, bg + bs + bk);
   if (e != hipSuccess) return set_err(FO_ERR_HIP, std::string("forward SOFT: ") + hipGetErrorString(e));
   return FO_OK;
 }

@@ -2534,77 +2534,126 @@ void launch_sph_mirror(hipStream_t s, int P, int Lmax, const SphPair* pd, double
 // for |m1|, |m2| <= L = n/2 - 1; w_k are the quadrature weights of
 // fastoverlap/soft.py:63-71.
 // ---------------------------------------------------------------------------
-__global__ void k_soft_weights(int bw, double* __restrict__ w) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < 2 * bw; k += gridDim.x * blockDim.x) {
-    const double a = (2.0 * k + 1.0) / (4.0 * bw);  // (2k+1) pi / (4 bw), in units of pi
-    double s = 0.0;
-    for (int j = 0; j < bw; ++j) s += 2.0 / (2.0 * j + 1.0) * sinpi((2.0 * j + 1.0) * a);
-    w[k] = s * sinpi(a) / bw;
-  }
-}
 
-// one workgroup per beta plane k: the 2D DFT of g[., k, .] at |m| <= L
-__global__ void k_soft_fwd_plane(int n, const double2* __restrict__ g,
-                                 const double2* __restrict__ tw, double2* __restrict__ S2) {
+// S2[m1][k][m2], already times w_k: one workgroup per 16 columns m2 and beta
+// plane k, both passes as FP64 matrix products of real and imaginary parts,
+//   T[j1][m2] = sum_{j2} g[j1][k][j2] e^{-2 pi i m2 j2/n},
+//   S2[m1][m2] = sum_{j1} e^{-2 pi i m1 j1/n} T[j1][m2],
+// with T in LDS between them.  Row tiles of 16 go round the wavefronts; what
+// lies past n is read as zero.
+// Tile layout of the FP64 product (lane = 16 r + c): A holds row c, inner r;
+// B inner r, column c; result i holds row 4 i + r, column c.
+constexpr int kSoftCols = 16;
+
+__global__ void __launch_bounds__(256) k_soft_fwd_plane(int n, const double2* __restrict__ g,
+                                                        const double2* __restrict__ tw,
+                                                        double2* __restrict__ S2) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int k = blockIdx.x, L = n / 2 - 1, W = 2 * L + 1, t = threadIdx.x;
-  double2* T = (double2*)smem;  // [n][W]: sum over j2 for each j1, m2
-  for (int e = t; e < n * W; e += blockDim.x) {
-    const int j1 = e / W, m2 = e % W - L;
-    double2 acc = make_double2(0.0, 0.0);
-    for (int j2 = 0; j2 < n; ++j2) {
-      // e^{-2 pi i m2 j2 / n} = conj(tw[(m2 j2) mod n])
-      const int q = ((m2 * j2) % n + n) % n;
-      acc = cadd(acc, cmul(g[((long long)j1 * n + k) * n + j2], cconj(tw[q])));
-    }
-    T[e] = acc;
+  const int k = blockIdx.y, L = n / 2 - 1, W = 2 * L + 1, t = threadIdx.x;
+  const int n16 = (n + 15) / 16 * 16;
+  double2* T = (double2*)smem;        // [n16][kSoftCols]
+  double2* E = T + n16 * kSoftCols;   // e^{-2 pi i q / n}
+  __shared__ double wk;
+  for (int q = t; q < n; q += blockDim.x) E[q] = cconj(tw[q]);
+  // quadrature weight of the plane, a term per lane
+  if (t < 64) {
+    const int bw = n / 2;
+    const double a = (2.0 * k + 1.0) / (4.0 * bw);  // (2k+1) pi / (4 bw), in units of pi
+    double v = 0.0;
+    for (int j = t; j < bw; j += 64) v += 2.0 / (2.0 * j + 1.0) * sinpi((2.0 * j + 1.0) * a);
+    v = wave_sum(v);
+    if (t == 0) wk = v * sinpi(a) / bw / ((double)n * n);
   }
   __syncthreads();
-  const double inv = 1.0 / ((double)n * n);
-  for (int e = t; e < W * W; e += blockDim.x) {
-    const int m1 = e / W - L, m2i = e % W;
-    double2 acc = make_double2(0.0, 0.0);
-    for (int j1 = 0; j1 < n; ++j1) {
-      const int q = ((m1 * j1) % n + n) % n;
-      acc = cadd(acc, cmul(T[j1 * W + m2i], cconj(tw[q])));
+  const int lane = t & 63, r = lane >> 4, c = lane & 15, wave = t >> 6;
+  const int m2 = blockIdx.x * kSoftCols + c;  // column of the row -L..L
+  // e^{-2 pi i m j / n} for j = r, r + 4, ...: index m j mod n, stepped by 4 m
+  const int mc = (m2 - L + n) % n;
+  const int step2 = 4 * mc % n, first2 = r * mc % n;
+  for (int rt = wave; rt * 16 < n; rt += 4) {
+    const int j1 = rt * 16 + c;
+    const double2* row = g + ((long long)j1 * n + k) * n;
+    v4d tr = {0, 0, 0, 0}, ti = {0, 0, 0, 0};
+    int q = first2;
+#pragma unroll 4
+    for (int j = r; j - r < n; j += 4) {
+      const double2 x = j1 < n && j < n ? row[j] : make_double2(0.0, 0.0);
+      const double2 e = E[q];
+      q += step2;
+      q -= q >= n ? n : 0;
+      tr = mfma64(x.x, e.x, tr);
+      ti = mfma64(x.x, e.y, ti);
+      tr = mfma64(-x.y, e.y, tr);
+      ti = mfma64(x.y, e.x, ti);
     }
-    S2[((long long)(m1 + L) * n + k) * W + m2i] = cscale(acc, inv);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      T[(rt * 16 + 4 * i + r) * kSoftCols + c] = make_double2(tr[i], ti[i]);
+  }
+  __syncthreads();
+  const double scale = wk;
+  for (int rt = wave; rt * 16 < W; rt += 4) {
+    const int m1 = rt * 16 + c;
+    const int mr = (m1 - L + n) % n;
+    const int step = 4 * mr % n;
+    int q = r * mr % n;
+    v4d sr = {0, 0, 0, 0}, si = {0, 0, 0, 0};
+#pragma unroll 4
+    for (int j = r; j - r < n; j += 4) {
+      const double2 x = T[j * kSoftCols + c], e = E[q];  // rows n.. of T are zero
+      q += step;
+      q -= q >= n ? n : 0;
+      sr = mfma64(e.x, x.x, sr);
+      si = mfma64(e.x, x.y, si);
+      sr = mfma64(-e.y, x.y, sr);
+      si = mfma64(e.y, x.x, si);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = rt * 16 + 4 * i + r;
+      if (row < W && m2 < W)
+        S2[((long long)row * n + k) * W + m2] = make_double2(scale * sr[i], scale * si[i]);
+    }
   }
 }
 
-// one thread per compact (l, m1, m2), l <= L
-__global__ void k_soft_fwd_beta(int n, long long Kt, const double* __restrict__ tab64,
-                                const double* __restrict__ w, const double2* __restrict__ S2,
-                                double2* __restrict__ f) {
-  const int L = n / 2 - 1, W = 2 * L + 1;
-  const long long K = kcount(L);
-  for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < K;
-       e += (long long)gridDim.x * blockDim.x) {
+// One compact (l, m1, m2), l <= L, per lane; the four wavefronts of a
+// workgroup take a quarter of the beta planes each.  Bound by the reads of the
+// Wigner table (22 MB at bandwidth 32: 14 us; 24 with one lane per sum).
+__global__ void __launch_bounds__(256) k_soft_fwd_beta(int n, long long Kt,
+                                                       const double* __restrict__ tab64,
+                                                       const double2* __restrict__ S2,
+                                                       double2* __restrict__ f) {
+  __shared__ double2 part[4][64];
+  const int L = n / 2 - 1, W = 2 * L + 1, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long long K = kcount(L), e = blockIdx.x * 64LL + lane;
+  double2 acc = make_double2(0.0, 0.0);
+  if (e < K) {
     int l = 0;
     while (kbase(l + 1) <= e) ++l;
     const int r = (int)(e - kbase(l));
     const int m1 = r / (2 * l + 1) - l, m2 = r % (2 * l + 1) - l;
-    double2 acc = make_double2(0.0, 0.0);
-    for (int k = 0; k < n; ++k)
-      acc = cadd(acc, cscale(S2[((long long)(m1 + L) * n + k) * W + (m2 + L)],
-                             w[k] * tab64[(long long)k * Kt + e]));
-    f[e] = acc;
+    const double2* S = S2 + (long long)(m1 + L) * n * W + (m2 + L);
+#pragma unroll 8
+    for (int k = wave; k < n; k += 4)
+      acc = cadd(acc, cscale(S[(long long)k * W], tab64[(long long)k * Kt + e]));
   }
+  part[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0 && e < K)
+    f[e] = cadd(cadd(acc, part[1][lane]), cadd(part[2][lane], part[3][lane]));
 }
 
 void launch_soft_forward(hipStream_t s, int n, long long Kt, const double* tab64,
-                         const double2* tw64, const double2* g, double* w, double2* S2,
-                         double2* f) {
-  const int L = n / 2 - 1, W = 2 * L + 1;
-  hipLaunchKernelGGL(k_soft_weights, dim3(1), dim3(256), 0, s, n / 2, w);
-  hipLaunchKernelGGL(k_soft_fwd_plane, dim3(n), dim3(256), sizeof(double2) * (size_t)n * W, s,
-                     n, g, tw64, S2);
-  const long long K = kcount(L);
-  hipLaunchKernelGGL(k_soft_fwd_beta, dim3((unsigned)std::min<long long>((K + 255) / 256, 4096)),
-                     dim3(256), 0, s, n, Kt, tab64, w, S2, f);
+                         const double2* tw64, const double2* g, double2* S2, double2* f) {
+  const int W = n - 1;
+  const size_t sm = sizeof(double2) * ((size_t)cdiv(n, 16) * 16 * kSoftCols + n);
+  hipLaunchKernelGGL(k_soft_fwd_plane, dim3(cdiv(W, kSoftCols), n), dim3(256), sm, s, n, g, tw64,
+                     S2);
+  const long long K = kcount(n / 2 - 1);
+  hipLaunchKernelGGL(k_soft_fwd_beta, dim3((unsigned)((K + 63) / 64)), dim3(256), 0, s, n, Kt,
+                     tab64, S2, f);
 }
-
-size_t soft_forward_smem(int n) { return sizeof(double2) * (size_t)n * (n - 1); }
 
 void launch_coef_to_plane(hipStream_t s, int P, int n, int Lmax, const SphPair* pd,
                           const double2* a, float2* b) {

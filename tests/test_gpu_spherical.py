@@ -131,6 +131,17 @@ def test_soft_forward_matches_oracle_and_round_trips(gpu):
     assert np.abs(back - f).max() <= 1e-5 * np.abs(f).max()
 
 
+@pytest.mark.parametrize("bw", [1, 2, 9, 16, 25, 33])
+def test_soft_forward_over_tiles(gpu, bw):
+    """Grid sides at the edges of the 16-row tiles and 4-row steps of the
+    forward transform's products (the bound is that of the test above)."""
+    say(f"case: SOFT({bw}).SOFT random grid")
+    rng = np.random.default_rng(bw)
+    data = rng.normal(size=(2 * bw,) * 3) + 1j * rng.normal(size=(2 * bw,) * 3)
+    ref = O.SOFTOracle(bw).SOFT(data)
+    np.testing.assert_allclose(fo.SOFT(bw).SOFT(data), ref, atol=1e-12 * np.abs(ref).max())
+
+
 def _oracle_pair(c, keep_grids=False):
     return O.spherical_align(c["pos1"], c["pos2"], c["L"], c["scale"], perm=c["groups"],
                              bw=c["grid_n"] // 2, fast=True, keep_grids=keep_grids)

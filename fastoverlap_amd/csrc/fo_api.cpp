@@ -42,11 +42,13 @@ void launch_coef_norm2(hipStream_t, int, const SphPair*, const double2*, double*
 void launch_sph_contract(hipStream_t, int, int, int, int, int, const SphPair*, const SphGroup*,
                          const double*, const double*, const double2*, const double2*,
                          const double*, const double*, double2*, float2*);
-size_t isoft_plane_smem(int, int, int);
-int isoft_plane_use_fft(int, int, size_t);
-void launch_isoft_plane(hipStream_t, int, int, int, int, long long, const SphPair*, const float*,
-                        const float2*, const float2*, const float2*, int, int, PlaneCand*, float*,
-                        double*, int, const float4*, int);
+size_t isoft_plane_smem(int, int, PlanePath, int);
+PlanePath isoft_plane_path(int, int, size_t);
+void launch_plane_basis(hipStream_t, int, int, float*);
+size_t plane_basis_floats(int, int);
+void launch_isoft_plane(hipStream_t, int, int, int, PlanePath, long long, int, const SphPair*,
+                        const float*, const float*, const float2*, const float2*, const float2*,
+                        int, int, PlaneCand*, float*, double*, int, const float4*, int);
 void launch_beta_gemm(hipStream_t, int, int, int, long long, int, const SphPair*, const float*,
                       const float2*, float4*, int, double*);
 void launch_sph_select(hipStream_t, int, int, long long, int, const SphPair*, const double*,
@@ -136,6 +138,7 @@ struct SphTable {
   float* tab32 = nullptr;
   double2* tw64 = nullptr;
   float2* tw32 = nullptr;
+  float* psi = nullptr;     // real functions of the folded planes
 };
 // Recurrence coefficients of the unnormalised Wigner d for every (l, m1, m2)
 // with l <= kRecL, shared by all batches of a context.
@@ -212,7 +215,8 @@ static int get_sph_table(fo_context* c, int n, const SphTable** out, bool build 
   t.Kp = plane_rows(t.Lt) * n;
   const size_t b64 = sizeof(double) * (size_t)t.Kt * n, b32 = sizeof(float) * (size_t)t.Kp * n;
   const size_t bt = (sizeof(double2) + sizeof(float2)) * (size_t)n;
-  const size_t total = b64 + b32 + bt + 1024;
+  const size_t bp = sizeof(float) * plane_basis_floats(n, t.Lt);
+  const size_t total = b64 + b32 + bt + bp + 1024;
   if (c->budget && c->used + total > c->budget)
     return set_err(FO_ERR_NOMEM, "Wigner table exceeds the context budget");
   void* base = nullptr;
@@ -228,6 +232,9 @@ static int get_sph_table(fo_context* c, int n, const SphTable** out, bool build 
   t.tw64 = (double2*)p;
   p += (sizeof(double2) * n + 255) / 256 * 256;
   t.tw32 = (float2*)p;
+  p += (sizeof(float2) * n + 255) / 256 * 256;
+  t.psi = (float*)p;
+  if (bp) launch_plane_basis(c->stream, n, t.Lt, t.psi);
   FO_HIP(hipMemsetAsync(t.tab32, 0, b32, c->stream));  // entries |m2| > l stay zero
   launch_wigner_table(c->stream, n, t.Lt, t.tab64, t.tab32);
   launch_twiddles(c->stream, n, 1.0, t.tw64, t.tw32);
@@ -457,7 +464,7 @@ struct fo_sph_batch {
   SphLaunch lc{};
   int flags = 0;
   int maxgroup = 1;
-  int fft_chunk = 0;  // 1: two-pass register transform in the plane kernel, 0: direct DFT
+  PlanePath path = kPlaneDirect;  // kernel of the beta planes
   long long Ntot = 0, Ktot = 0, C32tot = 0;
   // the last enqueued coefficient stage left the rows m1 < 0 of I64A unset
   bool mirror_pending = false;
@@ -567,8 +574,8 @@ static int sph_enqueue(fo_sph_batch* b, int stages) {
     if (b->S)
       launch_beta_gemm(s, P, L.n, L.Lmax, b->tab->Kp, L.Lt, b->pd, b->tab->tab32, b->I32A, b->S,
                        L.norient, b->abound);
-    launch_isoft_plane(s, P, L.n, L.Lmax, b->fft_chunk, b->tab->Kp, b->pd, b->tab->tab32,
-                       b->tab->tw32, b->I32A, b->I32B, L.mode, L.norient, b->cand, b->grid,
+    launch_isoft_plane(s, P, L.n, L.Lmax, b->path, b->tab->Kp, b->tab->Lt, b->pd,
+                       b->tab->tab32, b->tab->psi, b->tab->tw32, b->I32A, b->I32B, L.mode, L.norient, b->cand, b->grid,
                        b->abound, b->tune[0], b->S, L.Lmax + 1);
     mark(5);
     // split-BF16x3 products carry up to 3.1 * 2^-16 of each |d I| beyond FP32
@@ -744,13 +751,13 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
     gq += sp.ngroups;
     ga += ng;
   }
-  if (isoft_plane_smem(n, Lmax, 0) > c->max_lds)
+  if (isoft_plane_smem(n, Lmax, kPlaneDirect, 2) > c->max_lds)
     return set_err(FO_ERR_UNSUPPORTED, "grid_n and Jmax too large for one beta plane in LDS (" +
-                                           std::to_string(isoft_plane_smem(n, Lmax, 0)) + " > " +
+                                           std::to_string(isoft_plane_smem(n, Lmax, kPlaneDirect, 2)) + " > " +
                                            std::to_string(c->max_lds) + " bytes)");
-  b->fft_chunk = (d->flags & FO_SPH_DFT) ? 0 : isoft_plane_use_fft(n, Lmax, c->max_lds);
+  b->path = (d->flags & FO_SPH_DFT) ? kPlaneDirect : isoft_plane_path(n, Lmax, c->max_lds);
   const bool beta_gemm = (d->flags & FO_SPH_BETA_GEMM) != 0;
-  if (beta_gemm && (general || !b->fft_chunk))
+  if (beta_gemm && (general || b->path != kPlaneFft))
     return set_err(FO_ERR_UNSUPPORTED, "FO_SPH_BETA_GEMM needs the alignment mode and a "
                                        "power-of-two grid side in [16, 256]");
   if (lap_lds_bytes(b->maxgroup) > c->max_lds)
@@ -1074,7 +1081,7 @@ static int sph_autotune(fo_sph_batch* b) {
   const SphLaunch& L = b->lc;
   int bucket = 1;
   while (bucket < L.P) bucket <<= 1;
-  const auto key = std::make_tuple(L.n, L.Lmax, bucket, b->fft_chunk);
+  const auto key = std::make_tuple(L.n, L.Lmax, bucket, b->path);
   {
     std::lock_guard<std::mutex> g(c->mu);
     auto it = c->tuned.find(key);
@@ -1094,8 +1101,8 @@ static int sph_autotune(fo_sph_batch* b) {
   auto time_stage = [&](int knob, float* ms) -> int {
     auto launch = [&]() {
       if (knob == 0) {
-        launch_isoft_plane(s, L.P, L.n, L.Lmax, b->fft_chunk, b->tab->Kp, b->pd, b->tab->tab32,
-                           b->tab->tw32, b->I32A, b->I32B, L.mode, L.norient, b->cand, b->grid,
+        launch_isoft_plane(s, L.P, L.n, L.Lmax, b->path, b->tab->Kp, b->tab->Lt, b->pd,
+                           b->tab->tab32, b->tab->psi, b->tab->tw32, b->I32A, b->I32B, L.mode, L.norient, b->cand, b->grid,
                            b->abound, b->tune[0], b->S, L.Lmax + 1);
       } else {
         for (const CoefChunk& C : b->chunks)

@@ -57,7 +57,9 @@ FO_HD int rad_slot_deg(int s, int L) {
 // transform input k (m2 = k for k < n/2, k - n above) and zero where |m2| > l.
 // Inside a row, entry k sits at plane_pos(k, n): lane-major for the grid
 // sides of the two-pass transform (n = N1*N2, lane k1 owns k = k1 + N1*k2 and
-// its N2 entries are contiguous), in k order for other n.
+// its N2 entries are contiguous); for other even n the entries m2 and -m2 side
+// by side (2 m2 and 2 m2 + 1; m2 = 0 beside the unused k = n/2); in k order for
+// odd n.
 FO_HD int plane_n1(int n) {  // N1 of the two-pass transform, 0 if none
   switch (n) {
     case 16: return 4;
@@ -70,7 +72,9 @@ FO_HD long long plane_rows(int L) { return (long long)(L + 1) * (L + 2) / 2; }
 FO_HD int plane_k(int m2, int n) { return m2 < 0 ? m2 + n : m2; }
 FO_HD int plane_pos(int k, int n) {
   const int n1 = plane_n1(n);
-  return n1 ? (k % n1) * (n / n1) + k / n1 : k;
+  if (n1) return (k % n1) * (n / n1) + k / n1;
+  if (n & 1) return k;
+  return k < n / 2 ? 2 * k : k == n / 2 ? 1 : 2 * (n - k) + 1;
 }
 
 // ---- complex helpers (double2 / float2 = re, im) -------------------------
@@ -290,6 +294,7 @@ FO_DEV double2 load_d2(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
 // FP64 matrix product step.  Lane layout: A operand lane -> (row lane%16, k
 // lane/16), B operand lane -> (k lane/16, col lane%16), result register i of
 // a lane -> (row 4 i + lane/16, col lane%16).
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef double v4d __attribute__((ext_vector_type(4)));
 FO_DEV v4d mfma64(double a, double b, v4d c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);

@@ -39,6 +39,9 @@ __host__ __device__ inline long long harm_proj_doubles(int ngath, int L, int nma
   return basis ? 2LL * ngath * (L + 2 * nmax + 1) * (nmax + 1) : 0;
 }
 
+// Kernels of the beta planes.
+enum PlanePath { kPlaneDirect = 0, kPlaneFft = 1, kPlaneFold = 2 };
+
 // Per (pair, orientation, plane) candidate record written by the plane
 // kernels: the plane's values are split into kCandPerPlane parts (the
 // spherical kernels: one per wavefront) and entry r lists the largest value

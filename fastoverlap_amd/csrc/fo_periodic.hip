@@ -404,7 +404,6 @@ __global__ void __launch_bounds__(256) k_per_plane(
 // products read, four conversions and eight FP32 operations a term) and the
 // candidate test of every value.
 constexpr int kPlaneXP = 4;
-typedef float v4f __attribute__((ext_vector_type(4)));
 FO_HD double real_plane_delta(int NB) { return (9.0 * NB + 64.0) * 5.9604644775390625e-08; }
 FO_HD int real_plane_fs(int F) { return ((F + 15) & ~15) + 4; }  // row stride of phi
 FO_HD int real_plane_ks(int NB) { return ((NB + 3) & ~3) + 1; }  // row stride of R

@@ -7,8 +7,9 @@
 //   k_sph_radial     scaled i_l(x) * Gaussian radial kernel (FP64)
 //   k_sph_contract   C^l = Y1 . K_l . Y2^H per degree (FP64, fo_contract.hip)
 //   k_isoft_fft      inverse SOFT of both orientations per beta plane (FP32),
-//                    two-pass register transforms (power-of-two n); k_isoft_plane
-//                    is the direct-DFT form for other n;
+//                    two-pass register transforms (power-of-two n); k_isoft_fold
+//                    real matrix products (other even n), k_isoft_plane direct
+//                    sums (any n);
 //                    top candidates per plane
 //   k_sph_select     FP64 re-evaluation of every candidate within the FP32
 //                    error bound of the maximum -> exact argmax, parabolic
@@ -466,13 +467,13 @@ struct CandOne {
   float bv = -INFINITY, dm = -INFINITY;
   int bi = 0x7fffffff;
   FO_DEV void add(int flat, float val) {
-    if (val > bv) {
-      dm = fmaxf(dm, bv);
-      bv = val;
-      bi = flat;
-    } else {
-      dm = fmaxf(dm, val);
-    }
+    dm = __builtin_amdgcn_fmed3f(dm, bv, val);  // dm <= bv
+    bi = val > bv ? flat : bi;
+    bv = fmaxf(bv, val);
+  }
+  FO_DEV void merge(const CandOne& o) {
+    add(o.bi, o.bv);
+    dm = fmaxf(dm, o.dm);
   }
 };
 struct CandTrack {
@@ -885,6 +886,294 @@ __global__ void __launch_bounds__(256) k_isoft_fft(
     }
   }
   plane_candidates(ct, no, cand + ((long long)p * no) * n + ib, n);
+}
+
+// ---------------------------------------------------------------------------
+// Planes of even n as real matrix products (FP32).  A Hermitian set gives
+//   g[a][c] = sum_{r,k} R[r][k] psi_r(a) psi_k(c)
+// over the real functions psi = cos(2 pi m j / n), sin(2 pi m j / n), m <= L,
+// with R folded from S[m1][m2] = sum_l d^l_{m1m2} I^l_{m1m2} (m1 >= 0):
+// with P, Q = S[m1][m] +- S[m1][-m] and w = 1 (m1 = 0) or 2, the entries of
+// (cos m1, sin m1) x (cos m, sin m) are w (Re P, -Im Q; -Im P, -Re Q).
+// Moving j by n/2 changes the sign of the functions of odd m only, so both
+// products run over the first half of the grid side with the sums over even
+// and odd m apart, and the halves are their sum and difference.
+// Order of the functions: an even and an odd step of four alternate; function
+// e of a class (cos m: e = max(m - 1, 0), sin m: e = m; class m & 1) is entry
+// e & 3 of that class' step e >> 2.
+//   1. A thread forms S at +-m for two m of one row from 16-byte loads of the
+//      plane layout, and writes R [o][row][col] to LDS.
+//   2. G[row][c] = sum_k R psi_k(c) on v_mfma_f32_16x16x4f32 for 16 columns c
+//      of the half side, a wavefront per (orientation, 16 columns).
+//   3. g[c][a] = sum_row G psi_row(a): result register i of row tile tt of 2 is
+//      the A operand of step 4 tt + i of 3.
+// A wavefront's columns of the other half side are G_even - G_odd; with two or
+// fewer (orientation, tile) items the two halves go to different wavefronts.
+// Products run from the highest m down, so that a decaying spectrum is summed
+// from its small end: the grid's rms error at n = 42, degree 20 is 1.17e-7 of its
+// rms (upwards 1.8e-7, direct complex sums 1.4e-7).  Bound by vector
+// instructions (1 and the candidate test), the matrix products take a third.
+// ---------------------------------------------------------------------------
+FO_HD int fold_units(int L) { return (L + 4) / 4; }  // pairs of steps
+FO_HD int fold_row(int e, int cls) { return 8 * (e >> 2) + 4 * cls + (e & 3); }
+FO_HD int fold_col(int e, int cls) { return 8 * (e >> 2) + 2 * (e & 3) + cls; }
+FO_HD int fold_stride(int NU) { return 8 * NU + 4; }
+
+// psi in the column order, [j < n/2][8 NU]
+__global__ void k_plane_basis(int n, int NU, float* __restrict__ psi) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n / 2 * 8 * NU;
+       i += gridDim.x * blockDim.x) {
+    const int j = i / (8 * NU), c = i % (8 * NU);
+    const int cls = c & 1, e = 4 * (c >> 3) + ((c >> 1) & 3);
+    const bool sine = e && (e & 1) == cls;  // sin m has e = m
+    const int m = sine ? e : e + (e || cls);
+    double sv, cv;
+    sincospi(2.0 * (double)((m * j) % n) / (double)n, &sv, &cv);
+    psi[i] = (float)(sine ? sv : cv);
+  }
+}
+
+// TWO: two coefficient sets; else both orientations of one (even + odd, even -
+// odd degrees)
+template <int NT, bool TWO>
+__global__ void __launch_bounds__(256, NT <= 4 ? 4 : 2) k_isoft_fold(
+    const SphPair* __restrict__ pd, int P, int C, int n, long long Kp,
+    const float* __restrict__ tab32, const float* __restrict__ psig, int NUt,
+    const float2* __restrict__ IA, const float2* __restrict__ IB, int no,
+    PlaneCand* __restrict__ cand, float* __restrict__ grid, double* __restrict__ abound) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  // workgroups are dealt to the 8 XCDs round-robin; each XCD walks its
+  // pairs in chunks of C, beta-major inside a chunk, so the coefficient
+  // blocks of C pairs and a few beta slices of the table share its L2
+  const int wg = blockIdx.x;
+  const int sx = wg >> 3, chunk = sx / (C * n), rr = sx - chunk * C * n;
+  const int ib = rr / C, p = (wg & 7) + 8 * (chunk * C + rr % C);
+  if (p >= P) return;  // whole workgroup: padding of P to a multiple of 8 C
+  const SphPair d = pd[p];
+  const int L = d.L, t = threadIdx.x, n2 = n / 2;
+  const int NU = fold_units(L), KS = fold_stride(NU), rows = 8 * NU;
+  float* R = (float*)smem;             // [no][rows][KS]
+  float* psi = R + no * rows * KS;     // [n2][KS]
+  for (int e = t; e < no * rows * KS / 4; e += 256)
+    ((float4*)R)[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int e = t; e < n2 * 2 * NU; e += 256) {
+    const int j = e / (2 * NU), c = e - j * 2 * NU;
+    *(float4*)(psi + j * KS + 4 * c) = *(const float4*)(psig + (long long)j * 8 * NUt + 4 * c);
+  }
+  __syncthreads();
+
+  // ---- 1: items (m1, m = 2 mp and 2 mp + 1)
+  // (a lane whose second m is past L reads up to two entries past its row:
+  // not used, and inside the allocations also after the last row)
+  const int rbytes = (int)plane_rows(L) * n;
+  const __amdgpu_buffer_rsrc_t rtb = buf_rsrc(tab32 + (long long)ib * Kp, rbytes * 4 + 8);
+  const __amdgpu_buffer_rsrc_t ria = buf_rsrc(IA + d.c32_off, rbytes * 8 + 16);
+  const __amdgpu_buffer_rsrc_t rib = buf_rsrc(
+      TWO ? (const void*)(IB + d.c32_off) : (const void*)(IA + d.c32_off), rbytes * 8 + 16);
+  // the beta = 0 workgroup also sums the coefficient magnitudes for the
+  // selection's error bound (each entry is loaded once per workgroup)
+  const bool wantA = ib == 0;
+  double asum[2] = {0.0, 0.0};
+  const int MP = (L + 2) / 2, items = (L + 1) * MP;
+  for (int it = t; it - t < items; it += 256) {
+    const int m1 = it / MP, mp = it - m1 * MP;  // m1 > L: no item
+    const bool two = 2 * mp + 1 <= L;           // (else the second m is another row's)
+    float2 a[4], b[4];                          // +-2 mp, +-(2 mp + 1)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = b[i] = make_float2(0.f, 0.f);
+    {
+      const int vo = (m1 * n + 4 * mp) * 4;
+      // rows above the degree and degrees above L read as zero
+      auto step = [&](int l, float2(&sa)[4], float2(&sb)[4]) {
+        const bool in = m1 <= (l <= L ? l : -1);
+        const int so = qlm(l, 0) * n * 4;
+        const int v = in ? vo + so : 0x3ffffff0;
+        const float4 w = load_f4(rtb, v, 0);
+        const float4 c0 = load_f4(ria, 2 * v, 0), c1 = load_f4(ria, 2 * v + 16, 0);
+        const float dv[4] = {w.x, w.y, w.z, w.w};
+        const float2 ca[4] = {{c0.x, c0.y}, {c0.z, c0.w}, {c1.x, c1.y}, {c1.z, c1.w}};
+        float2 cb[4];
+        if constexpr (TWO) {
+          const float4 e0 = load_f4(rib, 2 * v, 0), e1 = load_f4(rib, 2 * v + 16, 0);
+          cb[0] = make_float2(e0.x, e0.y);
+          cb[1] = make_float2(e0.z, e0.w);
+          cb[2] = make_float2(e1.x, e1.y);
+          cb[3] = make_float2(e1.z, e1.w);
+        }
+        if (wantA) {
+          // weight sqrt((2l+1)/2), doubled for m1 > 0 (the m1 < 0 rows)
+          const float wl = sqrtf(l + 0.5f) * (m1 == 0 ? 1.f : 2.f);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (i >= 2 && !two) continue;
+            asum[0] += wl * sqrtf(ca[i].x * ca[i].x + ca[i].y * ca[i].y);
+            if constexpr (TWO) asum[1] += wl * sqrtf(cb[i].x * cb[i].x + cb[i].y * cb[i].y);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sa[i].x += dv[i] * ca[i].x;
+          sa[i].y += dv[i] * ca[i].y;
+          if constexpr (TWO) {
+            sb[i].x += dv[i] * cb[i].x;
+            sb[i].y += dv[i] * cb[i].y;
+          }
+        }
+      };
+      // from the wavefront's first row on, even and odd degrees in turn
+      for (int l = __builtin_amdgcn_readfirstlane(m1) & ~1; l <= L; l += 2) {
+        step(l, a, b);
+        if constexpr (TWO)
+          step(l + 1, a, b);
+        else
+          step(l + 1, b, a);
+      }
+    }
+    if (m1 > L) continue;
+    const int rc = fold_row(max(m1 - 1, 0), m1 & 1) * KS, rs = fold_row(m1, m1 & 1) * KS;
+    const float w = m1 == 0 ? 1.f : 2.f;
+    for (int o = 0; o < no; ++o) {
+      float* Ro = R + o * rows * KS;
+      const float sg = o == 0 ? 1.f : -1.f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int m = 2 * mp + h;
+        if (m > L) continue;
+        float2 u, v;
+        if constexpr (TWO) {
+          u = o == 0 ? a[2 * h] : b[2 * h];
+          v = o == 0 ? a[2 * h + 1] : b[2 * h + 1];
+        } else {
+          u = make_float2(a[2 * h].x + sg * b[2 * h].x, a[2 * h].y + sg * b[2 * h].y);
+          v = make_float2(a[2 * h + 1].x + sg * b[2 * h + 1].x,
+                          a[2 * h + 1].y + sg * b[2 * h + 1].y);
+        }
+        const int cc = fold_col(max(m - 1, 0), h), cs = fold_col(m, h);
+        Ro[rc + cc] = w * (u.x + v.x);
+        if (m) Ro[rc + cs] = -w * (u.y - v.y);
+        if (m1) {
+          Ro[rs + cc] = -2.f * (u.y + v.y);
+          if (m) Ro[rs + cs] = -2.f * (u.x - v.x);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  if (wantA) plane_abound(asum, TWO, no, abound + (long long)p * no);
+
+  // ---- 2 and 3
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6), ln = t & 63, col = ln & 15, q = ln >> 4;
+  const int JT = (n2 + 15) >> 4;
+  const bool split = JT * no <= 2;
+  const int nitems = JT * no * (split ? 2 : 1);
+  // candidate parts: a wavefront's item split at half of a where that gives
+  // at most kCandPerPlane parts, else one part per wavefront and orientation
+  const bool parts2 = no == 2 ? JT <= 2 : JT == 1;
+  int ro[NT];  // this lane's row of R, A operand of row tile tt (clamped rows are not used)
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt)
+    ro[tt] = min(16 * tt + 4 * (col & 3) + (col >> 2), rows - 1) * KS + 2 * q;
+  CandTrack ct;
+  PlaneCand* pc = cand + (long long)p * no * n + ib;
+  for (int item = wv; item < nitems; item += 4) {
+    const int half = split ? item & 1 : 0, x = split ? item >> 1 : item;
+    const int o = x / JT, jt = x - o * JT;
+    const float* Ro = R + o * rows * KS;
+    v4f G0[NT], G1[NT];
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) G0[tt] = G1[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+    const float* pb = psi + min(16 * jt + col, n2 - 1) * KS + 2 * q;
+#pragma unroll 2
+    for (int u = NU - 1; u >= 0; --u) {
+      const float2 bb = *(const float2*)(pb + 8 * u);
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        if (2 * tt >= NU) continue;  // uniform
+        const float2 aa = *(const float2*)(Ro + ro[tt] + 8 * u);
+        G0[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.x, bb.x, G0[tt], 0, 0, 0);
+        G1[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.y, bb.y, G1[tt], 0, 0, 0);
+      }
+    }
+    const float sg = half ? -1.f : 1.f;
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float ev = G0[tt][i], od = G1[tt][i];
+        G0[tt][i] = ev + sg * od;
+        G1[tt][i] = ev - od;  // the other half (not split)
+      }
+    // lanes and rows past n/2 start from -inf: never a candidate
+    v4f rowmask;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rowmask[i] = 16 * jt + 4 * q + i < n2 ? 0.f : -INFINITY;
+    CandOne c[2];  // a < n/2, a >= n/2: idx = 8 (tile of a) + 4 (half of c) + register
+    for (int at = 0; at < JT; ++at) {
+      const float* pa = psi + min(16 * at + col, n2 - 1) * KS + 2 * q;
+      v4f e0 = rowmask, e1;
+      if (16 * at + col >= n2) e0 = v4f{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      e1 = e0;
+      v4f d0 = v4f{0.f, 0.f, 0.f, 0.f}, d1 = d0;
+#pragma unroll
+      for (int u = 2 * NT - 1; u >= 0; --u) {
+        if (u >= NU) continue;  // uniform
+        const float2 bb = *(const float2*)(pa + 8 * u);
+        const int tt = u >> 1, i = 2 * (u & 1);
+        e0 = __builtin_amdgcn_mfma_f32_16x16x4f32(G0[tt][i], bb.x, e0, 0, 0, 0);
+        d0 = __builtin_amdgcn_mfma_f32_16x16x4f32(G0[tt][i + 1], bb.y, d0, 0, 0, 0);
+        if (!split) {  // uniform
+          e1 = __builtin_amdgcn_mfma_f32_16x16x4f32(G1[tt][i], bb.x, e1, 0, 0, 0);
+          d1 = __builtin_amdgcn_mfma_f32_16x16x4f32(G1[tt][i + 1], bb.y, d1, 0, 0, 0);
+        }
+      }
+      auto outputs = [&](int h, const v4f& e, const v4f& dd) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float lo = e[i] + dd[i], hi = e[i] - dd[i];
+          c[0].add(8 * at + 4 * h + i, lo);
+          c[1].add(8 * at + 4 * h + i, hi);
+          if (grid && 16 * at + col < n2 && 16 * jt + 4 * q + i < n2) {
+            const int cg = 16 * jt + 4 * q + i + h * n2;
+            float* gp = grid + ((long long)p * no + o) * n * n * n;
+            gp[((16 * at + col) * n + ib) * n + cg] = lo;
+            gp[((16 * at + col + n2) * n + ib) * n + cg] = hi;
+          }
+        }
+      };
+      outputs(half, e0, d0);
+      if (!split) outputs(1, e1, d1);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int id = c[h].bi;
+      if (c[h].bv > -INFINITY)
+        c[h].bi = ((16 * (id >> 3) + col + h * n2) * n + ib) * n + 16 * jt + 4 * q + (id & 3) +
+                  ((id >> 2) & 1) * n2;
+    }
+    if (parts2) {
+      float v[2] = {c[0].bv, c[1].bv}, r[2] = {c[0].dm, c[1].dm};
+      int id[2] = {c[0].bi, c[1].bi};
+      wave_top2(v, id, r);
+      if (ln == 0) {
+        PlaneCand* dst = pc + (long long)o * n;
+        const int e = 2 * (split ? (JT == 1 ? half : 0) : jt);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          dst->val[e + h] = v[h];
+          dst->idx[e + h] = id[h];
+          dst->rest[e + h] = r[h];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (o == 0)
+          ct.c0.merge(c[h]);
+        else
+          ct.c1.merge(c[h]);
+    }
+  }
+  if (!parts2) plane_candidates(ct, no, pc, n);
 }
 
 // Direct-DFT planes (any n): the beta contraction per (m1 >= 0, m2) entry,
@@ -2072,7 +2361,6 @@ namespace fo {
 // -> (row 4(lane/16) + r, column lane%16).
 // ---------------------------------------------------------------------------
 typedef short v4s __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 FO_DEV unsigned short bf16_rne(float x) {
   const unsigned u = __float_as_uint(x);
@@ -2261,32 +2549,54 @@ static bool fft_shape(int n, int& n1, int& n2) {
   return n1 != 0;
 }
 
-size_t isoft_plane_smem(int n, int Lmax, int use_fft) {
+size_t isoft_plane_smem(int n, int Lmax, PlanePath path, int norient) {
   int n1, n2;
-  if (use_fft && fft_shape(n, n1, n2)) {
-    const size_t ls = (size_t)((Lmax + 1) | 1);
-    const int tpf = std::max(n1, n2);
-    const size_t x = n1 == n2 ? 0 : (size_t)(256 / tpf) * (n + n / n1);
-    return sizeof(float2) * (2 * (size_t)n * ls + x);
+  switch (path) {
+    case kPlaneFft: {
+      fft_shape(n, n1, n2);
+      const size_t ls = (size_t)((Lmax + 1) | 1);
+      const int tpf = std::max(n1, n2);
+      const size_t x = n1 == n2 ? 0 : (size_t)(256 / tpf) * (n + n / n1);
+      return sizeof(float2) * (2 * (size_t)n * ls + x);
+    }
+    case kPlaneFold: {
+      const size_t NU = fold_units(Lmax), KS = fold_stride((int)NU);
+      return sizeof(float) * KS * (norient * 8 * NU + n / 2);
+    }
+    default:
+      return sizeof(float2) * ((size_t)n + 2 * (size_t)(Lmax + 1) * (2 * Lmax + 1) +
+                               2 * (size_t)(Lmax + 1) * n);
   }
-  return sizeof(float2) * ((size_t)n + 2 * (size_t)(Lmax + 1) * (2 * Lmax + 1) +
-                           2 * (size_t)(Lmax + 1) * n);
 }
 
-// 1 if the two-pass transform applies to n and fits max_lds, else 0.
-int isoft_plane_use_fft(int n, int Lmax, size_t max_lds) {
+// The power-of-two sides take the two-pass transform (64 planes of a pair of
+// degree 20: 3.6 ms for 4096 pairs, 4.4 with the folded products), other even
+// ones the folded products (96 pairs of n = 42, degree 20: 59 us, 198 with direct
+// sums); odd sides and planes beyond LDS the direct sums.
+PlanePath isoft_plane_path(int n, int Lmax, size_t max_lds) {
   int n1, n2;
-  return fft_shape(n, n1, n2) && isoft_plane_smem(n, Lmax, 1) <= max_lds ? 1 : 0;
+  if (fft_shape(n, n1, n2))
+    return isoft_plane_smem(n, Lmax, kPlaneFft, 2) <= max_lds ? kPlaneFft : kPlaneDirect;
+  return !(n & 1) && isoft_plane_smem(n, Lmax, kPlaneFold, 2) <= max_lds ? kPlaneFold
+                                                                         : kPlaneDirect;
 }
 
-void launch_isoft_plane(hipStream_t s, int P, int n, int Lmax, int use_fft, long long Kp,
-                        const SphPair* pd, const float* tab32, const float2* tw32,
-                        const float2* IA, const float2* IB, int mode, int norient,
-                        PlaneCand* cand, float* grid, double* abound, int chunk,
+// the folded planes' table of real functions, if the grid side uses it
+size_t plane_basis_floats(int n, int Lt) {
+  return (n & 1) || plane_n1(n) ? 0 : (size_t)(n / 2) * 8 * fold_units(Lt);
+}
+void launch_plane_basis(hipStream_t s, int n, int Lt, float* psi) {
+  const int NU = fold_units(Lt);
+  hipLaunchKernelGGL(k_plane_basis, dim3(cdiv(n / 2 * 8 * NU, 256)), dim3(256), 0, s, n, NU, psi);
+}
+
+void launch_isoft_plane(hipStream_t s, int P, int n, int Lmax, PlanePath path, long long Kp,
+                        int Lt, const SphPair* pd, const float* tab32, const float* psi,
+                        const float2* tw32, const float2* IA, const float2* IB, int mode,
+                        int norient, PlaneCand* cand, float* grid, double* abound, int chunk,
                         const float4* S, int Srows) {
-  const size_t sm = isoft_plane_smem(n, Lmax, use_fft);
-  int n1, n2;
-  if (!use_fft || !fft_shape(n, n1, n2)) {
+  const size_t sm = isoft_plane_smem(n, Lmax, path, norient);
+  if (path == kPlaneDirect) {
     hipLaunchKernelGGL(k_isoft_plane, dim3(n, P), dim3(256), sm, s, pd, n, Kp, tab32, tw32, IA,
                        IB, mode, norient, cand, grid, abound);
     return;
@@ -2295,6 +2605,30 @@ void launch_isoft_plane(hipStream_t s, int P, int n, int Lmax, int use_fft, long
   // beta-major); 16 unless chosen by the autotuner
   const int C = std::max(1, std::min(chunk > 0 ? chunk : 16, (P + 7) / 8));
   const dim3 g((unsigned)(8 * ((P + 8 * C - 1) / (8 * C)) * C * n)), b(256);
+  if (path == kPlaneFold) {
+    const int NUt = fold_units(Lt);
+#define FO_FOLD(NT)                                                                            \
+  case NT:                                                                                     \
+    if (mode == 0)                                                                             \
+      hipLaunchKernelGGL((k_isoft_fold<NT, false>), g, b, sm, s, pd, P, C, n, Kp, tab32, psi,  \
+                         NUt, IA, IB, norient, cand, grid, abound);                            \
+    else                                                                                       \
+      hipLaunchKernelGGL((k_isoft_fold<NT, true>), g, b, sm, s, pd, P, C, n, Kp, tab32, psi,   \
+                         NUt, IA, IB, norient, cand, grid, abound);                            \
+    break
+    switch ((fold_units(Lmax) + 1) / 2) {
+      FO_FOLD(1);
+      FO_FOLD(2);
+      FO_FOLD(3);
+      FO_FOLD(4);
+      FO_FOLD(5);
+      FO_FOLD(6);
+      FO_FOLD(7);
+      default: break;  // (degrees above 55: refused with the direct sums' LDS)
+    }
+#undef FO_FOLD
+    return;
+  }
 #define FO_FFT(N1, N2)                                                                         \
   if (S)                                                                                        \
     hipLaunchKernelGGL((k_isoft_fft<N1, N2, 0, true>), g, b, sm, s, pd, P, C, Kp, tab32, tw32,  \

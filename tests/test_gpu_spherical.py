@@ -666,3 +666,35 @@ def test_harmonics_split_over_workgroups(gpu):
     for got, (A, B) in zip(few, Xs):
         ref = O.so3_coeffs_species(A, B, [np.arange(len(A))], L, 0.4, fast=True)
         np.testing.assert_allclose(compact_to_dense(got, L), ref, atol=1e-12 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("n,L,invert", [
+    (2, 0, True), (6, 2, True), (10, 3, False), (18, 8, True), (30, 12, True), (34, 16, False),
+    (42, 20, False), (42, 20, True), (66, 24, True), (68, 31, False), (98, 40, True),
+    (100, 48, True), (100, 49, False)])
+def test_folded_planes_against_direct_planes(gpu, n, L, invert):
+    """The folded real products of even grid sides at the edges of their tiles
+    (16 columns of the half side, 4 functions a step, 16 rows), with one and
+    two orientations and ragged degrees, against the direct sums: every value
+    within the sum of both rounding bounds, the same argmax, and the listed
+    FP32 maximum equal to the grid's."""
+    say(f"case: n={n} L={L} invert={invert}")
+    rng = np.random.default_rng(n + L)
+    Ls = [L, max(L - 1, 0), L // 2]
+    Xs = rng.normal(size=(2, 3 * 11, 3))
+    out = []
+    for flag in (0, _lib.SPH_DFT):
+        flag |= _lib.SPH_KEEP_GRID | (0 if invert else _lib.SPH_NO_INVERT)
+        with SphericalBatch([11] * 3, Ls, 0.4, n, [[np.arange(11)]] * 3, flag) as b:
+            b.set_positions(Xs[0], Xs[1])
+            b.run(_lib.STAGE_PREP | _lib.STAGE_COEFF | _lib.STAGE_GRID)
+            out.append(([b.grid(p) for p in range(3)], b.peaks(), b.precision()))
+    (gf, pf, rf), (gd, pdir, rd) = out
+    for p in range(3):
+        for k in range(2 if invert else 1):
+            assert np.abs(gf[p][k] - gd[p][k]).max() <= 2 * rd["delta"][p, k], (p, k)
+            assert abs(rf["delta"][p, k] - rd["delta"][p, k]) <= 1e-6 * rd["delta"][p, k]
+            assert rf["val32"][p, k] == gf[p][k].max(), (p, k)
+            if Ls[p]:  # (degree 0: a constant grid)
+                np.testing.assert_array_equal(pf["ind"][p, k], pdir["ind"][p, k])
+                assert abs(pf["value"][p, k] - pdir["value"][p, k]) <= 1e-12 * pdir["value"][p, k]

@@ -56,7 +56,7 @@ void launch_sph_select(hipStream_t, int, int, long long, int, const SphPair*, co
                        double2*, long long, const double*, SphPeak*, double, int);
 void launch_sph_rotopt(hipStream_t, int, int, int, const SphPair*, const double2*, const double2*,
                        int, const SphPeak*, const double*, int, SphOpt*);
-void launch_rec_table(hipStream_t, int, double*, double*, double2*, double*);
+void launch_rec_table(hipStream_t, int, double*, double2*, double*);
 void launch_sph_finish(hipStream_t, int, int, const SphPair*, const SphGroup*, const int*,
                        const double*, const double*, const SphOpt*, int, double*, int*, int*,
                        double*, SphResult*);
@@ -65,7 +65,7 @@ void launch_soft_forward(hipStream_t, int, long long, const double*, const doubl
                          double2*, double2*);
 void launch_sph_mirror(hipStream_t, int, int, const SphPair*, double2*);
 void launch_sph_energy(hipStream_t, int, const double2*, double, double, double, const double*,
-                       const double*, int, double*);
+                       int, double*);
 void launch_wigner_D(hipStream_t, int, double, double, double, double2*, double2*);
 void launch_ylm_angles(hipStream_t, int, int, const double*, const double*, double2*);
 size_t per_sf_smem(int);
@@ -140,11 +140,10 @@ struct SphTable {
   float2* tw32 = nullptr;
   float* psi = nullptr;     // real functions of the folded planes
 };
-// Recurrence coefficients of the unnormalised Wigner d for every (l, m1, m2)
-// with l <= kRecL, shared by all batches of a context.
+// Seeds of the unnormalised Wigner d and the Legendre recurrence for degrees up
+// to kRecL, shared by all batches of a context.
 static constexpr int kRecL = 63;
 struct RecTable {
-  double* rec = nullptr;    // 3 * K(kRecL)
   double* seedu = nullptr;  // (2 kRecL + 1)^2
   double2* leg = nullptr;   // Legendre recurrence coefficients, q(kRecL, kRecL) + 1
   double* cm = nullptr;     // P_m^m prefactors, kRecL + 1
@@ -247,26 +246,24 @@ static int get_sph_table(fo_context* c, int n, const SphTable** out, bool build 
 
 static int get_rec_table(fo_context* c, const RecTable** out, bool build = true) {
   std::lock_guard<std::mutex> g(c->mu);
-  if (!c->rect.rec && !build)
+  if (!c->rect.seedu && !build)
     return set_err(FO_ERR_STATE, "recurrence tables not built (fo_sph_prepare builds them)");
-  if (!c->rect.rec) {
-    const size_t b1 = sizeof(double) * 3 * (size_t)kcount(kRecL);
+  if (!c->rect.seedu) {
     const size_t b2 = sizeof(double) * (size_t)(2 * kRecL + 1) * (2 * kRecL + 1);
     const size_t b3 = sizeof(double2) * (size_t)((kRecL + 1) * (kRecL + 2) / 2);
     const size_t b4 = sizeof(double) * (size_t)(kRecL + 1);
     auto up = [](size_t x) { return (x + 255) / 256 * 256; };
-    const size_t total = up(b1) + up(b2) + up(b3) + up(b4);
+    const size_t total = up(b2) + up(b3) + up(b4);
     void* base = nullptr;
     hipError_t e = hipMalloc(&base, total);
     if (e != hipSuccess) return set_err(FO_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     c->used += total;
     c->owned.push_back(base);
     char* cb = (char*)base;
-    c->rect.rec = (double*)cb;
-    c->rect.seedu = (double*)(cb + up(b1));
-    c->rect.leg = (double2*)(cb + up(b1) + up(b2));
-    c->rect.cm = (double*)(cb + up(b1) + up(b2) + up(b3));
-    launch_rec_table(c->stream, kRecL, c->rect.rec, c->rect.seedu, c->rect.leg, c->rect.cm);
+    c->rect.seedu = (double*)cb;
+    c->rect.leg = (double2*)(cb + up(b2));
+    c->rect.cm = (double*)(cb + up(b2) + up(b3));
+    launch_rec_table(c->stream, kRecL, c->rect.seedu, c->rect.leg, c->rect.cm);
     FO_CHECK_LAUNCH();
     FO_HIP(hipStreamSynchronize(c->stream));
   }
@@ -1425,7 +1422,7 @@ int fo_sph_energy(fo_context* c, int L, const double* X, const double* rot, doub
   double2* dI = (double2*)s.p;
   double* dout = (double*)((char*)s.p + (sizeof(double) * h.size() + 255) / 256 * 256);
   FO_HIP(hipMemcpyAsync(dI, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, c->stream));
-  launch_sph_energy(c->stream, L, dI, rot[0], rot[1], rot[2], rt->rec, rt->seedu, kRecL, dout);
+  launch_sph_energy(c->stream, L, dI, rot[0], rot[1], rot[2], rt->seedu, kRecL, dout);
   FO_CHECK_LAUNCH();
   double o[10];
   FO_HIP(hipMemcpyAsync(o, dout, sizeof(o), hipMemcpyDeviceToHost, c->stream));

@@ -1798,29 +1798,66 @@ __global__ void __launch_bounds__(256) k_sph_select(
 // exact gradient and Hessian (d, d', d'' by the differentiated recurrence)
 // converges to the same local optimum to full FP64 precision.
 //
-// The recurrence coefficients of the unnormalised d,
+// The recurrence is that of the unnormalised d,
 //   d^{l+1} = Bu_l (cos b - C_l) d^l - Au_l d^{l-1},
-//   Bu_l = B_l sqrt((2l+1)/(2l+3)),  Au_l = A_l sqrt((2l-1)/(2l+3)),
-// and the edge prefactor xi sqrt(binom(mu+nu, mu)) are precomputed once per
-// context (k_rec_table), so the inner loop has no FP64 square root or
-// division.
+// with coefficients from a table in LDS (RecLds); the edge prefactor
+// xi sqrt(binom(mu+nu, mu)) is precomputed once per context (k_seed_table), so
+// the inner loop has no FP64 square root or division.
 // ---------------------------------------------------------------------------
-__global__ void k_rec_table(int Lt, double* __restrict__ rec, double* __restrict__ seedu) {
+__global__ void k_seed_table(int Lt, double* __restrict__ seedu) {
   const int W = 2 * Lt + 1;
   for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < W * W; e += gridDim.x * blockDim.x) {
     const int m1 = e / W - Lt, m2 = e % W - Lt;
-    const int l0 = max(abs(m1), abs(m2));
-    const int mu = abs(m1 - m2), nu = abs(m1 + m2);
-    seedu[e] = seed_xi(m1, m2) * exp(seed_log_factor(mu, nu));
-    for (int l = l0; l <= Lt; ++l) {
-      double A = 0.0, B = 0.0, C = 0.0;
-      if (l < Lt) recurrence_terms(l, m1, m2, A, B, C);
-      double* r = rec + 3 * kidx(l, m1, m2);
-      // A_0 = 0 (no d^{-1} term); the square root is undefined at l = 0
-      r[0] = l > 0 ? A * sqrt((2.0 * l - 1.0) / (2.0 * l + 3.0)) : 0.0;
-      r[1] = B * sqrt((2.0 * l + 1.0) / (2.0 * l + 3.0));
-      r[2] = C;
-    }
+    seedu[e] = seed_xi(m1, m2) * exp(seed_log_factor(abs(m1 - m2), abs(m1 + m2)));
+  }
+}
+
+// Sums over the wavefront of ten values a lane, written to out[0..9]: two
+// halvings that keep one value per half, then a sum within rows of 16 lanes.
+// 60 instructions; ten butterflies over the lanes are 180 and wait 60 times.
+FO_DEV double swap_add32(double a, double b) {  // lanes 0-31: sum of a, 32-63: of b
+  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false,
+                                                   false);
+  return __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]) +
+         __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+}
+FO_DEV double swap_add16(double a, double b) {  // rows 0, 2: sums of a's, 1, 3: of b's halves
+  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false,
+                                                   false);
+  return __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]) +
+         __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+}
+template <int CTRL>
+FO_DEV double dpp_add(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), CTRL, 0xf, 0xf, true);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+FO_DEV double row_sum(double v) {  // over the 16 lanes of a row (rotations)
+  v = dpp_add<0x128>(v);
+  v = dpp_add<0x124>(v);
+  v = dpp_add<0x122>(v);
+  return dpp_add<0x121>(v);
+}
+FO_DEV void wave_sum10(const double (&v)[10], double* out) {
+  double u[5], w[3];
+#pragma unroll
+  for (int j = 0; j < 5; ++j) u[j] = swap_add32(v[j], v[j + 5]);
+  w[0] = row_sum(swap_add16(u[0], u[3]));
+  w[1] = row_sum(swap_add16(u[1], u[4]));
+  w[2] = row_sum(swap_add16(u[2], 0.0));
+  // rows: w[j] holds v[j], v[j + 3], v[j + 5], v[j + 8] (w[2]: v[2], -, v[7], -)
+  const int lane = threadIdx.x & 63, row = lane >> 4;
+  if ((lane & 15) == 0) {
+    const int at = row == 0 ? 0 : row == 1 ? 3 : row == 2 ? 5 : 8;
+    out[at] = w[0];
+    out[at + 1] = w[1];
+    if (!(row & 1)) out[at + 2] = w[2];
   }
 }
 
@@ -1828,59 +1865,63 @@ struct FGH {
   double v[10];  // f, fa, fb, fy, faa, fab, fay, fbb, fby, fyy
 };
 
-// Recurrence coefficients of the unnormalised d from two small tables in
-// LDS instead of the per-entry table: with s_l(m) = sqrt(l^2 - m^2) and
-// e_l = s_l(m1) s_l(m2),
+// Recurrence coefficients of the unnormalised d from a small table in LDS:
+// with s_l(m) = sqrt(l^2 - m^2) and e_l = s_l(m1) s_l(m2),
 //   Bu_l = (l+1)(2l+1) / e_{l+1},  Au_l = (l+1)/l e_l / e_{l+1},
-//   C_l = m1 m2 / (l(l+1))        (Au_0 = C_0 = 0),
-// the same values as k_rec_table's (to rounding).  st / ist hold s_l(m) and
-// 1 / s_l(m) (0 for m >= l) for l, m <= Lp1 - 1, row stride Lp1; al / cl
-// hold (l+1)/l and 1/(l(l+1)) (0 at l = 0).
+//   C_l = m1 m2 / (l(l+1))        (Au_0 = C_0 = 0).
+// sm holds (s_l(m), 1 / s_{l+1}(m)) (0 where m is too large) for l <= L,
+// m <= L, row stride L + 2; al / cl hold (l+1)/l and 1/(l(l+1)) (0 at l = 0).
 struct RecLds {
-  const double* st;
-  const double* ist;
+  const double2* sm;
   const double* al;
   const double* cl;
-  int Lp1;
+  int stride;
 };
-FO_DEV size_t rec_lds_doubles(int Lp1) { return 2 * (size_t)Lp1 * Lp1 + 2 * (size_t)Lp1; }
-FO_DEV RecLds build_rec_lds(double* t, int Lp1) {
-  double *st = t, *ist = t + Lp1 * Lp1, *al = ist + Lp1 * Lp1, *cl = al + Lp1;
-  for (int e = threadIdx.x; e < Lp1 * Lp1; e += blockDim.x) {
-    const int l = e / Lp1, m = e % Lp1;
-    const double v = m < l ? sqrt((double)(l * l - m * m)) : 0.0;
-    st[e] = v;
-    ist[e] = m < l ? 1.0 / v : 0.0;
+FO_HD size_t rec_lds_bytes(int L) {
+  return sizeof(double2) * (size_t)(L + 1) * (L + 2) + sizeof(double) * 2 * (size_t)(L + 2);
+}
+FO_DEV RecLds build_rec_lds(double2* t, int L) {
+  const int S = L + 2;
+  double *al = (double*)(t + (L + 1) * S), *cl = al + S;
+  for (int e = threadIdx.x; e < (L + 1) * S; e += blockDim.x) {
+    const int l = e / S, m = e % S;
+    t[e] = make_double2(m < l ? sqrt((double)(l * l - m * m)) : 0.0,
+                        m <= l ? 1.0 / sqrt((double)((l + 1) * (l + 1) - m * m)) : 0.0);
   }
-  for (int l = threadIdx.x; l < Lp1; l += blockDim.x) {
+  for (int l = threadIdx.x; l < S; l += blockDim.x) {
     al[l] = l > 0 ? (double)(l + 1) / l : 0.0;
     cl[l] = l > 0 ? 1.0 / ((double)l * (l + 1)) : 0.0;
   }
-  return RecLds{st, ist, al, cl, Lp1};
+  return RecLds{t, al, cl, S};
 }
 
-// `ph`: LDS for 3L + 2 phase factors; `part`: LDS for (kFghBlocks + 1) * 10
-// doubles; `ctr`: an LDS int.
+// `ph`: LDS for 3L + 3 phase factors; `pw`: LDS for 2 (2L + 1) powers; `part`:
+// LDS for kFghBlocks * 10 doubles; `ctr`: an LDS int.  The result is valid in
+// the first wavefront; a barrier must follow before the next call.
 constexpr int kEvalUnroll = 2;  // degrees per batch of operand loads
 constexpr int kFghBlocks = (64 * 64 + 63 + 63) / 64;  // item blocks at L = 63
-template <bool kLdsRec = false>
+constexpr int kFghPhases = 3 * 63 + 3, kFghPowers = 2 * (2 * 63 + 1);
 FO_DEV void eval_fgh(const double2* __restrict__ I, double sgn, int L, double a, double b,
-                     double y, const double* __restrict__ rec, const double* __restrict__ seedu,
-                     int Lt, FGH& out, double* part, double2* ph, int* ctr,
-                     RecLds rl = RecLds{}) {
-  const int W = 2 * L + 1, Wt = 2 * Lt + 1;
-  const double cb = cos(b), sb = sin(b), c2 = cos(0.5 * b), s2 = sin(0.5 * b);
-  // phase factors e^{-i m1 a} (m1 = 0..L) and e^{-i m2 y} (m2 = -L..L)
-  for (int q = threadIdx.x; q < 3 * L + 2; q += blockDim.x) {
+                     double y, const double* __restrict__ seedu, int Lt, FGH& out, double* part,
+                     double2* ph, double* pw, int* ctr, const RecLds& rl) {
+  const int Wt = 2 * Lt + 1;
+  const __amdgpu_buffer_rsrc_t ri = buf_rsrc(I, (int)(kcount(L) * sizeof(double2)));
+  double s2, c2;
+  sincos(0.5 * b, &s2, &c2);
+  // phase factors e^{-i m1 a} (m1 = 0..L), e^{-i m2 y} (m2 = -L..L) and e^{i b}
+  // from the first wavefronts on, powers of s2 and c2 from the last ones
+  for (int q = threadIdx.x; q < 3 * L + 3; q += blockDim.x) {
+    const double arg = q <= L ? -(q * a) : q < 3 * L + 2 ? -((q - L - 1 - L) * y) : b;
     double sp, cp;
-    if (q <= L)
-      sincos(-(q * a), &sp, &cp);
-    else
-      sincos(-((q - L - 1 - L) * y), &sp, &cp);
+    sincos(arg, &sp, &cp);
     ph[q] = make_double2(cp, sp);
   }
+  for (int q = blockDim.x - 1 - threadIdx.x; q < 2 * (2 * L + 1); q += blockDim.x)
+    pw[q] = q <= 2 * L ? ipow(s2, q) : ipow(c2, q - 2 * L - 1);
   if (threadIdx.x == 0) *ctr = blockDim.x >> 6;
   __syncthreads();
+  const double cb = ph[3 * L + 2].x, sb = ph[3 * L + 2].y;
+  const double *ps = pw, *pc = pw + 2 * L + 1;
   // The sum runs over the entries (m1 >= 0, m2).  d and its b-derivatives
   // obey d_{m1,m2} = (-1)^{m1-m2} d_{m2,m1} = d_{-m2,-m1}, so one recurrence
   // serves two entries: item (l0, m2), |m2| <= l0 (the row m1 = l0 of shell
@@ -1906,9 +1947,9 @@ FO_DEV void eval_fgh(const double2* __restrict__ I, double sgn, int L, double a,
       l0 = 0;
       row = true;
     } else if (act) {
-      l0 = (int)((sqrt(4.0 * e + 5.0) - 1.0) * 0.5);
-      while (l0 * l0 + l0 - 1 > e) --l0;
-      while ((l0 + 1) * (l0 + 1) + l0 <= e) ++l0;
+      l0 = (int)((sqrtf(4.f * e + 5.f) - 1.f) * 0.5f);  // off by one at most
+      if (l0 * l0 + l0 - 1 > e) --l0;
+      if ((l0 + 1) * (l0 + 1) + l0 <= e) ++l0;
       const int r = e - (l0 * l0 + l0 - 1);
       row = r <= 2 * l0;
       m1 = row ? l0 : 0;
@@ -1920,9 +1961,9 @@ FO_DEV void eval_fgh(const double2* __restrict__ I, double sgn, int L, double a,
     const int mu = abs(m1 - m2), nu = abs(m1 + m2);
     // edge element g = s2^mu c2^nu and its b-derivatives
     const double fct = seedu[(m1 + Lt) * Wt + (m2 + Lt)];
-    const double smu = ipow(s2, mu), cnu = ipow(c2, nu);
-    const double smu1 = mu ? ipow(s2, mu - 1) : 0.0, cnu1 = nu ? ipow(c2, nu - 1) : 0.0;
-    const double smu2 = mu > 1 ? ipow(s2, mu - 2) : 0.0, cnu2 = nu > 1 ? ipow(c2, nu - 2) : 0.0;
+    // (a power below 0 has the factor 0)
+    const double smu = ps[mu], smu1 = ps[max(mu - 1, 0)], smu2 = ps[max(mu - 2, 0)];
+    const double cnu = pc[nu], cnu1 = pc[max(nu - 1, 0)], cnu2 = pc[max(nu - 2, 0)];
     const double g0 = smu * cnu;
     const double g1 = 0.5 * (mu * smu1 * cnu * c2 - nu * smu * s2 * cnu1);
     // g'' = 1/4 [mu(mu-1) s^{mu-2} c^{nu+2} - (mu(nu+1) + nu(mu+1)) s^mu c^nu
@@ -1932,31 +1973,29 @@ FO_DEV void eval_fgh(const double2* __restrict__ I, double sgn, int L, double a,
                               nu * (nu - 1) * smu * s2 * s2 * cnu2);
     double c0x = 0, c0y = 0, c1x = 0, c1y = 0, c2x = 0, c2y = 0;
     double q0x = 0, q0y = 0, q1x = 0, q1y = 0, q2x = 0, q2y = 0;  // partner
-    double d0 = fct * g0, d1 = fct * g1, dd2 = fct * g2;
+    // sgn^l goes with d: into the seed and the terms that step l by one
+    const double f0 = (l0 & 1) ? sgn * fct : fct;
+    double d0 = f0 * g0, d1 = f0 * g1, dd2 = f0 * g2;
     double p0 = 0, p1 = 0, p2 = 0;
-    double sl = (l0 & 1) ? sgn : 1.0;
-    auto step = [&](int l, const double2& Iv, const double2& Pv, double Au, double Bu, double C) {
-      // conj(sgn^l I) * d
-      const double ix = sl * Iv.x, iy = -sl * Iv.y;
-      const double jx = sl * Pv.x, jy = -sl * Pv.y;
-      c0x += d0 * ix;
-      c0y += d0 * iy;
-      c1x += d1 * ix;
-      c1y += d1 * iy;
-      c2x += dd2 * ix;
-      c2y += dd2 * iy;
-      q0x += d0 * jx;
-      q0y += d0 * jy;
-      q1x += d1 * jx;
-      q1y += d1 * jy;
-      q2x += dd2 * jx;
-      q2y += dd2 * jy;
-      sl *= sgn;
-      if (l == L) return;
+    const double m12 = (double)(m1 * m2), sb2 = 2.0 * sb;
+    // sums of d I (the conjugate is taken at the end)
+    auto step = [&](const double2& Iv, const double2& Pv, double Au, double Bu, double C) {
+      c0x += d0 * Iv.x;
+      c0y += d0 * Iv.y;
+      c1x += d1 * Iv.x;
+      c1y += d1 * Iv.y;
+      c2x += dd2 * Iv.x;
+      c2y += dd2 * Iv.y;
+      q0x += d0 * Pv.x;
+      q0y += d0 * Pv.y;
+      q1x += d1 * Pv.x;
+      q1y += d1 * Pv.y;
+      q2x += dd2 * Pv.x;
+      q2y += dd2 * Pv.y;
       const double bc = Bu * (cb - C);
       const double n0 = bc * d0 - Au * p0;
-      const double n1 = bc * d1 - Bu * sb * d0 - Au * p1;
-      const double n2 = bc * dd2 - Bu * (cb * d0 + 2.0 * sb * d1) - Au * p2;
+      const double n1 = bc * d1 - Bu * (sb * d0) - Au * p1;
+      const double n2 = bc * dd2 - Bu * (cb * d0 + sb2 * d1) - Au * p2;
       p0 = d0;
       p1 = d1;
       p2 = dd2;
@@ -1964,56 +2003,51 @@ FO_DEV void eval_fgh(const double2* __restrict__ I, double sgn, int L, double a,
       d1 = n1;
       dd2 = n2;
     };
-    // operands (coefficients of the item and its partner, recurrence terms
-    // to l + 1) of kEvalUnroll degrees at a time, all loads issued before
-    // the steps.  The loaded degree is max(l, l0) clamped to L (terms of
-    // degree L are not used).
-    auto next_id = [&](int id, int l) { return next_kidx(id, l, l0, m1, L); };
-    // smallest l0 of the wavefront (the items (0, -l0) that follow the
-    // shells can share a wavefront with shell L)
-    int lmin = l0;
-    for (int off = 32; off > 0; off >>= 1) lmin = min(lmin, __shfl_xor(lmin, off, 64));
-    const int lw = __builtin_amdgcn_readfirstlane(lmin);
-    int id = act ? (int)kidx(l0, m1, m2) : 0;
-    int pid = hasp ? (int)kidx(l0, pm1, pm2) : 0;
-    for (int l = lw; l <= L; l += kEvalUnroll) {  // wavefront-uniform
-      int ids[kEvalUnroll], pids[kEvalUnroll];
+    // coefficients of the item and its partner for kEvalUnroll degrees at a
+    // time, loaded while the steps of the batch before run: entry (l, m1, m2)
+    // at kbase(l) + (m1 + l)(2l + 1) + m2 + l.  Reads outside the set give
+    // zero; below l0 and above L they are not used, and a lane without a
+    // partner reads as if (pm1, pm2) were one (its sums are not used).
+    struct Batch {
       double2 Iv[kEvalUnroll], Pv[kEvalUnroll];
-      double Au[kEvalUnroll], Bu[kEvalUnroll], C[kEvalUnroll];
-      ids[0] = id;
-      pids[0] = pid;
-#pragma unroll
-      for (int q = 1; q < kEvalUnroll; ++q) {
-        ids[q] = next_id(ids[q - 1], l + q - 1);
-        pids[q] = hasp ? next_kidx(pids[q - 1], l + q - 1, l0, pm1, L) : 0;
-      }
+    } ba, bb;
+    const int ms = 16 * m2, pms = 16 * pm2;
+    auto load = [&](Batch& B, int l) {
 #pragma unroll
       for (int q = 0; q < kEvalUnroll; ++q) {
-        Iv[q] = I[ids[q]];
-        Pv[q] = I[pids[q]];
-        if constexpr (kLdsRec) {
-          // degree lq = l + q (wavefront-uniform); lanes below their first
-          // degree take harmless values (their steps are skipped)
-          const int lq = min(l + q, L), am1 = m1, am2 = m2 < 0 ? -m2 : m2;
-          const double* s0 = rl.st + lq * rl.Lp1;
-          const double* i1 = rl.ist + (lq + 1) * rl.Lp1;
-          const double ie = i1[am1] * i1[am2];  // 1 / e_{l+1}
-          const double el = s0[am1] * s0[am2];  // e_l
-          Bu[q] = (double)((lq + 1) * (2 * lq + 1)) * ie;
-          Au[q] = rl.al[lq] * el * ie;
-          C[q] = (double)(m1 * m2) * rl.cl[lq];
-        } else {
-          Au[q] = rec[3 * ids[q]];
-          Bu[q] = rec[3 * ids[q] + 1];
-          C[q] = rec[3 * ids[q] + 2];
-        }
-        __builtin_amdgcn_sched_barrier(0);  // keep the loads in degree order
+        const int lq = l + q, W16 = 16 * (2 * lq + 1);
+        const int base = 16 * (lq * (2 * lq - 1) * (2 * lq + 1) / 3 + lq * (2 * lq + 2));  // (0, 0)
+        B.Iv[q] = load_d2(ri, base + ms + m1 * W16, 0);
+        B.Pv[q] = load_d2(ri, base + pms + pm1 * W16, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // issued before the steps that follow
+    };
+    const int am1 = m1, am2 = m2 < 0 ? -m2 : m2;
+    auto steps = [&](const Batch& B, int l) {
+      double Au[kEvalUnroll], Bu[kEvalUnroll], C[kEvalUnroll];
+#pragma unroll
+      for (int q = 0; q < kEvalUnroll; ++q) {
+        // degree lq (wavefront-uniform); lanes below their first degree take
+        // harmless values (their steps are skipped)
+        const int lq = min(l + q, L);
+        const double2 x1 = rl.sm[lq * rl.stride + am1], x2 = rl.sm[lq * rl.stride + am2];
+        const double ie = x1.y * x2.y;  // 1 / e_{l+1}
+        Bu[q] = sgn * (double)((lq + 1) * (2 * lq + 1)) * ie;
+        Au[q] = rl.al[lq] * (x1.x * x2.x) * ie;
+        C[q] = m12 * rl.cl[lq];
       }
 #pragma unroll
       for (int q = 0; q < kEvalUnroll; ++q)
-        if (l + q <= L && l + q >= l0) step(l + q, Iv[q], Pv[q], Au[q], Bu[q], C[q]);
-      id = next_id(ids[kEvalUnroll - 1], l + kEvalUnroll - 1);
-      pid = hasp ? next_kidx(pids[kEvalUnroll - 1], l + kEvalUnroll - 1, l0, pm1, L) : 0;
+        if (l + q <= L && l + q >= l0) step(B.Iv[q], B.Pv[q], Au[q], Bu[q], C[q]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    const int lw = __builtin_amdgcn_readfirstlane(l0);  // smallest of the wavefront
+    load(ba, lw);
+    for (int l = lw; l <= L; l += 2 * kEvalUnroll) {  // wavefront-uniform
+      load(bb, l + kEvalUnroll);
+      steps(ba, l);
+      load(ba, l + 2 * kEvalUnroll);
+      steps(bb, l + kEvalUnroll);
     }
     // the item's entry (m1, m2) and its partner (pm1, pm2): weight 2 for
     // m1 > 0 (the rows m1 < 0 by Hermitian symmetry), the partner's sign
@@ -2022,8 +2056,8 @@ FO_DEV void eval_fgh(const double2* __restrict__ I, double sgn, int L, double a,
     for (int k = 0; k < 2; ++k) {
       const int a1 = k ? pm1 : m1, a2 = k ? pm2 : m2;
       const double w = k ? (hasp ? (a1 == 0 ? psg : 2.0 * psg) : 0.0) : (a1 == 0 ? 1.0 : 2.0);
-      const double x0 = k ? q0x : c0x, y0 = k ? q0y : c0y, x1 = k ? q1x : c1x;
-      const double y1 = k ? q1y : c1y, x2 = k ? q2x : c2x, y2 = k ? q2y : c2y;
+      const double x0 = k ? q0x : c0x, y0 = k ? -q0y : -c0y, x1 = k ? q1x : c1x;
+      const double y1 = k ? -q1y : -c1y, x2 = k ? q2x : c2x, y2 = k ? -q2y : -c2y;
       const double2 ea = ph[a1], ey = ph[2 * L + 1 + a2];
       const double cp = ea.x * ey.x - ea.y * ey.y, sp = ea.x * ey.y + ea.y * ey.x;
       // Re(c E) and Re(-i c E) = Im(c E)
@@ -2042,29 +2076,23 @@ FO_DEV void eval_fgh(const double2* __restrict__ I, double sgn, int L, double a,
       acc[8] -= w * M2 * i1;
       acc[9] -= w * (-M2 * M2 * r0);
     }
-#pragma unroll
-    for (int q = 0; q < 10; ++q) {
-      const double v = wave_sum(acc[q]);
-      if (lane == 0) part[blk * 10 + q] = v;
-    }
+    wave_sum10(acc, part + blk * 10);
     int nb = 0;
     if (lane == 0) nb = atomicAdd(ctr, 1);
     blk = __builtin_amdgcn_readfirstlane(nb);
   }
   __syncthreads();
-  if (threadIdx.x < 10) {
+  if (threadIdx.x < 64) {
     double v = 0.0;
-    for (int b = 0; b < nblk; ++b) v += part[b * 10 + threadIdx.x];
-    part[kFghBlocks * 10 + threadIdx.x] = v;
-  }
-  __syncthreads();
-  // the sums are uniform over the workgroup: keep them in scalar registers
+#pragma unroll 4
+    for (int k = 0; k < nblk; ++k) v += part[k * 10 + min(lane, 9)];
+    const long long bits = __double_as_longlong(v);
 #pragma unroll
-  for (int q = 0; q < 10; ++q) {
-    const long long b = __double_as_longlong(part[kFghBlocks * 10 + q]);
-    const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffLL));
-    const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-    out.v[q] = __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    for (int q = 0; q < 10; ++q) {
+      const int lo = __builtin_amdgcn_readlane((int)(bits & 0xffffffffLL), q);
+      const int hi = __builtin_amdgcn_readlane((int)(bits >> 32), q);
+      out.v[q] = __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    }
   }
 }
 
@@ -2072,18 +2100,19 @@ FO_DEV bool chol3_solve(const double H[6], double lam, const double g[3], double
   // H = [haa hab hay; hab hbb hby; hay hby hyy] stored (aa,ab,ay,bb,by,yy)
   double a00 = H[0] + lam, a10 = H[1], a20 = H[2], a11 = H[3] + lam, a21 = H[4], a22 = H[5] + lam;
   if (!(a00 > 0)) return false;
-  const double l00 = sqrt(a00), l10 = a10 / l00, l20 = a20 / l00;
+  const double r00 = rsqrt(a00), l10 = a10 * r00, l20 = a20 * r00;
   const double t11 = a11 - l10 * l10;
   if (!(t11 > 0)) return false;
-  const double l11 = sqrt(t11), l21 = (a21 - l20 * l10) / l11;
+  const double r11 = rsqrt(t11), l21 = (a21 - l20 * l10) * r11;
   const double t22 = a22 - l20 * l20 - l21 * l21;
   if (!(t22 > 0)) return false;
-  const double l22 = sqrt(t22);
-  // solve L L^T x = -g
-  const double z0 = -g[0] / l00, z1 = (-g[1] - l10 * z0) / l11, z2 = (-g[2] - l20 * z0 - l21 * z1) / l22;
-  x[2] = z2 / l22;
-  x[1] = (z1 - l21 * x[2]) / l11;
-  x[0] = (z0 - l10 * x[1] - l20 * x[2]) / l00;
+  const double r22 = rsqrt(t22);
+  // solve L L^T x = -g (r: reciprocals of the diagonal)
+  const double z0 = -g[0] * r00, z1 = (-g[1] - l10 * z0) * r11,
+               z2 = (-g[2] - l20 * z0 - l21 * z1) * r22;
+  x[2] = z2 * r22;
+  x[1] = (z1 - l21 * x[2]) * r11;
+  x[0] = (z0 - l10 * x[1] - l20 * x[2]) * r00;
   return true;
 }
 
@@ -2142,7 +2171,8 @@ FO_DEV void newton_update(NewtonState& s, const FGH& r) {
   double dx[3];
   bool ok = chol3_solve(H, 0.0, g, dx);
   const bool pure = ok;  // undamped Newton step (positive definite Hessian)
-  for (int k = 0; !ok && k < 12; ++k) ok = chol3_solve(H, hs * pow(10.0, -8.0 + k), g, dx);
+  double lam = 1e-8 * hs;
+  for (int k = 0; !ok && k < 12; ++k, lam *= 10.0) ok = chol3_solve(H, lam, g, dx);
   if (!ok)
     for (int q = 0; q < 3; ++q) dx[q] = -g[q] / hs;
   for (int q = 0; q < 3; ++q) s.dx[q] = dx[q];
@@ -2168,6 +2198,13 @@ FO_DEV void newton_update(NewtonState& s, const FGH& r) {
   for (int q = 0; q < 3; ++q) s.xt[q] = s.x[q] + dx[q];
 }
 
+// One workgroup per (pair, orientation).  Bound by latency for a few pairs: an
+// evaluation is the phases and powers (2300 cycles), a block's edge elements
+// (2900), its degrees and the ten sums (1100); by FP64 issue for many: about 50
+// instructions per item and degree, 32 of them FP64.  One pair, degree 15: 55
+// -> 29 us, 64 pairs of degree 40: 292 -> 134, 4096 of 16..25: 900 -> 530,
+// against powers by squaring per item, index updates and a sign per degree, and
+// a butterfly per sum.
 // Converged when the gradient, the Newton model decrease -g.dx/2 or the step
 // reaches the level where rounding noise of f (a sum of ~K(L) terms)
 // dominates: |g| <= 1e-12 |f|, decrease <= 1e-13 |f|, step <= 1e-12 rad.
@@ -2178,15 +2215,15 @@ __global__ void __launch_bounds__(256, 3) k_sph_rotopt(const SphPair* __restrict
                                                     const SphPeak* __restrict__ peaks, int norient,
                                                     const double* __restrict__ seedu, int Lt,
                                                     int Lmax, SphOpt* __restrict__ opt, int P) {
-  __shared__ double part[(kFghBlocks + 1) * 10];
-  __shared__ double2 ph[3 * 64 + 2];
+  __shared__ double part[kFghBlocks * 10], pw[kFghPowers];
+  __shared__ double2 ph[kFghPhases];
   __shared__ int s_blk;
-  extern __shared__ __align__(16) double rtab[];  // rec_lds_doubles(Lmax + 2)
+  extern __shared__ __align__(16) double2 rtab[];  // rec_lds_bytes(Lmax)
   int p, o;
   if (!xcd_decode(P, norient, p, o)) return;
   const SphPair d = pd[p];
   const int L = d.L;
-  const RecLds rl = build_rec_lds(rtab, Lmax + 2);
+  const RecLds rl = build_rec_lds(rtab, L);
   __syncthreads();
   const double sgn = (mode == 0 && o == 1) ? -1.0 : 1.0;
   const double2* I = ((mode == 1 && o == 1) ? IB : IA) + d.coef_off;
@@ -2200,8 +2237,7 @@ __global__ void __launch_bounds__(256, 3) k_sph_rotopt(const SphPair* __restrict
   __syncthreads();
   for (;;) {
     FGH r;
-    eval_fgh<true>(I, sgn, L, ns.xt[0], ns.xt[1], ns.xt[2], nullptr, seedu, Lt, r, part, ph,
-                   &s_blk, rl);
+    eval_fgh(I, sgn, L, ns.xt[0], ns.xt[1], ns.xt[2], seedu, Lt, r, part, ph, pw, &s_blk, rl);
     if (threadIdx.x == 0) newton_update(ns, r);
     __syncthreads();
     if (ns.stop) break;
@@ -2672,8 +2708,7 @@ void launch_sph_select(hipStream_t s, int P, int n, long long Kt, int norient, c
 void launch_sph_rotopt(hipStream_t s, int P, int norient, int Lmax, const SphPair* pd,
                        const double2* IA, const double2* IB, int mode, const SphPeak* peaks,
                        const double* seedu, int Lt, SphOpt* opt) {
-  const size_t smem = sizeof(double) * (2 * (size_t)(Lmax + 2) * (Lmax + 2) + 2 * (Lmax + 2));
-  hipLaunchKernelGGL(k_sph_rotopt, dim3(xcd_grid(P, norient)), dim3(256), smem, s, pd, IA, IB,
+  hipLaunchKernelGGL(k_sph_rotopt, dim3(xcd_grid(P, norient)), dim3(256), rec_lds_bytes(Lmax), s, pd, IA, IB,
                      mode, peaks, norient, seedu, Lt, Lmax, opt, P);
 }
 
@@ -2748,14 +2783,16 @@ __global__ void k_coef_to_plane(const SphPair* __restrict__ pd, int n,
 // coefficient set given as conj(X) in compact layout.
 __global__ void __launch_bounds__(256) k_sph_energy(int L, const double2* __restrict__ Iconj,
                                                     double a, double b, double y,
-                                                    const double* __restrict__ rec,
                                                     const double* __restrict__ seedu, int Lt,
                                                     double* __restrict__ out) {
-  __shared__ double part[(kFghBlocks + 1) * 10];
-  __shared__ double2 ph[3 * 64 + 2];
+  __shared__ double part[kFghBlocks * 10], pw[kFghPowers];
+  __shared__ double2 ph[kFghPhases];
   __shared__ int s_blk;
+  extern __shared__ __align__(16) double2 rtab[];  // rec_lds_bytes(L)
+  const RecLds rl = build_rec_lds(rtab, L);
+  __syncthreads();
   FGH r;
-  eval_fgh(Iconj, 1.0, L, a, b, y, rec, seedu, Lt, r, part, ph, &s_blk);
+  eval_fgh(Iconj, 1.0, L, a, b, y, seedu, Lt, r, part, ph, pw, &s_blk, rl);
   if (threadIdx.x == 0)
     for (int q = 0; q < 10; ++q) out[q] = r.v[q];
 }
@@ -2996,15 +3033,14 @@ void launch_coef_to_plane(hipStream_t s, int P, int n, int Lmax, const SphPair* 
                      n, a, b);
 }
 void launch_sph_energy(hipStream_t s, int L, const double2* Iconj, double a, double b, double y,
-                       const double* rec, const double* seedu, int Lt, double* out) {
-  hipLaunchKernelGGL(k_sph_energy, dim3(1), dim3(256), 0, s, L, Iconj, a, b, y, rec, seedu, Lt,
-                     out);
+                       const double* seedu, int Lt, double* out) {
+  hipLaunchKernelGGL(k_sph_energy, dim3(1), dim3(256), rec_lds_bytes(L), s, L, Iconj, a, b, y,
+                     seedu, Lt, out);
 }
 
-void launch_rec_table(hipStream_t s, int Lt, double* rec, double* seedu, double2* leg,
-                      double* cm) {
+void launch_rec_table(hipStream_t s, int Lt, double* seedu, double2* leg, double* cm) {
   const int W = 2 * Lt + 1;
-  hipLaunchKernelGGL(k_rec_table, dim3((W * W + 127) / 128), dim3(128), 0, s, Lt, rec, seedu);
+  hipLaunchKernelGGL(k_seed_table, dim3((W * W + 127) / 128), dim3(128), 0, s, Lt, seedu);
   hipLaunchKernelGGL(k_leg_table, dim3((qlm(Lt, Lt) + 128) / 128), dim3(128), 0, s, Lt, leg, cm);
 }
 void launch_wigner_D(hipStream_t s, int L, double a, double b, double y, double2* D, double2* G) {

@@ -95,6 +95,7 @@ _PROTOS = {
     "fo_sph_batch_run": (C.c_int, [_vp, C.c_int, C.c_int]),
     "fo_sph_batch_sync": (C.c_int, [_vp]),
     "fo_sph_batch_results": (C.c_int, [_vp, _pd, _pd, _pd, _pi, _pd, _pd, _pi]),
+    "fo_sph_batch_read": (C.c_int, [_vp, _pd, _pi]),
     "fo_sph_batch_peaks": (C.c_int, [_vp, _pi, _pd, _pd, _pd, _pd, _pi, _pi]),
     "fo_sph_batch_opt": (C.c_int, [_vp, _pd, _pd, _pd, _pi, _pi]),
     "fo_sph_batch_scales": (C.c_int, [_vp, _pd]),
@@ -125,6 +126,7 @@ _PROTOS = {
     "fo_per_batch_set_disp": (C.c_int, [_vp, _pd]),
     "fo_per_batch_run": (C.c_int, [_vp, C.c_int, C.c_int]),
     "fo_per_batch_sync": (C.c_int, [_vp]),
+    "fo_per_batch_read": (C.c_int, [_vp, _pd, _pi]),
     "fo_per_batch_results": (C.c_int, [_vp, _pd, _pd, _pd, _pi, _pd]),
     "fo_per_batch_peaks": (C.c_int, [_vp, _pi, _pd, _pd, _pd, _pd, _pi, _pi]),
     "fo_per_batch_coeffs": (C.c_int, [_vp, _pd, _pd]),

@@ -69,6 +69,25 @@ def _groups_arrays(groups_per_pair):
     return ngroups, sizes, atoms
 
 
+def _pair_slices(offsets):
+    o = offsets.tolist()
+    return [slice(a, b) for a, b in zip(o, o[1:])]
+
+
+def per_pair(a, slices):
+    """The rows of each pair as views, 80 ns apiece (an index expression with
+    numpy integers takes 350)."""
+    return list(map(a.__getitem__, slices))
+
+
+def _split(a, *sizes):
+    out, at = [], 0
+    for n in sizes:
+        out.append(a[at:at + n])
+        at += n
+    return out
+
+
 def next_pow2(x: int) -> int:
     return 1 << max(0, (int(x) - 1).bit_length())
 
@@ -115,6 +134,7 @@ class SphericalBatch:
         self.natoms = natoms.astype(np.int64)
         self.L = L.astype(np.int64)
         self.offsets = np.concatenate([[0], np.cumsum(self.natoms)])
+        self._slices = _pair_slices(self.offsets)
         self.norient = 1 if (flags & _lib.SPH_NO_INVERT) and not (flags & _lib.SPH_GENERAL) else 2
         self.koff = np.concatenate([[0], np.cumsum([kcount(int(x)) for x in self.L])])
         self._nat = as_i32(self.natoms)
@@ -212,20 +232,40 @@ class SphericalBatch:
     # -- outputs -------------------------------------------------------------
     def results(self):
         N = int(self.offsets[-1])
-        dist = np.zeros(self.P)
-        X1 = np.zeros((N, 3))
-        X2 = np.zeros((N, 3))
-        perm = np.zeros(N, np.int32)
-        R = np.zeros((self.P, 3))
-        rmat = np.zeros((self.P, 3, 3))
-        inv = np.zeros(self.P, np.int32)
+        dist = np.empty(self.P)
+        X1 = np.empty((N, 3))
+        X2 = np.empty((N, 3))
+        perm = np.empty(N, np.int32)
+        R = np.empty((self.P, 3))
+        rmat = np.empty((self.P, 3, 3))
+        inv = np.empty(self.P, np.int32)
         call("fo_sph_batch_results", self.handle, dptr(dist), dptr(X1), dptr(X2), iptr(perm),
              dptr(R), dptr(rmat), iptr(inv))
-        o = self.offsets
         return dict(dist=dist, R=R, rmat=rmat, inverted=inv.astype(bool),
-                    X1=[X1[o[p]:o[p + 1]] for p in range(self.P)],
-                    X2=[X2[o[p]:o[p + 1]] for p in range(self.P)],
-                    perm=[perm[o[p]:o[p + 1]].astype(np.int64) for p in range(self.P)])
+                    X1=per_pair(X1, self._slices), X2=per_pair(X2, self._slices),
+                    perm=per_pair(perm.astype(np.int64), self._slices))
+
+    def read(self):
+        """``results()``, ``peaks()``, ``opt()`` and ``scales()`` in one transfer."""
+        P, N, m = self.P, int(self.offsets[-1]), self.P * self.norient
+        f = np.empty(14 * P + 6 * N + 8 * m)
+        q = np.empty(P + N + 7 * m, np.int32)
+        call("fo_sph_batch_read", self.handle, dptr(f), iptr(q))
+        sh = (P, self.norient)
+        dist, R, rmat, scale, X1, X2, fun, val, mar, dl, gn, oR = _split(
+            f, P, 3 * P, 9 * P, P, 3 * N, 3 * N, m, m, m, m, m, 3 * m)
+        inv, perm, ind, nc, no, it, ev = _split(q, P, N, 3 * m, m, m, m, m)
+        fun = fun.reshape(sh)
+        r = dict(dist=dist, R=R.reshape(P, 3), rmat=rmat.reshape(P, 3, 3),
+                 inverted=inv.astype(bool), X1=per_pair(X1.reshape(N, 3), self._slices),
+                 X2=per_pair(X2.reshape(N, 3), self._slices),
+                 perm=per_pair(perm.astype(np.int64), self._slices))
+        pk = dict(ind=ind.reshape(sh + (3,)), fun=fun, value=val.reshape(sh),
+                  margin=mar.reshape(sh), delta=dl.reshape(sh), ncand=nc.reshape(sh),
+                  noverflow=no.reshape(sh))
+        opt = dict(R=oR.reshape(sh + (3,)), fun=fun.copy(), gnorm=gn.reshape(sh),
+                   iters=it.reshape(sh), evals=ev.reshape(sh))
+        return r, pk, opt, scale
 
     def peaks(self):
         m = self.P * self.norient
@@ -406,6 +446,7 @@ class PeriodicBatch:
         self.P, self.nk, self.F, self.flags = P, int(nk), int(F), flags
         self.natoms = natoms
         self.offsets = np.concatenate([[0], np.cumsum(natoms)])
+        self._slices = _pair_slices(self.offsets)
         self.ngroups_total = sum(len(g) for g in groups)
         self._nat = as_i32(natoms)
         self._box = as_f64(box)
@@ -461,18 +502,31 @@ class PeriodicBatch:
 
     def results(self):
         N = int(self.offsets[-1])
-        dist = np.zeros(self.P)
-        X1 = np.zeros((N, 3))
-        X2 = np.zeros((N, 3))
-        perm = np.zeros(N, np.int32)
-        disp = np.zeros((self.P, 3))
+        dist = np.empty(self.P)
+        X1 = np.empty((N, 3))
+        X2 = np.empty((N, 3))
+        perm = np.empty(N, np.int32)
+        disp = np.empty((self.P, 3))
         call("fo_per_batch_results", self.handle, dptr(dist), dptr(X1), dptr(X2), iptr(perm),
              dptr(disp))
-        o = self.offsets
-        return dict(dist=dist, disp=disp,
-                    X1=[X1[o[p]:o[p + 1]] for p in range(self.P)],
-                    X2=[X2[o[p]:o[p + 1]] for p in range(self.P)],
-                    perm=[perm[o[p]:o[p + 1]].astype(np.int64) for p in range(self.P)])
+        return dict(dist=dist, disp=disp, X1=per_pair(X1, self._slices),
+                    X2=per_pair(X2, self._slices),
+                    perm=per_pair(perm.astype(np.int64), self._slices))
+
+    def read(self):
+        """``results()`` and ``peaks()`` in one transfer."""
+        P, N = self.P, int(self.offsets[-1])
+        f = np.empty(10 * P + 6 * N)
+        q = np.empty(N + 5 * P, np.int32)
+        call("fo_per_batch_read", self.handle, dptr(f), iptr(q))
+        dist, disp, X1, X2, disp0, val, mar, dl = _split(f, P, 3 * P, 3 * N, 3 * N, 3 * P, P, P, P)
+        perm, ind, nc, no = _split(q, N, 3 * P, P, P)
+        r = dict(dist=dist, disp=disp.reshape(P, 3),
+                 X1=per_pair(X1.reshape(N, 3), self._slices),
+                 X2=per_pair(X2.reshape(N, 3), self._slices),
+                 perm=per_pair(perm.astype(np.int64), self._slices))
+        return r, dict(ind=ind.reshape(P, 3), disp=disp0.reshape(P, 3), value=val, margin=mar,
+                       delta=dl, ncand=nc, noverflow=no)
 
     def peaks(self):
         P = self.P

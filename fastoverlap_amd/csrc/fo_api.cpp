@@ -170,7 +170,121 @@ struct fo_context {
   std::map<std::tuple<int, int, int, int>, std::array<int, 3>> tuned;
   RecTable rect;
   std::vector<void*> owned;  // table allocations
+  std::mutex slab_mu;
+  std::vector<void*> slabs;  // idle pinned staging buffers
 };
+
+// Pinned staging for small transfers: a buffer is one thread's from get to
+// put; at most kSlabsKept idle ones are kept.  One copy of a batch's adjacent
+// outputs through a buffer takes 10 us; a copy of each output into pageable
+// memory took 8..15 us apiece.  Larger transfers go to the caller's memory directly
+// (18 GB/s, as fast as the copy out of a buffer).
+static constexpr size_t kSlabBytes = 256 << 10;
+static constexpr size_t kSlabsKept = 16;
+static void* slab_get(fo_context* c) {
+  {
+    std::lock_guard<std::mutex> g(c->slab_mu);
+    if (!c->slabs.empty()) {
+      void* p = c->slabs.back();
+      c->slabs.pop_back();
+      return p;
+    }
+  }
+  void* p = nullptr;
+  if (hipHostMalloc(&p, kSlabBytes, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;  // the caller copies directly
+  }
+  return p;
+}
+static void slab_put(fo_context* c, void* p) {
+  if (!p) return;
+  {
+    std::lock_guard<std::mutex> g(c->slab_mu);
+    if (c->slabs.size() < kSlabsKept) {
+      c->slabs.push_back(p);
+      return;
+    }
+  }
+  (void)hipHostFree(p);
+}
+
+// Device memory read in one go: [dev, dev + bytes) through a staging buffer
+// into `use(const char*)`, if it is small enough and `own` (memory of the
+// context; a caller's arena never makes an allocation here).  Returns false if
+// the range has to be copied directly.
+template <class F>
+static bool read_staged(fo_context* c, bool own, hipStream_t s, const void* dev, size_t bytes,
+                        F&& use, hipError_t* err) {
+  if (!own || bytes > kSlabBytes) return false;
+  void* slab = slab_get(c);
+  if (!slab) return false;
+  *err = hipMemcpyAsync(slab, dev, bytes, hipMemcpyDeviceToHost, s);
+  if (*err == hipSuccess) *err = hipStreamSynchronize(s);
+  if (*err == hipSuccess) use((const char*)slab);
+  slab_put(c, slab);
+  return true;
+}
+
+template <class B>
+static void release_slab(B* b) {  // the batch's stream is idle
+  slab_put(b->ctx, b->slab);
+  b->slab = nullptr;
+}
+
+// Parts of the batch's memory, in ascending order, to where `to` is not NULL.
+template <class B, class Part, size_t K>
+static int read_parts(B* b, const Part (&parts)[K]) {
+  size_t lo = SIZE_MAX, hi = 0;
+  for (const Part& p : parts)
+    if (p.to) {
+      lo = std::min(lo, p.off);
+      hi = std::max(hi, p.off + p.bytes);
+    }
+  if (hi <= lo) return FO_OK;
+  const char* base = (const char*)b->base;
+  hipError_t e = hipSuccess;
+  const bool staged = read_staged(
+      b->ctx, b->own_mem, b->stream, base + lo, hi - lo,
+      [&](const char* h) {
+        for (const Part& p : parts)
+          if (p.to) memcpy(p.to, h + (p.off - lo), p.bytes);
+      },
+      &e);
+  if (!staged) {
+    for (const Part& p : parts)
+      if (p.to && p.bytes)
+        FO_HIP(hipMemcpyAsync(p.to, base + p.off, p.bytes, hipMemcpyDeviceToHost, b->stream));
+    e = hipStreamSynchronize(b->stream);
+  }
+  if (e != hipSuccess) return set_err(FO_ERR_HIP, hipGetErrorString(e));
+  release_slab(b);
+  return FO_OK;
+}
+
+// Host positions into a batch: pos2 lies at a fixed distance after pos1, so a
+// staged pair is one copy, which needs no wait (`slab` is the batch's until its
+// stream is next synchronised).
+static int write_positions(fo_context* c, bool own, hipStream_t s, double* d1, double* d2,
+                           const double* p1, const double* p2, size_t n, void** slab) {
+  const size_t gap = (char*)d2 - (char*)d1, bytes = gap + sizeof(double) * n;
+  if (own && bytes <= kSlabBytes) {
+    if (*slab)
+      FO_HIP(hipStreamSynchronize(s));  // an earlier copy may still read it
+    else
+      *slab = slab_get(c);
+    if (*slab) {
+      memcpy(*slab, p1, sizeof(double) * n);
+      memcpy((char*)*slab + gap, p2, sizeof(double) * n);
+      FO_HIP(hipMemcpyAsync(d1, *slab, bytes, hipMemcpyHostToDevice, s));
+      return FO_OK;
+    }
+  }
+  FO_HIP(hipMemcpyAsync(d1, p1, sizeof(double) * n, hipMemcpyHostToDevice, s));
+  FO_HIP(hipMemcpyAsync(d2, p2, sizeof(double) * n, hipMemcpyHostToDevice, s));
+  FO_HIP(hipStreamSynchronize(s));
+  return FO_OK;
+}
 
 static int ctx_alloc(fo_context* c, size_t bytes, void** p) {
   {
@@ -425,6 +539,7 @@ int fo_context_destroy(fo_context* c) {
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   for (void* p : c->owned) (void)hipFree(p);
+  for (void* p : c->slabs) (void)hipHostFree(p);
   (void)hipStreamDestroy(c->stream);
   delete c;
   return FO_OK;
@@ -504,6 +619,7 @@ struct fo_sph_batch {
   } off{};
   int gsum = 0;
   bool own_mem = false, own_stream = false;
+  void* slab = nullptr;  // staging buffer of the last host positions
   PeakScratch pk;  // multi-peak search buffers (allocated on first use)
   // FO_SPH_BETA_GEMM: even / odd-degree beta sums from k_beta_gemm
   // (split-BF16x3 on the matrix cores), [pair][beta][m1 <= Lmax][entry]
@@ -793,10 +909,15 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
   o.gath = lay.add<int>(b->hgath.size());
   o.pos1 = lay.add<double>(3 * Ntot);
   o.pos2 = lay.add<double>(3 * Ntot);
-  o.X1c = lay.add<double>(3 * Ntot);
   o.X2c = lay.add<double>(3 * Ntot);
   o.X2R = lay.add<double>(3 * Ntot);
+  // outputs, adjacent (sph_read)
+  o.X1c = lay.add<double>(3 * Ntot);
   o.X2out = lay.add<double>(3 * Ntot);
+  o.perm = lay.add<int>(Ntot);
+  o.res = lay.add<SphResult>(P);
+  o.peaks = lay.add<SphPeak>((size_t)P * no);
+  o.opt = lay.add<SphOpt>((size_t)P * no);
   o.scale = lay.add<double>(P);
   o.R = lay.add<double>(std::max(radmax, 1LL));
   o.Y1 = lay.add<double2>(std::max(ylmmax, 1LL));
@@ -808,10 +929,6 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
   o.I32B = general ? lay.add<float2>(C32tot) : 0;
   o.cand = lay.add<PlaneCand>((size_t)P * no * n);
   o.abound = lay.add<double>((size_t)P * no);
-  o.peaks = lay.add<SphPeak>((size_t)P * no);
-  o.opt = lay.add<SphOpt>((size_t)P * no);
-  o.res = lay.add<SphResult>(P);
-  o.perm = lay.add<int>(Ntot);
   o.rowsol = lay.add<int>(Ntot + 1);
   o.scr = lay.add<double2>((size_t)P * no * b->scr_stride);
   o.grid = lc.keep_grid ? lay.add<float>((size_t)P * no * n * n * n) : 0;
@@ -980,6 +1097,7 @@ int fo_sph_batch_coef_norm2(fo_sph_batch* b, double* norm2) {
 int fo_sph_batch_destroy(fo_sph_batch* b) {
   if (!b) return FO_OK;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
+  release_slab(b);
   for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second);
   if (b->ev_made) {
     for (auto& e : b->ev) (void)hipEventDestroy(e);
@@ -1004,10 +1122,8 @@ int fo_sph_batch_set_positions(fo_sph_batch* b, const double* p1, const double* 
   if (!b || !p1 || !p2) return set_err(FO_ERR_INVALID, "NULL argument");
   if (!all_finite(p1, 3 * b->Ntot) || !all_finite(p2, 3 * b->Ntot))
     return set_err(FO_ERR_INVALID, "positions must be finite");
-  FO_HIP(hipMemcpyAsync(b->pos1, p1, sizeof(double) * 3 * b->Ntot, hipMemcpyHostToDevice, b->stream));
-  FO_HIP(hipMemcpyAsync(b->pos2, p2, sizeof(double) * 3 * b->Ntot, hipMemcpyHostToDevice, b->stream));
-  FO_HIP(hipStreamSynchronize(b->stream));
-  return FO_OK;
+  return write_positions(b->ctx, b->own_mem, b->stream, b->pos1, b->pos2, p1, p2, 3 * b->Ntot,
+                         &b->slab);
 }
 
 int fo_sph_batch_set_positions_device(fo_sph_batch* b, const void* p1, const void* p2) {
@@ -1187,7 +1303,31 @@ int fo_sph_batch_run(fo_sph_batch* b, int stages, int use_graph) {
 int fo_sph_batch_sync(fo_sph_batch* b) {
   if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
   FO_HIP(hipStreamSynchronize(b->stream));
+  release_slab(b);
   return FO_OK;
+}
+
+// Outputs of a batch, each where its pointer is not NULL.
+struct SphOut {
+  double *X1 = nullptr, *X2 = nullptr, *scale = nullptr;
+  int* perm = nullptr;
+  SphResult* res = nullptr;
+  SphPeak* pk = nullptr;
+  SphOpt* op = nullptr;
+};
+static int sph_read(fo_sph_batch* b, const SphOut& w) {
+  const size_t P = b->lc.P, m = P * b->lc.norient, N = b->Ntot;
+  const struct {
+    size_t off, bytes;
+    void* to;
+  } parts[] = {{b->off.X1c, sizeof(double) * 3 * N, w.X1},
+               {b->off.X2out, sizeof(double) * 3 * N, w.X2},
+               {b->off.perm, sizeof(int) * N, w.perm},
+               {b->off.res, sizeof(SphResult) * P, w.res},
+               {b->off.peaks, sizeof(SphPeak) * m, w.pk},
+               {b->off.opt, sizeof(SphOpt) * m, w.op},
+               {b->off.scale, sizeof(double) * P, w.scale}};
+  return read_parts(b, parts);
 }
 
 int fo_sph_batch_results(fo_sph_batch* b, double* dist, double* X1, double* X2, int* perm,
@@ -1195,11 +1335,12 @@ int fo_sph_batch_results(fo_sph_batch* b, double* dist, double* X1, double* X2, 
   if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
   const int P = b->lc.P;
   std::vector<SphResult> r(P);
-  FO_HIP(hipMemcpyAsync(r.data(), b->res, sizeof(SphResult) * P, hipMemcpyDeviceToHost, b->stream));
-  if (X1) FO_HIP(hipMemcpyAsync(X1, b->X1c, sizeof(double) * 3 * b->Ntot, hipMemcpyDeviceToHost, b->stream));
-  if (X2) FO_HIP(hipMemcpyAsync(X2, b->X2out, sizeof(double) * 3 * b->Ntot, hipMemcpyDeviceToHost, b->stream));
-  if (perm) FO_HIP(hipMemcpyAsync(perm, b->perm, sizeof(int) * b->Ntot, hipMemcpyDeviceToHost, b->stream));
-  FO_HIP(hipStreamSynchronize(b->stream));
+  SphOut w;
+  w.X1 = X1;
+  w.X2 = X2;
+  w.perm = perm;
+  w.res = r.data();
+  if (int rc = sph_read(b, w)) return rc;
   for (int p = 0; p < P; ++p) {
     if (dist) dist[p] = r[p].dist;
     if (R)
@@ -1211,16 +1352,10 @@ int fo_sph_batch_results(fo_sph_batch* b, double* dist, double* X1, double* X2, 
   return FO_OK;
 }
 
-int fo_sph_batch_peaks(fo_sph_batch* b, int* ind, double* fun, double* peak_value, double* margin,
-                       double* delta, int* ncand, int* noverflow) {
-  if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
-  const size_t m = (size_t)b->lc.P * b->lc.norient;
-  std::vector<SphPeak> pk(m);
-  std::vector<SphOpt> op(m);
-  FO_HIP(hipMemcpyAsync(pk.data(), b->peaks, sizeof(SphPeak) * m, hipMemcpyDeviceToHost, b->stream));
-  FO_HIP(hipMemcpyAsync(op.data(), b->opt, sizeof(SphOpt) * m, hipMemcpyDeviceToHost, b->stream));
-  FO_HIP(hipStreamSynchronize(b->stream));
-  for (size_t i = 0; i < m; ++i) {
+static void put_peaks(const std::vector<SphPeak>& pk, const std::vector<SphOpt>& op, int* ind,
+                      double* fun, double* peak_value, double* margin, double* delta, int* ncand,
+                      int* noverflow) {
+  for (size_t i = 0; i < pk.size(); ++i) {
     if (ind)
       for (int k = 0; k < 3; ++k) ind[3 * i + k] = pk[i].ind[k];
     if (fun) fun[i] = op[i].f;
@@ -1230,17 +1365,10 @@ int fo_sph_batch_peaks(fo_sph_batch* b, int* ind, double* fun, double* peak_valu
     if (ncand) ncand[i] = pk[i].ncand;
     if (noverflow) noverflow[i] = pk[i].noverflow;
   }
-  return FO_OK;
 }
-
-int fo_sph_batch_opt(fo_sph_batch* b, double* R, double* fun, double* gnorm, int* iters,
-                     int* evals) {
-  if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
-  const size_t m = (size_t)b->lc.P * b->lc.norient;
-  std::vector<SphOpt> op(m);
-  FO_HIP(hipMemcpyAsync(op.data(), b->opt, sizeof(SphOpt) * m, hipMemcpyDeviceToHost, b->stream));
-  FO_HIP(hipStreamSynchronize(b->stream));
-  for (size_t i = 0; i < m; ++i) {
+static void put_opt(const std::vector<SphOpt>& op, double* R, double* fun, double* gnorm,
+                    int* iters, int* evals) {
+  for (size_t i = 0; i < op.size(); ++i) {
     if (R)
       for (int k = 0; k < 3; ++k) R[3 * i + k] = op[i].R[k];
     if (fun) fun[i] = op[i].f;
@@ -1248,13 +1376,65 @@ int fo_sph_batch_opt(fo_sph_batch* b, double* R, double* fun, double* gnorm, int
     if (iters) iters[i] = op[i].iters;
     if (evals) evals[i] = op[i].evals;
   }
+}
+
+int fo_sph_batch_peaks(fo_sph_batch* b, int* ind, double* fun, double* peak_value, double* margin,
+                       double* delta, int* ncand, int* noverflow) {
+  if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
+  const size_t m = (size_t)b->lc.P * b->lc.norient;
+  std::vector<SphPeak> pk(m);
+  std::vector<SphOpt> op(m);
+  SphOut w;
+  w.pk = pk.data();
+  w.op = op.data();
+  if (int rc = sph_read(b, w)) return rc;
+  put_peaks(pk, op, ind, fun, peak_value, margin, delta, ncand, noverflow);
+  return FO_OK;
+}
+
+int fo_sph_batch_opt(fo_sph_batch* b, double* R, double* fun, double* gnorm, int* iters,
+                     int* evals) {
+  if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
+  std::vector<SphOpt> op((size_t)b->lc.P * b->lc.norient);
+  SphOut w;
+  w.op = op.data();
+  if (int rc = sph_read(b, w)) return rc;
+  put_opt(op, R, fun, gnorm, iters, evals);
   return FO_OK;
 }
 
 int fo_sph_batch_scales(fo_sph_batch* b, double* scale) {
   if (!b || !scale) return set_err(FO_ERR_INVALID, "NULL argument");
-  FO_HIP(hipMemcpyAsync(scale, b->scale, sizeof(double) * b->lc.P, hipMemcpyDeviceToHost, b->stream));
-  FO_HIP(hipStreamSynchronize(b->stream));
+  SphOut w;
+  w.scale = scale;
+  return sph_read(b, w);
+}
+
+int fo_sph_batch_read(fo_sph_batch* b, double* f, int* q) {
+  if (!b || !f || !q) return set_err(FO_ERR_INVALID, "NULL argument");
+  const size_t P = b->lc.P, m = P * b->lc.norient, N = b->Ntot;
+  std::vector<SphResult> r(P);
+  std::vector<SphPeak> pk(m);
+  std::vector<SphOpt> op(m);
+  double *X = f + 14 * P, *g = X + 6 * N;
+  int *perm = q + P, *h = perm + N;
+  SphOut w;
+  w.X1 = X;
+  w.X2 = X + 3 * N;
+  w.scale = f + 13 * P;
+  w.perm = perm;
+  w.res = r.data();
+  w.pk = pk.data();
+  w.op = op.data();
+  if (int rc = sph_read(b, w)) return rc;
+  for (size_t p = 0; p < P; ++p) {
+    f[p] = r[p].dist;
+    for (int k = 0; k < 3; ++k) f[P + 3 * p + k] = r[p].R[k];
+    for (int k = 0; k < 9; ++k) f[4 * P + 9 * p + k] = r[p].rmat[k];
+    q[p] = r[p].inverted;
+  }
+  put_peaks(pk, op, h, g, g + m, g + 2 * m, g + 3 * m, h + 3 * m, h + 4 * m);
+  put_opt(op, g + 5 * m, nullptr, g + 4 * m, h + 5 * m, h + 6 * m);
   return FO_OK;
 }
 
@@ -1592,6 +1772,7 @@ struct fo_per_batch {
   } off{};
   bool keepc = false;
   bool own_mem = false, own_stream = false;
+  void* slab = nullptr;  // staging buffer of the last host positions
   float2* cgrid = nullptr;   // complex f (FO_PER_KEEP_FFT)
   // per-structure coefficients shared by the pairs (set_coeffs_indexed)
   void* csbuf = nullptr;
@@ -1720,16 +1901,17 @@ int per_batch_plan(fo_context* c, const fo_per_batch_desc* d, fo_per_batch** out
   o.at = lay.add<int>(b->hatoms.size());
   o.p1 = lay.add<double>(3 * Ntot);
   o.p2 = lay.add<double>(3 * Ntot);
+  // outputs, adjacent (per_read)
   o.x1 = lay.add<double>(3 * Ntot);
   o.x2 = lay.add<double>(3 * Ntot);
+  o.perm = lay.add<int>(Ntot);
+  o.res = lay.add<PerResult>(b->P);
+  o.pk = lay.add<PerPeak>(b->P);
   o.cp = lay.add<double2>((size_t)b->P * b->cube);
   o.c1 = b->keepc ? lay.add<double2>((size_t)std::max(gsum, 1) * b->cube) : 0;
   o.c2 = b->keepc ? lay.add<double2>((size_t)std::max(gsum, 1) * b->cube) : 0;
   o.cand = lay.add<PlaneCand>((size_t)b->P * b->F);
   o.ab = lay.add<double>((size_t)b->P * NB);
-  o.pk = lay.add<PerPeak>(b->P);
-  o.res = lay.add<PerResult>(b->P);
-  o.perm = lay.add<int>(Ntot);
   o.sp = lay.add<int>(Ntot);
   o.rs = lay.add<int>(Ntot + 1);
   // the selection's scratch, then the refinement's nearest rows (one per
@@ -1820,6 +2002,7 @@ int fo_per_batch_create(fo_context* c, const fo_per_batch_desc* d, fo_per_batch*
 int fo_per_batch_destroy(fo_per_batch* b) {
   if (!b) return FO_OK;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
+  release_slab(b);
   for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second);
   if (b->ev_made)
     for (auto& e : b->ev) (void)hipEventDestroy(e);
@@ -1841,10 +2024,8 @@ int fo_per_batch_set_positions(fo_per_batch* b, const double* p1, const double* 
   if (!b || !p1 || !p2) return set_err(FO_ERR_INVALID, "NULL argument");
   if (!all_finite(p1, 3 * b->Ntot) || !all_finite(p2, 3 * b->Ntot))
     return set_err(FO_ERR_INVALID, "positions must be finite");
-  FO_HIP(hipMemcpyAsync(b->pos1, p1, sizeof(double) * 3 * b->Ntot, hipMemcpyHostToDevice, b->stream));
-  FO_HIP(hipMemcpyAsync(b->pos2, p2, sizeof(double) * 3 * b->Ntot, hipMemcpyHostToDevice, b->stream));
-  FO_HIP(hipStreamSynchronize(b->stream));
-  return FO_OK;
+  return write_positions(b->ctx, b->own_mem, b->stream, b->pos1, b->pos2, p1, p2, 3 * b->Ntot,
+                         &b->slab);
 }
 
 int fo_per_batch_set_positions_device(fo_per_batch* b, const void* p1, const void* p2) {
@@ -1908,18 +2089,29 @@ int fo_per_batch_run(fo_per_batch* b, int stages, int use_graph) {
 int fo_per_batch_sync(fo_per_batch* b) {
   if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
   FO_HIP(hipStreamSynchronize(b->stream));
+  release_slab(b);
   return FO_OK;
+}
+
+static int per_read(fo_per_batch* b, double* X1, double* X2, int* perm, PerResult* res,
+                    PerPeak* pk) {
+  const size_t P = b->P, N = b->Ntot;
+  const struct {
+    size_t off, bytes;
+    void* to;
+  } parts[] = {{b->off.x1, sizeof(double) * 3 * N, X1},
+               {b->off.x2, sizeof(double) * 3 * N, X2},
+               {b->off.perm, sizeof(int) * N, perm},
+               {b->off.res, sizeof(PerResult) * P, res},
+               {b->off.pk, sizeof(PerPeak) * P, pk}};
+  return read_parts(b, parts);
 }
 
 int fo_per_batch_results(fo_per_batch* b, double* dist, double* X1, double* X2, int* perm,
                          double* disp) {
   if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
   std::vector<PerResult> r(b->P);
-  FO_HIP(hipMemcpyAsync(r.data(), b->res, sizeof(PerResult) * b->P, hipMemcpyDeviceToHost, b->stream));
-  if (X1) FO_HIP(hipMemcpyAsync(X1, b->X1out, sizeof(double) * 3 * b->Ntot, hipMemcpyDeviceToHost, b->stream));
-  if (X2) FO_HIP(hipMemcpyAsync(X2, b->X2out, sizeof(double) * 3 * b->Ntot, hipMemcpyDeviceToHost, b->stream));
-  if (perm) FO_HIP(hipMemcpyAsync(perm, b->perm, sizeof(int) * b->Ntot, hipMemcpyDeviceToHost, b->stream));
-  FO_HIP(hipStreamSynchronize(b->stream));
+  if (int rc = per_read(b, X1, X2, perm, r.data(), nullptr)) return rc;
   for (int p = 0; p < b->P; ++p) {
     if (dist) dist[p] = r[p].dist;
     if (disp)
@@ -1928,13 +2120,9 @@ int fo_per_batch_results(fo_per_batch* b, double* dist, double* X1, double* X2, 
   return FO_OK;
 }
 
-int fo_per_batch_peaks(fo_per_batch* b, int* ind, double* disp0, double* peak_value, double* margin,
-                       double* delta, int* ncand, int* noverflow) {
-  if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
-  std::vector<PerPeak> pk(b->P);
-  FO_HIP(hipMemcpyAsync(pk.data(), b->peaks, sizeof(PerPeak) * b->P, hipMemcpyDeviceToHost, b->stream));
-  FO_HIP(hipStreamSynchronize(b->stream));
-  for (int p = 0; p < b->P; ++p) {
+static void put_peaks(const std::vector<PerPeak>& pk, int* ind, double* disp0, double* peak_value,
+                      double* margin, double* delta, int* ncand, int* noverflow) {
+  for (size_t p = 0; p < pk.size(); ++p) {
     if (ind)
       for (int k = 0; k < 3; ++k) ind[3 * p + k] = pk[p].ind[k];
     if (disp0)
@@ -1945,6 +2133,30 @@ int fo_per_batch_peaks(fo_per_batch* b, int* ind, double* disp0, double* peak_va
     if (ncand) ncand[p] = pk[p].ncand;
     if (noverflow) noverflow[p] = pk[p].noverflow;
   }
+}
+
+int fo_per_batch_peaks(fo_per_batch* b, int* ind, double* disp0, double* peak_value, double* margin,
+                       double* delta, int* ncand, int* noverflow) {
+  if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
+  std::vector<PerPeak> pk(b->P);
+  if (int rc = per_read(b, nullptr, nullptr, nullptr, nullptr, pk.data())) return rc;
+  put_peaks(pk, ind, disp0, peak_value, margin, delta, ncand, noverflow);
+  return FO_OK;
+}
+
+int fo_per_batch_read(fo_per_batch* b, double* f, int* q) {
+  if (!b || !f || !q) return set_err(FO_ERR_INVALID, "NULL argument");
+  const size_t P = b->P, N = b->Ntot;
+  std::vector<PerResult> r(P);
+  std::vector<PerPeak> pk(P);
+  double *X = f + 4 * P, *g = X + 6 * N;
+  int* h = q + N;
+  if (int rc = per_read(b, X, X + 3 * N, q, r.data(), pk.data())) return rc;
+  for (size_t p = 0; p < P; ++p) {
+    f[p] = r[p].dist;
+    for (int k = 0; k < 3; ++k) f[P + 3 * p + k] = r[p].disp[k];
+  }
+  put_peaks(pk, h, g, g + 3 * P, g + 4 * P, g + 5 * P, h + 3 * P, h + 4 * P);
   return FO_OK;
 }
 

@@ -197,15 +197,15 @@ class PeriodicAlign(BasePeriodicAlignment):
                 b.set_positions(self.pos1, self.pos2)
                 b.set_coeffs(Cs[0], Cs[1])
                 b.run(_lib.PSTAGE_ALL)
-                r = b.results()
-                self.last = dict(peaks=b.peaks())
+                r, peaks = b.read()
+                self.last = dict(peaks=peaks)
         else:
             b, reused = self._plain_batch()
             b.set_positions(self.pos1, self.pos2)
             # repeated calls replay the captured launch graph
-            b.run(_lib.PSTAGE_ALL, graph=reused)
-            r = b.results()
-            self.last = dict(peaks=b.peaks())
+            b.run(_lib.PSTAGE_ALL, graph=reused, sync=False)
+            r, peaks = b.read()
+            self.last = dict(peaks=peaks)
         return (float(r["dist"][0]), r["X1"][0], r["X2"][0], r["perm"][0], r["disp"][0])
 
     def _plain_batch(self):

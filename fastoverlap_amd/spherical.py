@@ -193,11 +193,11 @@ class BaseSphericalAlignment:
             b.set_positions(pos1, pos2)
             # a repeated shape replays the captured launch graph; a new one
             # runs eagerly (a capture costs more than one eager pass)
-            b.run(_lib.STAGE_ALL, graph=reused)
-            r = b.results()
-            diag = dict(peaks=b.peaks(), opt=b.opt())
+            b.run(_lib.STAGE_ALL, graph=reused, sync=False)
+            r, peaks, opt, scales = b.read()
+            diag = dict(peaks=peaks, opt=opt)
             if self.calcScale:
-                self.scale = float(b.scales()[0])
+                self.scale = float(scales[0])
         else:
             A = dense_to_compact(np.asarray(calcCoeffs(False)))
             flags = _lib.SPH_GENERAL if invert else _lib.SPH_NO_INVERT
@@ -208,8 +208,8 @@ class BaseSphericalAlignment:
                 b.set_coeffs(A, Bc)
                 b.run(_lib.STAGE_PREP | _lib.STAGE_GRID | _lib.STAGE_ROTOPT |
                       _lib.STAGE_FINISH)
-                r = b.results()
-                diag = dict(peaks=b.peaks(), opt=b.opt())
+                r, peaks, opt, _ = b.read()
+                diag = dict(peaks=peaks, opt=opt)
         out = (float(r["dist"][0]), r["X1"][0], r["X2"][0])
         self.last = dict(perm=r["perm"][0], R=r["R"][0], rmat=r["rmat"][0],
                          inverted=bool(r["inverted"][0]), **diag)

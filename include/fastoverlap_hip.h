@@ -141,6 +141,13 @@ int fo_sph_batch_sync(fo_sph_batch* b);
  *  inverted[npairs] */
 int fo_sph_batch_results(fo_sph_batch* b, double* dist, double* X1, double* X2, int* perm,
                          double* R, double* rmat, int* inverted);
+/* every output of the calls around here in one transfer, with m = npairs *
+ * orientations, in this order:
+ *  f: dist[npairs], R[3 npairs], rmat[9 npairs], scale[npairs], X1[3N], X2[3N],
+ *     fun[m], peak_value[m], margin[m], delta[m], gnorm[m], optimal R[3m]
+ *  q: inverted[npairs], perm[N], ind[3m], ncand[m], noverflow[m], iters[m],
+ *     evals[m] */
+int fo_sph_batch_read(fo_sph_batch* b, double* f, int* q);
 /* per (pair, orientation): ind[3], fun, grid peak value, margin, error bound,
  * FP64 candidates, fully re-evaluated planes */
 int fo_sph_batch_peaks(fo_sph_batch* b, int* ind, double* fun, double* peak_value,
@@ -279,6 +286,11 @@ int fo_per_batch_run(fo_per_batch* b, int stages, int use_graph);
 int fo_per_batch_sync(fo_per_batch* b);
 int fo_per_batch_results(fo_per_batch* b, double* dist, double* X1, double* X2, int* perm,
                          double* disp);
+/* both calls' outputs (above and below) in one transfer:
+ *  f: dist[npairs], disp[3 npairs], X1[3N], X2[3N], disp0[3 npairs],
+ *     peak_value, margin, delta [npairs each]
+ *  q: perm[N], ind[3 npairs], ncand, noverflow [npairs each] */
+int fo_per_batch_read(fo_per_batch* b, double* f, int* q);
 int fo_per_batch_peaks(fo_per_batch* b, int* ind, double* disp0, double* peak_value,
                        double* margin, double* delta, int* ncand, int* noverflow);
 int fo_per_batch_coeffs(fo_per_batch* b, double* C1, double* C2);

@@ -319,3 +319,26 @@ def test_real_planes_within_the_selection_bound(gpu, nk, F, P):
         f = np.abs(np.fft.fftn(C[0], (F, F, F)))
         A = np.abs(C[0]).sum()
         assert np.abs(b.grid(0) - f).max() <= (4 * NB + 32) * 2.0 ** -24 * A
+
+
+@pytest.mark.parametrize("pairs", [1, 96])
+def test_periodic_read_back_in_one_transfer(gpu, pairs):
+    """``read()`` gives what ``results()`` and ``peaks()`` give, through the
+    staging buffer and directly (96 pairs of 64 atoms), with positions set
+    again before the first ones have run."""
+    say(f"case: {pairs} pairs")
+    rng = np.random.default_rng(pairs)
+    box = np.array([4.0, 4.4, 3.7])
+    x, y = (rng.random((pairs * 64, 3)) * box for _ in range(2))
+    with PeriodicBatch([64] * pairs, box, 0.25, 4, 16, None, 10, 0) as b:
+        b.set_positions(y, y)
+        b.set_positions(x, y)
+        b.run(sync=False)
+        r, pk = b.read()
+        for got, ref in ((r, b.results()), (pk, b.peaks())):
+            assert got.keys() == ref.keys()
+            for k in ref:
+                for u, v in zip(got[k], ref[k]):
+                    np.testing.assert_array_equal(u, v)
+        cells = (r["X1"][0] - x[:64]) / box  # the structure in the home cell
+        np.testing.assert_allclose(cells, np.round(cells), atol=1e-12)

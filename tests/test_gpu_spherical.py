@@ -698,3 +698,56 @@ def test_folded_planes_against_direct_planes(gpu, n, L, invert):
             if Ls[p]:  # (degree 0: a constant grid)
                 np.testing.assert_array_equal(pf["ind"][p, k], pdir["ind"][p, k])
                 assert abs(pf["value"][p, k] - pdir["value"][p, k]) <= 1e-12 * pdir["value"][p, k]
+
+
+@pytest.mark.parametrize("pairs", [1, 40, 200])
+def test_read_back_in_one_transfer(gpu, pairs):
+    """``read()`` gives what the single calls give, through the staging buffer
+    (few atoms) and directly (200 pairs of 60 atoms), also when positions are
+    set again before the first ones have run, and from two threads at once."""
+    import threading
+    N, L = 60, 5
+    rng = np.random.default_rng(pairs)
+    X = rng.normal(size=(3, pairs * N, 3))
+
+    def same(a, b):
+        if isinstance(a, dict):
+            assert a.keys() == b.keys()
+            for k in a:
+                same(a[k], b[k])
+        elif isinstance(a, list):
+            for x, y in zip(a, b):
+                same(x, y)
+        else:
+            assert a.dtype == b.dtype and a.shape == b.shape
+            np.testing.assert_array_equal(a, b)
+
+    errors = []
+
+    def work(shift):
+        try:
+            with SphericalBatch([N] * pairs, L, None, 12, None) as b:
+                outs = []
+                for k in range(3):
+                    say(f"case: {pairs} pairs, pass {k}, thread {shift}")
+                    b.set_positions(X[2] + shift, X[2])   # replaced before it runs
+                    b.set_positions(X[0], X[1] * (1 + 0.01 * k))
+                    b.run(sync=False)
+                    r, pk, opt, scale = b.read()
+                    same(r, b.results())
+                    same(pk, b.peaks())
+                    same(opt, b.opt())
+                    same(scale, b.scales())
+                    outs.append(r)
+                assert not np.array_equal(outs[0]["X2"][0], outs[2]["X2"][0])
+                np.testing.assert_allclose(outs[0]["X1"][0], X[0][:N] - X[0][:N].mean(0), atol=1e-12)
+        except BaseException as e:  # noqa: BLE001 - reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    if errors:
+        raise errors[0]

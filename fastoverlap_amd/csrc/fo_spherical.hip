@@ -1301,23 +1301,64 @@ struct GridCtx {
   double sgn;         // +1 / -1 (alignment mode)
 };
 
-// FP64 grid values at up to kEvalBatch points whose beta indices take at most
-// kEvalBeta distinct values, in one sweep over the coefficients (each
-// coefficient is read once for all points).  Point q: alpha pa[q], gamma
-// pg[q], beta slot pb[q] into betas[].  Each point's value is reduced with
-// the tree of block_sum.
+// Sums over the wavefront of several values a lane: two halvings that keep one
+// value per half, then a sum within rows of 16 lanes.  Ten values take 60
+// instructions; ten butterflies over the lanes are 180 and wait 60 times.
+FO_DEV double swap_add32(double a, double b) {  // lanes 0-31: sum of a, 32-63: of b
+  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false,
+                                                   false);
+  return __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]) +
+         __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+}
+FO_DEV double swap_add16(double a, double b) {  // rows 0, 2: sums of a's, 1, 3: of b's halves
+  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false,
+                                                   false);
+  return __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]) +
+         __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+}
+template <int CTRL>
+FO_DEV double dpp_add(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), CTRL, 0xf, 0xf, true);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+FO_DEV double row_sum(double v) {  // over the 16 lanes of a row (rotations)
+  v = dpp_add<0x128>(v);
+  v = dpp_add<0x124>(v);
+  v = dpp_add<0x122>(v);
+  return dpp_add<0x121>(v);
+}
+// eight values, written to out[0..7]
+FO_DEV void wave_sum8(const double (&v)[8], double* out) {
+  double u[4], w[2];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) u[j] = swap_add32(v[j], v[j + 4]);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) w[j] = row_sum(swap_add16(u[j], u[j + 2]));
+  // rows: w[j] holds v[j], v[j + 2], v[j + 4], v[j + 6]
+  const int lane = threadIdx.x & 63;
+  if ((lane & 15) == 0) {
+    out[2 * (lane >> 4)] = w[0];
+    out[2 * (lane >> 4) + 1] = w[1];
+  }
+}
+
 constexpr int kEvalBatch = 8;
 constexpr int kEvalBeta = 4;
-constexpr int kSelUnroll = 3;  // degrees per batch of operand loads
 
 // Entry e of the (m1 >= 0, m2) entries of degree <= L in shell order: shell
 // l0 = max(m1, |m2|) holds 4 l0 + 1 entries from e = l0 (2 l0 - 1) on
 // (m1 = l0, m2 = -l0..l0, then m1 < l0 with m2 = +-l0).  The lanes of a
-// wavefront then start their degree recurrences at nearly the same l.
+// wavefront then start their degree sums at nearly the same l.
 FO_DEV void shell_entry(int e, int& l0, int& m1, int& m2) {
-  l0 = (int)((1.0 + sqrt(1.0 + 8.0 * e)) * 0.25);
-  while (l0 * (2 * l0 - 1) > e) --l0;
-  while ((l0 + 1) * (2 * l0 + 1) <= e) ++l0;
+  l0 = (int)((1.f + sqrtf(1.f + 8.f * e)) * 0.25f);  // off by one at most
+  if (l0 * (2 * l0 - 1) > e) --l0;
+  if ((l0 + 1) * (2 * l0 + 1) <= e) ++l0;
   const int r = e - l0 * (2 * l0 - 1);
   if (r <= 2 * l0) {
     m1 = l0;
@@ -1327,12 +1368,78 @@ FO_DEV void shell_entry(int e, int& l0, int& m1, int& m2) {
     m2 = ((r - 2 * l0 - 1) & 1) ? -l0 : l0;
   }
 }
-// compact index of degree l + 1 from that of degree l (same m1, m2) once the
-// entry exists (l >= l0); held at the last existing degree otherwise
-FO_DEV int next_kidx(int id, int l, int l0, int m1, int L) {
-  return (l >= l0 && l < L) ? id + (2 * l + 1) * (2 * l + 1) + 2 * m1 + 4 * l + 4 : id;
+
+// S_b = sum_l sgn^l d^l_{m1 m2}(beta_b) I^l_{m1 m2} of the lane's entry, for the
+// first nb of NB beta planes.  The column entries of a shell (m1 < l0, m2 = +-l0)
+// read the table at the transposed entry, d_{m1 m2} = (-1)^{m1-m2} d_{m2 m1}, so
+// the lanes of a wavefront read consecutive table words (the rows of the
+// compact layout are contiguous, its columns 2l+1 words apart).  Two degrees
+// are loaded while the two before are summed, even and odd ones apart (the
+// sign is applied to the sums); reads outside a degree give zero or are not used.
+template <int NB>
+FO_DEV void beta_sums(__amdgpu_buffer_rsrc_t ri, const __amdgpu_buffer_rsrc_t (&rt)[NB], int nb,
+                      int L, double sgn, int l0, int m1, int m2, double2 (&s)[NB]) {
+  struct Batch {
+    double2 Iv[2];
+    double dv[2][NB];
+  } ba, bb;
+  const bool col = m1 < l0;
+  const int tm1 = col ? m2 : m1, tm2 = col ? m1 : m2;
+  auto load = [&](Batch& B, int l) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int lq = l + q, W = 2 * lq + 1;
+      const int base = lq * (2 * lq - 1) * W / 3 + lq * (2 * lq + 2);  // (m1, m2) = (0, 0)
+      B.Iv[q] = load_d2(ri, 16 * (base + m2 + m1 * W), 0);
+      const int tv = 8 * (base + tm2 + tm1 * W);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        if (b < nb) B.dv[q][b] = load_d(rt[b], tv, 0);  // uniform
+    }
+    __builtin_amdgcn_sched_barrier(0);  // issued before the sums that follow
+  };
+  double2 acc[2][NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) acc[0][b] = acc[1][b] = make_double2(0.0, 0.0);
+  auto sum = [&](const Batch& B, int l) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      if (l + q <= L && l + q >= l0) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          if (b < nb) {
+            acc[q][b].x += B.dv[q][b] * B.Iv[q].x;
+            acc[q][b].y += B.dv[q][b] * B.Iv[q].y;
+          }
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const int lw = __builtin_amdgcn_readfirstlane(l0);  // smallest of the wavefront
+  load(ba, lw);
+  for (int l = lw; l <= L; l += 4) {  // wavefront-uniform
+    load(bb, l + 2);
+    sum(ba, l);
+    load(ba, l + 4);
+    sum(bb, l + 2);
+  }
+  const double s0 = ((lw & 1) ? sgn : 1.0) * ((col && ((m1 - m2) & 1)) ? -1.0 : 1.0);
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    s[b] = make_double2(s0 * (acc[0][b].x + sgn * acc[1][b].x),
+                        s0 * (acc[0][b].y + sgn * acc[1][b].y));
 }
 
+// x mod n in [0, n) for |x| < 2^22, inv = 1 / n
+FO_DEV int mod_small(int x, int n, float inv) {
+  int r = x - (int)floorf((float)x * inv) * n;
+  r += r < 0 ? n : 0;
+  return r - (r >= n ? n : 0);
+}
+
+// FP64 grid values at up to kEvalBatch points whose beta indices take at most
+// kEvalBeta distinct values, in one sweep over the coefficients (each
+// coefficient is read once for all points).  Point q: alpha pa[q], gamma
+// pg[q], beta slot pb[q] into betas[]; stw: the n twiddles in LDS.
 // The entries are swept in blocks of 64 (one wavefront) in shell order, so
 // the first blocks carry the longest degree loops; a wavefront that finishes
 // its block takes the next untaken one (LDS counter ctr), which evens out the
@@ -1341,16 +1448,19 @@ FO_DEV int next_kidx(int id, int l, int l0, int m1, int L) {
 // in block order, so the result does not depend on which wavefront took
 // which block.
 FO_DEV void grid_eval64_batch(const GridCtx& c, int np, const int* pa, const int* pg,
-                              const int* pb, int nbeta, const int* betas, double* out,
-                              double* part, int* ctr) {
+                              const int* pb, int nbeta, const int* betas, const double2* stw,
+                              double* out, double* part, int* ctr) {
   const int L = c.L, W = 2 * L + 1, n = c.n;
-  const double2* I = c.IB ? c.IB : c.I;
+  const __amdgpu_buffer_rsrc_t ri = buf_rsrc(c.IB ? c.IB : c.I, (int)(kcount(L) * sizeof(double2)));
   const double sg = c.IB ? 1.0 : c.sgn;
-  const double* tb[kEvalBeta];
+  __amdgpu_buffer_rsrc_t rt[kEvalBeta];
 #pragma unroll
-  for (int b = 0; b < kEvalBeta; ++b) tb[b] = c.tab64 + (long long)betas[b < nbeta ? b : 0] * c.Kt;
-  // entries (m1 >= 0, m2) in shell order (shell_entry), so the degree loop of
-  // a wavefront is uniform and the operands of two degrees are loaded at once
+  for (int b = 0; b < kEvalBeta; ++b) {
+    const int ib = __builtin_amdgcn_readfirstlane(betas[b < nbeta ? b : 0]);
+    rt[b] = buf_rsrc(c.tab64 + (long long)ib * c.Kt, (int)(kcount(L) * sizeof(double)));
+  }
+  nbeta = __builtin_amdgcn_readfirstlane(nbeta);
+  const float inv = 1.f / n;
   const int ne = (L + 1) * W, nblk = (ne + 63) >> 6;
   const int lane = threadIdx.x & 63, nwv = blockDim.x >> 6;
   if (threadIdx.x == 0) *ctr = nwv;
@@ -1360,51 +1470,8 @@ FO_DEV void grid_eval64_batch(const GridCtx& c, int np, const int* pa, const int
     const bool act = e < ne;
     int l0 = L + 1, m1 = 0, m2 = 0;
     if (act) shell_entry(e, l0, m1, m2);
-    double sx[kEvalBeta], sy[kEvalBeta];
-#pragma unroll
-    for (int b = 0; b < kEvalBeta; ++b) sx[b] = sy[b] = 0.0;
-    // The column entries of a shell (m1 < l0, m2 = +-l0) read the table at
-    // the transposed entry, d_{m1 m2} = (-1)^{m1-m2} d_{m2 m1}: row m2, so
-    // the lanes of a wavefront read consecutive table words (the rows of
-    // the compact layout are contiguous, its columns 2l+1 words apart).
-    const bool col = m1 < l0;
-    const int tm1 = col ? m2 : m1, tm2 = col ? m1 : m2;
-    double sl = ((l0 & 1) ? sg : 1.0) * ((col && ((m1 - m2) & 1)) ? -1.0 : 1.0);
-    const int lw = __builtin_amdgcn_readfirstlane(l0);  // smallest l0 of the wavefront
-    int id = act ? (int)kidx(l0, m1, m2) : 0;
-    int td = act ? (int)kidx(l0, tm1, tm2) : 0;
-    for (int l = lw; l <= L; l += kSelUnroll) {  // wavefront-uniform
-      int ids[kSelUnroll], tds[kSelUnroll];
-      ids[0] = id;
-      tds[0] = td;
-#pragma unroll
-      for (int q = 1; q < kSelUnroll; ++q) {
-        ids[q] = next_kidx(ids[q - 1], l + q - 1, l0, m1, L);
-        tds[q] = next_kidx(tds[q - 1], l + q - 1, l0, tm1, L);
-      }
-      double2 Iv[kSelUnroll];
-      double dv[kSelUnroll][kEvalBeta];
-#pragma unroll
-      for (int q = 0; q < kSelUnroll; ++q) {
-        Iv[q] = I[ids[q]];
-#pragma unroll
-        for (int b = 0; b < kEvalBeta; ++b) dv[q][b] = b < nbeta ? tb[b][tds[q]] : 0.0;
-      }
-#pragma unroll
-      for (int q = 0; q < kSelUnroll; ++q) {
-        if (l + q <= L && l + q >= l0) {
-#pragma unroll
-          for (int b = 0; b < kEvalBeta; ++b) {
-            const double d = dv[q][b] * sl;
-            sx[b] += d * Iv[q].x;
-            sy[b] += d * Iv[q].y;
-          }
-          sl *= sg;
-        }
-      }
-      id = next_kidx(ids[kSelUnroll - 1], l + kSelUnroll - 1, l0, m1, L);
-      td = next_kidx(tds[kSelUnroll - 1], l + kSelUnroll - 1, l0, tm1, L);
-    }
+    double2 s[kEvalBeta];
+    beta_sums<kEvalBeta>(ri, rt, nbeta, L, sg, l0, m1, m2, s);
     const double wm = m1 == 0 ? 1.0 : 2.0;
     double acc[kEvalBatch];
 #pragma unroll
@@ -1412,24 +1479,15 @@ FO_DEV void grid_eval64_batch(const GridCtx& c, int np, const int* pa, const int
       acc[q] = 0.0;
       if (q < np) {
         const int b = pb[q];
-        double x = sx[0], y = sy[0];
+        double2 v = s[0];
 #pragma unroll
-        for (int bb = 1; bb < kEvalBeta; ++bb)
-          if (b == bb) {
-            x = sx[bb];
-            y = sy[bb];
-          }
-        int ph = (m1 * pa[q] + m2 * pg[q]) % n;  // |m1 pa + m2 pg| < 2 L n
-        if (ph < 0) ph += n;
-        const double2 w = c.tw64[ph];
-        acc[q] = wm * (x * w.x - y * w.y);
+        for (int k = 1; k < kEvalBeta; ++k)
+          if (b == k) v = s[k];
+        const double2 w = stw[mod_small(m1 * pa[q] + m2 * pg[q], n, inv)];
+        acc[q] = wm * (v.x * w.x - v.y * w.y);
       }
     }
-#pragma unroll
-    for (int q = 0; q < kEvalBatch; ++q) {
-      const double v = wave_sum(acc[q]);
-      if (lane == 0) part[blk * kEvalBatch + q] = v;
-    }
+    wave_sum8(acc, part + blk * kEvalBatch);
     int nb = 0;
     if (lane == 0) nb = atomicAdd(ctr, 1);
     blk = __builtin_amdgcn_readfirstlane(nb);
@@ -1437,32 +1495,34 @@ FO_DEV void grid_eval64_batch(const GridCtx& c, int np, const int* pa, const int
   __syncthreads();
   if (threadIdx.x < np) {
     double v = 0.0;
+#pragma unroll 4
     for (int b = 0; b < nblk; ++b) v += part[b * kEvalBatch + threadIdx.x];
     out[threadIdx.x] = v;
   }
 }
 
 // Full FP64 evaluation of one beta plane; returns its argmax (ties -> lower
-// flat index).  Three stages, each thread-parallel:
-//   S[m1][m2] = sum_l s_l d^l_{m1 m2}(beta) I^l_{m1 m2}   (entries in shell
-//     order, two degrees of loads in flight, as in grid_eval64_batch),
-//   T[m1][g]  = sum_m2 S[m1][m2] e^{i m2 g 2pi/n}          (thread per (m1, g)),
+// flat index).  256 threads, three stages:
+//   S[m1][m2] = sum_l s_l d^l_{m1 m2}(beta) I^l_{m1 m2}   (an entry a lane),
+//   T[m1][g]  = sum_m2 S[m1][m2] e^{i m2 g 2pi/n}  and
 //   v(a, g)   = Re T[0][g] + 2 sum_{m1>=1} Re(T[m1][g] e^{i m1 a 2pi/n})
-//     (thread per (g, kPlaneA values of a): each T load serves them all).
+// the last two as FP64 matrix products of real and imaginary parts, 16 columns g
+// a wavefront, four row tiles at a time; rows and terms past the end read as zero.
 // S lives in the LDS buffer sS when (L+1)(2L+1) <= kSelS (L <= 31), else
-// in the global scratch Sg; T in the global scratch Tg[(L+1)n]; the n
-// twiddles are staged in the LDS buffer stw (n <= 256).  Phases advance by
-// integer steps mod n, so every twiddle is a table entry.
+// in the global scratch Sg; T in the global scratch Tg[(L+1)n]; stw: the n
+// twiddles in LDS.  Phases advance by integer steps mod n, so every twiddle is a
+// table entry.  The largest of 128 selections at L = 40,
+// n = 128, with one or two such planes: 553 -> 230 us.
 constexpr int kSelS = 2048;
-constexpr int kPlaneA = 8;
 FO_DEV void plane_eval64(const GridCtx& c, int ib, double2* Sg, double2* Tg, double2* sS,
-                         double2* stw, double* red, int* redi, double& bestv, int& besti) {
+                         const double2* stw, double* red, int* redi, double& bestv, int& besti) {
   const int L = c.L, W = 2 * L + 1, n = c.n, t = threadIdx.x, nt = blockDim.x;
-  const double* tb = c.tab64 + (long long)ib * c.Kt;
-  const double2* I = c.IB ? c.IB : c.I;
+  const __amdgpu_buffer_rsrc_t ri = buf_rsrc(c.IB ? c.IB : c.I, (int)(kcount(L) * sizeof(double2)));
+  const __amdgpu_buffer_rsrc_t rt[1] = {
+      buf_rsrc(c.tab64 + (long long)__builtin_amdgcn_readfirstlane(ib) * c.Kt,
+               (int)(kcount(L) * sizeof(double)))};
   const double sg = c.IB ? 1.0 : c.sgn;
-  const bool sl_lds = (L + 1) * W <= kSelS;
-  for (int k = t; k < n; k += nt) stw[k] = c.tw64[k];
+  double2* S = (L + 1) * W <= kSelS ? sS : Sg;
   // (1) beta sums
   const int ne = (L + 1) * W;
   for (int e0 = 0; e0 < ne; e0 += nt) {
@@ -1470,86 +1530,92 @@ FO_DEV void plane_eval64(const GridCtx& c, int ib, double2* Sg, double2* Tg, dou
     const bool act = e < ne;
     int l0 = L + 1, m1 = 0, m2 = 0;
     if (act) shell_entry(e, l0, m1, m2);
-    const int lw = __builtin_amdgcn_readfirstlane(l0);  // smallest l0 of the wavefront
-    double sx = 0.0, sy = 0.0, sl = (l0 & 1) ? sg : 1.0;
-    int id = act ? (int)kidx(l0, m1, m2) : 0;
-    for (int l = lw; l <= L; l += 2) {  // wavefront-uniform
-      int ids[2];
-      ids[0] = id;
-      ids[1] = next_kidx(id, l, l0, m1, L);
-      double2 Iv[2];
-      double dv[2];
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        Iv[q] = I[ids[q]];
-        dv[q] = tb[ids[q]];
-      }
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        if (l + q <= L && l + q >= l0) {
-          const double d = dv[q] * sl;
-          sx += d * Iv[q].x;
-          sy += d * Iv[q].y;
-          sl *= sg;
-        }
-      }
-      id = next_kidx(ids[1], l + 1, l0, m1, L);
-    }
-    if (act) (sl_lds ? sS : Sg)[m1 * W + m2 + L] = make_double2(sx, sy);
+    double2 s[1];
+    beta_sums<1>(ri, rt, 1, L, sg, l0, m1, m2, s);
+    if (act) S[m1 * W + m2 + L] = s[0];
   }
   __threadfence_block();
   __syncthreads();
-  // (2) gamma sums
-  auto gamma = [&](const double2* S) {
-    for (int e = t; e < (L + 1) * n; e += nt) {
-      const int m1 = e / n, g = e % n;
-      int ph = (L * g) % n;
-      ph = ph ? n - ph : 0;  // (-L g) mod n
-      const double2* row = S + m1 * W;
-      double2 acc = make_double2(0.0, 0.0);
-#pragma unroll 4
-      for (int m2i = 0; m2i < W; ++m2i) {
-        acc = cadd(acc, cmul(row[m2i], stw[ph]));
-        ph += g;
-        if (ph >= n) ph -= n;
+  // (2) gamma sums; tile layout of the FP64 product (lane = 16 r + cl): A holds
+  // row cl, inner r; B inner r, column cl; result i holds row 4 i + r, column cl
+  const int lane = t & 63, r = lane >> 4, cl = lane & 15, wave = t >> 6;
+  const float inv = 1.f / n;
+  for (int ct = wave; ct * 16 < n; ct += nt >> 6) {
+    const int g = min(ct * 16 + cl, n - 1);
+    const int step = mod_small(4 * g, n, inv);
+    int q = mod_small((r - L) * g, n, inv);
+    v4d tr[4], ti[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) tr[k] = ti[k] = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+    for (int k0 = 0; k0 < W; k0 += 4) {
+      const int k = k0 + r;
+      const double2 e = stw[q];
+      q += step;
+      q -= q >= n ? n : 0;
+#pragma unroll
+      for (int rt4 = 0; rt4 < 4; ++rt4) {
+        if (16 * rt4 > L) continue;  // uniform
+        const int row = 16 * rt4 + cl;
+        const bool in = row <= L && k < W;
+        const double2 x = S[in ? row * W + k : 0];
+        const double xr = in ? x.x : 0.0, xi = in ? x.y : 0.0;
+        tr[rt4] = mfma64(xr, e.x, tr[rt4]);
+        ti[rt4] = mfma64(xr, e.y, ti[rt4]);
+        tr[rt4] = mfma64(-xi, e.y, tr[rt4]);
+        ti[rt4] = mfma64(xi, e.x, ti[rt4]);
       }
-      Tg[e] = acc;
     }
-  };
-  if (sl_lds)
-    gamma(sS);
-  else
-    gamma(Sg);
+    if (ct * 16 + cl < n)
+#pragma unroll
+      for (int rt4 = 0; rt4 < 4; ++rt4)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int row = 16 * rt4 + 4 * i + r;
+          if (row <= L) Tg[row * n + g] = make_double2(tr[rt4][i], ti[rt4][i]);
+        }
+  }
   __threadfence_block();
   __syncthreads();
-  // (3) alpha sums and the plane's argmax
+  // (3) alpha sums and the plane's argmax: rows a, columns g
   double bv = -INFINITY;
   int bi = 0x7fffffff;
-  const int nch = (n + kPlaneA - 1) / kPlaneA;
-  for (int it = t; it < n * nch; it += nt) {
-    const int g = it % n, a0 = (it / n) * kPlaneA;
-    double acc[kPlaneA];
-    int ph[kPlaneA];
-    const double t0 = Tg[g].x;
+  const int at4 = (n + 63) >> 6, ctn = (n + 15) >> 4;
+  for (int item = wave; item < ctn * at4; item += nt >> 6) {
+    const int ct = item % ctn, a0 = (item / ctn) * 64;
+    const int g = min(ct * 16 + cl, n - 1);
+    int q[4], step[4];
 #pragma unroll
-    for (int j = 0; j < kPlaneA; ++j) {
-      acc[j] = t0;
-      ph[j] = 0;
+    for (int j = 0; j < 4; ++j) {
+      const int a = min(a0 + 16 * j + cl, n - 1);
+      q[j] = mod_small(r * a, n, inv);
+      step[j] = mod_small(4 * a, n, inv);
     }
-#pragma unroll 2
-    for (int m1 = 1; m1 <= L; ++m1) {
-      const double2 v = Tg[m1 * n + g];
+    v4d v[4];
 #pragma unroll
-      for (int j = 0; j < kPlaneA; ++j) {
-        ph[j] += a0 + j < n ? a0 + j : 0;  // (values of a >= n are not used)
-        if (ph[j] >= n) ph[j] -= n;
-        const double2 w = stw[ph[j]];
-        acc[j] += 2.0 * (v.x * w.x - v.y * w.y);
+    for (int j = 0; j < 4; ++j) v[j] = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+    for (int k0 = 0; k0 <= L; k0 += 4) {
+      const int m1 = k0 + r;
+      const double2 x = Tg[min(m1, L) * n + g];
+      const double w = m1 > L ? 0.0 : m1 ? 2.0 : 1.0;
+      const double xr = w * x.x, xi = m1 ? -w * x.y : 0.0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const double2 e = stw[q[j]];
+        q[j] += step[j];
+        q[j] -= q[j] >= n ? n : 0;
+        v[j] = mfma64(e.x, xr, v[j]);
+        v[j] = mfma64(e.y, xi, v[j]);
       }
     }
 #pragma unroll
-    for (int j = 0; j < kPlaneA; ++j)
-      if (a0 + j < n) argmax_merge(bv, bi, acc[j], ((a0 + j) * n + ib) * n + g);
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int a = a0 + 16 * j + 4 * i + r;
+        if (a < n && ct * 16 + cl < n) argmax_merge(bv, bi, v[j][i], (a * n + ib) * n + g);
+      }
   }
   block_argmax(bv, bi, red, redi);
   bestv = bv;
@@ -1566,7 +1632,7 @@ FO_DEV void plane_eval64(const GridCtx& c, int ib, double2* Sg, double2* Tg, dou
 // re-evaluated in FP64; planes whose unlisted values could be within delta
 // are re-evaluated in full (all_planes: every plane, the exhaustive check).
 
-__global__ void __launch_bounds__(256) k_sph_select(
+__global__ void __launch_bounds__(1024) k_sph_select(
     const SphPair* __restrict__ pd, int n, long long Kt, const double* __restrict__ tab64,
     const double2* __restrict__ tw64, const double2* __restrict__ IA,
     const double2* __restrict__ IB, int mode, int norient, const PlaneCand* __restrict__ cand,
@@ -1582,7 +1648,7 @@ __global__ void __launch_bounds__(256) k_sph_select(
   // s_planeS also holds the block sums of grid_eval64_batch (L <= 63)
   static_assert(2 * kSelS >= kEvalBatch * ((64 * 127 + 63) / 64), "block sums");
   __shared__ double s_val[kEvalBatch];
-  __shared__ double2 s_planeS[kSelS], s_planeTw[256];  // full-plane evaluation only
+  __shared__ double2 s_planeS[kSelS], s_planeTw[256];
   int p, o;
   if (!xcd_decode(P, norient, p, o)) return;
   const SphPair d = pd[p];
@@ -1597,6 +1663,7 @@ __global__ void __launch_bounds__(256) k_sph_select(
   c.IB = (mode == 1 && o == 1) ? IB + d.coef_off : nullptr;
   c.sgn = (mode == 0 && o == 1) ? -1.0 : 1.0;
   const PlaneCand* pc = cand + ((long long)p * norient + o) * n;
+  for (int k = t; k < n; k += blockDim.x) s_planeTw[k] = tw64[k];
   // FP32 maximum over planes
   float mv = -INFINITY;
   int mi = 0x7fffffff;
@@ -1708,7 +1775,8 @@ __global__ void __launch_bounds__(256) k_sph_select(
       }
       __syncthreads();
       const int np = s_np;
-      grid_eval64_batch(c, np, s_pa, s_pg, s_pb, s_nb, s_beta, s_val, (double*)s_planeS, &s_blk);
+      grid_eval64_batch(c, np, s_pa, s_pg, s_pb, s_nb, s_beta, s_planeTw, s_val,
+                        (double*)s_planeS, &s_blk);
       __syncthreads();
       for (int q = 0; q < np; ++q) {
         const int f = s_cand[q0 + q];
@@ -1762,8 +1830,8 @@ __global__ void __launch_bounds__(256) k_sph_select(
       }
   }
   __syncthreads();
-  grid_eval64_batch(c, q0 + 6, s_pa, s_pg, s_pb, s_nb, s_beta, s_val, (double*)s_planeS,
-                    &s_blk);
+  grid_eval64_batch(c, q0 + 6, s_pa, s_pg, s_pb, s_nb, s_beta, s_planeTw, s_val,
+                    (double*)s_planeS, &s_blk);
   __syncthreads();
   if (merged) best = s_val[0];
   double off[3];
@@ -1812,38 +1880,7 @@ __global__ void k_seed_table(int Lt, double* __restrict__ seedu) {
   }
 }
 
-// Sums over the wavefront of ten values a lane, written to out[0..9]: two
-// halvings that keep one value per half, then a sum within rows of 16 lanes.
-// 60 instructions; ten butterflies over the lanes are 180 and wait 60 times.
-FO_DEV double swap_add32(double a, double b) {  // lanes 0-31: sum of a, 32-63: of b
-  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
-  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false,
-                                                   false);
-  return __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]) +
-         __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
-}
-FO_DEV double swap_add16(double a, double b) {  // rows 0, 2: sums of a's, 1, 3: of b's halves
-  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
-  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
-  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false,
-                                                   false);
-  return __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]) +
-         __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
-}
-template <int CTRL>
-FO_DEV double dpp_add(double v) {
-  const long long x = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), CTRL, 0xf, 0xf, true);
-  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-FO_DEV double row_sum(double v) {  // over the 16 lanes of a row (rotations)
-  v = dpp_add<0x128>(v);
-  v = dpp_add<0x124>(v);
-  v = dpp_add<0x122>(v);
-  return dpp_add<0x121>(v);
-}
+// Sums over the wavefront of ten values a lane, written to out[0..9].
 FO_DEV void wave_sum10(const double (&v)[10], double* out) {
   double u[5], w[3];
 #pragma unroll
@@ -2209,7 +2246,7 @@ FO_DEV void newton_update(NewtonState& s, const FGH& r) {
 // reaches the level where rounding noise of f (a sum of ~K(L) terms)
 // dominates: |g| <= 1e-12 |f|, decrease <= 1e-13 |f|, step <= 1e-12 rad.
 // The line search halves at most 8 times.
-__global__ void __launch_bounds__(256, 3) k_sph_rotopt(const SphPair* __restrict__ pd,
+__global__ void __launch_bounds__(512, 3) k_sph_rotopt(const SphPair* __restrict__ pd,
                                                     const double2* __restrict__ IA,
                                                     const double2* __restrict__ IB, int mode,
                                                     const SphPeak* __restrict__ peaks, int norient,
@@ -2695,12 +2732,19 @@ void launch_beta_gemm(hipStream_t s, int P, int n, int Lmax, long long Kp, int L
   hipLaunchKernelGGL(k_coef_abound, dim3(P), dim3(256), 0, s, pd, n, IA, norient, abound);
 }
 
+// Up to two workgroups a CU, the selection and the refinement take eight
+// wavefronts each instead of four (64 pairs of degree 40: 300 -> 233 and 136 ->
+// 105 us); beyond, the larger workgroups wait longer for each other (4096 pairs:
+// 487 -> 559 and 542 -> 942 us).  The results do not depend on the number.
+static bool few_workgroups(int P, int norient) { return (long long)P * norient <= 512; }
+
 void launch_sph_select(hipStream_t s, int P, int n, long long Kt, int norient, const SphPair* pd,
                        const double* tab64, const double2* tw64, const double2* IA,
                        const double2* IB, int mode, const PlaneCand* cand, double2* scratch,
                        long long scratch_stride, const double* abound, SphPeak* peaks,
                        double extra_rel, int all_planes) {
-  hipLaunchKernelGGL(k_sph_select, dim3(xcd_grid(P, norient)), dim3(256), 0, s, pd, n, Kt, tab64,
+  const int threads = few_workgroups(P, norient) ? 512 : 256;
+  hipLaunchKernelGGL(k_sph_select, dim3(xcd_grid(P, norient)), dim3(threads), 0, s, pd, n, Kt, tab64,
                      tw64, IA, IB, mode, norient, cand, scratch, scratch_stride, abound, peaks, P,
                      extra_rel, all_planes);
 }
@@ -2708,7 +2752,8 @@ void launch_sph_select(hipStream_t s, int P, int n, long long Kt, int norient, c
 void launch_sph_rotopt(hipStream_t s, int P, int norient, int Lmax, const SphPair* pd,
                        const double2* IA, const double2* IB, int mode, const SphPeak* peaks,
                        const double* seedu, int Lt, SphOpt* opt) {
-  hipLaunchKernelGGL(k_sph_rotopt, dim3(xcd_grid(P, norient)), dim3(256), rec_lds_bytes(Lmax), s, pd, IA, IB,
+  const int threads = few_workgroups(P, norient) ? 512 : 256;
+  hipLaunchKernelGGL(k_sph_rotopt, dim3(xcd_grid(P, norient)), dim3(threads), rec_lds_bytes(Lmax), s, pd, IA, IB,
                      mode, peaks, norient, seedu, Lt, Lmax, opt, P);
 }
 

@@ -751,3 +751,23 @@ def test_read_back_in_one_transfer(gpu, pairs):
         t.join()
     if errors:
         raise errors[0]
+
+
+@pytest.mark.parametrize("n,L", [(7, 2), (16, 7), (37, 15), (64, 31), (66, 32), (128, 40), (99, 48)])
+def test_full_plane_evaluation_finds_the_argmax(gpu, n, L):
+    """FO_SPH_EXACT_PLANES evaluates every plane in FP64: the same argmax and
+    value (to FP64 rounding) as the candidates' evaluation, at the edges of the
+    16-row tiles, the four-term steps and the LDS buffer of a plane (L = 31, 32)."""
+    say(f"case: n={n} L={L}")
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(2, 9, 3))
+    out = []
+    for flag in (0, _lib.SPH_EXACT_PLANES):
+        with SphericalBatch([9], [L], 0.4, n, None, flag) as b:
+            b.set_positions(X[0], X[1])
+            b.run(_lib.STAGE_PREP | _lib.STAGE_COEFF | _lib.STAGE_GRID)
+            out.append((b.peaks(), b.precision()))
+    (p0, _), (p1, _) = out
+    assert (p1["noverflow"] == n).all()
+    np.testing.assert_array_equal(p0["ind"], p1["ind"])
+    np.testing.assert_allclose(p1["value"], p0["value"], rtol=1e-12)

@@ -261,43 +261,81 @@ FO_DEV bool lap_solve(int n, KeyF key, Fin fin, Near near, LapShared s, int* row
   return true;
 }
 
-// Cyclic Jacobi eigen-decomposition of a symmetric 4x4 matrix (FP64).
+// Eigenvalues w and eigenvectors (columns of V) of a symmetric 4x4 matrix by
+// Jacobi sweeps.  The six rotations of a sweep go as three pairs of disjoint
+// ones, whose angles are formed side by side: a rotation is a chain of a square
+// root, a quotient and a reciprocal root, and the solve one lane's latency.
+// The matrix is scaled by a power of two first, so that squares of its
+// entries neither overflow nor vanish.  One rotation after another by
+// quotients took 25000 cycles, more than the rest of a fit of 38 atoms.
 FO_DEV void jacobi4(double A[4][4], double V[4][4], double w[4]) {
+  double big = 0.0;
+#pragma unroll
   for (int i = 0; i < 4; ++i)
-    for (int j = 0; j < 4; ++j) V[i][j] = (i == j) ? 1.0 : 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      V[i][j] = (i == j) ? 1.0 : 0.0;
+      big = fmax(big, fabs(A[i][j]));
+    }
+  const int ex = big > 0.0 && big < INFINITY ? ilogb(big) : 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) A[i][j] = ldexp(A[i][j], -ex);
+  auto angle = [](double app, double aqq, double apq, double& c, double& s) {
+    const double d = 0.5 * (aqq - app), r2 = d * d + apq * apq;
+    const double den = fabs(d) + (r2 > 0.0 ? r2 * rsqrt(r2) : 0.0);
+    const double t = den > 0.0 ? (d < 0.0 ? -apq : apq) / den : 0.0;
+    c = rsqrt(t * t + 1.0);
+    s = t * c;
+  };
+  auto turn = [&](auto P, auto Q, double c, double s) {
+    constexpr int p = decltype(P)::value, q = decltype(Q)::value;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double akp = A[k][p], akq = A[k][q];
+      A[k][p] = c * akp - s * akq;
+      A[k][q] = s * akp + c * akq;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double apk = A[p][k], aqk = A[q][k];
+      A[p][k] = c * apk - s * aqk;
+      A[q][k] = s * apk + c * aqk;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double vkp = V[k][p], vkq = V[k][q];
+      V[k][p] = c * vkp - s * vkq;
+      V[k][q] = s * vkp + c * vkq;
+    }
+  };
+  auto two = [&](auto P, auto Q, auto R, auto S) {
+    double c0, s0, c1, s1;
+    angle(A[P.value][P.value], A[Q.value][Q.value], A[P.value][Q.value], c0, s0);
+    angle(A[R.value][R.value], A[S.value][S.value], A[R.value][S.value], c1, s1);
+    turn(P, Q, c0, s0);
+    turn(R, S, c1, s1);
+  };
+  constexpr std::integral_constant<int, 0> i0{};
+  constexpr std::integral_constant<int, 1> i1{};
+  constexpr std::integral_constant<int, 2> i2{};
+  constexpr std::integral_constant<int, 3> i3{};
   for (int sweep = 0; sweep < 60; ++sweep) {
     double off = 0.0, dia = 0.0;
+#pragma unroll
     for (int p = 0; p < 4; ++p) {
       dia += A[p][p] * A[p][p];
+#pragma unroll
       for (int q = p + 1; q < 4; ++q) off += A[p][q] * A[p][q];
     }
     if (off == 0.0 || off < 1e-36 * dia) break;
-    for (int p = 0; p < 4; ++p) {
-      for (int q = p + 1; q < 4; ++q) {
-        double apq = A[p][q];
-        if (apq == 0.0) continue;
-        double theta = (A[q][q] - A[p][p]) / (2.0 * apq);
-        double tt = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-        double c = 1.0 / sqrt(tt * tt + 1.0), sn = tt * c;
-        for (int k = 0; k < 4; ++k) {
-          double akp = A[k][p], akq = A[k][q];
-          A[k][p] = c * akp - sn * akq;
-          A[k][q] = sn * akp + c * akq;
-        }
-        for (int k = 0; k < 4; ++k) {
-          double apk = A[p][k], aqk = A[q][k];
-          A[p][k] = c * apk - sn * aqk;
-          A[q][k] = sn * apk + c * aqk;
-        }
-        for (int k = 0; k < 4; ++k) {
-          double vkp = V[k][p], vkq = V[k][q];
-          V[k][p] = c * vkp - sn * vkq;
-          V[k][q] = sn * vkp + c * vkq;
-        }
-      }
-    }
+    two(i0, i1, i2, i3);
+    two(i0, i2, i1, i3);
+    two(i0, i3, i1, i2);
   }
-  for (int i = 0; i < 4; ++i) w[i] = A[i][i];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = ldexp(A[i][i], ex);
 }
 
 // Quaternion -> rotation matrix (fastoverlap/utils.py:255-275), row-major.
@@ -342,19 +380,25 @@ FO_DEV void kearsley_solve(const double q[10], double* dist, double MR[9]) {
                     {q[3], q[6], q[8], q[9]}};
   double V[4][4], w[4];
   jacobi4(A, V, w);
-  int im = 0;
+  double e = w[0], qv[4] = {V[0][0], V[1][0], V[2][0], V[3][0]};
+#pragma unroll
   for (int i = 1; i < 4; ++i)
-    if (w[i] < w[im]) im = i;
-  double e = w[im];
+    if (w[i] < e) {
+      e = w[i];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) qv[k] = V[k][i];
+    }
   if (e < 0.0) e = (fabs(e) < 1e-6) ? 0.0 : -e;
   *dist = sqrt(e);
-  double qv[4] = {V[0][im], V[1][im], V[2][im], V[3][im]};
   q2mx(qv, MR);
 }
 
 // EulerM(a, b, y) = My . Mb . Ma  (fastoverlap/utils.py:447-460), row-major.
 FO_HD void euler_matrix(double a, double b, double y, double M[9]) {
-  double sa = sin(a), ca = cos(a), sb = sin(b), cb = cos(b), sy = sin(y), cy = cos(y);
+  double sa, ca, sb, cb, sy, cy;
+  sincos(a, &sa, &ca);
+  sincos(b, &sb, &cb);
+  sincos(y, &sy, &cy);
   // Mb . Ma
   double T[9] = {cb * ca, -cb * sa, -sb, sa, ca, 0.0, sb * ca, -sb * sa, cb};
   // My . T

@@ -2298,8 +2298,11 @@ __global__ void __launch_bounds__(512, 3) k_sph_rotopt(const SphPair* __restrict
 // sphericalAlignment.py:184-187), X2 <- (+-X2) EulerM(R) (:124), per-group
 // LAP on squared distances with rows = X1 (utils.py:49-56, :82-167), and the
 // quaternion fit (utils.py:169-275): X2out = X2R[perm] MR^T (:126-127).
+// Bound by latency: one pair of 38 atoms 25 -> 17 us with the sums halved across
+// the lanes and the fit's rotations in disjoint pairs; the rest is the
+// assignment's chain of row searches.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_sph_finish(
+__global__ void __launch_bounds__(512) k_sph_finish(
     const SphPair* __restrict__ pd, const SphGroup* __restrict__ grp, const int* __restrict__ gath,
     const double* __restrict__ X1c, const double* __restrict__ X2c, const SphOpt* __restrict__ opt,
     int norient, int lap_nmax, int pos_lds, double* __restrict__ X2R, int* __restrict__ perm,
@@ -2362,21 +2365,26 @@ __global__ void __launch_bounds__(256) k_sph_finish(
   // depend on the block size)
   __shared__ double sMR[9];
   __shared__ double sdist;
+  __shared__ double sums[18];
   if (t < 64) {
-    double c[6] = {0, 0, 0, 0, 0, 0};
+    double v8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int a = t; a < N; a += 64)
       for (int k = 0; k < 3; ++k) {
-        c[k] += x1[3 * a + k];
-        c[3 + k] += xr[3 * pm[a] + k];
+        v8[k] += x1[3 * a + k];
+        v8[3 + k] += xr[3 * pm[a] + k];
       }
-    for (int k = 0; k < 6; ++k) c[k] = wave_sum(c[k]) / (double)N;
-    double q[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    wave_sum8(v8, sums);
+    wave_sync();
+    double c[6], q[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    for (int k = 0; k < 6; ++k) c[k] = sums[k] / (double)N;
     for (int a = t; a < N; a += 64) {
       const double* B = xr + 3 * pm[a];
       qmat_accum(q, x1[3 * a] - c[0], x1[3 * a + 1] - c[1], x1[3 * a + 2] - c[2], B[0] - c[3],
                  B[1] - c[4], B[2] - c[5]);
     }
-    for (int k = 0; k < 10; ++k) q[k] = wave_sum(q[k]);
+    wave_sum10(q, sums + 8);
+    wave_sync();
+    for (int k = 0; k < 10; ++k) q[k] = sums[8 + k];
     if (t == 0) {
       double MR[9], dist;
       kearsley_solve(q, &dist, MR);
@@ -2763,14 +2771,15 @@ void launch_sph_finish(hipStream_t s, int P, int lap_nmax, const SphPair* pd, co
                        SphResult* res) {
   // one wavefront per pair: the assignment search is a chain of small
   // reductions, cheapest without cross-wave barriers, until the largest
-  // group reaches 192 atoms: then four, whose column scans are shorter (the
-  // assignment and the fit do not depend on the block size)
+  // group reaches 192 atoms: then four, whose column scans are shorter, and
+  // eight from 512 on (64 pairs of 1000 atoms: 505 -> 447 us; the assignment
+  // and the fit do not depend on the block size)
   // positions of the largest group in LDS beside the assignment arrays when
   // that stays within 64 KiB
   const size_t lap = (lap_lds_bytes(lap_nmax) + 15) & ~(size_t)15;
   const size_t pos = 6 * sizeof(double) * (size_t)lap_nmax;
   const int pos_lds = lap + pos <= 65536 ? 1 : 0;
-  const int nthr = lap_nmax >= 192 ? 256 : 64;
+  const int nthr = lap_nmax >= 512 ? 512 : lap_nmax >= 192 ? 256 : 64;
   hipLaunchKernelGGL(k_sph_finish, dim3(P), dim3(nthr), lap + (pos_lds ? pos : 0), s, pd, grp,
                      gath, X1c, X2c, opt, norient, lap_nmax, pos_lds, X2R, perm, rowsol, X2out,
                      res);

@@ -541,9 +541,8 @@ def main():
             ach = fl / (kt[k] * 1e-3)
             per_kernel[name] = {"ms": round(kt[k], 4), "achieved_tflops": ach / 1e12,
                                 "peak_tflops": peak / 1e12, "frac": ach / peak}
-    # the dominant kernel: the stage with the largest time, except that the
-    # contraction stage is three kernels (degrees 0..7, 8..15 and >= 16),
-    # each well below the plane kernel, so it is not one kernel to roofline
+    # the dominant kernel: the largest stage beside the contraction, which is
+    # two launches when a batch has pairs on both sides of its split size
     dom = max((k for k in kt if k != "contract"), key=kt.get)
     # compute-bound kernels: the engine whose published peak bounds each one
     # ("valu": vector ALU, "mfma": matrix cores)

@@ -388,6 +388,22 @@ FO_DEV void kearsley_solve(const double q[10], double* dist, double MR[9]) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) qv[k] = V[k][i];
     }
+  // one first-order correction of the eigenvector against the matrix itself
+  // takes out what the rotations rounded; near-equal eigenvalues are left
+  const double rv[4] = {
+      q[0] * qv[0] + q[1] * qv[1] + q[2] * qv[2] + q[3] * qv[3] - e * qv[0],
+      q[1] * qv[0] + q[4] * qv[1] + q[5] * qv[2] + q[6] * qv[3] - e * qv[1],
+      q[2] * qv[0] + q[5] * qv[1] + q[7] * qv[2] + q[8] * qv[3] - e * qv[2],
+      q[3] * qv[0] + q[6] * qv[1] + q[8] * qv[2] + q[9] * qv[3] - e * qv[3]};
+  const double wmax = fmax(fmax(w[0], w[1]), fmax(w[2], w[3])), e0 = e;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const double gap = w[i] - e0;
+    const double dot = V[0][i] * rv[0] + V[1][i] * rv[1] + V[2][i] * rv[2] + V[3][i] * rv[3];
+    const double f = gap > 1e-6 * wmax ? dot / gap : 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) qv[k] -= f * V[k][i];
+  }
   if (e < 0.0) e = (fabs(e) < 1e-6) ? 0.0 : -e;
   *dist = sqrt(e);
   q2mx(qv, MR);

@@ -1232,8 +1232,8 @@ static int sph_autotune(fo_sph_batch* b) {
     FO_HIP(hipEventElapsedTime(ms, e0, e1));
     return FO_OK;
   };
-  // knob 1 is reserved (it chose the contraction's tile class below degree
-  // 16, where one fused kernel now runs).  The first candidate of each knob
+  // knob 1 is reserved (it chose a tile class that the contraction no longer
+  // has).  The first candidate of each knob
   // is the default shape; another replaces the best so far only when its
   // stage runs at least kTuneMargin faster, so timing noise (a few percent
   // between launches) cannot trade the default for an equal or slower

@@ -2239,7 +2239,7 @@ FO_DEV void newton_update(NewtonState& s, const FGH& r) {
 // evaluation is the phases and powers (2300 cycles), a block's edge elements
 // (2900), its degrees and the ten sums (1100); by FP64 issue for many: about 50
 // instructions per item and degree, 32 of them FP64.  One pair, degree 15: 55
-// -> 29 us, 64 pairs of degree 40: 292 -> 134, 4096 of 16..25: 900 -> 530,
+// -> 29 us, 64 pairs of degree 40: 292 -> 105, 4096 of 16..25: 900 -> 530,
 // against powers by squaring per item, index updates and a sign per degree, and
 // a butterfly per sum.
 // Converged when the gradient, the Newton model decrease -g.dx/2 or the step

@@ -268,7 +268,10 @@ static int read_parts(B* b, const Part (&parts)[K]) {
 static int write_positions(fo_context* c, bool own, hipStream_t s, double* d1, double* d2,
                            const double* p1, const double* p2, size_t n, void** slab) {
   const size_t gap = (char*)d2 - (char*)d1, bytes = gap + sizeof(double) * n;
-  if (own && bytes <= kSlabBytes) {
+  // (a captured copy would read the buffer at every replay: refused below)
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  FO_HIP(hipStreamIsCapturing(s, &cap));
+  if (own && bytes <= kSlabBytes && cap == hipStreamCaptureStatusNone) {
     if (*slab)
       FO_HIP(hipStreamSynchronize(s));  // an earlier copy may still read it
     else

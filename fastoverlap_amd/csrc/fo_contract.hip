@@ -46,14 +46,15 @@ namespace fo {
 // wavefronts hold registers), one pair of 160 atoms 75 us with one and 32 with
 // four.
 //
-// All degrees share a launch: as one launch per class it took 110 -> 44 us
-// more for one pair of 100 atoms (each class waits for its slowest item) and
-// 2.06 against 1.99 ms for the 4096 pairs, although the joint kernel spills 241
-// registers, outside its product loops.
+// All degrees share a launch: with one launch per class one pair of 100 atoms
+// took 110 us instead of 44 (each class waits for its slowest item) and the 4096
+// pairs 2.06 ms instead of 1.99, although the joint kernel spills 241 registers,
+// outside its product loops.
 //
-// Bound: reading K and Y.  1000 atoms, degree 40: 18.7 GB for 64 pairs (a
-// slot once for every item of its degrees), 3.6 TB/s; of the 5.2 ms the
-// products take 2.1 at the matrix rate.  4096 pairs of 13..147 atoms, degrees
+// Bound: reading K and Y.  1000 atoms, degree 40: 25.6 GB for 64 pairs (a
+// slot once for every item of its degrees), 5 TB/s; of the 5.1 ms the
+// products take 2.2 at the matrix rate.  Items with all row tiles of a degree
+// read a slot 40 times instead of 63 but leave one wavefront a SIMD: 6.3 ms.  4096 pairs of 13..147 atoms, degrees
 // 16..25: products 0.62 of 1.99 ms, waits on loads (two wavefronts a SIMD)
 // most of the rest.  Against the two kernels it replaces (a workgroup per
 // degree with A through LDS, the complex form, and for degrees <= 15 a fused

@@ -771,3 +771,30 @@ def test_full_plane_evaluation_finds_the_argmax(gpu, n, L):
     assert (p1["noverflow"] == n).all()
     np.testing.assert_array_equal(p0["ind"], p1["ind"])
     np.testing.assert_allclose(p1["value"], p0["value"], rtol=1e-12)
+
+
+def test_result_is_the_same_in_any_batch_size(gpu):
+    """The selection and the refinement take eight wavefronts a workgroup in a
+    small batch and four in a large one (P x orientations above 512): every
+    output of a pair is the same, bit for bit, also for symmetric structures
+    whose equal maxima put whole planes through the FP64 evaluation."""
+    say("case: 3 pairs alone and 300 together")
+    rng = np.random.default_rng(11)
+    cube = np.array([[x, y, z] for x in (-1, 1) for y in (-1, 1) for z in (-1, 1)], float)
+    q, _ = np.linalg.qr(rng.normal(size=(3, 3)))
+    pairs = [(cube, cube @ q), (cube * [1, 1, 1.3], (cube * [1, 1, 1.3]) @ q),
+             tuple(rng.normal(size=(2, 8, 3)))]
+
+    def run(sel):
+        with SphericalBatch([8] * len(sel), 10, 0.4, 32, None) as b:
+            b.set_positions([pairs[i][0] for i in sel], [pairs[i][1] for i in sel])
+            b.run(sync=False)
+            return b.read()
+
+    big = run([i % 3 for i in range(300)])
+    for i in range(3):
+        small = run([i])
+        for got, one in zip(big[:3], small[:3]):
+            for k in one:
+                for p in (i, 297 + i):
+                    np.testing.assert_array_equal(got[k][p], one[k][0], err_msg=f"{i} {k}")

@@ -52,10 +52,12 @@ FO_DEV double overlap_weight(const PerPair& d, int a, int b, int c) {
 // CT = ceil(NB / 16) column tiles; 2 NB rows are at most 4 tiles for CT <= 2
 // and 8 above (two per wave).  Bound: the latency of the phase stage, which
 // every a repeats (one sincospi per atom and axis, multiples by products) and
-// its barriers; the products take 23 us of the 114 below at the matrix rate
-// (34 of 48 rows and 17 of 32 columns used at nk = 8).  Against the complex
+// its barriers; the products take 23 us of the 93 below at the matrix rate
+// (34 of 48 rows and 17 of 32 columns used at nk = 8).  For CT <= 2 registers are
+// held to 128, two workgroups a CU, so that one's phases run beside the other's
+// products (114 -> 93 and 145 -> 125 us below, 19 spilled outside the product loop).  Against the complex
 // VALU sum over the full cube: 256 atoms, nk = 8: 145 -> 23 us for one pair,
-// 565 -> 114 us for 128; 24 pairs of 601..1024 atoms, nk = 14: 1428 -> 145 us;
+// 565 -> 93 us for 128; 24 pairs of 601..1024 atoms, nk = 14: 1428 -> 125 us;
 // relative error against 64-bit-exact phases 1.6e-15 -> 0.8e-15 (256 atoms).
 // ---------------------------------------------------------------------------
 constexpr int kSFTile = 64;   // atoms per LDS tile
@@ -64,7 +66,7 @@ constexpr int kSFThreads = 512;
 FO_HD int sf_stride(int NB) { return 2 * NB + 3; }  // doubles per atom (odd)
 
 template <int CT>
-__global__ void __launch_bounds__(kSFThreads) k_per_sf(
+__global__ void __launch_bounds__(kSFThreads, CT <= 2 ? 4 : 1) k_per_sf(
     const PerPair* __restrict__ pd, const PerGroup* __restrict__ grp,
     const int* __restrict__ atoms, const double* __restrict__ pos1,
     const double* __restrict__ pos2, int nk, double2* __restrict__ Cprod,

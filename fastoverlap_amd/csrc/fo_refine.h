@@ -233,6 +233,10 @@ FO_DEV bool lap_solve(int n, KeyF key, Fin fin, Near near, LapShared s, int* row
           __syncthreads();
           return false;
         }
+        // whether the column is free is read before the barrier: behind it the
+        // first lane may already be at the augmentation, whose first store is
+        // this entry, and a wavefront that read it late would stay in the loop
+        const int row = s.p[bj];
         const double delta = best;
         for (int j = t; j <= n; j += bd) {
           if (s.used[j]) {
@@ -244,7 +248,7 @@ FO_DEV bool lap_solve(int n, KeyF key, Fin fin, Near near, LapShared s, int* row
         }
         __syncthreads();
         j0 = bj;
-        if (s.p[j0] == 0) break;
+        if (row == 0) break;
       }
       if (t == 0) {
         do {

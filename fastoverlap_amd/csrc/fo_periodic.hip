@@ -391,15 +391,25 @@ __global__ void __launch_bounds__(256) k_per_plane(
 //      +-b into the real coefficients R[r over c][k over b] (LDS);
 //   2. G[r][y] = sum_k R[r][k] phi_k(y)  and
 //   3. g[y][z] = sum_r G[r][y] phi_r(z)  on v_mfma_f32_16x16x4f32: a
-//      wavefront owns 16 columns y, and register i of lane group q, row
-//      r = 4 q + i of a result tile of 2, is the A operand of 3 at the step
-//      that takes the rows 4 q + i, q = 0..3 (any order of r will do).
-// phi: (NB + 1) rows of F in LDS, the last one zero (padding of r and k).
+//      wavefront owns 16 columns y, and register i of lane group q, row 4 q + i
+//      of a result tile of 2, is the A operand of 3 at the step i of the tile; it
+//      holds the function r = 4 i + 3 - q of the tile, so that a step takes four
+//      consecutive functions.
+// All three sums run from the highest order down, +-a together in 1: the
+// structure factors fall off with it, and a sum that starts at its small end
+// rounds less.  rms error over the rms of the grid: 0.46e-7 for 256 atoms, nk = 8
+// (upwards 1.6e-7, the complex transform 1.2e-7), 0.31e-7 for 1000, nk = 14 (1.5
+// and 1.3e-7).
+// phi: (NB + 1) rows of F in LDS, the last one zero (padding of r and k); the row
+// stride is an odd multiple of 16, so the four rows of a step start in different
+// banks.
 // XP planes share the table; their products read C through the caches.
-// Rounding: the folds and the three sums of at most NB terms stay below
-// real_plane_delta(NB) sum |C|: stage 1 (2 NB + 4) u sum|C|, times sqrt 2 for each
-// of |cos| + |sin| in 2 and 3, whose own NB roundings add 3 NB u: 7.5 NB + 19
-// units u = 2^-24 in all.
+// Rounding, in units u = 2^-24 of sum |C| to first order: stage 1 rounds C, the
+// twiddles, 2 NB additions a component and the fold, 2 NB + 3, times 2 for both
+// components with |cos| + |sin| over b and c; 2 and 3 round phi, NB products and
+// their sums, NB + 2 each, times sqrt 2 (sum |R| |phi| |phi| <= sqrt 2 sum |C|):
+// 6.9 NB + 12 in all.  real_plane_delta, 9 NB + 64, is that with room for the
+// second order and for matrix units that round products apart from sums.
 // Against the complex transform on the vector units, which formed every F^2 NB
 // term of a plane: 259 -> 75 us for 128 pairs of nk = 8, F = 64, 111 -> 36 us for
 // 24 of nk = 14, F = 60, 20 -> 12 us for one pair.  Bound: stage 1 (two FP64
@@ -407,7 +417,7 @@ __global__ void __launch_bounds__(256) k_per_plane(
 // candidate test of every value.
 constexpr int kPlaneXP = 4;
 FO_HD double real_plane_delta(int NB) { return (9.0 * NB + 64.0) * 5.9604644775390625e-08; }
-FO_HD int real_plane_fs(int F) { return ((F + 15) & ~15) + 4; }  // row stride of phi
+FO_HD int real_plane_fs(int F) { return ((F + 15) & ~15) | 16; }  // row stride of phi
 FO_HD int real_plane_ks(int NB) { return ((NB + 3) & ~3) + 1; }  // row stride of R
 
 template <int NT>
@@ -432,19 +442,27 @@ __global__ void __launch_bounds__(256) k_per_plane_real(
     const double2* Cp = C + (nk + b) * NB + nk + c;
     const double2* Cm = C + (nk - b) * NB + nk + c;
     float2 hp = make_float2(0.f, 0.f), hm = hp;
-    int ph = (F - nk * x % F) % F;  // (-nk x) mod F
-#pragma unroll 4
-    for (int a = 0; a < NB; ++a) {
-      const double2 u = Cp[(long long)a * plane], v = Cm[(long long)a * plane];
-      const float2 w = tw[ph];
-      const float ux = (float)u.x, uy = (float)u.y, vx = (float)v.x, vy = (float)v.y;
-      hp.x += ux * w.x - uy * w.y;
-      hp.y += ux * w.y + uy * w.x;
-      hm.x += vx * w.x - vy * w.y;
-      hm.y += vx * w.y + vy * w.x;
-      ph += x;
-      if (ph >= F) ph -= F;
+    auto add = [&](float2& h, double2 z, float2 w) {
+      const float zx = (float)z.x, zy = (float)z.y;
+      h.x += zx * w.x - zy * w.y;
+      h.y += zx * w.y + zy * w.x;
+    };
+    const long long mid = (long long)nk * plane;
+    int ph = nk * x % F;
+#pragma unroll 2
+    for (int a = nk; a > 0; --a) {  // +-a together, the twiddle of -a is conjugate
+      const long long o = (long long)a * plane;
+      const float2 w = tw[ph], wc = make_float2(w.x, -w.y);
+      const double2 up = Cp[mid + o], um = Cp[mid - o], vp = Cm[mid + o], vm = Cm[mid - o];
+      add(hp, up, w);
+      add(hp, um, wc);
+      add(hm, vp, w);
+      add(hm, vm, wc);
+      ph -= x;
+      if (ph < 0) ph += F;
     }
+    add(hp, Cp[mid], make_float2(1.f, 0.f));
+    add(hm, Cm[mid], make_float2(1.f, 0.f));
     const float sc = c ? 2.f : 1.f;  // the terms of -c
     float* re = R + ((long long)xi * NB + (c ? 2 * c - 1 : 0)) * KS;
     float* im = re + KS;  // c > 0 only
@@ -476,7 +494,8 @@ __global__ void __launch_bounds__(256) k_per_plane_real(
   __syncthreads();
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6), ln = t & 63, col = ln & 15, q = ln >> 4;
   const int nyt = (F + 15) >> 4, ksteps = (NB + 3) >> 2;
-  // this lane's rows of phi in stage 3, register i of tile tt: 16 tt + 4 q + i
+  // function of row col of a result tile of stage 2
+  const int fr = 4 * (col & 3) + 3 - (col >> 2);
   for (int xi = 0; xi < XP; ++xi) {
     const int x = x0 + xi;
     if (x >= F) break;  // uniform
@@ -487,12 +506,12 @@ __global__ void __launch_bounds__(256) k_per_plane_real(
       v4f G[NT];
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) G[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-      for (int s = 0; s < ksteps; ++s) {
-        const int k = 4 * s + q;
+      for (int s = ksteps - 1; s >= 0; --s) {
+        const int k = 4 * s + 3 - q;
         const float b = phi[min(k, NB) * FS + 16 * yt + col];
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) {
-          const float a = Rx[min(16 * tt + col, NB - 1) * KS + k];
+          const float a = Rx[min(16 * tt + fr, NB - 1) * KS + k];
           G[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, G[tt], 0, 0, 0);
         }
       }
@@ -500,11 +519,11 @@ __global__ void __launch_bounds__(256) k_per_plane_real(
         const float* pz = phi + 16 * zt + col;
         v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int tt = 0; tt < NT; ++tt)
+        for (int tt = NT - 1; tt >= 0; --tt)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if (16 * tt + i >= NB) continue;  // uniform
-            const float b = pz[min(16 * tt + 4 * q + i, NB) * FS];
+          for (int i = 3; i >= 0; --i) {
+            if (16 * tt + 4 * i >= NB) continue;  // uniform
+            const float b = pz[min(16 * tt + 4 * i + 3 - q, NB) * FS];
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(G[tt][i], b, acc, 0, 0, 0);
           }
         const int z = 16 * zt + col;

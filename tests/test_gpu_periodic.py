@@ -342,3 +342,30 @@ def test_periodic_read_back_in_one_transfer(gpu, pairs):
                     np.testing.assert_array_equal(u, v)
         cells = (r["X1"][0] - x[:64]) / box  # the structure in the home cell
         np.testing.assert_allclose(cells, np.round(cells), atol=1e-12)
+
+
+@pytest.mark.parametrize("nk,F,N", [(4, 20, 30), (8, 64, 256), (14, 60, 1000), (16, 70, 500)])
+def test_real_planes_round_no_more_than_complex_planes(gpu, nk, F, N):
+    """|f| against a 64-bit FFT of the same product: the rms error of the
+    real-basis planes is no larger than that of the complex transform (the same
+    coefficients supplied), also for structures that nearly match, whose product
+    falls off slowest."""
+    rng = np.random.default_rng(nk)
+    box = np.array([1.0, 1.1, 0.95]) * (N / 1.185) ** (1 / 3)
+    err = np.zeros(2)
+    for seed in range(3):
+        say(f"case: nk={nk} F={F} N={N} seed {seed}")
+        x = rng.random((N, 3)) * box
+        y = rng.random((N, 3)) * box if seed == 2 else x + 0.3 * box + rng.normal(scale=0.02, size=x.shape)
+        coef = None
+        for k, flag in enumerate((_lib.PER_KEEP_COEFFS, _lib.PER_INPUT_COEFFS)):
+            with PeriodicBatch([N], box, 0.3, nk, F, None, 10, _lib.PER_KEEP_GRID | flag) as b:
+                b.set_positions(x, y)
+                if k:
+                    b.set_coeffs(*coef)
+                b.run(_lib.PSTAGE_SF | _lib.PSTAGE_GRID)
+                coef = coef or b.coeffs()
+                f = np.abs(np.fft.fftn(b.product()[0], (F, F, F)))
+                err[k] += np.square(b.grid(0) - f).mean() / np.square(f).mean()
+    say("rms error, real and complex:", np.sqrt(err / 3))
+    assert err[0] <= err[1]

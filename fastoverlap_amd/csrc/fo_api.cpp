@@ -23,6 +23,7 @@
 #include "fo_host.h"
 #include "fo_internal.h"
 #include "fo_refine.h"
+#include "fo_staging.h"
 
 namespace fo {
 // launchers (fo_spherical.hip / fo_periodic.hip)
@@ -170,67 +171,8 @@ struct fo_context {
   std::map<std::tuple<int, int, int, int>, std::array<int, 3>> tuned;
   RecTable rect;
   std::vector<void*> owned;  // table allocations
-  std::mutex slab_mu;
-  std::vector<void*> slabs;  // idle pinned staging buffers
+  SlabPool slabs;  // pinned staging buffers
 };
-
-// Pinned staging for small transfers: a buffer is one thread's from get to
-// put; at most kSlabsKept idle ones are kept.  One copy of a batch's adjacent
-// outputs through a buffer takes 10 us; a copy of each output into pageable
-// memory took 8..15 us apiece.  Larger transfers go to the caller's memory directly
-// (18 GB/s, as fast as the copy out of a buffer).
-static constexpr size_t kSlabBytes = 256 << 10;
-static constexpr size_t kSlabsKept = 16;
-static void* slab_get(fo_context* c) {
-  {
-    std::lock_guard<std::mutex> g(c->slab_mu);
-    if (!c->slabs.empty()) {
-      void* p = c->slabs.back();
-      c->slabs.pop_back();
-      return p;
-    }
-  }
-  void* p = nullptr;
-  if (hipHostMalloc(&p, kSlabBytes, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;  // the caller copies directly
-  }
-  return p;
-}
-static void slab_put(fo_context* c, void* p) {
-  if (!p) return;
-  {
-    std::lock_guard<std::mutex> g(c->slab_mu);
-    if (c->slabs.size() < kSlabsKept) {
-      c->slabs.push_back(p);
-      return;
-    }
-  }
-  (void)hipHostFree(p);
-}
-
-// Device memory read in one go: [dev, dev + bytes) through a staging buffer
-// into `use(const char*)`, if it is small enough and `own` (memory of the
-// context; a caller's arena never makes an allocation here).  Returns false if
-// the range has to be copied directly.
-template <class F>
-static bool read_staged(fo_context* c, bool own, hipStream_t s, const void* dev, size_t bytes,
-                        F&& use, hipError_t* err) {
-  if (!own || bytes > kSlabBytes) return false;
-  void* slab = slab_get(c);
-  if (!slab) return false;
-  *err = hipMemcpyAsync(slab, dev, bytes, hipMemcpyDeviceToHost, s);
-  if (*err == hipSuccess) *err = hipStreamSynchronize(s);
-  if (*err == hipSuccess) use((const char*)slab);
-  slab_put(c, slab);
-  return true;
-}
-
-template <class B>
-static void release_slab(B* b) {  // the batch's stream is idle
-  slab_put(b->ctx, b->slab);
-  b->slab = nullptr;
-}
 
 // Parts of the batch's memory, in ascending order, to where `to` is not NULL.
 template <class B, class Part, size_t K>
@@ -244,48 +186,42 @@ static int read_parts(B* b, const Part (&parts)[K]) {
   if (hi <= lo) return FO_OK;
   const char* base = (const char*)b->base;
   hipError_t e = hipSuccess;
-  const bool staged = read_staged(
-      b->ctx, b->own_mem, b->stream, base + lo, hi - lo,
-      [&](const char* h) {
-        for (const Part& p : parts)
-          if (p.to) memcpy(p.to, h + (p.off - lo), p.bytes);
-      },
-      &e);
+  // (a caller's arena never makes an allocation here)
+  const bool staged =
+      b->own_mem && read_staged(
+                        b->ctx->slabs, b->slab, b->stream, base + lo, hi - lo,
+                        [&](const char* h) {
+                          for (const Part& p : parts)
+                            if (p.to) memcpy(p.to, h + (p.off - lo), p.bytes);
+                        },
+                        &e);
   if (!staged) {
     for (const Part& p : parts)
       if (p.to && p.bytes)
         FO_HIP(hipMemcpyAsync(p.to, base + p.off, p.bytes, hipMemcpyDeviceToHost, b->stream));
-    e = hipStreamSynchronize(b->stream);
+    e = sync_staged(b->ctx->slabs, b->slab, b->stream);
   }
   if (e != hipSuccess) return set_err(FO_ERR_HIP, hipGetErrorString(e));
-  release_slab(b);
   return FO_OK;
 }
 
 // Host positions into a batch: pos2 lies at a fixed distance after pos1, so a
-// staged pair is one copy, which needs no wait (`slab` is the batch's until its
-// stream is next synchronised).
-static int write_positions(fo_context* c, bool own, hipStream_t s, double* d1, double* d2,
-                           const double* p1, const double* p2, size_t n, void** slab) {
-  const size_t gap = (char*)d2 - (char*)d1, bytes = gap + sizeof(double) * n;
+// staged pair is one copy, which needs no wait.
+template <class B>
+static int write_positions(B* b, const double* p1, const double* p2) {
+  const size_t bytes = sizeof(double) * 3 * b->Ntot, gap = (char*)b->pos2 - (char*)b->pos1;
   // (a captured copy would read the buffer at every replay: refused below)
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  FO_HIP(hipStreamIsCapturing(s, &cap));
-  if (own && bytes <= kSlabBytes && cap == hipStreamCaptureStatusNone) {
-    if (*slab)
-      FO_HIP(hipStreamSynchronize(s));  // an earlier copy may still read it
-    else
-      *slab = slab_get(c);
-    if (*slab) {
-      memcpy(*slab, p1, sizeof(double) * n);
-      memcpy((char*)*slab + gap, p2, sizeof(double) * n);
-      FO_HIP(hipMemcpyAsync(d1, *slab, bytes, hipMemcpyHostToDevice, s));
-      return FO_OK;
-    }
+  FO_HIP(hipStreamIsCapturing(b->stream, &cap));
+  hipError_t e = hipSuccess;
+  if (b->own_mem && cap == hipStreamCaptureStatusNone &&
+      write_staged(b->ctx->slabs, b->slab, b->stream, b->pos1, gap, p1, p2, bytes, &e)) {
+    if (e != hipSuccess) return set_err(FO_ERR_HIP, hipGetErrorString(e));
+    return FO_OK;
   }
-  FO_HIP(hipMemcpyAsync(d1, p1, sizeof(double) * n, hipMemcpyHostToDevice, s));
-  FO_HIP(hipMemcpyAsync(d2, p2, sizeof(double) * n, hipMemcpyHostToDevice, s));
-  FO_HIP(hipStreamSynchronize(s));
+  FO_HIP(hipMemcpyAsync(b->pos1, p1, bytes, hipMemcpyHostToDevice, b->stream));
+  FO_HIP(hipMemcpyAsync(b->pos2, p2, bytes, hipMemcpyHostToDevice, b->stream));
+  FO_HIP(hipStreamSynchronize(b->stream));
   return FO_OK;
 }
 
@@ -542,7 +478,7 @@ int fo_context_destroy(fo_context* c) {
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   for (void* p : c->owned) (void)hipFree(p);
-  for (void* p : c->slabs) (void)hipHostFree(p);
+  c->slabs.clear();
   (void)hipStreamDestroy(c->stream);
   delete c;
   return FO_OK;
@@ -622,7 +558,7 @@ struct fo_sph_batch {
   } off{};
   int gsum = 0;
   bool own_mem = false, own_stream = false;
-  void* slab = nullptr;  // staging buffer of the last host positions
+  SlabSlot slab{nullptr};  // staging buffer of the last host positions
   PeakScratch pk;  // multi-peak search buffers (allocated on first use)
   // FO_SPH_BETA_GEMM: even / odd-degree beta sums from k_beta_gemm
   // (split-BF16x3 on the matrix cores), [pair][beta][m1 <= Lmax][entry]
@@ -1099,8 +1035,7 @@ int fo_sph_batch_coef_norm2(fo_sph_batch* b, double* norm2) {
 
 int fo_sph_batch_destroy(fo_sph_batch* b) {
   if (!b) return FO_OK;
-  if (b->stream) (void)hipStreamSynchronize(b->stream);
-  release_slab(b);
+  if (b->stream) (void)sync_staged(b->ctx->slabs, b->slab, b->stream);
   for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second);
   if (b->ev_made) {
     for (auto& e : b->ev) (void)hipEventDestroy(e);
@@ -1125,8 +1060,7 @@ int fo_sph_batch_set_positions(fo_sph_batch* b, const double* p1, const double* 
   if (!b || !p1 || !p2) return set_err(FO_ERR_INVALID, "NULL argument");
   if (!all_finite(p1, 3 * b->Ntot) || !all_finite(p2, 3 * b->Ntot))
     return set_err(FO_ERR_INVALID, "positions must be finite");
-  return write_positions(b->ctx, b->own_mem, b->stream, b->pos1, b->pos2, p1, p2, 3 * b->Ntot,
-                         &b->slab);
+  return write_positions(b, p1, p2);
 }
 
 int fo_sph_batch_set_positions_device(fo_sph_batch* b, const void* p1, const void* p2) {
@@ -1305,8 +1239,7 @@ int fo_sph_batch_run(fo_sph_batch* b, int stages, int use_graph) {
 
 int fo_sph_batch_sync(fo_sph_batch* b) {
   if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
-  FO_HIP(hipStreamSynchronize(b->stream));
-  release_slab(b);
+  FO_HIP(sync_staged(b->ctx->slabs, b->slab, b->stream));
   return FO_OK;
 }
 
@@ -1775,7 +1708,7 @@ struct fo_per_batch {
   } off{};
   bool keepc = false;
   bool own_mem = false, own_stream = false;
-  void* slab = nullptr;  // staging buffer of the last host positions
+  SlabSlot slab{nullptr};  // staging buffer of the last host positions
   float2* cgrid = nullptr;   // complex f (FO_PER_KEEP_FFT)
   // per-structure coefficients shared by the pairs (set_coeffs_indexed)
   void* csbuf = nullptr;
@@ -2004,8 +1937,7 @@ int fo_per_batch_create(fo_context* c, const fo_per_batch_desc* d, fo_per_batch*
 
 int fo_per_batch_destroy(fo_per_batch* b) {
   if (!b) return FO_OK;
-  if (b->stream) (void)hipStreamSynchronize(b->stream);
-  release_slab(b);
+  if (b->stream) (void)sync_staged(b->ctx->slabs, b->slab, b->stream);
   for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second);
   if (b->ev_made)
     for (auto& e : b->ev) (void)hipEventDestroy(e);
@@ -2027,8 +1959,7 @@ int fo_per_batch_set_positions(fo_per_batch* b, const double* p1, const double* 
   if (!b || !p1 || !p2) return set_err(FO_ERR_INVALID, "NULL argument");
   if (!all_finite(p1, 3 * b->Ntot) || !all_finite(p2, 3 * b->Ntot))
     return set_err(FO_ERR_INVALID, "positions must be finite");
-  return write_positions(b->ctx, b->own_mem, b->stream, b->pos1, b->pos2, p1, p2, 3 * b->Ntot,
-                         &b->slab);
+  return write_positions(b, p1, p2);
 }
 
 int fo_per_batch_set_positions_device(fo_per_batch* b, const void* p1, const void* p2) {
@@ -2091,8 +2022,7 @@ int fo_per_batch_run(fo_per_batch* b, int stages, int use_graph) {
 
 int fo_per_batch_sync(fo_per_batch* b) {
   if (!b) return set_err(FO_ERR_INVALID, "NULL batch");
-  FO_HIP(hipStreamSynchronize(b->stream));
-  release_slab(b);
+  FO_HIP(sync_staged(b->ctx->slabs, b->slab, b->stream));
   return FO_OK;
 }
 

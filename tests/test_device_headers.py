@@ -1,4 +1,4 @@
-"""Device headers on the CPU: workgroups emulated lane by lane
+"""Headers of the library on the CPU: workgroups emulated lane by lane
 (tests/host/hip/hip_runtime.h), wavefronts running ahead of each other as far as
 the barriers let them."""
 
@@ -41,3 +41,11 @@ def test_assignment_search_in_any_wavefront_order(lap_block, threads, n, reverse
     got = np.array(rows.split(), int)
     c = np.array(costs.split(), float).reshape(n, n)
     np.testing.assert_array_equal(got, linear_sum_assignment(c)[1])
+
+
+def test_staging_buffers_change_hands_between_threads(tmp_path_factory):
+    """Positions set while another thread reads the same batch, two readers and
+    two writers: no buffer serves two batches, none is lost or freed twice."""
+    r = subprocess.run([build(tmp_path_factory, "staging")], capture_output=True, text=True,
+                       timeout=60)
+    assert (r.returncode, r.stdout) == (0, "ok\n"), r.stdout + r.stderr

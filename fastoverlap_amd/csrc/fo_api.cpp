@@ -765,6 +765,8 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
       b->maxgroup = std::max(b->maxgroup, sz);
     }
     sp.ngath = ng;
+    if (harm_nmax < 0 && !contract_in_reach(ng, Lp))
+      return set_err(FO_ERR_UNSUPPORTED, "too many grouped atoms in one pair");
     sp.coef_off = Ktot;
     sp.c32_off = C32tot;
     Ktot += kcount(Lp);

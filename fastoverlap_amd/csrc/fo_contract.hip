@@ -78,30 +78,37 @@ struct ContractArgs {
 // Row tiles of a degree: T / 2 pairs, (re, im) of m = 16 pair + r, and for odd
 // T one mixed tile, r < 8: re, r >= 8: im of m = 8 (T - 1) + r % 8.  A pair's
 // operands are one 16-byte load a lane.  Offsets (bytes) of the T tiles from
-// even tile t0 on at atom go + lane/16 of a harmonics block, one per pair and
-// one for the mixed tile (m beyond l repeat the last).
+// even tile t0 on at atom go + lane/16 of degree l's harmonics, one per pair and
+// one for the mixed tile (m beyond l repeat the last).  Descriptors and offsets
+// (unsigned) cover the degrees lb..l of one item, not the pair's whole block, which
+// passes 2^31 bytes at 156000 grouped atoms of degree 40 (contract_in_reach).
 FO_HD constexpr int row_units(int T) { return (T + 1) / 2; }
+FO_DEV __amdgpu_buffer_rsrc_t degree_rsrc(const double2* Y, int lb, int l, int Ng) {
+  const unsigned rows = qlm(l, l) + 1 - qlm(lb, 0);
+  return buf_rsrc(Y + (long long)qlm(lb, 0) * Ng, (int)(rows * Ng * 16u));
+}
 template <int T>
-FO_DEV void row_offsets(int (&off)[row_units(T)], int l, int t0, int Ng) {
+FO_DEV void row_offsets(unsigned (&off)[row_units(T)], int lb, int l, int t0, int Ng) {
   const int col = threadIdx.x & 15, q = (threadIdx.x >> 4) & 3;
 #pragma unroll
   for (int u = 0; u < row_units(T); ++u) {
     const bool mixed = 2 * u + 1 == T;
     const int m = 8 * (t0 + 2 * u) + (mixed ? col & 7 : col);
-    off[u] = (qlm(l, min(m, l)) * Ng + q) * 16 + (mixed ? (col >> 3) * 8 : 0);
+    off[u] = ((unsigned)(qlm(l, min(m, l)) - qlm(lb, 0)) * Ng + q) * 16u +
+             (mixed ? (col >> 3) * 8 : 0);
   }
 }
 // the T operands of those tiles, shifted by `add` bytes
 template <int T>
-FO_DEV void row_load(double (&v)[T], __amdgpu_buffer_rsrc_t r, const int (&off)[row_units(T)],
-                     int add) {
+FO_DEV void row_load(double (&v)[T], __amdgpu_buffer_rsrc_t r,
+                     const unsigned (&off)[row_units(T)], unsigned add) {
 #pragma unroll
   for (int u = 0; u < T / 2; ++u) {
-    const double2 x = load_d2(r, off[u] + add, 0);
+    const double2 x = load_d2(r, (int)(off[u] + add), 0);
     v[2 * u] = x.x;
     v[2 * u + 1] = x.y;
   }
-  if constexpr (T & 1) v[T - 1] = load_d(r, off[T / 2] + add, 0);
+  if constexpr (T & 1) v[T - 1] = load_d(r, (int)(off[T / 2] + add), 0);
 }
 // Tiles of atoms k: CNT / 2 pairs, tile 2 p + e holding the atoms 32 p + 2 r +
 // e of the block, and for odd CNT one tile of 16 consecutive ones; again one
@@ -227,8 +234,8 @@ FO_DEV void store_degree(const ContractArgs& a, const SphPair& d, int l, int rt0
 // with the next ones' operands loading meanwhile.
 template <int D, int CT, int RT, int CNT>
 FO_DEV void second_product(v4d (&P)[D][CT][RT], const v4d (&A)[D][CNT][RT],
-                           __amdgpu_buffer_rsrc_t ry2, const int (&o2)[D][row_units(CT)], int k0,
-                           int go, int Ns) {
+                           __amdgpu_buffer_rsrc_t ry2, const unsigned (&o2)[D][row_units(CT)],
+                           int k0, int go, int Ns) {
   constexpr int U = CT <= 2 ? 4 : (CT <= 4 ? 2 : 1), NU = 4 / U, NG = D * CNT * NU;
   const int q = (threadIdx.x >> 4) & 3;
   double y[2][U][CT];
@@ -239,7 +246,8 @@ FO_DEV void second_product(v4d (&P)[D][CT][RT], const v4d (&A)[D][CNT][RT],
     const int kt = (g / NU) % CNT;
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      row_load<CT>(v[u], ry2, o2[g / (NU * CNT)], (go + atom(kt, U * (g % NU) + u) - q) * 16);
+      row_load<CT>(v[u], ry2, o2[g / (NU * CNT)],
+                   (unsigned)(go + atom(kt, U * (g % NU) + u) - q) * 16u);
   };
   load(0, y[0]);
 #pragma unroll
@@ -290,12 +298,11 @@ FO_DEV void contract_high(const ContractArgs& a, const SphPair& d, int l, int rt
   const int q = (threadIdx.x >> 4) & 3;
   const int wv = WV > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int Ng = d.ngath;
-  const int ybytes = (int)(plane_rows(d.L) * Ng * 16);
-  const __amdgpu_buffer_rsrc_t ry1 = buf_rsrc(a.Y1 + d.ylm_off, ybytes);
-  const __amdgpu_buffer_rsrc_t ry2 = buf_rsrc(a.Y2 + d.ylm_off, ybytes);
-  int oy[row_units(RT)], o2[1][row_units(CT)];
-  row_offsets<RT>(oy, l, rt0, Ng);
-  row_offsets<CT>(o2[0], l, 0, Ng);
+  const __amdgpu_buffer_rsrc_t ry1 = degree_rsrc(a.Y1 + d.ylm_off, l, l, Ng);
+  const __amdgpu_buffer_rsrc_t ry2 = degree_rsrc(a.Y2 + d.ylm_off, l, l, Ng);
+  unsigned oy[row_units(RT)], o2[1][row_units(CT)];
+  row_offsets<RT>(oy, l, l, rt0, Ng);
+  row_offsets<CT>(o2[0], l, l, 0, Ng);
   v4d P[1][CT][RT];
 #pragma unroll
   for (int c = 0; c < CT; ++c)
@@ -318,7 +325,7 @@ FO_DEV void contract_high(const ContractArgs& a, const SphPair& d, int l, int rt
       double ka[CNT], kb[CNT], ya[RT], yb[RT];
       auto load = [&](double(&k)[CNT], double(&y)[RT], int s) {
         col_load<CNT>(k, rk, vk + s * (32 * Ns));
-        row_load<RT>(y, ry1, oy, go * 16 + s * 64);
+        row_load<RT>(y, ry1, oy, go * 16u + s * 64u);
         __builtin_amdgcn_sched_barrier(0);  // step by step, so that waits count
       };
       auto mul = [&](const double(&k)[CNT], const double(&y)[RT]) {
@@ -350,18 +357,18 @@ FO_DEV void contract_low_tiles(const ContractArgs& a, const SphPair& d, int h, d
   const int ln = threadIdx.x & 63, col = ln & 15, q = ln >> 4;
   const int wv = WV > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int Ng = d.ngath, Ns = G.size, go = G.gath_off, n4 = (Ns + 3) >> 2, nt = (Ns + 15) >> 4;
-  const int ybytes = (int)(plane_rows(d.L) * Ng * 16);
-  const __amdgpu_buffer_rsrc_t ry1 = buf_rsrc(a.Y1 + d.ylm_off, ybytes);
-  const __amdgpu_buffer_rsrc_t ry2 = buf_rsrc(a.Y2 + d.ylm_off, ybytes);
+  const int lt = h - PRE, lb = max(lt - (D - 1), 0);  // the item's degrees
+  const __amdgpu_buffer_rsrc_t ry1 = degree_rsrc(a.Y1 + d.ylm_off, lb, lt, Ng);
+  const __amdgpu_buffer_rsrc_t ry2 = degree_rsrc(a.Y2 + d.ylm_off, lb, lt, Ng);
   const double c0 = 2.0 * h + 1.0;
   const long long ss = (long long)Ns * Ns;
   const double* K = a.R + d.rad_off + G.rad_off;
   const __amdgpu_buffer_rsrc_t rk0 = buf_rsrc(K + 2 * BLK * ss, (int)(ss * 8));
   const __amdgpu_buffer_rsrc_t rk1 = buf_rsrc(K + (2 * BLK + 1) * ss, (int)(ss * 8));
   const __amdgpu_buffer_rsrc_t rr1 = buf_rsrc(a.rad1 + d.gath_off + go, Ns * 8);
-  int oy[D][row_units(RT)];
+  unsigned oy[D][row_units(RT)];
 #pragma unroll
-  for (int dd = 0; dd < D; ++dd) row_offsets<RT>(oy[dd], max(h - PRE - dd, 0), 0, Ng);
+  for (int dd = 0; dd < D; ++dd) row_offsets<RT>(oy[dd], lb, max(lt - dd, 0), 0, Ng);
   tile_blocks<KT>(nt * wv / WV, nt * (wv + 1) / WV, [&](auto CN, int tile) {
     constexpr int CNT = decltype(CN)::value;
     v4d A[D][CNT][RT];
@@ -386,7 +393,7 @@ FO_DEV void contract_low_tiles(const ContractArgs& a, const SphPair& d, int h, d
       col_load<CNT>(t.k1, rk1, vk + s * (32 * Ns));
       t.r = load_d(rr1, (4 * s + q) * 8, 0);
 #pragma unroll
-      for (int dd = 0; dd < D; ++dd) row_load<RT>(t.y[dd], ry1, oy[dd], go * 16 + s * 64);
+      for (int dd = 0; dd < D; ++dd) row_load<RT>(t.y[dd], ry1, oy[dd], go * 16u + s * 64u);
       __builtin_amdgcn_sched_barrier(0);  // step by step, so that waits count
     };
     auto mul = [&](Step& t) {

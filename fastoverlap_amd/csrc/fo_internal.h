@@ -39,6 +39,13 @@ __host__ __device__ inline long long harm_proj_doubles(int ngath, int L, int nma
   return basis ? 2LL * ngath * (L + 2 * nmax + 1) * (nmax + 1) : 0;
 }
 
+// Whether the contraction's 32-bit byte offsets reach a pair's harmonics: an
+// item reads the rows of one degree, or of up to four below 16 (at most 31),
+// 16 bytes an atom, with a step's reads past the end.
+__host__ __device__ inline bool contract_in_reach(int ngath, int L) {
+  return 16LL * (L + 1 > 31 ? L + 1 : 31) * ngath <= (1LL << 32) - 4096;
+}
+
 // Kernels of the beta planes.
 enum PlanePath { kPlaneDirect = 0, kPlaneFft = 1, kPlaneFold = 2 };
 

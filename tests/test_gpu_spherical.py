@@ -798,3 +798,22 @@ def test_result_is_the_same_in_any_batch_size(gpu):
             for k in one:
                 for p in (i, 297 + i):
                     np.testing.assert_array_equal(got[k][p], one[k][0], err_msg=f"{i} {k}")
+
+
+def test_coefficients_of_a_pair_past_32_bit_offsets(gpu):
+    """320000 grouped atoms at degree 40, whose harmonics take more than 2^32
+    bytes a structure: 5000 equal groups of 64 atoms give 5000 times the
+    coefficients of one."""
+    say("case: 5000 groups of 64 atoms, Jmax 40")
+    L, n, reps = 40, 64, 5000
+    rng = np.random.default_rng(40)
+    X1, X2 = (rng.normal(size=(n, 3)) for _ in range(2))
+    groups = list(np.arange(reps * n).reshape(reps, n))
+    with SphericalBatch([reps * n], [L], 0.35, 2 * (L + 1), [groups],
+                        _lib.SPH_NO_INVERT | _lib.SPH_NO_CENTER) as b:
+        b.set_positions(np.tile(X1, (reps, 1)), np.tile(X2, (reps, 1)))
+        b.run(_lib.STAGE_PREP | _lib.STAGE_COEFF)
+        got = compact_to_dense(b.coeffs()[0], L) / reps
+    ref = O.so3_coeffs_species(X1, X2, [np.arange(n)], L, 0.35, fast=True)
+    # the bound of the tests above, and a rounding of the sum for every group
+    np.testing.assert_allclose(got, ref, atol=(1e-12 + reps * 2.0 ** -53) * np.abs(ref).max())

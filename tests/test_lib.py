@@ -66,3 +66,39 @@ def test_compact_layout_roundtrip():
     np.testing.assert_array_equal(k, np.arange(kcount(L)))
     c = np.arange(kcount(L)) * (1 + 2j)
     np.testing.assert_array_equal(dense_to_compact(compact_to_dense(c, L)), c)
+
+
+def test_contraction_reach_is_the_offsets_range():
+    """The largest pair whose harmonics the contraction's 32-bit offsets reach:
+    an item's rows of 16 bytes an atom below 2^32, with a step to spare."""
+    import subprocess
+    import tempfile
+    src = r"""
+#include "fo_internal.h"
+#include <stdio.h>
+int main() {
+  for (int L = 0; L <= 63; ++L) {
+    long long lo = 1, hi = 1LL << 30;
+    while (hi - lo > 1) {
+      const long long mid = (lo + hi) / 2;
+      (fo::contract_in_reach((int)mid, L) ? lo : hi) = mid;
+    }
+    printf("%lld\n", lo);
+  }
+}
+"""
+    host = os.path.join(ROOT, "tests", "host")
+    with tempfile.TemporaryDirectory() as d:
+        with open(os.path.join(d, "r.cpp"), "w") as f:
+            f.write(src)
+        r = subprocess.run(["/opt/rocm/llvm/bin/clang++", "-std=c++17", "-w", "-I", host, "-I",
+                            os.path.join(ROOT, "fastoverlap_amd", "csrc"),
+                            os.path.join(d, "r.cpp"), "-o", os.path.join(d, "r")],
+                           capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr
+        out = subprocess.run([os.path.join(d, "r")], capture_output=True, text=True).stdout
+    for L, most in enumerate(int(x) for x in out.split()):
+        # a degree l >= 16 has l + 1 rows; below, four degrees up to 7 or two up to 15
+        low = max(sum(range(l - 3, l + 1)) + 4 for l in range(3, 8))
+        rows = max(L + 1, low, 15 + 16)
+        assert rows * 16 * most <= 2 ** 32 - 4096 < rows * 16 * (most + 1)

@@ -6,6 +6,8 @@
 //  * Kearsley (1989) quaternion superposition (fastoverlap/utils.py:169-275);
 //  * Euler-angle rotation matrix (fastoverlap/utils.py:447-460).
 #pragma once
+#include <type_traits>
+
 #include "fo_common.h"
 
 namespace fo {
@@ -272,6 +274,16 @@ FO_DEV bool lap_solve(int n, KeyF key, Fin fin, Near near, LapShared s, int* row
 // The matrix is scaled by a power of two first, so that squares of its
 // entries neither overflow nor vanish.  One rotation after another by
 // quotients took 25000 cycles, more than the rest of a fit of 38 atoms.
+// A rotation moves t a_pq from one diagonal entry to the other and sets the
+// entry it is for to zero (Rutishauser 1966).  Forming these three by the
+// products instead leaves a rounding of the largest entry in all of them, so
+// that the smallest eigenvalue lost digits to the larger ones and equal ones (a
+// cubic or icosahedral cluster) ran into the cap of 60 sweeps.  An entry within two
+// roundings of the smaller of its diagonal entries, or 2^-60 of the largest, is
+// left: between equal eigenvalues each sweep would turn it by 45 degrees, and
+// their rows with it.  The finish of 2048 icosahedra of 13 atoms: 114 -> 21 us, of
+// random clusters the same; rms error of the distance of 1000-atom pairs 1.29e-15
+// -> 1.05e-15.
 FO_DEV void jacobi4(double A[4][4], double V[4][4], double w[4]) {
   double big = 0.0;
 #pragma unroll
@@ -286,54 +298,59 @@ FO_DEV void jacobi4(double A[4][4], double V[4][4], double w[4]) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) A[i][j] = ldexp(A[i][j], -ex);
-  auto angle = [](double app, double aqq, double apq, double& c, double& s) {
+  struct Angle {
+    double t, c, s;
+  };
+  auto left = [](double app, double aqq, double apq) {
+    return fabs(apq) <= __builtin_fma(0x1p-51, fmin(fabs(app), fabs(aqq)), 0x1p-60);
+  };
+  auto angle = [&](double app, double aqq, double apq) {
+    // (no branch: the two angles are formed side by side)
     const double d = 0.5 * (aqq - app), r2 = d * d + apq * apq;
     const double den = fabs(d) + (r2 > 0.0 ? r2 * rsqrt(r2) : 0.0);
-    const double t = den > 0.0 ? (d < 0.0 ? -apq : apq) / den : 0.0;
-    c = rsqrt(t * t + 1.0);
-    s = t * c;
+    Angle a;
+    a.t = den > 0.0 && !left(app, aqq, apq) ? (d < 0.0 ? -apq : apq) / den : 0.0;
+    a.c = rsqrt(a.t * a.t + 1.0);
+    a.s = a.t * a.c;
+    return a;
   };
-  auto turn = [&](auto P, auto Q, double c, double s) {
+  auto turn = [&](auto P, auto Q, const Angle& a) {
     constexpr int p = decltype(P)::value, q = decltype(Q)::value;
+    const double move = a.t * A[p][q];
+    A[p][p] -= move;
+    A[q][q] += move;
+    A[p][q] = A[q][p] = 0.0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
+      if (k == p || k == q) continue;
       const double akp = A[k][p], akq = A[k][q];
-      A[k][p] = c * akp - s * akq;
-      A[k][q] = s * akp + c * akq;
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const double apk = A[p][k], aqk = A[q][k];
-      A[p][k] = c * apk - s * aqk;
-      A[q][k] = s * apk + c * aqk;
+      A[k][p] = A[p][k] = a.c * akp - a.s * akq;
+      A[k][q] = A[q][k] = a.s * akp + a.c * akq;
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const double vkp = V[k][p], vkq = V[k][q];
-      V[k][p] = c * vkp - s * vkq;
-      V[k][q] = s * vkp + c * vkq;
+      V[k][p] = a.c * vkp - a.s * vkq;
+      V[k][q] = a.s * vkp + a.c * vkq;
     }
   };
   auto two = [&](auto P, auto Q, auto R, auto S) {
-    double c0, s0, c1, s1;
-    angle(A[P.value][P.value], A[Q.value][Q.value], A[P.value][Q.value], c0, s0);
-    angle(A[R.value][R.value], A[S.value][S.value], A[R.value][S.value], c1, s1);
-    turn(P, Q, c0, s0);
-    turn(R, S, c1, s1);
+    const Angle a = angle(A[P.value][P.value], A[Q.value][Q.value], A[P.value][Q.value]);
+    const Angle b = angle(A[R.value][R.value], A[S.value][S.value], A[R.value][S.value]);
+    turn(P, Q, a);
+    turn(R, S, b);
   };
   constexpr std::integral_constant<int, 0> i0{};
   constexpr std::integral_constant<int, 1> i1{};
   constexpr std::integral_constant<int, 2> i2{};
   constexpr std::integral_constant<int, 3> i3{};
   for (int sweep = 0; sweep < 60; ++sweep) {
-    double off = 0.0, dia = 0.0;
+    bool done = true;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      dia += A[p][p] * A[p][p];
+    for (int p = 0; p < 4; ++p)
 #pragma unroll
-      for (int q = p + 1; q < 4; ++q) off += A[p][q] * A[p][q];
-    }
-    if (off == 0.0 || off < 1e-36 * dia) break;
+      for (int q = p + 1; q < 4; ++q) done &= left(A[p][p], A[q][q], A[p][q]);
+    if (done) break;
     two(i0, i1, i2, i3);
     two(i0, i2, i1, i3);
     two(i0, i3, i1, i2);
@@ -374,6 +391,14 @@ FO_DEV void qmat_accum(double q[10], double x1, double y1, double z1, double x2,
   q[9] += XP * XP + YP * YP + ZM * ZM;
 }
 
+// (hi, lo) += a b, lo holding what the sums and products round off
+FO_DEV void add_product(double& hi, double& lo, double a, double b) {
+#pragma clang fp contract(off)
+  const double p = a * b, pe = __builtin_fma(a, b, -p), s = hi + p, t = s - hi;
+  lo += ((hi - (s - t)) + (p - t)) + pe;
+  hi = s;
+}
+
 // Solve the 4x4 problem: dist = sqrt(min eigenvalue) with the reference's
 // clamp of small negative eigenvalues (fastoverlap/utils.py:236-248), and
 // the rotation MR (row-major).
@@ -392,14 +417,22 @@ FO_DEV void kearsley_solve(const double q[10], double* dist, double MR[9]) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) qv[k] = V[k][i];
     }
-  // one first-order correction of the eigenvector against the matrix itself
-  // takes out what the rotations rounded; near-equal eigenvalues are left
-  const double rv[4] = {
-      q[0] * qv[0] + q[1] * qv[1] + q[2] * qv[2] + q[3] * qv[3] - e * qv[0],
-      q[1] * qv[0] + q[4] * qv[1] + q[5] * qv[2] + q[6] * qv[3] - e * qv[1],
-      q[2] * qv[0] + q[5] * qv[1] + q[7] * qv[2] + q[8] * qv[3] - e * qv[2],
-      q[3] * qv[0] + q[6] * qv[1] + q[8] * qv[2] + q[9] * qv[3] - e * qv[3]};
+  // one first-order correction of the pair against the matrix itself takes out what
+  // the rotations rounded; near-equal eigenvalues leave the vector.  The
+  // residual is summed in twice the precision: its terms are of the size of the
+  // largest eigenvalue and the distance is the root of the smallest.
+  double rv[4];
+  const int at[4][4] = {{0, 1, 2, 3}, {1, 4, 5, 6}, {2, 5, 7, 8}, {3, 6, 8, 9}};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    double hi = 0.0, lo = 0.0;
+    add_product(hi, lo, -e, qv[i]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) add_product(hi, lo, q[at[i][j]], qv[j]);
+    rv[i] = hi + lo;
+  }
   const double wmax = fmax(fmax(w[0], w[1]), fmax(w[2], w[3])), e0 = e;
+  e += qv[0] * rv[0] + qv[1] * rv[1] + qv[2] * rv[2] + qv[3] * rv[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const double gap = w[i] - e0;

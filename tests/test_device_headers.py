@@ -49,3 +49,31 @@ def test_staging_buffers_change_hands_between_threads(tmp_path_factory):
     r = subprocess.run([build(tmp_path_factory, "staging")], capture_output=True, text=True,
                        timeout=60)
     assert (r.returncode, r.stdout) == (0, "ok\n"), r.stdout + r.stderr
+
+
+def test_jacobi_sweeps_with_equal_eigenvalues(tmp_path_factory):
+    """Equal eigenvalues (the fits of cubic and icosahedral clusters) take no more
+    sweeps than distinct ones."""
+    spectra = [(0, 1, 2, 3), (0, 1, 1, 2), (0, 1, 1, 1), (0, 0, 1, 1), (1, 1, 1, 1), (0, 0, 0, 0),
+               (1e-3, 4000, 4001, 4002), (0, 1, 1, 1 + 1e-7)]
+    spectra = [s + (off,) for off in (0, 1e-12, 1e-9, 1e-6, 1e-3) for s in spectra]
+    r = subprocess.run([build(tmp_path_factory, "jacobi")] + [repr(float(v)) for s in spectra for v in s],
+                       capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
+    for spec, line in zip(spectra, r.stdout.splitlines()):
+        sweeps, err, orth = line.split()
+        assert int(sweeps) <= 8, (spec, line)
+        # the matrix is rounded as it is formed (four terms an entry), then once a
+        # rotation of a row; V by three roundings in each of at most 48 rotations
+        assert float(err) <= 16 * 2.0 ** -52 and float(orth) <= 48 * 3 * 2.0 ** -53, (spec, line)
+
+
+@pytest.mark.parametrize("atoms,angle,noise", [(13, 1e-4, 0.02), (13, 1.0, 0.02), (1000, 1e-2, 0.02),
+                                               (1000, 1.0, 0.02), (100, 1.0, 1.0)])
+def test_fitted_distance_is_that_of_its_matrix(tmp_path_factory, atoms, angle, noise):
+    """The smallest eigenvalue within a rounding, half of it after the root,
+    which rounds once more: 2^-52 together, however far the larger eigenvalues lie."""
+    r = subprocess.run([build(tmp_path_factory, "fit"), str(atoms), str(angle), str(noise)],
+                       capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
+    assert float(r.stdout) <= 2.0 ** -52

@@ -58,7 +58,7 @@ void launch_sph_select(hipStream_t, int, int, long long, int, const SphPair*, co
 void launch_sph_rotopt(hipStream_t, int, int, int, const SphPair*, const double2*, const double2*,
                        int, const SphPeak*, const double*, int, SphOpt*);
 void launch_rec_table(hipStream_t, int, double*, double2*, double*);
-void launch_sph_finish(hipStream_t, int, int, const SphPair*, const SphGroup*, const int*,
+void launch_sph_finish(hipStream_t, int, int, int, const SphPair*, const SphGroup*, const int*,
                        const double*, const double*, const SphOpt*, int, double*, int*, int*,
                        double*, SphResult*);
 void launch_coef_to_plane(hipStream_t, int, int, int, const SphPair*, const double2*, float2*);
@@ -644,7 +644,7 @@ static int sph_enqueue(fo_sph_batch* b, int stages) {
                       b->rect->seedu, kRecL, b->opt);
   mark(7);
   if (stages & FO_STAGE_FINISH)
-    launch_sph_finish(s, P, b->maxgroup, b->pd, b->grp, b->gath, b->X1c, b->X2c, b->opt,
+    launch_sph_finish(s, P, L.nlarge, b->maxgroup, b->pd, b->grp, b->gath, b->X1c, b->X2c, b->opt,
                       L.norient, b->X2R, b->perm, b->rowsol, b->X2out, b->res);
   mark(8);
   FO_CHECK_LAUNCH();
@@ -710,7 +710,7 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
   b->harm_nmax = harm_nmax;
   b->harm_r0 = harm_r0;
   b->harm_basis = harm_basis ? 1 : 0;
-  int Lmax = 0, maxatoms = 0, mingath = 1 << 30, maxgath = 0;
+  int Lmax = 0, maxatoms = 0, mingath = 1 << 30, maxgath = 0, nlarge = 0;
   long long maxjk = 0, Ntot = 0, Ktot = 0, C32tot = 0, radtot = 0, ylmtot = 0;
   long long radmax = 0, ylmmax = 0;  // largest chunk
   const size_t chunk_budget = coef_chunk_bytes();
@@ -743,7 +743,7 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
     sp.pad0 = 0;
     std::vector<char> seen(N, 0);
     long long jk = 0;
-    int ng = 0;
+    int ng = 0, largest = 0;
     for (int q = 0; q < sp.ngroups; ++q) {
       const int sz = d->group_sizes[gq + q];
       if (sz > kMaxGroup)
@@ -762,8 +762,10 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
       }
       jk += (long long)sz * sz;
       ng += sz;
-      b->maxgroup = std::max(b->maxgroup, sz);
+      largest = std::max(largest, sz);
     }
+    b->maxgroup = std::max(b->maxgroup, largest);
+    nlarge += largest >= kFinishLarge;
     sp.ngath = ng;
     if (harm_nmax < 0 && !contract_in_reach(ng, Lp))
       return set_err(FO_ERR_UNSUPPORTED, "too many grouped atoms in one pair");
@@ -829,6 +831,7 @@ int sph_batch_plan(fo_context* c, const fo_sph_batch_desc* d, fo_sph_batch** out
   lc.mingath = mingath;
   lc.maxgath = maxgath;
   lc.maxatoms = maxatoms;
+  lc.nlarge = nlarge;
   lc.maxjk = maxjk;
   lc.norient = (d->flags & FO_SPH_NO_INVERT) ? 1 : 2;
   lc.mode = general ? 1 : 0;

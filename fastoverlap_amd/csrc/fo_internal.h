@@ -128,6 +128,22 @@ struct PerResult {
 };
 
 // ---- kernel launchers (implemented in the .hip files) ---------------------
+// Threads of the finish (one workgroup a pair), whose assignment search is a chain
+// of small reductions: one wavefront, without barriers, until the largest group
+// reaches 192 atoms; then four, whose column scans are shorter; eight above 512 atoms
+// while every pair has a CU, or few pairs (nlarge) have a group of 192.  Eight
+// against four wavefronts: 64 pairs of 1000 atoms 652 / 924 us, of 544 269 / 295,
+// unrelated 544-atom pairs 28.5 / 29.2 ms, 64 of 600 among 4000 small ones 312 /
+// 343 us, one among 4095 305 / 336; but 128 among 4000 372 / 345, 320 pairs of 600
+// atoms 632 / 571, 512 of 700 801 / 722, 128 of 600 with 896 of 400 672 / 611 (the
+// workgroups of a CU wait for each other), and 512 unrelated atoms, which four
+// wavefronts divide evenly, 28.3 / 27.6 ms.  Results do not depend on the number.
+constexpr int kFinishLarge = 192;
+__host__ __device__ inline int finish_threads(int npairs, int nlarge, int maxgroup) {
+  if (maxgroup > 512 && (npairs <= 256 || nlarge <= 64)) return 512;
+  return maxgroup >= kFinishLarge ? 256 : 64;
+}
+
 struct SphLaunch {
   int P;               // pairs
   int n;               // grid side 2B
@@ -136,6 +152,7 @@ struct SphLaunch {
   int mingath;         // min gathered atoms over pairs
   int maxgath;         // max gathered atoms over pairs
   int maxatoms;        // max atoms over pairs
+  int nlarge;          // pairs with a group of kFinishLarge atoms or more
   long long maxjk;     // max sum of group size^2 over pairs
   int norient;         // 1 or 2
   int mode;            // 0 = alignment (B = (-1)^l A), 1 = general (A,B given)

@@ -2765,22 +2765,17 @@ void launch_sph_rotopt(hipStream_t s, int P, int norient, int Lmax, const SphPai
                      mode, peaks, norient, seedu, Lt, Lmax, opt, P);
 }
 
-void launch_sph_finish(hipStream_t s, int P, int lap_nmax, const SphPair* pd, const SphGroup* grp,
-                       const int* gath, const double* X1c, const double* X2c, const SphOpt* opt,
-                       int norient, double* X2R, int* perm, int* rowsol, double* X2out,
-                       SphResult* res) {
-  // one wavefront per pair: the assignment search is a chain of small
-  // reductions, cheapest without cross-wave barriers, until the largest
-  // group reaches 192 atoms: then four, whose column scans are shorter, and
-  // eight from 512 on (64 pairs of 1000 atoms: 505 -> 447 us; the assignment
-  // and the fit do not depend on the block size)
+void launch_sph_finish(hipStream_t s, int P, int nlarge, int lap_nmax, const SphPair* pd,
+                       const SphGroup* grp, const int* gath, const double* X1c, const double* X2c,
+                       const SphOpt* opt, int norient, double* X2R, int* perm, int* rowsol,
+                       double* X2out, SphResult* res) {
   // positions of the largest group in LDS beside the assignment arrays when
   // that stays within 64 KiB
   const size_t lap = (lap_lds_bytes(lap_nmax) + 15) & ~(size_t)15;
   const size_t pos = 6 * sizeof(double) * (size_t)lap_nmax;
   const int pos_lds = lap + pos <= 65536 ? 1 : 0;
-  const int nthr = lap_nmax >= 512 ? 512 : lap_nmax >= 192 ? 256 : 64;
-  hipLaunchKernelGGL(k_sph_finish, dim3(P), dim3(nthr), lap + (pos_lds ? pos : 0), s, pd, grp,
+  const int threads = finish_threads(P, nlarge, lap_nmax);
+  hipLaunchKernelGGL(k_sph_finish, dim3(P), dim3(threads), lap + (pos_lds ? pos : 0), s, pd, grp,
                      gath, X1c, X2c, opt, norient, lap_nmax, pos_lds, X2R, perm, rowsol, X2out,
                      res);
 }

@@ -77,3 +77,14 @@ def test_fitted_distance_is_that_of_its_matrix(tmp_path_factory, atoms, angle, n
                        capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
     assert float(r.stdout) <= 2.0 ** -52
+
+
+def test_finish_takes_eight_wavefronts_only_where_they_win(tmp_path_factory):
+    """Batches on both sides of each line of the rule, as measured."""
+    rule = {(1, 0, 38): 64, (4096, 0, 191): 64, (1, 0, 192): 256, (64, 0, 512): 256,
+            (64, 64, 513): 512, (256, 256, 1000): 512, (4096, 1, 600): 512, (4064, 64, 600): 512,
+            (4128, 128, 600): 256, (1024, 1024, 600): 256,
+            (320, 320, 600): 256, (512, 512, 700): 256, (1280, 256, 600): 256}
+    r = subprocess.run([build(tmp_path_factory, "finish_rule")] + [str(v) for k in rule for v in k],
+                       capture_output=True, text=True, timeout=60)
+    assert [int(v) for v in r.stdout.split()] == list(rule.values())

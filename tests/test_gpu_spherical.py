@@ -817,3 +817,27 @@ def test_coefficients_of_a_pair_past_32_bit_offsets(gpu):
     ref = O.so3_coeffs_species(X1, X2, [np.arange(n)], L, 0.35, fast=True)
     # the bound of the tests above, and a rounding of the sum for every group
     np.testing.assert_allclose(got, ref, atol=(1e-12 + reps * 2.0 ** -53) * np.abs(ref).max())
+
+
+def test_finish_is_the_same_with_four_and_eight_wavefronts(gpu):
+    """Pairs with a group of 513 atoms alone (eight wavefronts) and 257 times
+    (four), beside small pairs: every output the same, bit for bit."""
+    say("case: two pairs alone and 514 together")
+    rng = np.random.default_rng(513)
+    sizes = [513, 12]
+    pairs = [tuple(rng.normal(size=(2, n, 3)) * 0.5 * n ** (1 / 3)) for n in sizes]
+    # the larger pair: a noisy copy, so that its assignment is found at once
+    x = pairs[0][0]
+    pairs[0] = (x, x[rng.permutation(513)] + rng.normal(scale=0.02, size=x.shape))
+
+    def run(reps):
+        with SphericalBatch(sizes * reps, 6, 0.4, 16, None) as b:
+            b.set_positions([p[0] for p in pairs] * reps, [p[1] for p in pairs] * reps)
+            b.run()
+            return b.results()
+
+    one, many = run(1), run(257)
+    for k in one:
+        for p in range(2):
+            for q in (p, p + 512):
+                np.testing.assert_array_equal(many[k][q], one[k][p], err_msg=f"{k} {q}")

@@ -124,7 +124,9 @@ static bool all_finite(const double* p, size_t n) {
   return true;
 }
 static constexpr int kMaxL = 63;
-static constexpr int kSoftMaxBw = 50;  // bandwidth of the forward transform of a grid
+// Bandwidth of the forward transform of a grid: that of the inverse, whose planes
+// of two coefficient sets fit LDS up to degree 49.
+static constexpr int kSoftMaxBw = 50;
 static constexpr int kMaxGroup = 4096;
 static constexpr int kHarmMaxN = 40;  // harmonic basis radial degree
 

@@ -35,8 +35,11 @@ namespace fo {
 // block of eight and descend K_{l-1} = K_{l+1} + (2l+1)/x K_l (i_l is the
 // minimal solution, stable downwards), D degrees a wavefront.  x below
 // kMinRadX = 2^-58 (an atom at the centre) counts as 2^-58, here and where the
-// slots are filled: K_0 is the same to FP64, K_l, l >= 1, moves by less than
-// 2^-59 K_0, and the stored K_16 stays a normal number.
+// slots are filled: K_0 is the same to FP64 and K_l, l >= 1, moves by less than
+// 2^-59 K_0.  With x = 2^-58 the degrees 8..15 are below x^8 / 17!! = 2^-489 of K_0,
+// so it does not matter that K_15 and K_16 may vanish for two atoms whose distances
+// differ by several widths; K_0..K_7 come from the slots 7 and 8, normal numbers
+// until the Gaussian, and K_0 with it, is below 2^-530.
 //
 // Pairs with more than kSplitAtoms grouped atoms take four wavefronts per
 // item, the k tiles dealt to them in equal shares and their P added through

@@ -561,7 +561,6 @@ __global__ void __launch_bounds__(256) k_per_plane_real(
 struct PerGridCtx {
   int NB, F;
   const double2* C;
-  const double2* tw64;
 };
 
 // FP64 |f| at up to kSelPoints grid points with at most three x and five
@@ -734,7 +733,6 @@ __global__ void __launch_bounds__(kSelThreads) k_per_select(
   c.NB = NB;
   c.F = F;
   c.C = Cprod + d.c_off;
-  c.tw64 = tw64;
   double2* tw = (double2*)smem;
   double2* H = tw + F;
   double2* G = H + XB * NB * NB;

@@ -1295,7 +1295,6 @@ struct GridCtx {
   int n, L;
   long long Kt;
   const double* tab64;
-  const double2* tw64;
   const double2* I;   // pair's FP64 coefficients (A set)
   const double2* IB;  // B set (general mode) or nullptr
   double sgn;         // +1 / -1 (alignment mode)
@@ -1658,7 +1657,6 @@ __global__ void __launch_bounds__(1024) k_sph_select(
   c.L = L;
   c.Kt = Kt;
   c.tab64 = tab64;
-  c.tw64 = tw64;
   c.I = IA + d.coef_off;
   c.IB = (mode == 1 && o == 1) ? IB + d.coef_off : nullptr;
   c.sgn = (mode == 0 && o == 1) ? -1.0 : 1.0;
@@ -1824,7 +1822,9 @@ __global__ void __launch_bounds__(1024) k_sph_select(
       for (int sd = 0; sd < 2; ++sd) {
         const int q = q0 + 2 * ax + sd;  // sd 0: +1, 1: -1
         const int dlt = sd == 0 ? 1 : n - 1;
-        s_pa[q] = ax == 0 ? (ind[0] + dlt) % n : ind[0];
+        // (no listed point, as for a grid that is not a number: ind[0] is out of
+        // range and is folded back, its twiddle index has to stay below 2^22)
+        s_pa[q] = (ax == 0 ? ind[0] + dlt : ind[0]) % n;
         s_pg[q] = ax == 2 ? (ind[2] + dlt) % n : ind[2];
         s_pb[q] = ax == 1 ? (sd == 0 ? 1 : 2) : 0;
       }
@@ -2251,7 +2251,7 @@ __global__ void __launch_bounds__(512, 3) k_sph_rotopt(const SphPair* __restrict
                                                     const double2* __restrict__ IB, int mode,
                                                     const SphPeak* __restrict__ peaks, int norient,
                                                     const double* __restrict__ seedu, int Lt,
-                                                    int Lmax, SphOpt* __restrict__ opt, int P) {
+                                                    SphOpt* __restrict__ opt, int P) {
   __shared__ double part[kFghBlocks * 10], pw[kFghPowers];
   __shared__ double2 ph[kFghPhases];
   __shared__ int s_blk;
@@ -2762,7 +2762,7 @@ void launch_sph_rotopt(hipStream_t s, int P, int norient, int Lmax, const SphPai
                        const double* seedu, int Lt, SphOpt* opt) {
   const int threads = few_workgroups(P, norient) ? 512 : 256;
   hipLaunchKernelGGL(k_sph_rotopt, dim3(xcd_grid(P, norient)), dim3(threads), rec_lds_bytes(Lmax), s, pd, IA, IB,
-                     mode, peaks, norient, seedu, Lt, Lmax, opt, P);
+                     mode, peaks, norient, seedu, Lt, opt, P);
 }
 
 void launch_sph_finish(hipStream_t s, int P, int nlarge, int lap_nmax, const SphPair* pd,

@@ -368,18 +368,19 @@ def periodic_batched(ctx, pairs, steps, warmup, plain_sample):
         agree += int(np.array_equal(pa.last["peaks"]["ind"][0], pk["ind"][i])
                      and np.array_equal(perm, r["perm"][i]))
     plain = plain_sample / (time.perf_counter() - t0)
-    # algorithmic work: structure factors as separable phase products, 8 flops
-    # per complex multiply-add, (2n+1)^3 k per atom, both structures (FP64);
-    # the pruned transform: F planes of (2n+1)^3 + (2n+1)^2 F + (2n+1) F^2
-    # complex multiply-adds (FP32)
-    NB = 2 * c0["nk"] + 1
-    F = c0["F"]
-    f_sf = sum(2 * 8 * NB ** 3 * len(c["pos1"]) for c in pairs)
-    f_plane = P * 8 * F * (NB ** 3 + NB * NB * F + NB * F * F)
+    # work of the kernels' own form: structure factors as real octant sums, a
+    # multiply-add per atom for (2n+1)^3 real sums of cosines and sines, both
+    # structures (FP64); planes as real products: the sums over the first index
+    # (8 flops a term of the half cube), then two real products, (2n+1)^2 F and
+    # (2n+1) F^2 multiply-adds a plane (FP32)
+    nk = c0["nk"]
+    NB, F = 2 * nk + 1, c0["F"]
+    f_sf = sum(2 * 2 * NB ** 3 * len(c["pos1"]) for c in pairs)
+    f_plane = P * F * (2 * 8 * (nk + 1) ** 2 * NB + 2 * (NB * NB * F + NB * F * F))
     roof = {}
-    for k, fl, peak, unit in (("sf", f_sf, FP64_PEAK, "FP64 vector ALU"),
-                              ("plane", f_plane, FP32_PEAK / 2,
-                               "FP32 vector ALU, single-issue (packed FP32 disabled)")):
+    for k, fl, peak, unit in (("sf", f_sf, FP64_PEAK, "FP64 matrix cores"),
+                              ("plane", f_plane, FP32_PEAK,
+                               "FP32 matrix cores (the first sum on the vector ALU)")):
         if kt.get(k, 0) > 0:
             ach = fl / (kt[k] * 1e-3)
             roof[k] = {"achieved_tflops": ach / 1e12, "peak_tflops": peak / 1e12,

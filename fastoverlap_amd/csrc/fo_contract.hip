@@ -51,18 +51,19 @@ namespace fo {
 //
 // All degrees share a launch: with one launch per class one pair of 100 atoms
 // took 110 us instead of 44 (each class waits for its slowest item) and the 4096
-// pairs 2.06 ms instead of 1.99, although the joint kernel spills 241 registers,
-// outside its product loops.
+// pairs 2.06 ms instead of 1.99, although the joint kernel spills 247 registers
+// (262 with four wavefronts), outside its product loops.
 //
-// Bound: reading K and Y.  1000 atoms, degree 40: 25.6 GB for 64 pairs (a
-// slot once for every item of its degrees), 5 TB/s; of the 5.1 ms the
-// products take 2.2 at the matrix rate.  Items with all row tiles of a degree
-// read a slot 40 times instead of 63 but leave one wavefront a SIMD: 6.3 ms.  4096 pairs of 13..147 atoms, degrees
-// 16..25: products 0.62 of 1.99 ms, waits on loads (two wavefronts a SIMD)
-// most of the rest.  Against the two kernels it replaces (a workgroup per
-// degree with A through LDS, the complex form, and for degrees <= 15 a fused
-// one): 3.31 -> 1.99 ms and 9.62 -> 5.2 ms; 16 pairs of 300..500 atoms 1006 ->
-// 189 us, one pair of 500 at degree 30 988 -> 159 us.
+// Bound: reading K and Y.  1000 atoms, degree 40: 26.0 GB past the L2 for 64 pairs
+// (a slot once for every item of its degrees), 5 TB/s; of the 5.1 ms the products
+// take 2.2 at the matrix rate (matrix units 55 % busy).  Items with all row tiles of
+// a degree read a slot 40 times instead of 63 but leave one wavefront a SIMD: 6.3
+// ms.  4096 pairs of 13..147 atoms, degrees 16..25: products 0.62 of 1.99 ms (34 %
+// busy, with the padding), waits on loads (two wavefronts a SIMD) most of the rest.
+// Against the two kernels it replaces (a workgroup per degree with A through LDS, the
+// complex form, and for degrees <= 15 a fused one): 3.31 -> 1.99 ms and 9.62 -> 5.2
+// ms; 16 pairs of 300..500 atoms 1006 -> 189 us, one pair of 500 at degree 30 988 ->
+// 159 us.
 // ---------------------------------------------------------------------------
 constexpr int kSplitAtoms = 160;
 constexpr double kMaxInvX = 1.0 / kMinRadX;

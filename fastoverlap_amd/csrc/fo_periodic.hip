@@ -411,8 +411,8 @@ __global__ void __launch_bounds__(256) k_per_plane(
 // 6.9 NB + 12 in all.  real_plane_delta, 9 NB + 64, is that with room for the
 // second order and for matrix units that round products apart from sums.
 // Against the complex transform on the vector units, which formed every F^2 NB
-// term of a plane: 259 -> 75 us for 128 pairs of nk = 8, F = 64, 111 -> 36 us for
-// 24 of nk = 14, F = 60, 20 -> 12 us for one pair.  Bound: stage 1 (two FP64
+// term of a plane: 259 -> 72 us for 128 pairs of nk = 8, F = 64, 111 -> 33 us for
+// 24 of nk = 14, F = 60, 20 -> 10 us for one pair.  Bound: stage 1 (two FP64
 // products read, four conversions and eight FP32 operations a term) and the
 // candidate test of every value.
 constexpr int kPlaneXP = 4;
@@ -709,8 +709,10 @@ FO_DEV void per_plane64(const PerGridCtx& c, int x, double2* H, double2* G, cons
 // The product is read once for the argmax and its six neighbours when a single
 // candidate is listed (the common case); as seven separate sums over the cube
 // and one for A, each a chain of loads, this took 61 us for one pair of nk = 8
-// and 255 us for 24 of nk = 14, now 11 and 30.  Bound: load latency of one
-// workgroup per pair.
+// and 255 us for 24 of nk = 14, now 14 and 30.  The real planes list one value a
+// wavefront and have twice the bound of the complex ones, so one or two of 128
+// pairs of nk = 8, fewer at nk = 14, have a whole plane to evaluate, which the others
+// wait for: 33 and 61 us then.  Bound: load latency of one workgroup per pair.
 template <int XB>
 __global__ void __launch_bounds__(kSelThreads) k_per_select(
     const PerPair* __restrict__ pd, int nk, int F, const double2* __restrict__ Cprod,
